@@ -67,7 +67,8 @@ typedef enum msco_dtype {
   MSCO_DT_U64 = 4,
   MSCO_DT_F16 = 5,
   MSCO_DT_BF16 = 6,
-  MSCO_DT_F32 = 7
+  MSCO_DT_F32 = 7,
+  MSCO_DT_I4 = 8     /* weights only: two signed 4-bit values per byte, the even-indexed one in the low nibble */
 } msco_dtype;
 
 /* Storage of the weight tensor.  The reference keeps its weights in the device's own blocked format (FRACTAL_NZ,
@@ -104,7 +105,7 @@ enum {
  * (grouped_matmul_v4_cops.cc:94-97). */
 enum {
   MSCO_IN_X = 0,               /* [M,K] int8 (W8A8) or bf16/f16 (W8A16) */
-  MSCO_IN_WEIGHT = 1,          /* [E,K,N] int8, or [E,N,K] when transpose_b, or packed (weight_layout) */
+  MSCO_IN_WEIGHT = 1,          /* [E,K,N] int8, or [E,N,K] when transpose_b, or packed (weight_layout), or [E,K,N/2] 4-bit */
   MSCO_IN_BIAS = 2,            /* [E,N] int32, optional */
   MSCO_IN_SCALE = 3,           /* [E,N] f32 / bf16 / int64|uint64 carrying f32 bits in the low word; optional */
   MSCO_IN_GROUP_LIST = 4,      /* [E] int32 / int64; NULL = E equal groups of M/E rows (dense / batched) */
@@ -119,7 +120,7 @@ enum {
 typedef struct msco_gmm_desc {
   int32_t abi_version;       /* MSCO_GMM_ABI_VERSION */
   int32_t x_dtype;           /* I8 | BF16 | F16 */
-  int32_t weight_dtype;      /* I8 */
+  int32_t weight_dtype;      /* I8 | I4 ([E,K,N/2] bytes, row-major, transpose_b 0) */
   int32_t out_dtype;         /* BF16 | F16 | I32 (raw accumulator + bias; scales are not applied) */
   int32_t group_list_dtype;  /* I32 | I64 | NONE */
   int32_t group_list_type;   /* 0 cumulative row ends, 1 per-group row counts */
@@ -135,7 +136,8 @@ typedef struct msco_gmm_desc {
                               * 2 128 x 128, 3 64 x 128, 4 decode (streaming) kernels, 5 generic, 6 persistent four-wave
                               * 256 x 256 (16 x 16 x 64 MFMAs), 7 128 x 256, 8 the persistent kernel's 32 x 32 x 32 MFMA form,
                               * 9 / 10 / 11 packed weights: chunks of up to 128 / 256 / 160 rows through LDS and weights
-                              * straight into MFMA operands
+                              * straight into MFMA operands, 12 [E,K,N] weights transposed in registers (4-bit weights:
+                              * every other value widens them to int8 first and forces the family on the result)
                               * (msco_gmm_plan_info names what was planned) */
   int32_t weight_layout;     /* MSCO_WL_ROW_MAJOR: as transpose_b says; MSCO_WL_PACKED: written by msco_pack_weight */
   int32_t act_type;          /* msco_act: activation applied to the dequantised float32 value before the output cast */
@@ -200,12 +202,12 @@ MSCO_API int msco_gmm_a8w4(const int8_t *x, const void *weight, const int32_t *g
                            const float *weight_scale, void *out, int64_t m, int64_t k, int64_t n, int64_t e,
                            int64_t group_size, void *stream);
 
-/* 4-bit weights of grouped_matmul_v4_cops widened to int8 on the device.  The reference hands its qint4x2 weight
+/* 4-bit values widened to int8 on the device: byte i of src holds element 2 i in its low nibble and element 2 i + 1 in its
+ * high nibble (tests/st/test_grouped_matmul_v4_cops.py:458-460), each a signed 4-bit value; dst receives 2 * src_bytes
+ * int8 values.  For callers that keep 4-bit weights as int8 from load time on; the reference hands its qint4x2 weight
  * [E, K, N / 2] to aclnnGroupedMatmulV4 as an int4 tensor of shape [E, K, N] (UnifyWeightShape,
- * ops/c_api/grouped_matmul_v4_cops/grouped_matmul_v4_cops.cc:56-66,274-295); this backend multiplies int8, so the op
- * layer widens the nibbles first: byte i of src holds element 2 i in its low nibble and element 2 i + 1 in its high
- * nibble (tests/st/test_grouped_matmul_v4_cops.py:458-460), each a signed 4-bit value; dst receives 2 * src_bytes
- * int8 values.  Both pointers 16-byte aligned.  Enqueued on the given stream, nothing is allocated. */
+ * ops/c_api/grouped_matmul_v4_cops/grouped_matmul_v4_cops.cc:56-66,274-295), which here is a launch with weight_dtype I4.
+ * Both pointers 16-byte aligned.  Enqueued on the given stream, nothing is allocated. */
 MSCO_API int msco_unpack_int4(const void *src, void *dst, int64_t src_bytes, void *stream);
 
 /* Weight prepack, once at load time -- the counterpart of the reference's trans_data ND -> FRACTAL_NZ step

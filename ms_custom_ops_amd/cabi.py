@@ -17,14 +17,14 @@ LIB_PATH = os.environ.get("MSCO_GMM_LIB") or os.path.join(_HERE, "lib", "libmsco
 ABI_VERSION = 1
 
 # msco_dtype
-DT_NONE, DT_I8, DT_I32, DT_I64, DT_U64, DT_F16, DT_BF16, DT_F32 = range(8)
+DT_NONE, DT_I8, DT_I32, DT_I64, DT_U64, DT_F16, DT_BF16, DT_F32, DT_I4 = range(9)
 
 # positional launch inputs
 IN_X, IN_WEIGHT, IN_BIAS, IN_SCALE, IN_GROUP_LIST, IN_PER_TOKEN_SCALE, IN_ANTIQUANT_SCALE, IN_ANTIQUANT_OFFSET = range(8)
 IN_COUNT = 8
 
 # msco_gmm_desc.kernel_override
-OV_AUTO, OV_TILE_256, OV_TILE_128, OV_TILE_64, OV_SKINNY, OV_GENERIC, OV_TILE_256_W4, OV_TILE_128x256, OV_TILE_256_W4_MFMA32, OV_ROWS128, OV_ROWS256, OV_ROWS160 = range(12)
+OV_AUTO, OV_TILE_256, OV_TILE_128, OV_TILE_64, OV_SKINNY, OV_GENERIC, OV_TILE_256_W4, OV_TILE_128x256, OV_TILE_256_W4_MFMA32, OV_ROWS128, OV_ROWS256, OV_ROWS160, OV_REGT = range(13)
 
 # msco_gmm_desc.act_type
 ACT_NONE, ACT_RELU, ACT_GELU_TANH, ACT_GELU_ERF, ACT_FAST_GELU, ACT_SILU = range(6)

@@ -43,10 +43,8 @@ inline unsigned chunk_slots(const GmmParams &p, int rows_per_chunk) {
 // range; waves split K and reduce through LDS, workgroups split K and reduce through the workspace.
 // wide16: the 16-wave / 128-column-strip variant for small weight sets, else 4 waves / 256-column strips
 hipError_t launch_skinny_w8a8(const GmmParams &p, bool nk, bool wide16, hipStream_t stream);
-hipError_t launch_skinny_a16w8(const GmmParams &p, hipStream_t stream);
 size_t skinny_workspace_bytes(int64_t m, int64_t n, int64_t e, int split_k, int cols);
 size_t skinny_counter_count(int64_t m, int64_t n, int64_t e, int cols);
-size_t a16w8_workspace_bytes(int64_t m, int64_t n, int64_t e, int split_k);
 
 // Decode kernels for weights in the packed layout (gmm_stream.hip): 4 waves, strips of up to 256 columns, K slices of
 // at most 128 blocks of 64 bytes (split_k chosen accordingly); workspace and counters as for the 4-wave skinny kernel.
@@ -62,6 +60,13 @@ int stream_blocks_per_wave(int64_t k, int split_k);
 size_t packed_weight_bytes(int64_t k, int64_t n);   // bytes of one group's weights in the packed layout
 hipError_t launch_pack_weight(const void *src, void *dst, long long e, long long k, long long n, bool src_nk,
                               hipStream_t stream);
+
+// Row-major [E,K,N] weights of 4 or 8 bits transposed and converted in registers (gmm_regt.hip): chunks of 16 row_blocks rows
+// (1 or 2), strips of strip_cols columns (256 or 512), p.split_k slices of K
+hipError_t launch_regt(const GmmParams &p, int weight_bits, int row_blocks, int strip_cols, hipStream_t stream);
+size_t regt_slice_bytes(int row_blocks, int strip_cols);   // workspace bytes of one (chunk, strip, K slice) partial tile
+// 4-bit values widened to int8 (gmm_w4.hip)
+hipError_t launch_unpack_int4(const void *src, void *dst, long long src_bytes, hipStream_t stream);
 
 // Shape-agnostic fallback kernels (one output element per thread), any K / N.
 // layout: 0 [E,K,N], 1 [E,N,K], 2 packed

@@ -223,6 +223,19 @@ __global__ void __launch_bounds__(256) unpack_int4_kernel(const uint4 *__restric
 }
 
 }  // namespace
+
+hipError_t launch_unpack_int4(const void *src, void *dst, long long src_bytes, hipStream_t stream) {
+  const long long pieces = src_bytes / 16;
+  const int tail = (int)(src_bytes % 16);
+  const long long threads = pieces > tail ? pieces : tail;
+  if (threads == 0) return hipSuccess;
+  if ((threads + 255) / 256 > 0x7FFFFFFFll) return hipErrorInvalidValue;
+  const unsigned char *s8 = static_cast<const unsigned char *>(src);
+  hipLaunchKernelGGL(unpack_int4_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
+                     static_cast<const uint4 *>(src), static_cast<uint4 *>(dst), pieces, s8 + pieces * 16,
+                     static_cast<signed char *>(dst) + pieces * 32, tail);
+  return hipGetLastError();
+}
 }  // namespace msco
 
 extern "C" int msco_unpack_int4(const void *src, void *dst, int64_t src_bytes, void *stream) {
@@ -231,15 +244,8 @@ extern "C" int msco_unpack_int4(const void *src, void *dst, int64_t src_bytes, v
   if (src_bytes == 0) return MSCO_OK;
   if (src == nullptr || dst == nullptr) return MSCO_ERR_INVALID_ARG;
   if ((reinterpret_cast<uintptr_t>(src) & 15) != 0 || (reinterpret_cast<uintptr_t>(dst) & 15) != 0) return MSCO_ERR_INVALID_ARG;
-  const long long pieces = src_bytes / 16;
-  const int tail = (int)(src_bytes % 16);
-  const long long threads = pieces > tail ? pieces : tail;
-  if ((threads + 255) / 256 > 0x7FFFFFFFll) return MSCO_ERR_SHAPE;
-  const unsigned char *s8 = static_cast<const unsigned char *>(src);
-  hipLaunchKernelGGL(unpack_int4_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint4 *>(src), static_cast<uint4 *>(dst), pieces, s8 + pieces * 16,
-                     static_cast<signed char *>(dst) + pieces * 32, tail);
-  return hipGetLastError() == hipSuccess ? MSCO_OK : MSCO_ERR_DEVICE;
+  if ((src_bytes / 16 + 255) / 256 > 0x7FFFFFFFll) return MSCO_ERR_SHAPE;
+  return launch_unpack_int4(src, dst, src_bytes, static_cast<hipStream_t>(stream)) == hipSuccess ? MSCO_OK : MSCO_ERR_DEVICE;
 }
 
 extern "C" int msco_gmm_a8w4(const int8_t *x, const void *weight, const int32_t *group_list, const float *x_scale,

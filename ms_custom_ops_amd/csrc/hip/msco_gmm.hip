@@ -18,7 +18,7 @@ namespace {
 
 using namespace msco;
 
-enum Family : int { FAM_NONE = 0, FAM_TILE = 1, FAM_SKINNY = 2, FAM_GENERIC = 3 };
+enum Family : int { FAM_NONE = 0, FAM_TILE = 1, FAM_SKINNY = 2, FAM_GENERIC = 3, FAM_REGT = 4 };
 
 // values of msco_gmm_desc::kernel_override
 enum Override : int {
@@ -28,7 +28,8 @@ enum Override : int {
   OV_TILE_256_W4_MFMA32 = 8,  // the persistent kernel's 32 x 32 x 32 form (never planned)
   OV_ROWS128 = 9,  // packed weights: chunks of up to 128 rows through LDS, weights straight into MFMA operands (other layouts: 128 x 256 tiles)
   OV_ROWS256 = 10,  // the same with chunks of up to 256 rows (other layouts: the persistent kernel)
-  OV_ROWS160 = 11   // ... of up to 160 rows (other layouts: the persistent kernel)
+  OV_ROWS160 = 11,  // ... of up to 160 rows (other layouts: the persistent kernel)
+  OV_REGT = 12      // [E,K,N] weights transposed and converted in registers (other layouts: as planned)
 };
 
 constexpr int64_t kSkinnyMaxRows = 64;   // total rows up to which the weight-streaming kernel is planned
@@ -52,19 +53,20 @@ int env_int(const char *name, int fallback) {
 // library has no such switches.
 struct Tuning {
   int print_plan, tile_cfg, tile_target_wgs, tile_split_k, stream_max_slots, skinny_wide16, stream_min_wgs, stream_groups,
-      skinny_target_wgs, skinny_split_k, tile_wide_k, stream_tch, two_level;
+      skinny_target_wgs, skinny_split_k, tile_wide_k, stream_tch, two_level, regt_cols;
 };
 const Tuning &tuning() {
 #ifdef MSCO_TUNING_SWITCHES
-  static const Tuning t = {env_int("MSCO_PRINT_PLAN", 0),        env_int("MSCO_TILE_CFG", -1),
+  static thread_local Tuning t;   // read again at every plan: a sweep changes them between plans
+  t = Tuning{env_int("MSCO_PRINT_PLAN", 0),        env_int("MSCO_TILE_CFG", -1),
                            env_int("MSCO_TILE_TARGET_WGS", 0),   env_int("MSCO_TILE_SPLIT_K", 0),
                            env_int("MSCO_STREAM_MAX_SLOTS", 0),  env_int("MSCO_SKINNY_WIDE16", -1),
                            env_int("MSCO_STREAM_MIN_WGS", 0),    env_int("MSCO_STREAM_GROUPS", 0),
                            env_int("MSCO_SKINNY_TARGET_WGS", 0), env_int("MSCO_SKINNY_SPLIT_K", 0),
                            env_int("MSCO_TILE_WIDE_K", -1),      env_int("MSCO_STREAM_TCH", 0),
-                           env_int("MSCO_TWO_LEVEL", 1)};
+                           env_int("MSCO_TWO_LEVEL", 1),         env_int("MSCO_REGT_COLS", 0)};
 #else
-  static const Tuning t = {env_int("MSCO_PRINT_PLAN", 0), -1, 0, 0, 0, -1, 0, 0, 0, 0, -1, 0, 1};
+  static const Tuning t = {env_int("MSCO_PRINT_PLAN", 0), -1, 0, 0, 0, -1, 0, 0, 0, 0, -1, 0, 1, 0};
 #endif
   return t;
 }
@@ -88,6 +90,9 @@ struct msco_gmm_op {
   int wide_k_slabs = 0;      // small tile kernels on K-major weights: 128-byte K slabs
   int w_nontemporal = 0;     // small tile kernels on packed weights: non-temporal weight loads
   int small_group_rows = 0;  // > 0: the persistent kernel takes the groups with more rows, a second launch of 64 x 128 tiles the others
+  int row_blocks = 1;        // register-transpose kernels: 16-row blocks per chunk
+  int strip_cols = 256;      // ... and columns per strip
+  int64_t widen_bytes = 0;   // 4-bit weights without a kernel of their own for the shape: int8 copy of them at the front of the workspace
   size_t workspace_bytes = 0;
   unsigned *counters = nullptr;
   size_t counters_cap = 0;
@@ -100,17 +105,19 @@ namespace {
 
 bool is_w8a8(const msco_gmm_desc &d) { return d.x_dtype == MSCO_DT_I8; }
 bool is_a16w8(const msco_gmm_desc &d) { return d.x_dtype == MSCO_DT_BF16 || d.x_dtype == MSCO_DT_F16; }
+bool is_w4(const msco_gmm_desc &d) { return d.weight_dtype == MSCO_DT_I4; }
 bool is_packed(const msco_gmm_desc &d) { return d.weight_layout == MSCO_WL_PACKED; }
 // 0 [E,K,N], 1 [E,N,K], 2 packed
 int layout_of(const msco_gmm_desc &d) { return is_packed(d) ? 2 : (d.transpose_b ? 1 : 0); }
 
 int check_desc(const msco_gmm_desc &d) {
   if (d.abi_version != MSCO_GMM_ABI_VERSION) return MSCO_ERR_INVALID_ARG;
-  if (d.weight_dtype != MSCO_DT_I8) return MSCO_ERR_UNSUPPORTED;
+  if (d.weight_dtype != MSCO_DT_I8 && d.weight_dtype != MSCO_DT_I4) return MSCO_ERR_UNSUPPORTED;
+  if (d.weight_dtype == MSCO_DT_I4 && (d.weight_layout != MSCO_WL_ROW_MAJOR || d.transpose_b != 0)) return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_dtype != MSCO_DT_NONE && d.group_list_dtype != MSCO_DT_I32 && d.group_list_dtype != MSCO_DT_I64)
     return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_type != 0 && d.group_list_type != 1) return MSCO_ERR_INVALID_ARG;
-  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_ROWS160) return MSCO_ERR_INVALID_ARG;
+  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_REGT) return MSCO_ERR_INVALID_ARG;
   if (d.weight_layout != MSCO_WL_ROW_MAJOR && d.weight_layout != MSCO_WL_PACKED) return MSCO_ERR_INVALID_ARG;
   if (d.force_split_k < 0) return MSCO_ERR_INVALID_ARG;
   if (d.act_type < MSCO_ACT_NONE || d.act_type > MSCO_ACT_SILU) return MSCO_ERR_INVALID_ARG;
@@ -136,6 +143,71 @@ int check_desc(const msco_gmm_desc &d) {
     return MSCO_OK;
   }
   return MSCO_ERR_UNSUPPORTED;
+}
+
+// Row-major [E,K,N] weights transposed and converted in registers (gmm_regt.hip).  Called behind choose_plan's own pick:
+// takes the plan over where these kernels are the better ones, and sets up the widening where 4-bit weights go to a
+// kernel that reads int8.
+void plan_regt(msco_gmm_op *op) {
+  const msco_gmm_desc &d = op->desc;
+  const int64_t m = op->m, k = op->k, n = op->n, e = op->e;
+  const int bits = is_w4(d) ? 4 : 8;
+  const bool can = layout_of(d) == 0 && k % 16 == 0 && n % 16 == 0 && k < ((int64_t)1 << 17) && k * n * bits / 8 < ((int64_t)1 << 31) &&
+                   m * k < ((int64_t)1 << 31);
+  // rows a group is expected to hold (shapes only); real routings are uneven, hence 1.5 x the average
+  const int64_t avg = (m + e - 1) / e, rows = e == 1 ? m : avg + avg / 2;
+  // 4-bit weights: widening them first costs more than a second and third pass over the nibbles (8 experts, K = 4096,
+  // N = 14336: the widening alone 120 us; with 4 / 32 rows per group these kernels take 44 / 82 us with int8 x).
+  // Weight-only on 8-bit weights, one 16-row chunk per group: the decode form.
+  const bool want = d.kernel_override == OV_REGT ||
+                    (d.kernel_override == OV_AUTO && bits == 4 && rows <= 64) ||
+                    (op->family == FAM_SKINNY && bits == 8 && is_a16w8(d) && op->stream_tch == 1);
+  if (can && want) {
+    const int blocks = bits == 8 || rows <= 16 ? 1 : 2;
+    GmmParams p{};
+    p.m = (int)m;
+    p.e = (int)e;
+    const int64_t slots = chunk_slots(p, 16 * blocks);
+    const int64_t active = std::max<int64_t>(1, std::min<int64_t>(slots, std::min<int64_t>(m, e)));
+    const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
+    // Strips of 512 columns (eight waves, twice as many neighbouring bytes per K row) while they fill most of the CUs
+    // without a K split, strips of 256 (four waves) otherwise.  8 experts, K = 4096, N = 14336, 4 rows per group, 4-bit
+    // weights: 44 against 51 us (int8 x), 47 against 52 us (bf16); 8-bit weights 79 against 82 us.  One group, N = 11008:
+    // 20 against 17 us.
+    int64_t cols = ((n + 511) / 512) * active * 4 >= cus * 3 ? 512 : 256;
+    if (tuning().regt_cols > 0) cols = tuning().regt_cols;
+    const int64_t strips = (n + cols - 1) / cols;
+    if (slots <= 65535) {
+      op->family = FAM_REGT;
+      op->row_blocks = blocks;
+      op->strip_cols = (int)cols;
+      op->n_strips = (int)strips;
+      // K split across workgroups up to one of them per CU: of the splits that leave the fewest K steps to a wave (four
+      // waves share them, in rounds of four or two), the smallest.  K = 4096, N = 11008, one row, 8-bit weights, split
+      // 1 / 2 / 3 / 4 / 6 / 8: 27 / 20 / 17.4 / 17.0 / 19.6 / 19.9 us -- beyond one workgroup per CU the slower half of a
+      // CU's pair and the exchange of partial tiles cost more than the shorter walk saves.
+      const int64_t steps = is_w8a8(d) ? (k + 63) / 64 : (k + 31) / 32, round = is_w8a8(d) ? 2 : 4;
+      auto per_wave = [&](int64_t s) { return ((((steps + s - 1) / s + 3) / 4 + round - 1) / round) * round; };
+      const int64_t most = std::min<int64_t>({std::max<int64_t>(1, cus / std::max<int64_t>(strips * active, 1)), kMaxSplitK, steps});
+      int64_t split = 1;
+      for (int64_t s = 2; s <= most; ++s)
+        if (per_wave(s) + 1 < per_wave(split)) split = s;
+      if (d.force_split_k > 0) split = std::min<int64_t>(d.force_split_k, steps);
+      const size_t tile = (size_t)slots * strips * regt_slice_bytes(blocks, (int)cols);
+      while (split > 1 && tile * split > kTileSplitMaxWorkspace) --split;
+      op->split_k = (int)split;
+      op->workspace_bytes = op->split_k > 1 ? tile * op->split_k : 0;
+      return;
+    }
+  }
+  if (op->family == FAM_SKINNY && layout_of(d) == 0 && is_a16w8(d) && op->stream_tch == 1) {   // (what the kernels above cannot take)
+    op->family = FAM_GENERIC;
+    op->split_k = 1;
+  }
+  if (bits == 4) {
+    op->widen_bytes = (e * k * n + 255) / 256 * 256;
+    op->workspace_bytes += (size_t)op->widen_bytes;
+  }
 }
 
 void choose_plan(msco_gmm_op *op) {
@@ -495,18 +567,21 @@ void choose_plan(msco_gmm_op *op) {
                                               : skinny_counter_count(m, n, e, op->skinny_cols);
       op->workspace_bytes = op->split_k > 1 ? tiles * (size_t)op->split_k * tile_bytes : 0;
     } else {
-      op->workspace_bytes = is_w8a8(d) ? skinny_workspace_bytes(m, n, e, op->split_k, op->skinny_cols)
-                                       : a16w8_workspace_bytes(m, n, e, op->split_k);
+      op->workspace_bytes = is_w8a8(d) ? skinny_workspace_bytes(m, n, e, op->split_k, op->skinny_cols) : 0;   // (weight-only: plan_regt's)
     }
   }
   op->family = family;
+  op->widen_bytes = 0;
+  plan_regt(op);
 
+  family = op->family;
   char buf[320];
-  const char *fam = family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
+  const char *fam = family == FAM_REGT ? "skinny_regt" : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
   std::snprintf(buf, sizeof(buf),
                 "msco_gmm plan: kernel=%s%s%s%s layout=%s m=%lld k=%lld n=%lld e=%lld split_k=%d strips=%d "
                 "workspace=%zu%s",
-                is_w8a8(d) ? "w8a8_" : "a16w8_", (family == FAM_SKINNY && is_packed(d)) ? (op->stream_tch > 1 ? "stream_rows" : "stream")
+                is_w4(d) ? (op->widen_bytes > 0 ? (is_w8a8(d) ? "a8w4_widened_" : "a16w4_widened_") : (is_w8a8(d) ? "a8w4_" : "a16w4_"))
+                         : is_w8a8(d) ? "w8a8_" : "a16w8_", (family == FAM_SKINNY && is_packed(d)) ? (op->stream_tch > 1 ? "stream_rows" : "stream")
                 : (family == FAM_SKINNY && op->stream_tch > 1)    ? "skinny_rows" : fam,
                 family == FAM_TILE ? (std::string("_") + tile_cfg_name(op->tile_cfg)).c_str() : "",
                 (family == FAM_SKINNY && op->skinny_wide16) ? "_16w" : "",
@@ -561,8 +636,12 @@ int msco_gmm_plan(msco_gmm_handle h, int64_t m, int64_t k, int64_t n, int64_t e,
   std::lock_guard<std::mutex> lock(h->mu);
   h->m = m; h->k = k; h->n = n; h->e = e;
   choose_plan(h);
-  if ((h->family == FAM_SKINNY || h->family == FAM_TILE) && h->split_k > 1) {
-    const size_t need = h->family == FAM_TILE ? tile_count_bound(h->tile_cfg, m, n, e)
+  if (h->family != FAM_GENERIC && h->split_k > 1) {
+    GmmParams p{};
+    p.m = (int)m;
+    p.e = (int)e;
+    const size_t need = h->family == FAM_REGT ? (size_t)chunk_slots(p, 16 * h->row_blocks) * h->n_strips
+                        : h->family == FAM_TILE ? tile_count_bound(h->tile_cfg, m, n, e)
                                               : skinny_counter_count(m, n, e, h->skinny_cols);
     if (need > h->counters_cap) {
       if (h->counters) (void)hipFree(h->counters);
@@ -630,6 +709,13 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   p.aq_offset = inputs[MSCO_IN_ANTIQUANT_OFFSET];
   p.out = out;
   p.partial = static_cast<int32_t *>(workspace);
+  if (is_w4(d) && (reinterpret_cast<uintptr_t>(p.w) & 15) != 0) return MSCO_ERR_INVALID_ARG;
+  if (h->widen_bytes > 0) {
+    // 4-bit weights on their way to a kernel that reads int8: the int8 copy sits at the front of the workspace
+    if (launch_unpack_int4(p.w, workspace, h->e * h->k * h->n / 2, static_cast<hipStream_t>(stream)) != hipSuccess) return MSCO_ERR_DEVICE;
+    p.w = static_cast<const int8_t *>(workspace);
+    p.partial = reinterpret_cast<int32_t *>(static_cast<char *>(workspace) + h->widen_bytes);
+  }
   p.counters = h->counters;
   p.m = (int)h->m; p.k = (int)h->k; p.n = (int)h->n; p.e = (int)h->e;
   p.gl_dtype = d.group_list_dtype;
@@ -656,7 +742,9 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   hipError_t err = hipSuccess;
   const bool nk = d.transpose_b != 0;
   const int layout = layout_of(d);
-  if (is_w8a8(d)) {
+  if (h->family == FAM_REGT) {
+    err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, s);
+  } else if (is_w8a8(d)) {
     if (h->family == FAM_TILE && h->small_group_rows > 0) {
       GmmParams big = p, small = p;
       big.rows_lo = h->small_group_rows;
@@ -673,7 +761,6 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   } else {
     if (h->family == FAM_SKINNY && h->stream_tch > 1) err = launch_streamm_a16w8(p, h->stream_tch, layout == 2, s);
     else if (h->family == FAM_SKINNY && layout == 2) err = launch_stream_a16w8(p, s);
-    else if (h->family == FAM_SKINNY) err = launch_skinny_a16w8(p, s);
     else err = launch_generic_a16w8(p, layout, s);
   }
   return err == hipSuccess ? MSCO_OK : MSCO_ERR_DEVICE;

@@ -10,9 +10,7 @@
 //   * group_type 0 (one x [M,K], one weight [E,K,N], one output [M,N]) is one grouped launch of the
 //     HIP backend: W8A8 with per-channel scale / per-token scale / int32 bias, or weight-only
 //     (bf16/f16 x, int8 weight, antiquant scale and offset [E,N]); with a qint4x2 weight [E,K,N/2] (A8W4,
-//     tests/st/test_grouped_matmul_v4_cops.py:429-485, and A16W4, :197-262) the nibble pairs are widened to int8 on the
-//     device first (msco_unpack_int4) and the W8A8 or the weight-only launch multiplies them: exact, at the price of
-//     one more pass over the weights;
+//     tests/st/test_grouped_matmul_v4_cops.py:429-485, and A16W4, :197-262) the launch has weight_dtype I4;
 //   * group_type -1 (independent x[i] @ weight[i]) is one dense launch per pair.
 // Not implemented on this backend and refused with a message: float x float matmuls,
 // uint64 scales with int8 output, `offset`, the activation inputs, group_type 1.  act_type selects an activation
@@ -92,10 +90,6 @@ struct OneLaunch {
   GmmProblem problem{};
   const void *addrs[MSCO_IN_COUNT] = {nullptr};
   void *out{nullptr};
-  // 4-bit weights: the nibble pairs (int4_bytes bytes at int4_src) are widened to int8 in a staging buffer of twice that
-  // size first, and addrs[MSCO_IN_WEIGHT] is set to the staging buffer
-  const void *int4_src{nullptr};
-  size_t int4_bytes{0};
 };
 const char *const kBackendOpName = "GroupedMatmulV4";
 
@@ -113,7 +107,7 @@ OneLaunch BuildOne(const ms::Tensor &x, const ms::Tensor &w, const ms::Tensor &b
   const void **addrs = one.addrs;
   d.abi_version = MSCO_GMM_ABI_VERSION;
   d.x_dtype = ToBackendDtype(xt);
-  d.weight_dtype = MSCO_DT_I8;
+  d.weight_dtype = int4 ? MSCO_DT_I4 : MSCO_DT_I8;
   d.out_dtype = ToBackendDtype(out.data_type());
   d.group_list_dtype = group_list.is_defined() ? ToBackendDtype(group_list.data_type()) : MSCO_DT_NONE;
   d.group_list_type = static_cast<int32_t>(group_list_type);
@@ -126,11 +120,6 @@ OneLaunch BuildOne(const ms::Tensor &x, const ms::Tensor &w, const ms::Tensor &b
   d.act_type = static_cast<int32_t>(act_type);
   addrs[MSCO_IN_X] = x.GetDataPtr();
   addrs[MSCO_IN_WEIGHT] = w.GetDataPtr();
-  if (int4) {
-    one.int4_src = w.GetDataPtr();
-    one.int4_bytes = w.nbytes();
-    addrs[MSCO_IN_WEIGHT] = nullptr;   // the staging buffer, set by the caller
-  }
   addrs[MSCO_IN_GROUP_LIST] = group_list.is_defined() ? group_list.GetDataPtr() : nullptr;
   auto expect_en = [&](const ms::Tensor &t, const char *name) {
     if (t.is_defined() && t.numel() != e * n) {
@@ -261,25 +250,11 @@ std::vector<OneLaunch> BuildLaunches(const V4Args &a, const TensorVec &outputs) 
   return launches;
 }
 
-// 4-bit weights -> int8 in `staging` (2 * int4_bytes bytes), which becomes the launch's weight
-void WidenInt4(OneLaunch &one, void *staging, void *stream) {
-  const int rc = msco_unpack_int4(one.int4_src, staging, static_cast<int64_t>(one.int4_bytes), stream);
-  if (rc != MSCO_OK) {
-    MS_LOG_EXCEPTION << "For " << kGroupedMatmulV4CopsName << ", widening the 4-bit weights failed: " << msco_status_string(rc);
-  }
-  one.addrs[MSCO_IN_WEIGHT] = staging;
-}
-
 // Pynative: plan (cached), take the workspace from the framework's allocator, launch.
 void RunGroupedMatmulV4(const V4Args &a, const TensorVec &outputs) {
   void *stream = CurrentStream();
   for (OneLaunch &one : BuildLaunches(a, outputs)) {
     auto plan = GmmPlanCache::GetInstance().GetOrCreate(kBackendOpName, one.desc, one.problem, stream);
-    ms::Tensor widened;
-    if (one.int4_bytes > 0) {
-      widened = AllocateTensor(kNumberTypeInt8, ShapeVector{static_cast<int64_t>(2 * one.int4_bytes)});
-      WidenInt4(one, widened.GetDataPtr(), stream);
-    }
     ms::Tensor workspace;
     if (plan->workspace_bytes > 0) {
       workspace = AllocateTensor(kNumberTypeInt8, ShapeVector{static_cast<int64_t>(plan->workspace_bytes)});
@@ -329,7 +304,6 @@ class GroupedMatmulV4CopsHip : public KernelMod {
     void *stream = CurrentStream();
     for (const OneLaunch &one : BuildLaunches(ArgsFromGraphInputs(inputs), outputs)) {
       sizes.push_back(GmmPlanCache::GetInstance().GetOrCreate(kBackendOpName, one.desc, one.problem, stream)->workspace_bytes);
-      if (one.int4_bytes > 0) sizes.push_back(2 * one.int4_bytes);   // 4-bit weights widened to int8: one more slice
     }
     return sizes;
   }
@@ -337,25 +311,15 @@ class GroupedMatmulV4CopsHip : public KernelMod {
   bool Launch(const KernelTensorList &inputs, const std::vector<ms::Tensor> &workspace, const std::vector<ms::Tensor> &outputs,
               void *stream) override {
     std::vector<OneLaunch> launches = BuildLaunches(ArgsFromGraphInputs(inputs), outputs);
-    size_t slot = 0;   // workspace slices in Resize's order: per launch the plan's, then the widened weights if any
-    for (size_t li = 0; li < launches.size(); ++li) {
+    for (size_t i = 0; i < launches.size(); ++i) {   // workspace slices in Resize's order, one per launch
       // the plan of the stream this launch goes to (a cache hit unless the stream changed since Resize)
-      auto plan = GmmPlanCache::GetInstance().GetOrCreate(kBackendOpName, launches[li].desc, launches[li].problem, stream);
-      const size_t i = slot++;
-      if (launches[li].int4_bytes > 0) {
-        const size_t w_slot = slot++;
-        if (w_slot >= workspace.size() || workspace[w_slot].nbytes() < 2 * launches[li].int4_bytes) {
-          MS_LOG_EXCEPTION << "For " << kGroupedMatmulV4CopsName << ", Launch got no workspace for the widened 4-bit weights of launch "
-                           << li << ": Resize must run when shapes change.";
-        }
-        WidenInt4(launches[li], workspace[w_slot].GetDataPtr(), stream);
-      }
+      auto plan = GmmPlanCache::GetInstance().GetOrCreate(kBackendOpName, launches[i].desc, launches[i].problem, stream);
       const bool have = i < workspace.size() && workspace[i].is_defined();
       if (plan->workspace_bytes > 0 && (!have || workspace[i].nbytes() < plan->workspace_bytes)) {
         MS_LOG_EXCEPTION << "For " << kGroupedMatmulV4CopsName << ", Launch got no workspace of " << plan->workspace_bytes
-                         << " bytes for launch " << li << ": Resize must run when shapes change.";
+                         << " bytes for launch " << i << ": Resize must run when shapes change.";
       }
-      LaunchPlan(kBackendOpName, plan, launches[li].addrs, launches[li].out, have ? workspace[i].GetDataPtr() : nullptr,
+      LaunchPlan(kBackendOpName, plan, launches[i].addrs, launches[i].out, have ? workspace[i].GetDataPtr() : nullptr,
                  have ? workspace[i].nbytes() : 0, stream);
     }
     return true;

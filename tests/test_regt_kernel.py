@@ -1,0 +1,89 @@
+"""Kernels that transpose and convert row-major [E,K,N] weights in registers (kernel_override 12): 4-bit and 8-bit weights,
+int8 and 16-bit activations, at the edges of their chunks (16 / 32 rows), strips (256 / 512 columns), K steps (64 / 32) and
+K splits, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_utils import ptr, to_dev
+from ms_custom_ops_amd import cabi
+from oracle import gmm_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# (rows per group, K, N, forced K split); the last list entry is where the rows end, M is two more
+SHAPES = [([1], 16, 16, 0), ([16, 0, 17], 48, 256, 0), ([3, 33, 1], 2064, 272, 3), ([5] * 24, 80, 528, 0), ([31, 2], 4096, 512, 8),
+          ([0, 0, 64, 7], 96, 1040, 2), ([2] * 70, 64, 48, 0)]
+
+
+def _run(x_dtype, bits, x, w, counts, split, operands, out_dtype, **fields):
+    m, (e, k, n) = x.shape[0], w.shape
+    wd = to_dev(O.pack_int4(w) if bits == 4 else w)
+    gl = to_dev(np.asarray(counts, dtype=np.int64))
+    op = cabi.GmmOp(x_dtype=x_dtype, weight_dtype=cabi.DT_I4 if bits == 4 else cabi.DT_I8, out_dtype=out_dtype, group_list_dtype=cabi.DT_I64,
+                    group_list_type=1, kernel_override=cabi.OV_REGT, force_split_k=split, **fields)
+    ws = op.plan(m, k, n, e)
+    assert "regt" in op.plan_info(), op.plan_info()
+    tws = torch.empty(max(ws, 1), dtype=torch.uint8, device="cuda:0")
+    out = torch.full((m, n), 0x7FC0, dtype=torch.int32 if out_dtype == cabi.DT_I32 else torch.int16, device="cuda:0")
+    tx = to_dev(x)
+    ins = [ptr(tx), ptr(wd), None, None, ptr(gl), None, None, None]
+    for slot, t in operands.items():
+        ins[slot] = ptr(t)
+    for _ in range(2):   # the arrival counters of a K split reset themselves
+        op.launch(ins, out.data_ptr(), tws.data_ptr(), ws, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    op.close()
+    return out.cpu().numpy()
+
+
+def _weights(rng, bits, e, k, n):
+    return rng.integers(-8, 8, (e, k, n), dtype=np.int8) if bits == 4 else rng.integers(-128, 128, (e, k, n), dtype=np.int8)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("counts,k,n,split", SHAPES)
+def test_int8_activations_bit_exact(device, counts, k, n, split, bits):
+    rng = np.random.default_rng(k + n + bits)
+    e, rows = len(counts), sum(counts)
+    x = rng.integers(-128, 128, (rows + 2, k), dtype=np.int8)
+    w = _weights(rng, bits, e, k, n)
+    bias = rng.integers(-1000, 1001, (e, n), dtype=np.int32)
+    scale = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32)
+    pt = rng.uniform(1e-3, 1e-2, rows + 2).astype(np.float32)
+    want, acc = O.grouped_matmul_w8a8(x, w, np.cumsum(counts), bias, scale, pt, return_acc=True)
+    ops = {cabi.IN_BIAS: to_dev(bias), cabi.IN_SCALE: to_dev(scale), cabi.IN_PER_TOKEN_SCALE: to_dev(pt)}
+    got = _run(cabi.DT_I8, bits, x, w, counts, split, ops, cabi.DT_BF16, bias_dtype=cabi.DT_I32, scale_dtype=cabi.DT_F32, per_token_dtype=cabi.DT_F32)
+    assert np.array_equal(got[:rows].view(np.uint16), want[:rows])
+    assert (got[rows:] == 0x7FC0).all()                      # rows behind the last group are left alone
+    raw = _run(cabi.DT_I8, bits, x, w, counts, split, {cabi.IN_BIAS: ops[cabi.IN_BIAS]}, cabi.DT_I32, bias_dtype=cabi.DT_I32)
+    assert np.array_equal(raw[:rows], acc[:rows] + np.repeat(bias, counts, axis=0))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("counts,k,n,split", SHAPES)
+def test_16_bit_activations_within_one_rounding_and_equal_for_both_weight_widths(device, counts, k, n, split, dtype):
+    """One rounding of the output plus float32 accumulation noise (1e-5 of the sum of the terms' magnitudes: K <= 4096
+    additions of relative error 2^-24 each) against float64; 4-bit weights and 8-bit weights of the same values give the
+    same bits where both take 16-row chunks (the 4-bit operands are 16 times the values, a power of two)."""
+    rng = np.random.default_rng(k + n)
+    e, rows = len(counts), sum(counts)
+    to_bits = O.f32_to_bf16_bits if dtype == "bf16" else (lambda a: a.astype(np.float16).view(np.uint16))
+    to_f = O.bf16_bits_to_f32 if dtype == "bf16" else (lambda b: b.view(np.float16).astype(np.float32))
+    x = to_bits(rng.standard_normal((rows + 2, k)).astype(np.float32))
+    s = to_bits(rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32))
+    o = to_bits(rng.integers(-8, 9, (e, n)).astype(np.float32))
+    dt = cabi.DT_BF16 if dtype == "bf16" else cabi.DT_F16
+    ops = {cabi.IN_ANTIQUANT_SCALE: to_dev(s), cabi.IN_ANTIQUANT_OFFSET: to_dev(o)}
+    run = lambda bits, w: _run(dt, bits, x, w, counts, split, ops, dt, antiquant_dtype=dt, has_antiquant_offset=1).view(np.uint16)
+    ends, starts = np.cumsum(counts), np.cumsum(counts) - counts
+    for w in (_weights(rng, 8, e, k, n), _weights(rng, 4, e, k, n)):
+        got = run(8, w)
+        exact = O.a16w8_grouped_f64(to_f(x), w, to_f(s), to_f(o), ends)[:rows]
+        mag = np.concatenate([np.abs(to_f(x)[a:b]) @ (np.abs(w[g].astype(np.float64) + to_f(o)[g]) * to_f(s)[g]) for g, (a, b) in enumerate(zip(starts, ends))])
+        ulp = 2.0 ** -7 if dtype == "bf16" else 2.0 ** -10
+        assert (np.abs(to_f(got[:rows]).astype(np.float64) - exact) <= ulp * np.abs(exact) + 1e-5 * mag).all()
+        assert (got[rows:] == 0x7FC0).all()
+    avg = -(-(rows + 2) // e)
+    if (avg if e == 1 else avg + avg // 2) <= 16:   # chunks of 16 rows for both widths: the same order of summation
+        assert np.array_equal(got, run(4, w))
