@@ -14,11 +14,14 @@ enum TileCfg : int {
   TILE_ROWS256 = 6,   // packed weights only: chunks of up to 256 rows x strips of 256 columns, x through LDS, weights straight into MFMA operands: gmm_rows_w8a8.hip
   TILE_ROWS128 = 7,   // the same with chunks of up to 128 rows and two workgroups per CU
   TILE_ROWS160 = 8,   // ... of up to 160 rows, two workgroups per CU, two K blocks of weights in flight
-  TILE_CFG_COUNT = 9
+  TILE_64x256_W4B = 9,    // 4-bit weights [E,K,N/2]
+  TILE_128x256_W4B = 10,
+  TILE_CFG_COUNT = 11
 };
 
 // MFMA tile kernel for W8A8 (prefill shapes).  nk: weights stored [E,N,K]; packed: the packed layout (nk is ignored).
 hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool packed, hipStream_t stream);
+hipError_t launch_tile_a8w4(const GmmParams &p, int tile_cfg, hipStream_t stream);   // int8 x, 4-bit weights [E,K,N/2]
 const char *tile_cfg_name(int tile_cfg);
 hipError_t launch_tile4m_w8a8(const GmmParams &p, int layout, hipStream_t stream);  // layout 0 [E,N,K], 1 packed, 2 [E,K,N] (N % 16 == 0)
 hipError_t launch_tile4_w8a8(const GmmParams &p, int layout, hipStream_t stream);   // layout 0 [E,N,K], 1 packed, 2 [E,K,N] (N % 16 == 0)

@@ -82,6 +82,16 @@ __device__ __forceinline__ void lds_read_tr8_pair(const unsigned char *p, uint2 
   (void)p; lo = hi = uint2{0, 0};
 #endif
 }
+// One 4-bit transpose read (ds_read_b64_tr_b4): of a block of 16 lanes, lane i names 8 bytes = 16 nibbles M[i][0..15] and
+// lane j receives nibble i = M[i][j].  Hand-issued like the pair above.
+__device__ __forceinline__ void lds_read_tr4(const unsigned char *p, uint2 &v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const unsigned a = (unsigned)(unsigned long)(const __attribute__((address_space(3))) unsigned char *)p;
+  asm volatile("ds_read_b64_tr_b4 %0, %1" : "=v"(v) : "v"(a));
+#else
+  (void)p; v = uint2{0, 0};
+#endif
+}
 template <typename T>
 __device__ __forceinline__ void lds_reads_done(T &frags) {
   asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(frags));
@@ -120,10 +130,15 @@ __device__ __forceinline__ void wait_vmcnt() {
 // byte b = M[2 b + j / 8][j % 8]; with lanes 2 b and 2 b + 1 on the two halves of one chunk of K row b, lane j gets K
 // rows 0 .. 7 of the chunk's column j).  MFMA row q of a 32-column block is then column q itself, so a lane owns four
 // runs of 4 output columns instead of two of 8 and the epilogue parks 8-byte pieces.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK = false, int KS = 2, bool WNT = false, bool KT = false>
+// W4 (with KT): 4-bit weights [E,K,N/2].  A slab row is BN / 2 bytes, and one transpose read turns 16 K rows of 16 columns
+// into 16 K-consecutive nibbles per lane; (v << 4) & 0xF0.. and v & 0xF0.. make int8 operands of 16 times the values of
+// the even and the odd ones (6 instructions per 16 weights), and the lanes of a read name their K rows in the order that
+// puts both back into the order of x.  The int32 sums are exactly 16 times the true ones.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK = false, int KS = 2, bool WNT = false, bool KT = false, bool W4 = false>
 __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel(const GmmParams p) {
   static_assert(!WNT || PK || KT, "non-temporal weight loads: whole kilobytes of whole lines per instruction (packed blocks, [K,N] rows)");
   static_assert(KS == 2 || KS == 4, "64- or 128-byte K slabs");
+  static_assert(!W4 || (KT && BN == 256), "4-bit weights: K rows of 128 bytes");
   static_assert(!KT || (!PK && (BN == 128 || BN == 256)), "transpose reads: [K,N] rows of 128 or 256 columns");
   constexpr int BKT = 32 * KS;                      // bytes of K per slab
   constexpr int ROWS_PER_LOAD = 1024 / BKT;         // x rows one wave instruction (1 KiB) brings
@@ -135,8 +150,9 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
   constexpr int FM = WTM / 32, FN = WTN / 32;     // 32 x 32 MFMA blocks per wave
   constexpr int A_LD = BM / ROWS_PER_LOAD / NW;     // 1 KiB pieces (16 or 8 rows) of the x slab per wave
-  constexpr int B_LD = BN * BKT / 1024 / NW;        // same for an [N,K] weight slab
-  constexpr int A_STAGE = BM * BKT, B_STAGE = BN * BKT;
+  constexpr int WPB = W4 ? 2 : 1;                   // weights per byte
+  constexpr int A_STAGE = BM * BKT, B_STAGE = BN * BKT / WPB;
+  constexpr int B_LD = B_STAGE / 1024 / NW;         // same for a weight slab
   constexpr int PANEL = 8;                          // m-tiles that share a streamed weight panel
   constexpr unsigned OOB = 0x80000000u;             // buffer offset that always reads zero
   constexpr int VM_PER_SLAB = A_LD + B_LD;          // vector-memory loads a wave issues per slab
@@ -230,14 +246,14 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   // Buffer descriptors start at this tile's first x row / weight column, so per-lane offsets stay
   // small; anything past the end of the group's rows / the tensor reads as zero (no clamping, no branches in
   // the loop; zeros instead of the next group's rows cost neither memory traffic nor matrix-pipe power).
-  const long long w_elems = (long long)p.k * p.n;
+  const long long w_elems = (long long)p.k * p.n / WPB;   // bytes of a group's weights
   const int8_t *wg = p.w + (long long)grp * w_elems;
   const __amdgpu_buffer_rsrc_t rx =
     make_rsrc(reinterpret_cast<const int8_t *>(p.x) + (long long)m0 * p.k, (long long)(g_end - m0) * p.k);
   const int pk_blocks = (p.k + 63) / 64, pk_groups = (p.n + 15) / 16;   // packed layout: K blocks per column group, column groups
   const __amdgpu_buffer_rsrc_t rw =
     PK   ? make_rsrc(p.w + ((long long)grp * pk_groups + n0 / 16) * pk_blocks * 1024, (long long)(pk_groups - n0 / 16) * pk_blocks * 1024)
-    : KT ? make_rsrc(wg + n0, w_elems - n0)
+    : KT ? make_rsrc(wg + n0 / WPB, w_elems - n0 / WPB)
          : make_rsrc(wg + (long long)n0 * p.k, (long long)(p.n - n0) * p.k);
 
   // ---- operands loaded straight into LDS (x rows, [N,K] weights) -----------------------------
@@ -262,15 +278,16 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   // column 32 * block + col_of_q(q) of the tile.
   unsigned b_voff[B_LD];
   int b_chunk[B_LD];                                 // [N,K] weights: logical chunk of this lane in piece u; [K,N]: its K row
-  constexpr int KT_SLOTS = BN / 16, KT_ROWS = 1024 / BN;   // [K,N] slabs: 16-column chunks per K row, K rows per piece
+  constexpr int KT_SLOTS = BN / WPB / 16, KT_ROWS = 1024 * WPB / BN;   // [K,N] slabs: 16-byte chunks per K row, K rows per piece
+  auto kt_swz = [](int r) { return W4 ? (r >> 1) & 7 : swz_kt<BN>(r); };
   if constexpr (KT) {
 #pragma unroll
     for (int u = 0; u < B_LD; ++u) {
       const int krow = (wave * B_LD + u) * KT_ROWS + lane / KT_SLOTS;   // K row of the slab that this lane brings in piece u
-      const int chunk = (lane % KT_SLOTS) ^ swz_kt<BN>(krow);
+      const int chunk = (lane % KT_SLOTS) ^ kt_swz(krow);
       b_chunk[u] = krow;                               // (the K tail is a matter of rows here)
       // columns past N read as zero; the K row of the slab goes into the scalar offset, which nobody range-checks
-      b_voff[u] = (n0 + chunk * 16 < p.n) ? (unsigned)krow * (unsigned)p.n + chunk * 16 : OOB;
+      b_voff[u] = (n0 + chunk * 16 * WPB < p.n) ? (unsigned)krow * (unsigned)(p.n / WPB) + chunk * 16 : OOB;
     }
   } else {
 #pragma unroll
@@ -303,7 +320,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
         buffer_load_lds_b128<WNT ? 2 : 0>(rw, lds_b + stage * B_STAGE + blk * 1024, b_voff[u] | kill_w, kblock * 1024);
       } else if constexpr (KT) {
         const unsigned kill_b = (kbase + (unsigned)b_chunk[u] >= (unsigned)p.k) ? OOB : 0u;   // K rows past K
-        buffer_load_lds_b128<WNT ? 2 : 0>(rw, lds_b + stage * B_STAGE + blk * 1024, b_voff[u] | kill_b, kbase * (unsigned)p.n);
+        buffer_load_lds_b128<WNT ? 2 : 0>(rw, lds_b + stage * B_STAGE + blk * 1024, b_voff[u] | kill_b, kbase * (unsigned)(p.n / WPB));
       } else {
         const unsigned kill_b = (kbase + b_chunk[u] * 16 >= (unsigned)p.k) ? OOB : 0u;
         buffer_load_lds_b128(rw, lds_b + stage * B_STAGE + blk * 1024, b_voff[u] | kill_b, kbase);
@@ -342,6 +359,15 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
     }
   };
 
+  // 4-bit weights: lane i of a block of 16 names the K row whose nibble lands at position i.  Even positions become the low
+  // operand words, odd ones the high ones, so positions 0, 2, 4, 6, 1, 3, 5, 7 (and 8 more) are K rows 0 .. 7 (8 .. 15).
+  auto read_w4 = [&](int kt, int f, int kk, uint2 &v) {
+    const int i = lane & 15;
+    const int krow = 32 * kk + 16 * hh + (i & 8) + 4 * (i & 1) + ((i & 7) >> 1);
+    const int chunk = (wave_n * WTN + 32 * f) / 32;
+    lds_read_tr4(lds_b + (kt % NSTAGE) * B_STAGE + krow * (BN / WPB) + ((chunk ^ kt_swz(krow)) << 4) + ((lane >> 4) & 1) * 8, v);
+  };
+
   v16i acc[FN][FM];
 #pragma unroll
   for (int f = 0; f < FN; ++f)
@@ -375,10 +401,14 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   auto step = [&](int kt) {
     issue_direct(kt + AHEAD);
     v4i xf[KS][FM], wf[KS][FN];
+    uint2 w4[KS][FN];
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-      for (int f = 0; f < FN; ++f) wf[kk][f] = read_w(kt, f, kk);
+      for (int f = 0; f < FN; ++f) {
+        if constexpr (W4) read_w4(kt, f, kk, w4[kk][f]);
+        else wf[kk][f] = read_w(kt, f, kk);
+      }
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
@@ -388,7 +418,19 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-        for (int f = 0; f < FN; ++f) lds_reads_done(wf[kk][f]);
+        for (int f = 0; f < FN; ++f) {
+          if constexpr (!W4) lds_reads_done(wf[kk][f]);
+          else lds_reads_done(w4[kk][f]);
+        }
+    }
+    if constexpr (W4) {
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+        for (int f = 0; f < FN; ++f) {
+          const unsigned a = w4[kk][f].x, b = w4[kk][f].y;
+          wf[kk][f] = v4i{(int)((a << 4) & 0xF0F0F0F0u), (int)(a & 0xF0F0F0F0u), (int)((b << 4) & 0xF0F0F0F0u), (int)(b & 0xF0F0F0F0u)};
+        }
     }
     if constexpr (PINGPONG) {
       wait_vmcnt<(AHEAD - 1) * VM_PER_SLAB>();                // this wave's part of slab t+1 has landed
@@ -508,6 +550,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
     pt[i] = ep_pt[wave_m * WTM + 32 * i + l32];
   }
   // int32 rows are 256 bytes: one 32-column block per pass; 16-bit outputs take a single pass
+  constexpr int SHIFT = W4 ? 4 : 0;   // the operands were 16 times the nibbles: exact
   auto run_pass = [&](auto raw_c, auto pass_c) {
     constexpr bool raw = decltype(raw_c)::value;
     constexpr int pass = decltype(pass_c)::value;
@@ -532,14 +575,14 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
           unsigned char *dst = stage + (32 * i + l32) * EP_PITCH;
           if (raw) {
             int *d = reinterpret_cast<int *>(dst + (cw - 32 * f) * 4);
-            *reinterpret_cast<int4 *>(d) = make_int4(acc[f][i][8 * s2] + bi[0], acc[f][i][8 * s2 + 1] + bi[1],
-                                                     acc[f][i][8 * s2 + 2] + bi[2], acc[f][i][8 * s2 + 3] + bi[3]);
-            *reinterpret_cast<int4 *>(d + RUN2) = make_int4(acc[f][i][8 * s2 + 4] + bi[4], acc[f][i][8 * s2 + 5] + bi[5],
-                                                            acc[f][i][8 * s2 + 6] + bi[6], acc[f][i][8 * s2 + 7] + bi[7]);
+            *reinterpret_cast<int4 *>(d) = make_int4((acc[f][i][8 * s2] >> SHIFT) + bi[0], (acc[f][i][8 * s2 + 1] >> SHIFT) + bi[1],
+                                                     (acc[f][i][8 * s2 + 2] >> SHIFT) + bi[2], (acc[f][i][8 * s2 + 3] >> SHIFT) + bi[3]);
+            *reinterpret_cast<int4 *>(d + RUN2) = make_int4((acc[f][i][8 * s2 + 4] >> SHIFT) + bi[4], (acc[f][i][8 * s2 + 5] >> SHIFT) + bi[5],
+                                                            (acc[f][i][8 * s2 + 6] >> SHIFT) + bi[6], (acc[f][i][8 * s2 + 7] >> SHIFT) + bi[7]);
           } else {
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = dequant(acc[f][i][8 * s2 + j] + bi[j], sc[j], pt[i]);
+            for (int j = 0; j < 8; ++j) v[j] = dequant((acc[f][i][8 * s2 + j] >> SHIFT) + bi[j], sc[j], pt[i]);
             if (p.act_type != ACT_NONE) {
 #pragma unroll
               for (int j = 0; j < 8; ++j) v[j] = activate(v[j], p.act_type);
@@ -591,13 +634,13 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
 }
 
 // ---- host launcher ---------------------------------------------------------------------------------
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES = 4, bool PK = false, int KS = 2, bool WNT = false, bool KT = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES = 4, bool PK = false, int KS = 2, bool WNT = false, bool KT = false, bool W4 = false>
 static hipError_t launch_cfg(const GmmParams &p, hipStream_t stream) {
   constexpr int BKT = 32 * KS;
-  const size_t loop_lds = (size_t)STAGES * (BM + BN) * BKT;
+  const size_t loop_lds = (size_t)STAGES * (BM + BN / (W4 ? 2 : 1)) * BKT;
   const size_t epi_lds = (size_t)WAVES_M * WAVES_N * (BM / WAVES_M) * 144;   // epilogue staging, 144-byte row pitch
   const size_t lds = (loop_lds > epi_lds ? loop_lds : epi_lds) + 3 * 1024;   // + epilogue operand table
-  auto kern = gmm_w8a8_tile_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, PK, KS, WNT, KT>;
+  auto kern = gmm_w8a8_tile_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, PK, KS, WNT, KT, W4>;
   static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race between first launches repeats it at worst
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
@@ -665,6 +708,19 @@ hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool pack
   }
 }
 
+// 4-bit weights [E,K,N/2] (N a multiple of 16): 128-byte K rows per tile.  8 experts, K = 4096, N = 14336, 32 / 128 / 256 /
+// 1024 rows per group: 58 / 106 / 162 / 478 us, against 213 / 240 / 280 / 539 us for widening the weights to int8 first (120 us
+// of it) and the kernels of int8 weights.  The weight stream (235 MB: 36 us) bounds the first, the operand path from L2 the
+// last.  (A 256 x 256 tile of eight waves: 171 us at 256 and 485 us at 1024 rows per group.)
+hipError_t launch_tile_a8w4(const GmmParams &p, int tile_cfg, hipStream_t stream) {
+  if (p.n % 16 != 0) return hipErrorInvalidValue;
+  if (tile_cfg == TILE_64x256_W4B)
+    return p.w_nontemporal ? launch_cfg<64, 256, 1, 4, 4, false, 2, true, true, true>(p, stream) : launch_cfg<64, 256, 1, 4, 4, false, 2, false, true, true>(p, stream);
+  if (tile_cfg == TILE_128x256_W4B)
+    return p.w_nontemporal ? launch_cfg<128, 256, 1, 4, 4, false, 2, true, true, true>(p, stream) : launch_cfg<128, 256, 1, 4, 4, false, 2, false, true, true>(p, stream);
+  return hipErrorInvalidValue;
+}
+
 const char *tile_cfg_name(int tile_cfg) {
   switch (tile_cfg) {
     case TILE_256x256: return "256x256x64";
@@ -676,6 +732,8 @@ const char *tile_cfg_name(int tile_cfg) {
     case TILE_ROWS256: return "rows256";
     case TILE_ROWS128: return "rows128";
     case TILE_ROWS160: return "rows160";
+    case TILE_64x256_W4B: return "64x256_4bit";
+    case TILE_128x256_W4B: return "128x256_4bit";
     default: return "?";
   }
 }
@@ -699,7 +757,8 @@ void tile_cfg_dims(int tile_cfg, int *bm, int *bn) {
   switch (tile_cfg) {
     case TILE_256x256: case TILE_256x256_W4: case TILE_256x256_W4_MFMA32: case TILE_ROWS256: case TILE_ROWS160: *bm = 256; *bn = 256; break;
     case TILE_128x128: *bm = 128; *bn = 128; break;
-    case TILE_128x256: case TILE_ROWS128: *bm = 128; *bn = 256; break;
+    case TILE_128x256: case TILE_ROWS128: case TILE_128x256_W4B: *bm = 128; *bn = 256; break;
+    case TILE_64x256_W4B: *bm = 64; *bn = 256; break;
     default: *bm = 64; *bn = 128; break;
   }
 }

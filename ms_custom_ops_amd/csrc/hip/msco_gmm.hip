@@ -29,7 +29,8 @@ enum Override : int {
   OV_ROWS128 = 9,  // packed weights: chunks of up to 128 rows through LDS, weights straight into MFMA operands (other layouts: 128 x 256 tiles)
   OV_ROWS256 = 10,  // the same with chunks of up to 256 rows (other layouts: the persistent kernel)
   OV_ROWS160 = 11,  // ... of up to 160 rows (other layouts: the persistent kernel)
-  OV_REGT = 12      // [E,K,N] weights transposed and converted in registers (other layouts: as planned)
+  OV_REGT = 12,     // [E,K,N] weights transposed and converted in registers (other layouts: as planned)
+  OV_TILE_4BIT = 13   // 4-bit weights, int8 x: 64 x 256 or 128 x 256 tiles that read the nibbles (else: as planned)
 };
 
 constexpr int64_t kSkinnyMaxRows = 64;   // total rows up to which the weight-streaming kernel is planned
@@ -117,7 +118,7 @@ int check_desc(const msco_gmm_desc &d) {
   if (d.group_list_dtype != MSCO_DT_NONE && d.group_list_dtype != MSCO_DT_I32 && d.group_list_dtype != MSCO_DT_I64)
     return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_type != 0 && d.group_list_type != 1) return MSCO_ERR_INVALID_ARG;
-  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_REGT) return MSCO_ERR_INVALID_ARG;
+  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_TILE_4BIT) return MSCO_ERR_INVALID_ARG;
   if (d.weight_layout != MSCO_WL_ROW_MAJOR && d.weight_layout != MSCO_WL_PACKED) return MSCO_ERR_INVALID_ARG;
   if (d.force_split_k < 0) return MSCO_ERR_INVALID_ARG;
   if (d.act_type < MSCO_ACT_NONE || d.act_type > MSCO_ACT_SILU) return MSCO_ERR_INVALID_ARG;
@@ -156,12 +157,41 @@ void plan_regt(msco_gmm_op *op) {
                    m * k < ((int64_t)1 << 31);
   // rows a group is expected to hold (shapes only); real routings are uneven, hence 1.5 x the average
   const int64_t avg = (m + e - 1) / e, rows = e == 1 ? m : avg + avg / 2;
-  // 4-bit weights: widening them first costs more than a second and third pass over the nibbles (8 experts, K = 4096,
-  // N = 14336: the widening alone 120 us; with 4 / 32 rows per group these kernels take 44 / 82 us with int8 x).
+  // 4-bit weights with 16-bit x: widening them first (8 experts, K = 4096, N = 14336: 120 us for the widening alone) costs
+  // more than a second and third pass over the nibbles (4 / 32 rows per group: 47 / 95 us in all).
   // Weight-only on 8-bit weights, one 16-row chunk per group: the decode form.
   const bool want = d.kernel_override == OV_REGT ||
                     (d.kernel_override == OV_AUTO && bits == 4 && rows <= 64) ||
                     (op->family == FAM_SKINNY && bits == 8 && is_a16w8(d) && op->stream_tch == 1);
+  // 4-bit weights, int8 x, more than one 16-row chunk per group: tiles that read the nibbles through LDS (4 / 16 / 32 rows
+  // per group 52 / 53 / 58 us against 44 / 53 / 82 us in 32-row chunks)
+  if (can && bits == 4 && is_w8a8(d) && (d.kernel_override == OV_TILE_4BIT || (d.kernel_override == OV_AUTO && rows > 16))) {
+    const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, groups = std::min<int64_t>(e, m), n_tiles = (n + 255) / 256;
+    // 128-row tiles once 64 rows no longer hold a group and there are tiles for most CUs (64 / 128 rows per group 83 / 114 us
+    // with 64-row tiles, 68 / 106 us with 128; one group of 256 rows, N = 11008: 31.7 against 42.7 us)
+    const bool tall = rows > 64 && std::max<int64_t>((m + 127) / 128, groups) * n_tiles * 4 >= cus * 3;
+    op->family = FAM_TILE;
+    op->tile_cfg = tall ? TILE_128x256_W4B : TILE_64x256_W4B;
+    if (tuning().tile_cfg >= TILE_64x256_W4B) op->tile_cfg = tuning().tile_cfg;
+    op->wide_k_slabs = 0;
+    op->small_group_rows = 0;
+    const int bm = op->tile_cfg == TILE_128x256_W4B ? 128 : 64;
+    op->w_nontemporal = (rows + bm - 1) / bm <= 2 && e * k * n / 2 >= ((int64_t)32 << 20);   // (as for int8 weights)
+    // K split of the 64-row tiles up to one workgroup per CU, by the cost in 64-byte K slabs: a slice's slabs, 10 for the
+    // workgroup's ends and 5 per slice of the exchange (one group, 32 rows, N = 11008, split 2 / 4 / 5: 21.6 / 18.7 / 19.0 us; 8 x
+    // 38 rows, N = 1024, split 2 / 4 / 8: 21.4 / 18.0 / 20.9 us)
+    const int64_t tiles = std::max<int64_t>((m + bm - 1) / bm, groups) * n_tiles, slabs = (k + 63) / 64;
+    const int64_t most = bm == 64 ? std::min<int64_t>({cus / tiles, kMaxSplitK, std::max<int64_t>(1, slabs / kTileMinSlabs)}) : 1;
+    auto cost = [&](int64_t s) { return (slabs + s - 1) / s + (s > 1 ? 5 * s : 0); };
+    int64_t split = 1;
+    for (int64_t s = 2; s <= most; ++s)
+      if (cost(s) < cost(split)) split = s;
+    if (d.force_split_k > 0 && bm == 64) split = std::min<int64_t>(d.force_split_k, slabs);
+    while (split > 1 && tile_workspace_bytes(op->tile_cfg, m, n, e, (int)split) > kTileSplitMaxWorkspace) --split;
+    op->split_k = (int)split;
+    op->workspace_bytes = tile_workspace_bytes(op->tile_cfg, m, n, e, op->split_k);
+    return;
+  }
   if (can && want) {
     const int blocks = bits == 8 || rows <= 16 ? 1 : 2;
     GmmParams p{};
@@ -754,7 +784,8 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
       small.w_nontemporal = layout == 2 || !nk;   // each small group's weights are read by one m-tile (packed, [E,K,N])
       err = launch_tile_w8a8(big, h->tile_cfg, nk, layout == 2, s);
       if (err == hipSuccess) err = launch_tile_w8a8(small, TILE_64x128, nk, layout == 2, s);
-    } else if (h->family == FAM_TILE) err = launch_tile_w8a8(p, h->tile_cfg, nk, layout == 2, s);
+    } else if (h->family == FAM_TILE && is_w4(d) && h->widen_bytes == 0) err = launch_tile_a8w4(p, h->tile_cfg, s);
+    else if (h->family == FAM_TILE) err = launch_tile_w8a8(p, h->tile_cfg, nk, layout == 2, s);
     else if (h->family == FAM_SKINNY && layout == 2) err = h->stream_tch > 1 ? launch_streamm_w8a8(p, h->stream_tch, s) : launch_stream_w8a8(p, s);
     else if (h->family == FAM_SKINNY) err = launch_skinny_w8a8(p, nk, h->skinny_wide16 != 0, s);
     else err = launch_generic_w8a8(p, layout, s);

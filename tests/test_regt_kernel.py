@@ -1,6 +1,6 @@
-"""Kernels that transpose and convert row-major [E,K,N] weights in registers (kernel_override 12): 4-bit and 8-bit weights,
-int8 and 16-bit activations, at the edges of their chunks (16 / 32 rows), strips (256 / 512 columns), K steps (64 / 32) and
-K splits, against the oracle."""
+"""Kernels on row-major [E,K,N] weights of 4 and 8 bits, at the edges of their chunks, strips, K steps and K splits, against
+the oracle: the ones that transpose and convert in registers (kernel_override 12: chunks of 16 / 32 rows, strips of 256 / 512
+columns, steps of 64 / 32 K) and the tiles that read 4-bit weights through LDS (13: 64 or 128 x 256, slabs of 64 K)."""
 import numpy as np
 import pytest
 import torch
@@ -16,14 +16,14 @@ SHAPES = [([1], 16, 16, 0), ([16, 0, 17], 48, 256, 0), ([3, 33, 1], 2064, 272, 3
           ([0, 0, 64, 7], 96, 1040, 2), ([2] * 70, 64, 48, 0)]
 
 
-def _run(x_dtype, bits, x, w, counts, split, operands, out_dtype, **fields):
+def _run(x_dtype, bits, x, w, counts, split, operands, out_dtype, override=cabi.OV_REGT, **fields):
     m, (e, k, n) = x.shape[0], w.shape
     wd = to_dev(O.pack_int4(w) if bits == 4 else w)
     gl = to_dev(np.asarray(counts, dtype=np.int64))
     op = cabi.GmmOp(x_dtype=x_dtype, weight_dtype=cabi.DT_I4 if bits == 4 else cabi.DT_I8, out_dtype=out_dtype, group_list_dtype=cabi.DT_I64,
-                    group_list_type=1, kernel_override=cabi.OV_REGT, force_split_k=split, **fields)
+                    group_list_type=1, kernel_override=override, force_split_k=split, **fields)
     ws = op.plan(m, k, n, e)
-    assert "regt" in op.plan_info(), op.plan_info()
+    assert {cabi.OV_REGT: "regt", cabi.OV_TILE_4BIT: "4bit"}[override] in op.plan_info(), op.plan_info()
     tws = torch.empty(max(ws, 1), dtype=torch.uint8, device="cuda:0")
     out = torch.full((m, n), 0x7FC0, dtype=torch.int32 if out_dtype == cabi.DT_I32 else torch.int16, device="cuda:0")
     tx = to_dev(x)
@@ -41,9 +41,12 @@ def _weights(rng, bits, e, k, n):
     return rng.integers(-8, 8, (e, k, n), dtype=np.int8) if bits == 4 else rng.integers(-128, 128, (e, k, n), dtype=np.int8)
 
 
-@pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("counts,k,n,split", SHAPES)
-def test_int8_activations_bit_exact(device, counts, k, n, split, bits):
+TILE_SHAPES = [([65], 80, 16, 0), ([64, 1, 0, 63], 4096, 272, 4), ([129, 40, 128], 2064, 528, 0), ([100] * 9, 256, 6144, 0)]
+
+
+@pytest.mark.parametrize("counts,k,n,split,bits,override",
+                         [(*s, bits, cabi.OV_REGT) for s in SHAPES for bits in (4, 8)] + [(*s, 4, cabi.OV_TILE_4BIT) for s in SHAPES + TILE_SHAPES])
+def test_int8_activations_bit_exact(device, counts, k, n, split, bits, override):
     rng = np.random.default_rng(k + n + bits)
     e, rows = len(counts), sum(counts)
     x = rng.integers(-128, 128, (rows + 2, k), dtype=np.int8)
@@ -53,10 +56,10 @@ def test_int8_activations_bit_exact(device, counts, k, n, split, bits):
     pt = rng.uniform(1e-3, 1e-2, rows + 2).astype(np.float32)
     want, acc = O.grouped_matmul_w8a8(x, w, np.cumsum(counts), bias, scale, pt, return_acc=True)
     ops = {cabi.IN_BIAS: to_dev(bias), cabi.IN_SCALE: to_dev(scale), cabi.IN_PER_TOKEN_SCALE: to_dev(pt)}
-    got = _run(cabi.DT_I8, bits, x, w, counts, split, ops, cabi.DT_BF16, bias_dtype=cabi.DT_I32, scale_dtype=cabi.DT_F32, per_token_dtype=cabi.DT_F32)
+    got = _run(cabi.DT_I8, bits, x, w, counts, split, ops, cabi.DT_BF16, override, bias_dtype=cabi.DT_I32, scale_dtype=cabi.DT_F32, per_token_dtype=cabi.DT_F32)
     assert np.array_equal(got[:rows].view(np.uint16), want[:rows])
     assert (got[rows:] == 0x7FC0).all()                      # rows behind the last group are left alone
-    raw = _run(cabi.DT_I8, bits, x, w, counts, split, {cabi.IN_BIAS: ops[cabi.IN_BIAS]}, cabi.DT_I32, bias_dtype=cabi.DT_I32)
+    raw = _run(cabi.DT_I8, bits, x, w, counts, split, {cabi.IN_BIAS: ops[cabi.IN_BIAS]}, cabi.DT_I32, override, bias_dtype=cabi.DT_I32)
     assert np.array_equal(raw[:rows], acc[:rows] + np.repeat(bias, counts, axis=0))
 
 
