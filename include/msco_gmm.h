@@ -137,7 +137,8 @@ typedef struct msco_gmm_desc {
                               * 256 x 256 (16 x 16 x 64 MFMAs), 7 128 x 256, 8 the persistent kernel's 32 x 32 x 32 MFMA form,
                               * 9 / 10 / 11 packed weights: chunks of up to 128 / 256 / 160 rows through LDS and weights
                               * straight into MFMA operands, 12 [E,K,N] weights transposed in registers, 13 tiles on 4-bit
-                              * weights (4-bit weights: every other value widens them to int8 first and forces the family on the result)
+                              * weights (4-bit weights: every other value widens them to int8 first and forces the family on the result),
+                              * 14 weight-only: equal chunks of up to 128 rows x strips of 512 columns
                               * (msco_gmm_plan_info names what was planned) */
   int32_t weight_layout;     /* MSCO_WL_ROW_MAJOR: as transpose_b says; MSCO_WL_PACKED: written by msco_pack_weight */
   int32_t act_type;          /* msco_act: activation applied to the dequantised float32 value before the output cast */

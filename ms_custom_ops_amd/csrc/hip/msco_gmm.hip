@@ -18,7 +18,7 @@ namespace {
 
 using namespace msco;
 
-enum Family : int { FAM_NONE = 0, FAM_TILE = 1, FAM_SKINNY = 2, FAM_GENERIC = 3, FAM_REGT = 4 };
+enum Family : int { FAM_NONE = 0, FAM_TILE = 1, FAM_SKINNY = 2, FAM_GENERIC = 3, FAM_REGT = 4, FAM_ROWS16 = 5 };
 
 // values of msco_gmm_desc::kernel_override
 enum Override : int {
@@ -30,7 +30,8 @@ enum Override : int {
   OV_ROWS256 = 10,  // the same with chunks of up to 256 rows (other layouts: the persistent kernel)
   OV_ROWS160 = 11,  // ... of up to 160 rows (other layouts: the persistent kernel)
   OV_REGT = 12,     // [E,K,N] weights transposed and converted in registers (other layouts: as planned)
-  OV_TILE_4BIT = 13   // 4-bit weights, int8 x: 64 x 256 or 128 x 256 tiles that read the nibbles (else: as planned)
+  OV_TILE_4BIT = 13,  // 4-bit weights, int8 x: 64 x 256 or 128 x 256 tiles that read the nibbles (else: as planned)
+  OV_ROWS16 = 14      // weight-only: equal chunks of up to 128 rows x strips of 512 columns (else: as planned)
 };
 
 constexpr int64_t kSkinnyMaxRows = 64;   // total rows up to which the weight-streaming kernel is planned
@@ -118,7 +119,7 @@ int check_desc(const msco_gmm_desc &d) {
   if (d.group_list_dtype != MSCO_DT_NONE && d.group_list_dtype != MSCO_DT_I32 && d.group_list_dtype != MSCO_DT_I64)
     return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_type != 0 && d.group_list_type != 1) return MSCO_ERR_INVALID_ARG;
-  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_TILE_4BIT) return MSCO_ERR_INVALID_ARG;
+  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_ROWS16) return MSCO_ERR_INVALID_ARG;
   if (d.weight_layout != MSCO_WL_ROW_MAJOR && d.weight_layout != MSCO_WL_PACKED) return MSCO_ERR_INVALID_ARG;
   if (d.force_split_k < 0) return MSCO_ERR_INVALID_ARG;
   if (d.act_type < MSCO_ACT_NONE || d.act_type > MSCO_ACT_SILU) return MSCO_ERR_INVALID_ARG;
@@ -238,6 +239,32 @@ void plan_regt(msco_gmm_op *op) {
     op->widen_bytes = (e * k * n + 255) / 256 * 256;
     op->workspace_bytes += (size_t)op->widen_bytes;
   }
+}
+
+// Weight-only on packed or [E,K,N] weights: tiles of 128 rows x 512 columns (gmm_rows_a16w8.hip) where they fill the chip.  One
+// workgroup per CU, and a tile takes about 19 us + 1.2 .. 1.4 us per 64 K, so what counts is how full the rounds are and that a
+// tile has rows enough; otherwise the 32- to 128-row kernels with their narrower strips and K split stay (us, before -> this,
+// packed / [E,K,N]):
+//   8 experts, K = 4096, N = 14336, 32 / 48 / 96 / 192 / 512 rows per group: 91 -> 96, 117 -> 101, 139 -> 118, 270 -> 197, 572 -> 435 /
+//   95 -> 93, 111 -> 95, 142 -> 122, 270 -> 222, 577 -> 456; 64 experts, K = 2048, N = 1408, 64 / 160 rows: 65 -> 53, 137 -> 106 / 63 -> 59,
+//   139 -> 118; one group, N = 11008, 512 (88 tiles) / 1024 (176) / 4096 rows: 91 -> 113, 158 -> 108, 444 -> 327 / 90 -> 107, 141 -> 116, 464 -> 347;
+//   128 tiles (8 experts, 4096 x 4096, 160 rows): 92 -> 89 / 95 -> 102; 288 tiles (16 experts, 2048 x 2816, 320 rows): 123 -> 113 / 112 -> 124;
+//   a strip and a half (128 experts, 1024 x 768, 100 rows): 53 -> 72 / 50 -> 81.  Short K, 64 experts x 64 rows, N = 2048, K = 512 / 768 / 1408: 32 -> 37,
+//   38.5 -> 36.5, 57 -> 53 / 31.5 -> 34.5, 38.2 -> 38.8, 57 -> 56 (the weights not in the caches 52 -> 54); x 150 rows, K = 512: 66 -> 60 / 62 -> 61.
+void plan_rows16(msco_gmm_op *op) {
+  const msco_gmm_desc &d = op->desc;
+  if (op->family != FAM_SKINNY || !is_a16w8(d) || layout_of(d) == 1 || op->k >= ((int64_t)1 << 22)) return;   // (128 rows of x through 32-bit offsets)
+  const int64_t m = op->m, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
+  const int64_t strips = (n + 511) / 512, groups = std::max<int64_t>(1, std::min<int64_t>(e, m)), avg = (m + e - 1) / e;
+  const int64_t rows = e == 1 ? m : avg + avg / 10;   // (real routings are uneven)
+  const int64_t tiles = strips * groups * ((rows + 127) / 128), rounds = (tiles + cus - 1) / cus;
+  const bool full = tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65;
+  const int64_t k_min = rows > 128 ? 512 : is_packed(d) ? 1024 : 2048;
+  if (d.kernel_override != OV_ROWS16 && !(d.kernel_override == OV_AUTO && d.force_split_k == 0 && op->k >= k_min && avg >= 48 && full && n * 100 >= strips * 512 * 85)) return;
+  op->family = FAM_ROWS16;
+  op->n_strips = (int)strips;
+  op->split_k = 1;
+  op->workspace_bytes = 0;
 }
 
 void choose_plan(msco_gmm_op *op) {
@@ -602,11 +629,12 @@ void choose_plan(msco_gmm_op *op) {
   }
   op->family = family;
   op->widen_bytes = 0;
+  plan_rows16(op);
   plan_regt(op);
 
   family = op->family;
   char buf[320];
-  const char *fam = family == FAM_REGT ? "skinny_regt" : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
+  const char *fam = family == FAM_REGT ? "skinny_regt" : family == FAM_ROWS16 ? "rows128" : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
   std::snprintf(buf, sizeof(buf),
                 "msco_gmm plan: kernel=%s%s%s%s layout=%s m=%lld k=%lld n=%lld e=%lld split_k=%d strips=%d "
                 "workspace=%zu%s",
@@ -774,6 +802,8 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   const int layout = layout_of(d);
   if (h->family == FAM_REGT) {
     err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, s);
+  } else if (h->family == FAM_ROWS16) {
+    err = launch_rows_a16w8(p, layout == 2, s);
   } else if (is_w8a8(d)) {
     if (h->family == FAM_TILE && h->small_group_rows > 0) {
       GmmParams big = p, small = p;
