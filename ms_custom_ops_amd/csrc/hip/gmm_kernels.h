@@ -26,7 +26,8 @@ const char *tile_cfg_name(int tile_cfg);
 hipError_t launch_tile4m_w8a8(const GmmParams &p, int layout, hipStream_t stream);  // layout 0 [E,N,K], 1 packed, 2 [E,K,N] (N % 16 == 0)
 hipError_t launch_tile4_w8a8(const GmmParams &p, int layout, hipStream_t stream);   // layout 0 [E,N,K], 1 packed, 2 [E,K,N] (N % 16 == 0)
 void tile_cfg_dims(int tile_cfg, int *bm, int *bn);
-// packed weights, several groups of a few dozen to a few hundred rows: chunks of 16 rbmax rows (rbmax = 8, 10 or 16), see gmm_rows_w8a8.hip
+// packed weights, several groups of a few dozen to a few hundred rows: chunks of 16 rbmax rows (rbmax = 8, 10 or 16), see gmm_rows_w8a8.hip;
+// p.w_nontemporal as for the tiles
 hipError_t launch_rows_w8a8(const GmmParams &p, int rbmax, hipStream_t stream);
 // K split across workgroups (p.split_k > 1; four-wave tile shapes only): partial tiles and arrival counters
 size_t tile_count_bound(int tile_cfg, int64_t m, int64_t n, int64_t e);
@@ -40,6 +41,11 @@ inline unsigned chunk_slots(const GmmParams &p, int rows_per_chunk) {
   const long long held = (p.m < p.e ? p.m : p.e) + p.m / rows_per_chunk;
   const long long slots = all < held ? all : held;
   return (unsigned)(slots > 1 ? slots : 1);
+}
+
+// workgroups of a launch that finds its work with chunk_of_xcd_slot: an XCD holds at most ceil(strips / 8) strips of a group
+inline long long xcd_slots(const GmmParams &p, int rows_per_chunk) {
+  return (long long)kNumXcd * ((p.n_strips + kNumXcd - 1) / kNumXcd) * chunk_slots(p, rows_per_chunk);
 }
 
 // Skinny (decode) kernels: one workgroup streams a 128-column weight strip of one group over a K

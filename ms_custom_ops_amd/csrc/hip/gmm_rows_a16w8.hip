@@ -96,40 +96,6 @@ __device__ __forceinline__ void xa_load_lds(__amdgpu_buffer_rsrc_t rsrc, unsigne
 #endif
 }
 
-// number of v < y (y >= 0) with v % kNumXcd == xcd
-__device__ __forceinline__ int xa_on_xcd(int y, int xcd) { return (y - xcd + kNumXcd - 1) / kNumXcd; }
-
-// Position `pos` of XCD `xcd` -> group, strip and rows.  The groups that hold rows are numbered; strip s of the r-th is unit
-// r strips + s and runs on XCD unit % 8, all its chunks in turn.  False past the last one.  Every lane of the wave calls it.
-__device__ __forceinline__ bool xa_locate(const GmmParams &p, int xcd, int pos, int lane, int &grp, int &strip, int &m0, int &chunk_rows) {
-  int carry = 0, seen = 0, rank0 = 0;
-  for (int g0 = 0; g0 < p.e; g0 += 64) {
-    int start, end;
-    group_rows_chunk(p, g0, lane, carry, start, end);
-    const int rows = end - start, chunks = (rows + XA_ROWS - 1) / XA_ROWS;
-    const unsigned long long held = __ballot(rows > 0);
-    const int rank = rank0 + __popcll(held & ((1ull << lane) - 1ull));
-    const int first = rank * p.n_strips;
-    const int units = xa_on_xcd(first + p.n_strips, xcd) - xa_on_xcd(first, xcd);
-    const int mine = units * chunks, upto = seen + wave_scan_add(mine, lane);
-    const unsigned long long beyond = __ballot(upto > pos);
-    if (beyond != 0) {
-      const int l = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(beyond));
-      const int c = wave_bcast(chunks, l), f = wave_bcast(first, l), r = wave_bcast(rows, l);
-      const int local = pos - (wave_bcast(upto, l) - wave_bcast(mine, l));
-      const int unit = local / c, i = local - unit * c;
-      grp = g0 + l;
-      strip = ((xcd - f) & (kNumXcd - 1)) + kNumXcd * unit;
-      const int blocks = (r + 15) / 16, b0 = (int)((long long)i * blocks / c), b1 = (int)((long long)(i + 1) * blocks / c);
-      m0 = wave_bcast(start, l) + 16 * b0;
-      chunk_rows = min(16 * (b1 - b0), r - 16 * b0);
-      return true;
-    }
-    seen = wave_bcast(upto, 63);
-    rank0 += __popcll(held);
-  }
-  return false;
-}
 }  // namespace
 
 // RB = 16-row blocks of the chunk
@@ -348,7 +314,7 @@ __global__ void __launch_bounds__(XA_THREADS, 2) gmm_a16w8_rows128_kernel(const 
   __shared__ __align__(16) unsigned char smem[XA_STAGES];
   const int lane = threadIdx.x & 63;
   int grp, strip, m0, chunk_rows;
-  if (!xa_locate(p, (int)(blockIdx.x % kNumXcd), (int)(blockIdx.x / kNumXcd), lane, grp, strip, m0, chunk_rows)) return;
+  if (!chunk_of_xcd_slot(p, XA_ROWS, (int)blockIdx.x, lane, grp, strip, m0, chunk_rows)) return;
   const int rb = (chunk_rows + 15) / 16;
   bool done = false;
   static_for<XA_RB>([&](auto i_c) {   // one copy of the K loop per number of 16-row blocks
@@ -366,8 +332,7 @@ hipError_t launch_rows_a16w8(const GmmParams &p_in, bool packed, hipStream_t str
   if (p_in.k % 16 != 0 || p_in.n % 16 != 0 || p_in.split_k != 1) return hipErrorInvalidValue;
   GmmParams p = p_in;
   p.n_strips = (p.n + XA_COLS - 1) / XA_COLS;
-  // an XCD holds at most ceil(strips / 8) strips of every group with rows, each with its chunks
-  const long long grid = (long long)kNumXcd * ((p.n_strips + kNumXcd - 1) / kNumXcd) * chunk_slots(p, XA_ROWS);
+  const long long grid = xcd_slots(p, XA_ROWS);
   if (grid > 0x7FFFFFFFll) return hipErrorInvalidValue;
   const bool bf = p.x_dtype == DT_BF16;
   auto kern = bf ? (packed ? gmm_a16w8_rows128_kernel<true, false> : gmm_a16w8_rows128_kernel<true, true>)

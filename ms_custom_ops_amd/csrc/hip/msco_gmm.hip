@@ -351,12 +351,24 @@ void choose_plan(msco_gmm_op *op) {
     // (narrower strips for fewer columns do not pay: with one or two column groups per wave, strips of 6 / 3 column groups,
     // 8 experts, 1024 rows, K = 5120, N = 2688 / 1344: 55 / 40 us against 46 / 24 us for the 64 x 128 tiles)
     const bool rows_kernel_ok = is_packed(d) && e > 1 && k >= 1024 && ((n + 255) / 256) * std::min<int64_t>(e, m) >= num_cus;
+    // The 160-row form again where a group is two or three equal chunks that share its weights through the L2.  What it beats is the
+    // second 256-row m-tile of a group of just more than 256 rows (us, persistent -> this): 8 experts, K = 4096, N = 14336, 240 / 256 /
+    // 272 / 300 / 400 / 512 rows per group: 126 -> 141, 164 -> 141, 191 -> 155, 206 -> 159, 208 -> 206, 255 -> 239; 64 experts, K = 2048, N = 1408,
+    // 256 / 300 / 330 / 400 rows: 89 -> 79, 99 -> 90, 98 -> 111, 100 -> 122 (few columns, narrow strips); and 128 x 128 tiles where
+    // larger ones do not fill the chip but these workgroups do: 8 experts, K = 7168, N = 4096, 200 / 240 / 300 rows: 91 -> 69, 120 -> 74,
+    // 141 -> 80; 2 experts, K = 4096, N = 11008, 200 / 512 rows: 47 -> 38, 78 -> 65; 8 experts, 4096 x 2048, 200 rows (128 workgroups): 28 -> 38.
+    const int64_t row_wgs = ((n + 255) / 256) * std::min<int64_t>(e, m) * ((avg_rows + avg_rows / 20 + 159) / 160);
+    const bool rows_chunks_ok = is_packed(d) && e > 1 && k >= 2048 &&
+                                ((avg_rows >= 244 && avg_rows <= 296 && row_wgs >= 172) || (avg_rows > 296 && avg_rows <= 520 && n >= 4096 && row_wgs >= 256) ||
+                                 (avg_rows >= 192 && avg_rows < 244 && n >= 2048 && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));
     if (rows_kernel_ok && avg_rows <= 116) {
       op->tile_cfg = TILE_ROWS128;
     } else if (rows_kernel_ok && avg_rows <= 146) {
       op->tile_cfg = TILE_ROWS160;
     } else if (rows_kernel_ok && avg_rows <= 155) {
       op->tile_cfg = TILE_ROWS256;
+    } else if (rows_chunks_ok) {
+      op->tile_cfg = TILE_ROWS160;
     } else if (e > 1 && w4_ok && cover > 174 && cover <= 384 && group_tiles(256, 256) >= busy) {
       op->tile_cfg = TILE_256x256_W4;
     } else if (e > 1 && cover > 64 && cover <= 192 && group_tiles(128, 128) >= busy) {
@@ -473,13 +485,13 @@ void choose_plan(msco_gmm_op *op) {
     // least: ceil(workgroups / CUs) x (strip bytes + x bytes of a chunk), one chunk per group expected.  8 experts x 14336
     // columns on 256 CUs: 448 workgroups of 16 column groups cost two per CU as 512 of 14 do (c3_t64 82.2 -> 72.8 us).
     const int64_t cus = num_cus > 0 ? num_cus : kDefaultCUs;
-    const int64_t col_groups = (n + 15) / 16, chunks = std::max<int64_t>(1, std::min<int64_t>(e, m));
+    const int64_t col_groups = (n + 15) / 16, groups = std::max<int64_t>(1, std::min<int64_t>(e, m));
     const int64_t chunk_rows = op->tile_cfg == TILE_ROWS128 ? 128 : op->tile_cfg == TILE_ROWS160 ? 160 : 256;
-    const int64_t x_bytes = std::min<int64_t>(avg_rows, chunk_rows) * k;
+    const int64_t group_chunks = (avg_rows + chunk_rows - 1) / chunk_rows, x_bytes = (avg_rows + group_chunks - 1) / group_chunks * k;
     int best = 16;
     int64_t best_cost = INT64_MAX;
     for (int sg = 16; sg >= 10; --sg) {
-      const int64_t wgs = ((col_groups + sg - 1) / sg) * chunks;
+      const int64_t wgs = ((col_groups + sg - 1) / sg) * groups * group_chunks;
       const int64_t cost = ((wgs + cus - 1) / cus) * ((int64_t)sg * 16 * k + x_bytes);
       if (cost < best_cost) { best_cost = cost; best = sg; }
     }
@@ -487,6 +499,7 @@ void choose_plan(msco_gmm_op *op) {
     const int forced_groups = tuning().stream_groups;
     if (forced_groups >= 1 && forced_groups <= 16) op->strip_groups = forced_groups;
     op->n_strips = (int)((col_groups + op->strip_groups - 1) / op->strip_groups);
+    op->w_nontemporal = avg_rows <= chunk_rows;   // (the 128- and 256-row forms are planned for one chunk per group and always set the bit)
   }
   // Many experts with uneven loads (a skewed routing): every group of a few rows costs the persistent kernel a whole
   // 256-row m-tile per n-tile.  The groups of at most 64 rows go to a second launch of 64 x 128 tiles instead, which
