@@ -125,8 +125,9 @@ def as_qint4x2(tensor: torch.Tensor) -> QInt4x2:
 def widen_qint4x2(weight) -> torch.Tensor:
     """4-bit weights widened to int8 once, at load time: [..., N / 2] nibble pairs (a QInt4x2 or the int8 / uint8 bytes
     themselves; low nibble first, signed) become an int8 tensor [..., N] that grouped_matmul_v4_cops takes like any int8
-    weight.  The op widens a qint4x2 weight on every call (one more pass over the weights); a caller whose weights do
-    not change does it here and keeps the result.  No counterpart in the reference, whose kernels read 4-bit weights
+    weight.  The op reads the 4-bit values directly for groups of up to a few dozen rows (int8 x: any number)
+    and widens them on every call beyond that (one more pass over the weights); a caller with large groups and weights that
+    do not change may do it here and keep the result.  No counterpart in the reference, whose kernels read 4-bit weights
     directly (ops/c_api/grouped_matmul_v4_cops/grouped_matmul_v4_cops.cc:56-66)."""
     t = weight.tensor if isinstance(weight, QInt4x2) else QInt4x2(weight).tensor
     if not t.is_cuda:
