@@ -357,10 +357,12 @@ void choose_plan(msco_gmm_op *op) {
     // 256 / 300 / 330 / 400 rows: 89 -> 79, 99 -> 90, 98 -> 111, 100 -> 122 (few columns, narrow strips); and 128 x 128 tiles where
     // larger ones do not fill the chip but these workgroups do: 8 experts, K = 7168, N = 4096, 200 / 240 / 300 rows: 91 -> 69, 120 -> 74,
     // 141 -> 80; 2 experts, K = 4096, N = 11008, 200 / 512 rows: 47 -> 38, 78 -> 65; 8 experts, 4096 x 2048, 200 rows (128 workgroups): 28 -> 38.
+    // Where 256-row tiles fill the chip the line is the one m-tile that holds an even group: up to 256 rows an even routing is faster there
+    // (240 rows: 126 against 141 us) and only an uneven one with 256 on average is not (164 against 141 us).
     const int64_t row_wgs = ((n + 255) / 256) * std::min<int64_t>(e, m) * ((avg_rows + avg_rows / 20 + 159) / 160);
     const bool rows_chunks_ok = is_packed(d) && e > 1 && k >= 2048 &&
-                                ((avg_rows >= 244 && avg_rows <= 296 && row_wgs >= 172) || (avg_rows > 296 && avg_rows <= 520 && n >= 4096 && row_wgs >= 256) ||
-                                 (avg_rows >= 192 && avg_rows < 244 && n >= 2048 && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));
+                                ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172) || (avg_rows > 296 && avg_rows <= 520 && n >= 4096 && row_wgs >= 256) ||
+                                 (avg_rows >= 192 && avg_rows <= 256 && n >= 2048 && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));
     if (rows_kernel_ok && avg_rows <= 116) {
       op->tile_cfg = TILE_ROWS128;
     } else if (rows_kernel_ok && avg_rows <= 146) {
