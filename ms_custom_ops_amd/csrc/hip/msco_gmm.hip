@@ -251,6 +251,7 @@ void plan_regt(msco_gmm_op *op) {
 //   128 tiles (8 experts, 4096 x 4096, 160 rows): 92 -> 89 / 95 -> 102; 288 tiles (16 experts, 2048 x 2816, 320 rows): 123 -> 113 / 112 -> 124;
 //   a strip and a half (128 experts, 1024 x 768, 100 rows): 53 -> 72 / 50 -> 81.  Short K, 64 experts x 64 rows, N = 2048, K = 512 / 768 / 1408: 32 -> 37,
 //   38.5 -> 36.5, 57 -> 53 / 31.5 -> 34.5, 38.2 -> 38.8, 57 -> 56 (the weights not in the caches 52 -> 54); x 150 rows, K = 512: 66 -> 60 / 62 -> 61.
+//   [E,K,N], 64 experts, N = 4096: K = 768 x 200 rows 161 -> 152, three tiles per group (270 rows) K = 576 / 1024: 181 -> 189, 253 -> 255.
 void plan_rows16(msco_gmm_op *op) {
   const msco_gmm_desc &d = op->desc;
   if (op->family != FAM_SKINNY || !is_a16w8(d) || layout_of(d) == 1 || op->k >= ((int64_t)1 << 22)) return;   // (128 rows of x through 32-bit offsets)
@@ -259,7 +260,7 @@ void plan_rows16(msco_gmm_op *op) {
   const int64_t rows = e == 1 ? m : avg + avg / 10;   // (real routings are uneven)
   const int64_t tiles = strips * groups * ((rows + 127) / 128), rounds = (tiles + cus - 1) / cus;
   const bool full = tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65;
-  const int64_t k_min = rows > 128 ? 512 : is_packed(d) ? 1024 : 2048;
+  const int64_t k_min = rows <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : rows <= 256 ? 768 : 1280;
   if (d.kernel_override != OV_ROWS16 && !(d.kernel_override == OV_AUTO && d.force_split_k == 0 && op->k >= k_min && avg >= 48 && full && n * 100 >= strips * 512 * 85)) return;
   op->family = FAM_ROWS16;
   op->n_strips = (int)strips;
@@ -353,15 +354,17 @@ void choose_plan(msco_gmm_op *op) {
     const bool rows_kernel_ok = is_packed(d) && e > 1 && k >= 1024 && ((n + 255) / 256) * std::min<int64_t>(e, m) >= num_cus;
     // The 160-row form again where a group is two or three equal chunks that share its weights through the L2.  What it beats is the
     // second 256-row m-tile of a group of just more than 256 rows (us, persistent -> this): 8 experts, K = 4096, N = 14336, 240 / 256 /
-    // 272 / 300 / 400 / 512 rows per group: 126 -> 141, 164 -> 141, 191 -> 155, 206 -> 159, 208 -> 206, 255 -> 239; 64 experts, K = 2048, N = 1408,
+    // 272 / 300 / 400 rows per group: 126 -> 141, 164 -> 141, 191 -> 155, 206 -> 159, 208 -> 208; 64 experts, K = 2048, N = 1408,
     // 256 / 300 / 330 / 400 rows: 89 -> 79, 99 -> 90, 98 -> 111, 100 -> 122 (few columns, narrow strips); and 128 x 128 tiles where
     // larger ones do not fill the chip but these workgroups do: 8 experts, K = 7168, N = 4096, 200 / 240 / 300 rows: 91 -> 69, 120 -> 74,
-    // 141 -> 80; 2 experts, K = 4096, N = 11008, 200 / 512 rows: 47 -> 38, 78 -> 65; 8 experts, 4096 x 2048, 200 rows (128 workgroups): 28 -> 38.
+    // 141 -> 80; 2 experts, K = 4096, N = 11008, 200 rows: 47 -> 38; 8 experts, 4096 x 2048, 200 rows (128 workgroups): 28 -> 38.
+    // Up to 340 rows: 8 experts, K = 2816, N = 5664, 330 / 400 / 450 rows 80 -> 73, 70 -> 77, 74 -> 81; 32 experts, K = 2048, N = 4608, 330 rows 148 -> 128;
+    // 16 experts, K = 2784, N = 7504, 480 rows 183 -> 190.
     // Where 256-row tiles fill the chip the line is the one m-tile that holds an even group: up to 256 rows an even routing is faster there
     // (240 rows: 126 against 141 us) and only an uneven one with 256 on average is not (164 against 141 us).
     const int64_t row_wgs = ((n + 255) / 256) * std::min<int64_t>(e, m) * ((avg_rows + avg_rows / 20 + 159) / 160);
     const bool rows_chunks_ok = is_packed(d) && e > 1 && k >= 2048 &&
-                                ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172) || (avg_rows > 296 && avg_rows <= 520 && n >= 4096 && row_wgs >= 256) ||
+                                ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172) || (avg_rows > 296 && avg_rows <= 340 && n >= 4096 && row_wgs >= 256) ||
                                  (avg_rows >= 192 && avg_rows <= 256 && n >= 2048 && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));
     if (rows_kernel_ok && avg_rows <= 116) {
       op->tile_cfg = TILE_ROWS128;
