@@ -167,7 +167,7 @@ void plan_regt(msco_gmm_op *op) {
   // 4-bit weights, int8 x, more than one 16-row chunk per group: tiles that read the nibbles through LDS (4 / 16 / 32 rows
   // per group 52 / 53 / 58 us against 44 / 53 / 82 us in 32-row chunks)
   if (can && bits == 4 && is_w8a8(d) && (d.kernel_override == OV_TILE_4BIT || (d.kernel_override == OV_AUTO && rows > 16))) {
-    const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, groups = std::min<int64_t>(e, m), n_tiles = (n + 255) / 256;
+    const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, groups = std::max<int64_t>(1, std::min<int64_t>(e, m)), n_tiles = (n + 255) / 256;
     // 128-row tiles once 64 rows no longer hold a group and there are tiles for most CUs (64 / 128 rows per group 83 / 114 us
     // with 64-row tiles, 68 / 106 us with 128; one group of 256 rows, N = 11008: 31.7 against 42.7 us)
     const bool tall = rows > 64 && std::max<int64_t>((m + 127) / 128, groups) * n_tiles * 4 >= cus * 3;
@@ -492,7 +492,7 @@ void choose_plan(msco_gmm_op *op) {
     const int64_t cus = num_cus > 0 ? num_cus : kDefaultCUs;
     const int64_t col_groups = (n + 15) / 16, groups = std::max<int64_t>(1, std::min<int64_t>(e, m));
     const int64_t chunk_rows = op->tile_cfg == TILE_ROWS128 ? 128 : op->tile_cfg == TILE_ROWS160 ? 160 : 256;
-    const int64_t group_chunks = (avg_rows + chunk_rows - 1) / chunk_rows, x_bytes = (avg_rows + group_chunks - 1) / group_chunks * k;
+    const int64_t group_chunks = std::max<int64_t>(1, (avg_rows + chunk_rows - 1) / chunk_rows), x_bytes = (avg_rows + group_chunks - 1) / group_chunks * k;
     int best = 16;
     int64_t best_cost = INT64_MAX;
     for (int sg = 16; sg >= 10; --sg) {

@@ -4,6 +4,8 @@ workload generators.  No kernel is launched here."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -124,6 +126,34 @@ def test_plan_of_the_serving_range_on_packed_weights_without_a_gpu():
     assert "tile_256x256x128_w4" in plan(896, packed=False, override=cabi.OV_ROWS256)[0]
     assert "tile_rows256" in plan(300, n=512, k=256, e=2, override=cabi.OV_ROWS256)[0]
     assert "tile_rows160" in plan(300, n=512, k=256, e=2, override=cabi.OV_ROWS160)[0]
+
+
+def _plan_fields(x, bits=8, packed=False):
+    half = x in ("bf16", "f16")
+    dt = {"i8": cabi.DT_I8, "bf16": cabi.DT_BF16, "f16": cabi.DT_F16}[x]
+    fields = dict(x_dtype=dt, weight_dtype=cabi.DT_I4 if bits == 4 else cabi.DT_I8, out_dtype=dt if half else cabi.DT_BF16,
+                  group_list_dtype=cabi.DT_I64, weight_layout=cabi.WL_PACKED if packed else cabi.WL_ROW_MAJOR)
+    return dict(fields, antiquant_dtype=dt) if half else dict(fields, scale_dtype=cabi.DT_F32, scale_per_group=1)
+
+
+def _plan(m, k, n, e, x="i8", bits=8, packed=False, override=0, force_split_k=0):
+    """(workspace bytes, plan info) of a shape; no device needed as long as K is not split across workgroups."""
+    op = cabi.GmmOp(kernel_override=override, force_split_k=force_split_k, **_plan_fields(x, bits, packed))
+    try:
+        return op.plan(m, k, n, e), op.plan_info()
+    finally:
+        op.close()
+
+
+def test_no_rows_can_be_planned_under_every_kernel_override():
+    # an empty batch is a valid call (launching its plan does nothing); the plans are made in a process of their own, so that one that
+    # ends the process (an integer division by zero rows) fails this test and not the run (N: enough strips that K is not split)
+    cases = [(x, bits, packed) for x in ("i8", "bf16") for bits, packed in ((8, False), (8, True), (4, False))]
+    code = ("import sys; sys.path[:0] = %r; from test_host_logic import _plan\n"
+            "for c in %r:\n    for ov in range(15):\n        print(c, ov, flush=True); _plan(0, 4096, 131072, 8, *c, ov)\n"
+            % ([REPO, os.path.join(REPO, "tests")], cases))
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert done.returncode == 0, (done.stdout.splitlines()[-1:], done.stderr[-500:])
 
 
 def test_grouped_matmul_infer_shape_and_type():
