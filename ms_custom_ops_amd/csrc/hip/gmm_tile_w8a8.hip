@@ -31,6 +31,7 @@
 
 #include "gmm_common.h"
 #include "gmm_kernels.h"
+#include "gmm_w4_piece.h"
 
 #include <type_traits>
 
@@ -253,7 +254,8 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   const int pk_blocks = (p.k + 63) / 64, pk_groups = (p.n + 15) / 16;   // packed layout: K blocks per column group, column groups
   const __amdgpu_buffer_rsrc_t rw =
     PK   ? make_rsrc(p.w + ((long long)grp * pk_groups + n0 / 16) * pk_blocks * 1024, (long long)(pk_groups - n0 / 16) * pk_blocks * 1024)
-    : KT ? make_rsrc(wg + n0 / WPB, w_elems - n0 / WPB)
+    : W4 ? make_rsrc(wg, w_elems)
+    : KT ? make_rsrc(wg + n0, w_elems - n0)
          : make_rsrc(wg + (long long)n0 * p.k, (long long)(p.n - n0) * p.k);
 
   // ---- operands loaded straight into LDS (x rows, [N,K] weights) -----------------------------
@@ -287,7 +289,10 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
       const int chunk = (lane % KT_SLOTS) ^ kt_swz(krow);
       b_chunk[u] = krow;                               // (the K tail is a matter of rows here)
       // columns past N read as zero; the K row of the slab goes into the scalar offset, which nobody range-checks
-      b_voff[u] = (n0 + chunk * 16 * WPB < p.n) ? (unsigned)krow * (unsigned)(p.n / WPB) + chunk * 16 : OOB;
+      // (4-bit weights: no piece ends behind its K row, see gmm_w4_piece.h)
+      const int col = n0 + chunk * 16 * WPB;
+      if constexpr (W4) b_voff[u] = col < p.n ? w4_piece_offset(krow, col, p.n) : OOB;
+      else b_voff[u] = col < p.n ? (unsigned)krow * (unsigned)p.n + chunk * 16 : OOB;
     }
   } else {
 #pragma unroll
@@ -365,7 +370,8 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
     const int i = lane & 15;
     const int krow = 32 * kk + 16 * hh + (i & 8) + 4 * (i & 1) + ((i & 7) >> 1);
     const int chunk = (wave_n * WTN + 32 * f) / 32;
-    lds_read_tr4(lds_b + (kt % NSTAGE) * B_STAGE + krow * (BN / WPB) + ((chunk ^ kt_swz(krow)) << 4) + ((lane >> 4) & 1) * 8, v);
+    const int half = w4_half_offset(krow, n0 + 32 * chunk, p.n, (lane >> 4) & 1);   // (the same for every kk)
+    lds_read_tr4(lds_b + (kt % NSTAGE) * B_STAGE + krow * (BN / WPB) + ((chunk ^ kt_swz(krow)) << 4) + half, v);
   };
 
   v16i acc[FN][FM];

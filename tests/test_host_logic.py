@@ -156,6 +156,38 @@ def test_no_rows_can_be_planned_under_every_kernel_override():
     assert done.returncode == 0, (done.stdout.splitlines()[-1:], done.stderr[-500:])
 
 
+_PIECE_WALK = r"""
+#include "gmm_w4_piece.h"
+// every piece that the 4-bit tiles request of one group's [K, N/2] bytes: false if one lies outside them or if a column is
+// not where the fragment reads look for it
+extern "C" int walk(int k, int n) {
+  const long long pitch = n / 2, bytes = k * pitch;
+  for (int kbase = 0; kbase < k; kbase += 64)
+    for (int krow = 0; krow < 64 && kbase + krow < k; ++krow)
+      for (int col = 0; col < n; col += 32) {
+        const long long at = kbase * pitch + msco::w4_piece_offset(krow, col, n);
+        if (at < 0 || at + 16 > bytes) return 0;
+        for (int half = 0; half < 2 && col + 16 * half < n; ++half)
+          if (at + msco::w4_half_offset(krow, col, n, half) != (kbase + krow) * pitch + (col + 16 * half) / 2) return 0;
+        if (msco::w4_half_offset(krow, col, n, 1) > 8 || msco::w4_half_offset(krow, col, n, 0) != msco::w4_half_offset(krow % 32, col, n, 0)) return 0;
+      }
+  return 1;
+}
+"""
+
+
+def test_4_bit_tiles_read_inside_the_weights(tmp_path):
+    # N = 16 (mod 32): the last piece of a K row has 16 of its 32 columns; neither it nor any other may reach past the group's
+    # bytes, and its columns are found where they were put
+    src, lib = tmp_path / "walk.cc", tmp_path / "walk.so"
+    src.write_text(_PIECE_WALK)
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(REPO, "ms_custom_ops_amd", "csrc", "hip"), str(src), "-o", str(lib)])
+    walk = ctypes.CDLL(str(lib)).walk
+    for k in (16, 48, 64, 80, 112, 2064):
+        for n in (16, 32, 48, 256, 272, 528, 1040, 1056):
+            assert walk(k, n), (k, n)
+
+
 def test_grouped_matmul_infer_shape_and_type():
     shapes, types = _C._graph_infer("grouped_matmul", _gmm_args())
     assert shapes == [[64, 128]] and types == [F16]          # the reference's float16 output
