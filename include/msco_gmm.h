@@ -120,7 +120,7 @@ enum {
 typedef struct msco_gmm_desc {
   int32_t abi_version;       /* MSCO_GMM_ABI_VERSION */
   int32_t x_dtype;           /* I8 | BF16 | F16 */
-  int32_t weight_dtype;      /* I8 | I4 ([E,K,N/2] bytes, row-major, transpose_b 0) */
+  int32_t weight_dtype;      /* I8 | I4 ([E,K,N/2] bytes, N even, row-major, transpose_b 0) */
   int32_t out_dtype;         /* BF16 | F16 | I32 (raw accumulator + bias; scales are not applied) */
   int32_t group_list_dtype;  /* I32 | I64 | NONE */
   int32_t group_list_type;   /* 0 cumulative row ends, 1 per-group row counts */

@@ -709,6 +709,7 @@ int msco_gmm_plan(msco_gmm_handle h, int64_t m, int64_t k, int64_t n, int64_t e,
   if (m < 0 || k <= 0 || n <= 0 || e <= 0) return MSCO_ERR_SHAPE;
   if (m > INT32_MAX || k > INT32_MAX || n > INT32_MAX || e > 65535 || m * n > ((int64_t)1 << 40)) return MSCO_ERR_SHAPE;
   if (h->desc.group_list_dtype == MSCO_DT_NONE && m % e != 0) return MSCO_ERR_SHAPE;
+  if (is_w4(h->desc) && n % 2 != 0) return MSCO_ERR_SHAPE;   // [E,K,N/2] bytes hold pairs of columns
   std::lock_guard<std::mutex> lock(h->mu);
   h->m = m; h->k = k; h->n = n; h->e = e;
   choose_plan(h);

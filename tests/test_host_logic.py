@@ -188,6 +188,14 @@ def test_4_bit_tiles_read_inside_the_weights(tmp_path):
             assert walk(k, n), (k, n)
 
 
+def test_4_bit_weights_come_in_pairs_of_columns():
+    assert "widened" in _plan(4, 7, 6, 1, bits=4)[1]
+    for x in ("i8", "bf16"):
+        with pytest.raises(cabi.BackendError) as e:   # [E,K,N/2] does not exist for an odd N
+            _plan(4, 7, 5, 1, x, bits=4)
+        assert e.value.status == 3
+
+
 def test_grouped_matmul_infer_shape_and_type():
     shapes, types = _C._graph_infer("grouped_matmul", _gmm_args())
     assert shapes == [[64, 128]] and types == [F16]          # the reference's float16 output
