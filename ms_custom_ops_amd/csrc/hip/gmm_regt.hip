@@ -9,7 +9,7 @@
 //   int8 x    v_mfma_i32_16x16x64_i8, KR = 16.  Four rows of a word are transposed as bytes (8 v_perm per 16 bytes).  8-bit
 //             weights: that is the operand.  4-bit weights: a byte holds an even and an odd column, and both become int8
 //             operands of 16 times their value ((c << 4) & 0xF0.., c & 0xF0..): 20 instructions per 32 weights, nothing to
-//             sign-extend, and the int32 sums are exactly 16 times the true ones (K x 2^14 < 2^31 is checked by the plan).
+//             sign-extend, and the int32 sums are exactly 16 times the true ones (K x 2^14 < 2^31 is checked by the plan, for this form alone).
 //   16-bit x  v_mfma_f32_16x16x32, KR = 8.  A signed byte of two rows each goes through v_cvt_f32_i32 (byte select) and
 //             one pack: exact in bf16 and f16.  4-bit weights enter as 16 times their value (the same masks as above):
 //             every product and every rounding is 16 times the one 8-bit weights of the same value give, so with the
@@ -132,7 +132,7 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
     for (int t = 0; t < L; ++t)
       xbuf[B][t] = __builtin_amdgcn_raw_buffer_load_b128(rx, ok ? x_lane[t] : kBufferOob, (unsigned)(step * S::kStep * SX), 0);
 #pragma unroll
-    for (int i = 0; i < KR; ++i) load_words<DW>(wbuf[B][i], rw, wo, (unsigned)((step * S::kStep + i) * pitch));
+    for (int i = 0; i < KR; ++i) load_words<DW>(wbuf[B][i], rw, wo, (unsigned)(step * S::kStep + i) * (unsigned)pitch);
   };
   auto multiply = [&](auto b_c) {
     constexpr int B = decltype(b_c)::value;

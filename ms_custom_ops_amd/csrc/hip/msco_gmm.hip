@@ -154,10 +154,14 @@ void plan_regt(msco_gmm_op *op) {
   const msco_gmm_desc &d = op->desc;
   const int64_t m = op->m, k = op->k, n = op->n, e = op->e;
   const int bits = is_w4(d) ? 4 : 8;
-  const bool can = layout_of(d) == 0 && k % 16 == 0 && n % 16 == 0 && k < ((int64_t)1 << 17) && k * n * bits / 8 < ((int64_t)1 << 31) &&
-                   m * k < ((int64_t)1 << 31);
   // rows a group is expected to hold (shapes only); real routings are uneven, hence 1.5 x the average
   const int64_t avg = (m + e - 1) / e, rows = e == 1 ? m : avg + avg / 2;
+  const int blocks = bits == 8 || rows <= 16 ? 1 : 2;
+  // int8 x on 4-bit weights: int32 sums of 16 times the products, K x 2^14 < 2^31.  16-bit x is summed in float32, whatever K.
+  // A chunk's x rows and a group's weights are addressed through 32-bit offsets.
+  const bool sums_fit = !(is_w8a8(d) && bits == 4) || k < ((int64_t)1 << 17);
+  const bool can = layout_of(d) == 0 && k % 16 == 0 && n % 16 == 0 && sums_fit && k * n * bits / 8 < ((int64_t)1 << 31) &&
+                   m * k < ((int64_t)1 << 31) && std::min<int64_t>(m, 16 * blocks) * k * (is_w8a8(d) ? 1 : 2) < ((int64_t)1 << 31);
   // 4-bit weights with 16-bit x: widening them first (8 experts, K = 4096, N = 14336: 120 us for the widening alone) costs
   // more than a second and third pass over the nibbles (4 / 32 rows per group: 47 / 95 us in all).
   // Weight-only on 8-bit weights, one 16-row chunk per group: the decode form.
@@ -194,7 +198,6 @@ void plan_regt(msco_gmm_op *op) {
     return;
   }
   if (can && want) {
-    const int blocks = bits == 8 || rows <= 16 ? 1 : 2;
     GmmParams p{};
     p.m = (int)m;
     p.e = (int)e;

@@ -196,6 +196,15 @@ def test_4_bit_weights_come_in_pairs_of_columns():
         assert e.value.status == 3
 
 
+def test_long_k_keeps_the_weight_only_decode_kernel():
+    # the int32 sums of int8 x on 4-bit weights bound K; float32 sums do not, nor do int32 sums of 8-bit weights
+    for k in (131056, 131072, 1 << 20):
+        for bits in (8, 4):
+            assert "skinny_regt" in _plan(1, k, 64, 1, "bf16", bits, force_split_k=1)[1], (k, bits)
+    assert "regt" in _plan(1, 131056, 64, 1, "i8", 4, force_split_k=1)[1]
+    assert "widened" in _plan(1, 131072, 131072 // 16, 1, "i8", 4, override=cabi.OV_GENERIC)[1]
+
+
 def test_grouped_matmul_infer_shape_and_type():
     shapes, types = _C._graph_infer("grouped_matmul", _gmm_args())
     assert shapes == [[64, 128]] and types == [F16]          # the reference's float16 output

@@ -90,3 +90,23 @@ def test_16_bit_activations_within_one_rounding_and_equal_for_both_weight_widths
     avg = -(-(rows + 2) // e)
     if (avg if e == 1 else avg + avg // 2) <= 16:   # chunks of 16 rows for both widths: the same order of summation
         assert np.array_equal(got, run(4, w))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_16_bit_activations_long_k_exact(device, dtype, bits):
+    """K beyond 2^17 and beyond what int32 sums of 16 times the products could hold.  x is -1, 0 or 1, so every float32 partial sum
+    is exact (|sum| <= 127 K < 2^24; 4-bit weights: multiples of 16 below 2^28) and the output is two roundings of it: the same bits."""
+    rng = np.random.default_rng(bits)
+    k, n, counts = 131088, 48, [2, 1]
+    xv = rng.integers(-1, 2, (5, k)).astype(np.float32)
+    x = O.f32_to_bf16_bits(xv) if dtype == "bf16" else xv.astype(np.float16).view(np.uint16)
+    w = np.maximum(_weights(rng, bits, 2, k, n), -127)
+    sv = (2.0 ** rng.integers(-8, -4, (2, n))).astype(np.float32) if dtype == "bf16" else np.full((2, n), 2.0 ** -10, np.float32)
+    s = O.f32_to_bf16_bits(sv) if dtype == "bf16" else sv.astype(np.float16).view(np.uint16)
+    dt = cabi.DT_BF16 if dtype == "bf16" else cabi.DT_F16
+    got = _run(dt, bits, x, w, counts, 0, {cabi.IN_ANTIQUANT_SCALE: to_dev(s)}, dt, antiquant_dtype=dt).view(np.uint16)
+    acc = np.concatenate([xv[:2].astype(np.int64) @ w[0].astype(np.int64), xv[2:3].astype(np.int64) @ w[1].astype(np.int64)])
+    want = acc.astype(np.float32) * np.repeat(sv, counts, axis=0)
+    assert np.array_equal(got[:3], O.f32_to_bf16_bits(want) if dtype == "bf16" else want.astype(np.float16).view(np.uint16))
+    assert (got[3:] == 0x7FC0).all()
