@@ -202,7 +202,9 @@ void plan_regt(msco_gmm_op *op) {
     p.m = (int)m;
     p.e = (int)e;
     const int64_t slots = chunk_slots(p, 16 * blocks);
-    const int64_t active = std::max<int64_t>(1, std::min<int64_t>(slots, std::min<int64_t>(m, e)));
+    // chunks expected to hold rows (an average group's, not one per group: 8 experts, 40 rows each, K = N = 4096, 4-bit weights: a K
+    // split for 16 chunks instead of 8 and 45.3 -> 37.0 us)
+    const int64_t active = std::max<int64_t>(1, std::min<int64_t>(slots, std::min<int64_t>(m, e) * ((avg + 16 * blocks - 1) / (16 * blocks))));
     const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
     // Strips of 512 columns (eight waves, twice as many neighbouring bytes per K row) while they fill most of the CUs
     // without a K split, strips of 256 (four waves) otherwise.  8 experts, K = 4096, N = 14336, 4 rows per group, 4-bit
