@@ -73,8 +73,8 @@ hipError_t launch_pack_weight(const void *src, void *dst, long long e, long long
                               hipStream_t stream);
 
 // Row-major [E,K,N] weights of 4 or 8 bits transposed and converted in registers (gmm_regt.hip): chunks of 16 row_blocks rows
-// (1 or 2), strips of strip_cols columns (256 or 512), p.split_k slices of K
-hipError_t launch_regt(const GmmParams &p, int weight_bits, int row_blocks, int strip_cols, hipStream_t stream);
+// (1 or 2), strips of strip_cols columns (256 or 512), p.split_k slices of K; shallow (16-bit x on 8-bit weights): more workgroups per CU
+hipError_t launch_regt(const GmmParams &p, int weight_bits, int row_blocks, int strip_cols, bool shallow, hipStream_t stream);
 size_t regt_slice_bytes(int row_blocks, int strip_cols);   // workspace bytes of one (chunk, strip, K slice) partial tile
 // 4-bit values widened to int8 (gmm_w4.hip)
 hipError_t launch_unpack_int4(const void *src, void *dst, long long src_bytes, hipStream_t stream);

@@ -26,6 +26,11 @@
 // workgroups.  With the slices slowest these empty ones stood between the slices, and CUs that had got one were passed over
 // for the next slice while others took two of it (weight-only, 8 x 4 rows, K = 8192, N = 4096, two slices on 256 CUs: 69.3 -> 49.2 us;
 // 4-bit weights, 8 x 8 rows, K = N = 4096: 32.0 -> 21.5 us).
+//
+// SHALLOW (16-bit x, 8-bit weights): one K step in flight per wave and four waves per SIMD in place of three steps and two
+// waves.  Where a CU gets several workgroups, one's ends (first requests, reduction, stores) lie under the other's walk: 64
+// experts, N = 4096, 8 rows per group, K = 512 / 1024: 38.3 -> 29.2, 55.9 -> 48.9 us; 8 experts, K = 4096, N = 14336, 4 rows: 76.1 -> 74.6
+// us.  With one workgroup per CU or less it has too few requests in flight (one row, K = 4096, N = 11008: 16.4 -> 17.8 us).
 #include <type_traits>
 
 #include "gmm_common.h"
@@ -86,14 +91,14 @@ __device__ __forceinline__ void rt_mfma(v4f &acc, const v4i &a, const v4i &b) {
 }  // namespace
 
 // L = 16-row blocks of the chunk that hold rows
-template <int XT, int WB, int R, int CPL, int WN, int L>
+template <int XT, int WB, int R, int CPL, int WN, bool SHALLOW, int L>
 __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem, int grp, int m0, int chunk_rows) {
   using S = RtShape<XT, WB, R, CPL, WN>;
   using Acc = std::conditional_t<XT == DT_I8, v4i, v4f>;
   using Elem = std::conditional_t<XT == DT_I8, int, float>;
   constexpr int WK = S::kWk, KR = S::kKr, DW = S::kDw, SX = XT == DT_I8 ? 1 : 2;
   constexpr bool FP = XT != DT_I8, BF16 = XT == DT_BF16;
-  constexpr int NB = FP ? (R == 1 && WB == 4 ? 4 : 3) : 2;   // steps in flight per wave, the one being multiplied included
+  constexpr int NB = SHALLOW ? 1 : FP ? (R == 1 && WB == 4 ? 4 : 3) : 2;   // steps in flight per wave, the one being multiplied included
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -355,8 +360,8 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
   }
 }
 
-template <int XT, int WB, int R, int CPL, int WN>
-__global__ void __launch_bounds__(64 * WN * CPL / 4, 2) gmm_regt_kernel(const GmmParams p) {
+template <int XT, int WB, int R, int CPL, int WN, bool SHALLOW>
+__global__ void __launch_bounds__(64 * WN * CPL / 4, SHALLOW ? 4 : 2) gmm_regt_kernel(const GmmParams p) {
   extern __shared__ __align__(16) unsigned char rt_smem[];
   const int lane = threadIdx.x & 63;
   // (grid.z enumerates the chunks that hold rows, group after group: a slot past the last one has nothing to do)
@@ -369,17 +374,17 @@ __global__ void __launch_bounds__(64 * WN * CPL / 4, 2) gmm_regt_kernel(const Gm
   static_for<R>([&](auto i_c) {   // one copy of the loop per number of live row blocks
     constexpr int L = decltype(i_c)::value + 1;
     if (!done && live <= L) {
-      regt_run<XT, WB, R, CPL, WN, L>(p, rt_smem, grp, m0, chunk_rows);
+      regt_run<XT, WB, R, CPL, WN, SHALLOW, L>(p, rt_smem, grp, m0, chunk_rows);
       done = true;
     }
   });
 }
 
 namespace {
-template <int XT, int WB, int R, int CPL, int WN>
+template <int XT, int WB, int R, int CPL, int WN, bool SHALLOW = false>
 hipError_t regt_launch(const GmmParams &p, hipStream_t stream) {
   using S = RtShape<XT, WB, R, CPL, WN>;
-  auto kern = gmm_regt_kernel<XT, WB, R, CPL, WN>;
+  auto kern = gmm_regt_kernel<XT, WB, R, CPL, WN, SHALLOW>;
   static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race between first launches repeats it at worst
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLds);
@@ -393,35 +398,41 @@ hipError_t regt_launch(const GmmParams &p, hipStream_t stream) {
   return hipGetLastError();
 }
 template <int XT, int WB, int WN>
-hipError_t regt_dispatch(const GmmParams &p, int row_blocks, hipStream_t stream) {
-  if (row_blocks == 1) return regt_launch<XT, WB, 1, 16, WN>(p, stream);
+hipError_t regt_dispatch(const GmmParams &p, int row_blocks, bool shallow, hipStream_t stream) {
+  if constexpr (XT != DT_I8 && WB == 8) {
+    if (row_blocks == 1 && shallow) return regt_launch<XT, WB, 1, 16, WN, true>(p, stream);
+  }
+  if (shallow) return hipErrorInvalidValue;
+  if constexpr (XT == DT_I8 || WB == 4 || WN == 1) {   // (16-bit x on 8-bit weights: strips of 512 columns are always shallow)
+    if (row_blocks == 1) return regt_launch<XT, WB, 1, 16, WN>(p, stream);
+  }
   if constexpr (WB == 4) {   // (8-bit weights of more than 16 rows per group have LDS kernels of their own)
     if (row_blocks == 2) return regt_launch<XT, WB, 2, 16, WN>(p, stream);
   }
   return hipErrorInvalidValue;
 }
 template <int XT, int WB>
-hipError_t regt_by_strip(const GmmParams &p, int row_blocks, int strip_cols, hipStream_t stream) {
-  if (strip_cols == 256) return regt_dispatch<XT, WB, 1>(p, row_blocks, stream);
-  if (strip_cols == 512) return regt_dispatch<XT, WB, 2>(p, row_blocks, stream);
+hipError_t regt_by_strip(const GmmParams &p, int row_blocks, int strip_cols, bool shallow, hipStream_t stream) {
+  if (strip_cols == 256) return regt_dispatch<XT, WB, 1>(p, row_blocks, shallow, stream);
+  if (strip_cols == 512) return regt_dispatch<XT, WB, 2>(p, row_blocks, shallow, stream);
   return hipErrorInvalidValue;
 }
 }  // namespace
 
 size_t regt_slice_bytes(int row_blocks, int strip_cols) { return (size_t)row_blocks * (16 * strip_cols / 2 + 8) * 8; }
 
-// row_blocks = 16-row blocks per chunk (1 or 2), strip_cols = columns per strip (256 or 512)
-hipError_t launch_regt(const GmmParams &p, int weight_bits, int row_blocks, int strip_cols, hipStream_t stream) {
+// row_blocks = 16-row blocks per chunk (1 or 2), strip_cols = columns per strip (256 or 512), shallow: 16-bit x on 8-bit weights only
+hipError_t launch_regt(const GmmParams &p, int weight_bits, int row_blocks, int strip_cols, bool shallow, hipStream_t stream) {
   if (p.m == 0) return hipSuccess;
   if (p.k % 16 != 0 || p.n % 16 != 0) return hipErrorInvalidValue;
   if (weight_bits == 4) {
-    if (p.x_dtype == DT_I8) return regt_by_strip<DT_I8, 4>(p, row_blocks, strip_cols, stream);
-    if (p.x_dtype == DT_BF16) return regt_by_strip<DT_BF16, 4>(p, row_blocks, strip_cols, stream);
-    return regt_by_strip<DT_F16, 4>(p, row_blocks, strip_cols, stream);
+    if (p.x_dtype == DT_I8) return regt_by_strip<DT_I8, 4>(p, row_blocks, strip_cols, shallow, stream);
+    if (p.x_dtype == DT_BF16) return regt_by_strip<DT_BF16, 4>(p, row_blocks, strip_cols, shallow, stream);
+    return regt_by_strip<DT_F16, 4>(p, row_blocks, strip_cols, shallow, stream);
   }
-  if (p.x_dtype == DT_I8) return regt_by_strip<DT_I8, 8>(p, row_blocks, strip_cols, stream);
-  if (p.x_dtype == DT_BF16) return regt_by_strip<DT_BF16, 8>(p, row_blocks, strip_cols, stream);
-  return regt_by_strip<DT_F16, 8>(p, row_blocks, strip_cols, stream);
+  if (p.x_dtype == DT_I8) return regt_by_strip<DT_I8, 8>(p, row_blocks, strip_cols, shallow, stream);
+  if (p.x_dtype == DT_BF16) return regt_by_strip<DT_BF16, 8>(p, row_blocks, strip_cols, shallow, stream);
+  return regt_by_strip<DT_F16, 8>(p, row_blocks, strip_cols, shallow, stream);
 }
 
 }  // namespace msco

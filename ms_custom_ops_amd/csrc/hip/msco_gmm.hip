@@ -94,6 +94,7 @@ struct msco_gmm_op {
   int small_group_rows = 0;  // > 0: the persistent kernel takes the groups with more rows, a second launch of 64 x 128 tiles the others
   int row_blocks = 1;        // register-transpose kernels: 16-row blocks per chunk
   int strip_cols = 256;      // ... and columns per strip
+  bool shallow = false;      // ... and the form with one K step in flight per wave (several workgroups per CU)
   int64_t widen_bytes = 0;   // 4-bit weights without a kernel of their own for the shape: int8 copy of them at the front of the workspace
   size_t workspace_bytes = 0;
   unsigned *counters = nullptr;
@@ -208,8 +209,7 @@ void plan_regt(msco_gmm_op *op) {
     const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
     // Strips of 512 columns (eight waves, twice as many neighbouring bytes per K row) while they fill most of the CUs
     // without a K split, strips of 256 (four waves) otherwise.  8 experts, K = 4096, N = 14336, 4 rows per group, 4-bit
-    // weights: 44 against 51 us (int8 x), 47 against 52 us (bf16); 8-bit weights 79 against 82 us.  One group, N = 11008:
-    // 20 against 17 us.
+    // weights: 44 against 51 us (int8 x), 47 against 52 us (bf16).  One group, N = 11008: 20 against 17 us.
     int64_t cols = ((n + 511) / 512) * active * 4 >= cus * 3 ? 512 : 256;
     if (tuning().regt_cols > 0) cols = tuning().regt_cols;
     const int64_t strips = (n + cols - 1) / cols;
@@ -233,6 +233,11 @@ void plan_regt(msco_gmm_op *op) {
       while (split > 1 && tile * split > kTileSplitMaxWorkspace) --split;
       op->split_k = (int)split;
       op->workspace_bytes = op->split_k > 1 ? tile * op->split_k : 0;
+      // One K step in flight per wave and twice the waves where CUs get more than one workgroup: strips of 512 columns (8
+      // experts, K = 512, N = 14336, 8 rows per group, 224 workgroups: 18.2 -> 15.7 us) and 256 workgroups of 256 (64 experts, K = 4096,
+      // N = 1024: 50.9 -> 47.1 us; 8 experts, K = N = 4096, two slices: 31.1 -> 30.2 us); below that three steps (176 workgroups, 8
+      // experts, K = 4096, N = 5632: 35.5 against 42.6 us; 224, N = 7168: 43.2 against 44.3 us).
+      op->shallow = bits == 8 && is_a16w8(d) && (cols == 512 || strips * active * split >= cus);
       return;
     }
   }
@@ -288,6 +293,7 @@ void choose_plan(msco_gmm_op *op) {
   op->wide_k_slabs = 0;
   op->w_nontemporal = 0;
   op->small_group_rows = 0;
+  op->shallow = false;
 
   int family;
   // All three W8A8 weight layouts follow the same tile rules: packed weights are K-contiguous per column like [E,N,K],
@@ -657,7 +663,7 @@ void choose_plan(msco_gmm_op *op) {
 
   family = op->family;
   char buf[320];
-  const char *fam = family == FAM_REGT ? "skinny_regt" : family == FAM_ROWS16 ? "rows128" : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
+  const char *fam = family == FAM_REGT ? (op->shallow ? "skinny_regt_shallow" : "skinny_regt") : family == FAM_ROWS16 ? "rows128" : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
   std::snprintf(buf, sizeof(buf),
                 "msco_gmm plan: kernel=%s%s%s%s layout=%s m=%lld k=%lld n=%lld e=%lld split_k=%d strips=%d "
                 "workspace=%zu%s",
@@ -825,7 +831,7 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   const bool nk = d.transpose_b != 0;
   const int layout = layout_of(d);
   if (h->family == FAM_REGT) {
-    err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, s);
+    err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, h->shallow, s);
   } else if (h->family == FAM_ROWS16) {
     err = launch_rows_a16w8(p, layout == 2, s);
   } else if (is_w8a8(d)) {

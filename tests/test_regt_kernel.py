@@ -16,14 +16,14 @@ SHAPES = [([1], 16, 16, 0), ([16, 0, 17], 48, 256, 0), ([3, 33, 1], 2064, 272, 3
           ([0, 0, 64, 7], 96, 1040, 2), ([2] * 70, 64, 48, 0)]
 
 
-def _run(x_dtype, bits, x, w, counts, split, operands, out_dtype, override=cabi.OV_REGT, **fields):
+def _run(x_dtype, bits, x, w, counts, split, operands, out_dtype, override=cabi.OV_REGT, must="", **fields):
     m, (e, k, n) = x.shape[0], w.shape
     wd = to_dev(O.pack_int4(w) if bits == 4 else w)
     gl = to_dev(np.asarray(counts, dtype=np.int64))
     op = cabi.GmmOp(x_dtype=x_dtype, weight_dtype=cabi.DT_I4 if bits == 4 else cabi.DT_I8, out_dtype=out_dtype, group_list_dtype=cabi.DT_I64,
                     group_list_type=1, kernel_override=override, force_split_k=split, **fields)
     ws = op.plan(m, k, n, e)
-    assert {cabi.OV_REGT: "regt", cabi.OV_TILE_4BIT: "4bit"}[override] in op.plan_info(), op.plan_info()
+    assert {cabi.OV_AUTO: must, cabi.OV_REGT: "regt", cabi.OV_TILE_4BIT: "4bit"}[override] in op.plan_info(), op.plan_info()
     tws = torch.empty(max(ws, 1), dtype=torch.uint8, device="cuda:0")
     out = torch.full((m, n), 0x7FC0, dtype=torch.int32 if out_dtype == cabi.DT_I32 else torch.int16, device="cuda:0")
     tx = to_dev(x)
@@ -110,3 +110,32 @@ def test_16_bit_activations_long_k_exact(device, dtype, bits):
     want = acc.astype(np.float32) * np.repeat(sv, counts, axis=0)
     assert np.array_equal(got[:3], O.f32_to_bf16_bits(want) if dtype == "bf16" else want.astype(np.float16).view(np.uint16))
     assert (got[3:] == 0x7FC0).all()
+
+
+# (rows per group, K, N, what the plan names): the form with one K step in flight per wave, planned from 256 workgroups on, in
+# strips of 256 columns without and with a K split and in strips of 512; groups of up to 17 rows, the last strip cut at 16 columns
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("counts,k,n,must", [([1, 16, 0, 17, 3, 2, 0, 1] * 4, 80, 2320, "split_k=1 strips=10 "), ([3, 0, 1, 2] * 8, 2064, 784, "split_k=2 strips=4 "),
+                                             ([1, 16, 0, 17, 3, 2, 0, 1] * 4, 48, 3600, "split_k=1 strips=8 "), ([1] * 32, 16, 3072 + 16, "split_k=1 strips=7 ")])
+def test_shallow_form_within_one_rounding(device, counts, k, n, must, dtype):
+    """Tolerance as above; the same values given as 4-bit weights take the other form and give the same bits."""
+    rng = np.random.default_rng(k + n)
+    e, rows = len(counts), sum(counts)
+    to_bits = O.f32_to_bf16_bits if dtype == "bf16" else (lambda a: a.astype(np.float16).view(np.uint16))
+    to_f = O.bf16_bits_to_f32 if dtype == "bf16" else (lambda b: b.view(np.float16).astype(np.float32))
+    x = to_bits(rng.standard_normal((rows + 2, k)).astype(np.float32))
+    s = to_bits(rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32))
+    o = to_bits(rng.integers(-8, 9, (e, n)).astype(np.float32))
+    dt = cabi.DT_BF16 if dtype == "bf16" else cabi.DT_F16
+    ops = {cabi.IN_ANTIQUANT_SCALE: to_dev(s), cabi.IN_ANTIQUANT_OFFSET: to_dev(o)}
+    run = lambda bits, w, name: _run(dt, bits, x, w, counts, 0, ops, dt, cabi.OV_AUTO, name, antiquant_dtype=dt, has_antiquant_offset=1).view(np.uint16)
+    ends, starts = np.cumsum(counts), np.cumsum(counts) - counts
+    for bits in (8, 4):
+        w = _weights(rng, bits, e, k, n)
+        got = run(8, w, "regt_shallow layout=[E,K,N] m=%d k=%d n=%d e=%d %s" % (rows + 2, k, n, e, must))
+        exact = O.a16w8_grouped_f64(to_f(x), w, to_f(s), to_f(o), ends)[:rows]
+        mag = np.concatenate([np.abs(to_f(x)[a:b]) @ (np.abs(w[g].astype(np.float64) + to_f(o)[g]) * to_f(s)[g]) for g, (a, b) in enumerate(zip(starts, ends))])
+        ulp = 2.0 ** -7 if dtype == "bf16" else 2.0 ** -10
+        assert (np.abs(to_f(got[:rows]).astype(np.float64) - exact) <= ulp * np.abs(exact) + 1e-5 * mag).all()
+        assert (got[rows:] == 0x7FC0).all()
+    assert np.array_equal(got, run(4, w, "skinny_regt "))
