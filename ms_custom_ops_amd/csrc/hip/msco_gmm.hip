@@ -171,7 +171,15 @@ void plan_regt(msco_gmm_op *op) {
                     (op->family == FAM_SKINNY && bits == 8 && is_a16w8(d) && op->stream_tch == 1);
   // 4-bit weights, int8 x, more than one 16-row chunk per group: tiles that read the nibbles through LDS (4 / 16 / 32 rows
   // per group 52 / 53 / 58 us against 44 / 53 / 82 us in 32-row chunks)
-  if (can && bits == 4 && is_w8a8(d) && (d.kernel_override == OV_TILE_4BIT || (d.kernel_override == OV_AUTO && rows > 16))) {
+  // ... up to some two thousand rows per group, where the persistent kernel, a sixth to an eighth faster, makes up for widening
+  // the weights first (3 us and 1 us per 3.9 M weights) by the time that is 11.6 % of the products (2.2 Pop/s).  4-bit tiles
+  // against widening, us: 8 experts, K = 4096, N = 14336, 2048 / 3072 / 4096 rows per group 920 / 1367 / 1800 against 937 / 1321 / 1712;
+  // one group, N = 11008, 2048 / 3072 / 16384 rows 101 / 152 / 674 against 101 / 144 / 590; K = N = 4096, 4096 / 8192 rows 66 / 126 against
+  // 67 / 114; 16 experts, 2048 x 2816, 1792 / 4096 rows 194 / 407 against 204 / 388.  The line is not sharp: 128 experts, 2048 x 768,
+  // 2048 rows (14.6 %) 502 against 475, 32 experts, 4096 x 1024, 2048 rows (14.9 %) 297 against 310.
+  const bool widen_pays = d.kernel_override == OV_AUTO && op->family == FAM_TILE && op->tile_cfg == TILE_256x256_W4 &&
+                          3.0 + (double)(e * k * n) / 3.9e6 <= 0.116 * 2.0 * (double)(m * k) * (double)n / 2.2e9;
+  if (can && bits == 4 && is_w8a8(d) && (d.kernel_override == OV_TILE_4BIT || (d.kernel_override == OV_AUTO && rows > 16 && !widen_pays))) {
     const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, groups = std::max<int64_t>(1, std::min<int64_t>(e, m)), n_tiles = (n + 255) / 256;
     // 128-row tiles once 64 rows no longer hold a group and there are tiles for most CUs (64 / 128 rows per group 83 / 114 us
     // with 64-row tiles, 68 / 106 us with 128; one group of 256 rows, N = 11008: 31.7 against 42.7 us)

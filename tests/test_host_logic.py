@@ -205,6 +205,15 @@ def test_long_k_keeps_the_weight_only_decode_kernel():
     assert "widened" in _plan(1, 131072, 131072 // 16, 1, "i8", 4, override=cabi.OV_GENERIC)[1]
 
 
+def test_large_a8w4_calls_widen_in_front_of_the_persistent_kernel():
+    for m, k, n, e, widened in ((16384, 4096, 14336, 8, False), (32768, 4096, 14336, 8, True), (2048, 4096, 11008, 1, False), (16384, 4096, 11008, 1, True),
+                                (8192, 1024, 1024, 1, False), (32768, 4096, 11008, 16, False)):
+        ws, info = _plan(m, k, n, e, bits=4)
+        assert ("a8w4_widened_tile_256x256x128_w4" if widened else "4bit") in info, info
+        assert ws == (e * k * n if widened else 0)
+    assert "4bit" in _plan(32768, 4096, 14336, 8, bits=4, override=cabi.OV_TILE_4BIT)[1]
+
+
 def test_grouped_matmul_infer_shape_and_type():
     shapes, types = _C._graph_infer("grouped_matmul", _gmm_args())
     assert shapes == [[64, 128]] and types == [F16]          # the reference's float16 output

@@ -139,3 +139,22 @@ def test_shallow_form_within_one_rounding(device, counts, k, n, must, dtype):
         assert (np.abs(to_f(got[:rows]).astype(np.float64) - exact) <= ulp * np.abs(exact) + 1e-5 * mag).all()
         assert (got[rows:] == 0x7FC0).all()
     assert np.array_equal(got, run(4, w, "skinny_regt "))
+
+
+def test_large_a8w4_call_widens_first(device):
+    """A call large enough for the persistent kernel: the int8 copy at the front of the workspace gives the bits that int8
+    weights of the same values give, and those of the oracle on the first and last rows of every group."""
+    rng = np.random.default_rng(0)
+    counts, k, n = [40000, 26001], 512, 1040
+    e, rows = len(counts), sum(counts)
+    x, w = rng.integers(-128, 128, (rows + 2, k), dtype=np.int8), _weights(rng, 4, e, k, n)
+    scale = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32)
+    ops = {cabi.IN_SCALE: to_dev(scale)}
+    run = lambda bits, name: _run(cabi.DT_I8, bits, x, w, counts, 0, ops, cabi.DT_BF16, cabi.OV_AUTO, name, scale_dtype=cabi.DT_F32, scale_per_group=1)
+    got = run(4, "a8w4_widened_tile_256x256x128_w4")
+    assert np.array_equal(got, run(8, "w8a8_tile_256x256x128_w4"))
+    for g, (a, b) in enumerate(((0, 40000), (40000, rows))):
+        pick = np.r_[a:a + 8, b - 8:b]
+        want = O.grouped_matmul_w8a8(x[pick], w[g:g + 1], np.array([16]), None, scale[g:g + 1], None)
+        assert np.array_equal(got[pick].view(np.uint16), want)
+    assert (got[rows:] == 0x7FC0).all()
