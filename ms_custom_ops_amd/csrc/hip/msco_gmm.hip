@@ -371,20 +371,24 @@ void choose_plan(msco_gmm_op *op) {
     // (narrower strips for fewer columns do not pay: with one or two column groups per wave, strips of 6 / 3 column groups,
     // 8 experts, 1024 rows, K = 5120, N = 2688 / 1344: 55 / 40 us against 46 / 24 us for the 64 x 128 tiles)
     const bool rows_kernel_ok = is_packed(d) && e > 1 && k >= 1024 && ((n + 255) / 256) * std::min<int64_t>(e, m) >= num_cus;
-    // The 160-row form again where a group is two or three equal chunks that share its weights through the L2.  What it beats is the
-    // second 256-row m-tile of a group of just more than 256 rows (us, persistent -> this): 8 experts, K = 4096, N = 14336, 240 / 256 /
-    // 272 / 300 / 400 rows per group: 126 -> 141, 164 -> 141, 191 -> 155, 206 -> 159, 208 -> 208; 64 experts, K = 2048, N = 1408,
-    // 256 / 300 / 330 / 400 rows: 89 -> 79, 99 -> 90, 98 -> 111, 100 -> 122 (few columns, narrow strips); and 128 x 128 tiles where
-    // larger ones do not fill the chip but these workgroups do: 8 experts, K = 7168, N = 4096, 200 / 240 / 300 rows: 91 -> 69, 120 -> 74,
-    // 141 -> 80; 2 experts, K = 4096, N = 11008, 200 rows: 47 -> 38; 8 experts, 4096 x 2048, 200 rows (128 workgroups): 28 -> 38.
-    // Up to 340 rows: 8 experts, K = 2816, N = 5664, 330 / 400 / 450 rows 80 -> 73, 70 -> 77, 74 -> 81; 32 experts, K = 2048, N = 4608, 330 rows 148 -> 128;
-    // 16 experts, K = 2784, N = 7504, 480 rows 183 -> 190.
-    // Where 256-row tiles fill the chip the line is the one m-tile that holds an even group: up to 256 rows an even routing is faster there
-    // (240 rows: 126 against 141 us) and only an uneven one with 256 on average is not (164 against 141 us).
+    // The 160-row form again where a group is two or three equal chunks that share its weights through the L2.  All figures are
+    // routings by the top-2 of random logits (groups as uneven as real ones), us, former plan -> this.
+    //   257 .. 296 rows per group on average: the persistent kernel gives a group of just more than 256 rows a second 256-row
+    //   m-tile.  8 experts, K = 4096, N = 14336, 260 / 290 rows: 167 -> 149, 197 -> 160; 64 experts, 2048 x 1408, 260 / 275 / 290: 84 -> 79,
+    //   90 -> 82, 90 -> 89; 128 experts, 4096 x 1024, 270: 213 -> 188.
+    //   297 .. 340 (three chunks): 8 experts, 4096 x 14336, 300 / 335 rows: 205 -> 177, 199 -> 189; 2816 x 5664, 330: 80 -> 72; 16 experts,
+    //   4096 x 4096, 320: 112 -> 113; not beyond: 8 experts, 2816 x 5664, 400 rows 70 -> 77.
+    //   192 .. 256 where larger tiles than 128 x 128 do not fill the chip but these workgroups do: 8 experts, 7168 x 4096, 200 / 250
+    //   rows: 91 -> 73, 120 -> 79; 2816 x 4096, 200 / 250: 38 -> 33, 55 -> 37.  A short K needs the 250: 2048 x 4096, 210 / 250 rows 24.2 ->
+    //   28.8, 36.6 -> 33.9; 16 experts, 2048 x 2048, 230 / 250: 29.9 -> 33.8, 36.4 -> 35.4.
+    // Popularity falling as 1 / rank^0.6 and 1 / rank^1.2 in place of even: the first two bands lie between 0.90 and 1.14, the third
+    // between 1.0 and 1.5 times the former plan's speed; which it will be only the device knows.
+    // Where 256-row tiles fill the chip, 256 rows on average and fewer stay with them: even groups of 240 rows, one m-tile each, take
+    // 126 us there (8 experts, 4096 x 14336) and 141 us here; random routings of 256 rows on average 158 and 147 us.
     const int64_t row_wgs = ((n + 255) / 256) * std::min<int64_t>(e, m) * ((avg_rows + avg_rows / 20 + 159) / 160);
     const bool rows_chunks_ok = is_packed(d) && e > 1 && k >= 2048 &&
                                 ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172) || (avg_rows > 296 && avg_rows <= 340 && n >= 4096 && row_wgs >= 256) ||
-                                 (avg_rows >= 192 && avg_rows <= 256 && n >= 2048 && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));
+                                 (avg_rows >= 192 && avg_rows <= 256 && n >= 2048 && (k >= 2816 || avg_rows >= 250) && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));
     if (rows_kernel_ok && avg_rows <= 116) {
       op->tile_cfg = TILE_ROWS128;
     } else if (rows_kernel_ok && avg_rows <= 146) {

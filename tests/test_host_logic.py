@@ -214,6 +214,12 @@ def test_large_a8w4_calls_widen_in_front_of_the_persistent_kernel():
     assert "4bit" in _plan(32768, 4096, 14336, 8, bits=4, override=cabi.OV_TILE_4BIT)[1]
 
 
+def test_chunks_of_200_rows_need_a_long_k():
+    for m, k, n, e, chunks in ((8 * 210, 2048, 4096, 8, False), (16 * 200, 2048, 2048, 16, False), (16 * 230, 2048, 2048, 16, False),
+                               (8 * 250, 2048, 4096, 8, True), (8 * 200, 2816, 4096, 8, True), (8 * 200, 7168, 4096, 8, True)):
+        assert ("rows160" in _plan(m, k, n, e, packed=True)[1]) == chunks, (m, k, n, e)
+
+
 def test_grouped_matmul_infer_shape_and_type():
     shapes, types = _C._graph_infer("grouped_matmul", _gmm_args())
     assert shapes == [[64, 128]] and types == [F16]          # the reference's float16 output
