@@ -326,10 +326,11 @@ __global__ void __launch_bounds__(XA_THREADS, 2) gmm_a16w8_rows128_kernel(const 
   });
 }
 
-// packed or [E,K,N] weights; K % 16 == 0, N % 16 == 0, 2 M K and one group's weights below 2^31 bytes
+// packed or [E,K,N] weights; K % 16 == 0, N % 16 == 0, K < 2^22 (an out-of-range mark plus the offset of a chunk's last row, 256 K
+// bytes, stays a 32-bit offset out of range) and one group's weights below 2^31 bytes; M is not bounded by offsets
 hipError_t launch_rows_a16w8(const GmmParams &p_in, bool packed, hipStream_t stream) {
   if (p_in.m == 0) return hipSuccess;
-  if (p_in.k % 16 != 0 || p_in.n % 16 != 0 || p_in.split_k != 1) return hipErrorInvalidValue;
+  if (p_in.k % 16 != 0 || p_in.n % 16 != 0 || p_in.k >= (1 << 22) || p_in.split_k != 1) return hipErrorInvalidValue;
   GmmParams p = p_in;
   p.n_strips = (p.n + XA_COLS - 1) / XA_COLS;
   const long long grid = xcd_slots(p, XA_ROWS);
