@@ -42,6 +42,7 @@ namespace {
 typedef long long i64;
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+typedef unsigned short v8us __attribute__((ext_vector_type(8), aligned(2)));   // antiquant rows may start at any element
 
 template <int XT, int WB, int R, int CPL, int WN>
 struct RtShape {
@@ -244,13 +245,12 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
     float f[8];
     if constexpr (FP) {
       const long long at = ((long long)grp * p.n + n) * 2;
-      const uint4 sw = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p.aq_scale) + at);
-      uint4 ow = make_uint4(0, 0, 0, 0);
-      if (p.aq_offset) ow = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p.aq_offset) + at);
-      const unsigned s4[4] = {sw.x, sw.y, sw.z, sw.w}, o4[4] = {ow.x, ow.y, ow.z, ow.w};
+      const v8us s8 = *reinterpret_cast<const v8us *>(static_cast<const char *>(p.aq_scale) + at);
+      v8us o8 = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (p.aq_offset) o8 = *reinterpret_cast<const v8us *>(static_cast<const char *>(p.aq_offset) + at);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const unsigned short sb = (unsigned short)(s4[j >> 1] >> (16 * (j & 1))), ob = (unsigned short)(o4[j >> 1] >> (16 * (j & 1)));
+        const unsigned short sb = s8[j], ob = o8[j];
         const float sc = BF16 ? bf16_bits_to_f32(sb) : f16_bits_to_f32(sb);
         const float of = BF16 ? bf16_bits_to_f32(ob) : f16_bits_to_f32(ob);
         f[j] = fmaf(of, xs, v[j] * (1.0f / (1 << shift))) * sc;

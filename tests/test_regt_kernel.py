@@ -158,3 +158,40 @@ def test_large_a8w4_call_widens_first(device):
         want = O.grouped_matmul_w8a8(x[pick], w[g:g + 1], np.array([16]), None, scale[g:g + 1], None)
         assert np.array_equal(got[pick].view(np.uint16), want)
     assert (got[rows:] == 0x7FC0).all()
+
+
+# (weight bits, override, groups x rows, what the plan names): register transpose with three and one K steps in flight, 4-bit weights,
+# the kernel of up to 128-row chunks
+@pytest.mark.parametrize("bits,override,counts,must", [(8, cabi.OV_AUTO, [5, 16], "skinny_regt layout"), (8, cabi.OV_AUTO, [3] * 40, "regt_shallow"),
+                                                       (4, cabi.OV_AUTO, [5, 16], "skinny_regt layout"), (8, cabi.OV_ROWS16, [100, 30], "rows128")])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_16_bit_operands_may_start_at_any_element(device, dtype, bits, override, counts, must):
+    """x, scale and offset one element behind a 16-byte boundary: the same bits as on one."""
+    rng = np.random.default_rng(bits)
+    e, m, k, n = len(counts), sum(counts), 80, 1808
+    dt, t16 = (cabi.DT_BF16, torch.bfloat16) if dtype == "bf16" else (cabi.DT_F16, torch.float16)
+    half = lambda a: torch.from_numpy(a.astype(np.float32)).cuda().to(t16)
+    x, s, o = half(rng.standard_normal((m, k))), half(rng.uniform(1e-3, 1e-2, (e, n))), half(rng.integers(-8, 9, (e, n)))
+    w = _weights(rng, bits, e, k, n)
+    wd, gl = to_dev(O.pack_int4(w) if bits == 4 else w), to_dev(np.asarray(counts, dtype=np.int64))
+
+    def shifted(t):
+        whole = torch.zeros(t.numel() + 16, dtype=t16, device="cuda")
+        assert whole.data_ptr() % 16 == 0
+        view = whole[1:1 + t.numel()].view(t.shape)
+        return view.copy_(t)
+
+    op = cabi.GmmOp(x_dtype=dt, weight_dtype=cabi.DT_I4 if bits == 4 else cabi.DT_I8, out_dtype=dt, group_list_dtype=cabi.DT_I64, group_list_type=1,
+                    antiquant_dtype=dt, has_antiquant_offset=1, kernel_override=override)
+    ws = op.plan(m, k, n, e)
+    assert must in op.plan_info(), op.plan_info()
+    tws = torch.empty(max(ws, 1), dtype=torch.uint8, device="cuda")
+    outs = []
+    for ins in ((x, s, o), (shifted(x), s, o), (x, shifted(s), shifted(o))):
+        out = torch.zeros((m, n), dtype=t16, device="cuda")
+        op.launch([ptr(ins[0]), ptr(wd), None, None, ptr(gl), None, ptr(ins[1]), ptr(ins[2])], out.data_ptr(), tws.data_ptr(), ws,
+                  torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        outs.append(out.view(torch.int16))
+    op.close()
+    assert outs[0].any() and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
