@@ -175,3 +175,27 @@ def test_act_type_errors():
         cabi.GmmOp(x_dtype=cabi.DT_I8, out_dtype=cabi.DT_I32, group_list_dtype=cabi.DT_I64, act_type=cabi.ACT_RELU)
     with pytest.raises(cabi.BackendError):
         cabi.GmmOp(x_dtype=cabi.DT_I8, out_dtype=cabi.DT_BF16, group_list_dtype=cabi.DT_I64, act_type=cabi.ACT_GELU_ERF)
+
+
+@pytest.mark.parametrize("act", ACTS)
+@pytest.mark.parametrize("packed", [False, True])
+def test_fused_activation_weight_only_128_row_chunks(act, packed):
+    """The kernel of up to 128-row chunks x 512 columns, ragged groups: bars as for the other weight-only kernels."""
+    from gpu_utils import run_a16w8
+    rng = np.random.default_rng(5)
+    m, k, n, e, gl = 333, 144, 528, 3, [129, 130, 333]
+    x_bits = O.f32_to_bf16_bits(rng.standard_normal((m, k)).astype(np.float32))
+    w = rng.integers(-127, 128, (e, k, n), dtype=np.int8)
+    s_bits = O.f32_to_bf16_bits(rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32))
+    o_bits = O.f32_to_bf16_bits(rng.integers(-8, 9, (e, n)).astype(np.float32))
+    plain, info = run_a16w8(x_bits, w, s_bits, o_bits, gl, packed=packed, override=cabi.OV_ROWS16)
+    bits, info = run_a16w8(x_bits, w, s_bits, o_bits, gl, packed=packed, override=cabi.OV_ROWS16, act_type=act)
+    assert "rows128" in info, info
+    xv, sv, ov = (O.bf16_bits_to_f32(b) for b in (x_bits, s_bits, o_bits))
+    exact = O.a16w8_grouped_f64(xv, w, sv, ov, gl)
+    mag = np.abs(xv).astype(np.float64).sum(1, keepdims=True) * 140.0 * float(np.abs(sv).max())
+    ref, got = O.activation(exact.astype(np.float32), act), O.bf16_bits_to_f32(bits).astype(np.float64)
+    assert (np.abs(got - ref) <= 2.0 ** -7 * np.abs(ref) + 1.13 * (2.0 ** -7 * np.abs(exact) + 1e-5 * mag) + 1e-30).all(), info
+    assert not np.array_equal(bits, plain)
+    if act == O.ACT_RELU:
+        assert np.array_equal(bits, np.where(O.bf16_bits_to_f32(plain) < 0, np.uint16(0), plain))

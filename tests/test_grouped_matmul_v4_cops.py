@@ -341,7 +341,7 @@ def test_v4_a16w4_reference_case(device, mode, dtype):
     assert w_int4.shape == (e, k, n // 2)
     x, s, o = _t(x_np.astype(np.float32), dtype), _t(s_np.astype(np.float32), dtype), _t(o_np.astype(np.float32), dtype)
     with ms_custom_ops.exec_mode(mode):
-        for _ in range(2):   # the second call reuses the graph-mode module and its staging slice
+        for _ in range(2):   # the second call reuses the graph-mode module and its workspace slice
             res = ms_custom_ops.grouped_matmul_v4_cops([x], [ms_custom_ops.as_qint4x2(_t(w_int4))], None, None, None, [s], [o],
                                                        None, _t(ends), None, None, None, 3, 0, 0)
             assert res[0].dtype == dtype and res[0].shape == (m, n)
@@ -362,7 +362,8 @@ def test_v4_a16w4_reference_case(device, mode, dtype):
 
 def test_v4_a16w4_signed_nibbles_ragged_groups_equal_the_a16w8_path(device):
     """Every 4-bit value (-8 .. 7), empty groups, rows behind the last boundary: the A16W4 result is bit for bit the a16w8
-    result on the same values given as int8 (the nibbles are widened, then the same kernels run), in both modes."""
+    result on the same values given as int8, in both modes (both widths take the register-transpose kernel, whose 4-bit operands are
+    16 times the values, a power of two)."""
     rng = np.random.default_rng(12)
     e, m, k, n = 8, 70, 192, 96
     w = rng.integers(-8, 8, (e, k, n), dtype=np.int8)
@@ -385,7 +386,8 @@ def test_v4_a16w4_signed_nibbles_ragged_groups_equal_the_a16w8_path(device):
 
 
 def test_widen_qint4x2_once_then_the_int8_paths(device):
-    """Weights widened at load time give the same bits as the op's per-call widening, for A8W4 and for A16W4."""
+    """Weights widened at load time give the same bits as the 4-bit ones, for A8W4 and for A16W4 (these few rows per group are
+    multiplied without widening; calls that widen: the test below)."""
     rng = np.random.default_rng(13)
     e, m, k, n = 4, 40, 128, 64
     w = rng.integers(-8, 8, (e, k, n), dtype=np.int8)
@@ -411,6 +413,34 @@ def test_widen_qint4x2_once_then_the_int8_paths(device):
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
     with pytest.raises(RuntimeError, match="GPU tensor"):
         ms_custom_ops.widen_qint4x2(packed.cpu())
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("x_type,counts,k,n", [("bf16", [150, 0, 90, 130], 192, 96), ("f16", [200], 2048, 256), ("i8", [3, 9], 88, 24)])
+def test_calls_that_widen_4_bit_weights_in_their_workspace(device, mode, x_type, counts, k, n):
+    """More rows per group than the kernels for 4-bit weights take (the second case splits K, its partial sums behind the int8
+    copy) and K or N that are no multiple of 16: the bits of the same call on int8 weights, twice in a row."""
+    from ms_custom_ops_amd import cabi
+    rng = np.random.default_rng(k)
+    e, m = len(counts), sum(counts)
+    w = rng.integers(-8, 8, (e, k, n), dtype=np.int8)
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "i8": torch.int8}[x_type]
+    i8 = dt == torch.int8
+    code = {"bf16": cabi.DT_BF16, "f16": cabi.DT_F16, "i8": cabi.DT_I8}[x_type]
+    op = cabi.GmmOp(x_dtype=code, weight_dtype=cabi.DT_I4, out_dtype=cabi.DT_BF16 if i8 else code, group_list_dtype=cabi.DT_I64, group_list_type=1,
+                    scale_per_group=1, **(dict(scale_dtype=cabi.DT_F32) if i8 else dict(antiquant_dtype=code)))
+    op.plan(m, k, n, e)
+    assert "widened" in op.plan_info() and ("split_k=1 " in op.plan_info()) == (e > 1), op.plan_info()
+    op.close()
+    x = _t(rng.integers(-128, 128, (m, k), dtype=np.int8)) if i8 else _t(rng.standard_normal((m, k)).astype(np.float32), dt)
+    s = _t(rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32)) if i8 else _t(rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), dt)
+    kw = dict(scale=[s], output_dtype=torch.bfloat16) if i8 else dict(antiquant_scale=[s])
+    f = ms_custom_ops.grouped_matmul_v4_cops
+    call = lambda wt: f([x], [wt], group_list=_t(np.array(counts, dtype=np.int64)), split_item=3, group_type=0, group_list_type=1, **kw)[0].view(torch.int16)
+    with ms_custom_ops.exec_mode(mode):
+        want = call(_t(w))
+        for _ in range(2):
+            assert torch.equal(call(ms_custom_ops.as_qint4x2(_t(O.pack_int4(w)))), want)
 
 
 def test_unpack_int4_through_the_c_abi(device):

@@ -24,6 +24,7 @@ def _run(x_dtype, bits, x, w, counts, split, operands, out_dtype, override=cabi.
                     group_list_type=1, kernel_override=override, force_split_k=split, **fields)
     ws = op.plan(m, k, n, e)
     assert {cabi.OV_AUTO: must, cabi.OV_REGT: "regt", cabi.OV_TILE_4BIT: "4bit"}[override] in op.plan_info(), op.plan_info()
+    assert must in op.plan_info(), op.plan_info()
     tws = torch.empty(max(ws, 1), dtype=torch.uint8, device="cuda:0")
     out = torch.full((m, n), 0x7FC0, dtype=torch.int32 if out_dtype == cabi.DT_I32 else torch.int16, device="cuda:0")
     tx = to_dev(x)
@@ -195,3 +196,73 @@ def test_16_bit_operands_may_start_at_any_element(device, dtype, bits, override,
         outs.append(out.view(torch.int16))
     op.close()
     assert outs[0].any() and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+# (x type, rows per group, K, N, forced K split, what the plan names)
+WIDENED = [("bf16", [100, 90], 192, 96, 0, "a16w4_widened_"), ("f16", [70, 0, 230], 2048, 1040, 0, "a16w4_widened_"),
+           ("bf16", [198], 2048, 272, 4, "a16w4_widened_skinny_rows layout=[E,K,N] m=200 k=2048 n=272 e=1 split_k=4"),
+           ("f16", [5, 6], 100, 24, 0, "a16w4_widened_generic"), ("i8", [5, 6], 100, 24, 0, "a8w4_widened_generic"),
+           ("i8", [3], 131072, 48, 8, "a8w4_widened_skinny")]
+
+
+@pytest.mark.parametrize("x_type,counts,k,n,split,must", WIDENED)
+def test_widened_by_the_backend_like_8_bit_weights(device, x_type, counts, k, n, split, must):
+    """4-bit weights that no kernel reads directly: an int8 copy at the front of the workspace, the partial tiles of a K split
+    behind it.  The bits of the same call on int8 weights of the same values, and int8 x against the oracle."""
+    rng = np.random.default_rng(k + n)
+    e, rows = len(counts), sum(counts)
+    w = _weights(rng, 4, e, k, n)
+    w[:, ::2, ::3] = -8
+    if x_type == "i8":
+        x, dt, out = rng.integers(-128, 128, (rows + 2, k), dtype=np.int8), cabi.DT_I8, cabi.DT_BF16
+        s = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32)
+        ops, fields = {cabi.IN_SCALE: to_dev(s)}, dict(scale_dtype=cabi.DT_F32, scale_per_group=1)
+    else:
+        to_bits = O.f32_to_bf16_bits if x_type == "bf16" else (lambda a: a.astype(np.float16).view(np.uint16))
+        x, dt = to_bits(rng.standard_normal((rows + 2, k)).astype(np.float32)), cabi.DT_BF16 if x_type == "bf16" else cabi.DT_F16
+        out = dt
+        s, o = to_bits(rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32)), to_bits(rng.integers(-8, 9, (e, n)).astype(np.float32))
+        ops, fields = {cabi.IN_ANTIQUANT_SCALE: to_dev(s), cabi.IN_ANTIQUANT_OFFSET: to_dev(o)}, dict(antiquant_dtype=dt, has_antiquant_offset=1)
+    run = lambda bits, name: _run(dt, bits, x, w, counts, split, ops, out, cabi.OV_AUTO, name, **fields).view(np.uint16)
+    got, wide = run(4, must), run(8, "8_")
+    assert np.array_equal(got[:rows], wide[:rows])
+    if x_type == "i8":
+        assert np.array_equal(got[:rows], O.grouped_matmul_w8a8(x, w, np.cumsum(counts), None, s, None)[:rows])
+    else:
+        to_f = O.bf16_bits_to_f32 if x_type == "bf16" else (lambda b: b.view(np.float16).astype(np.float32))
+        exact = O.a16w8_grouped_f64(to_f(x), w, to_f(s), to_f(o), np.cumsum(counts))[:rows]
+        assert np.abs(to_f(got[:rows]) - exact).max() <= 2.0 ** (-7 if x_type == "bf16" else -10) * np.abs(exact).max()
+
+
+# (x type, override, rows per group, K, N, what the plan names)
+ACTIVATED = [("i8", cabi.OV_REGT, [3, 33, 1], 272, 272, "a8w4_skinny_regt"), ("i8", cabi.OV_TILE_4BIT, [3, 33, 1], 272, 272, "64x256_4bit"),
+             ("i8", cabi.OV_TILE_4BIT, [100] * 9, 256, 6128, "128x256_4bit"), ("bf16", cabi.OV_REGT, [3, 33, 1], 272, 272, "a16w4_skinny_regt")]
+
+
+@pytest.mark.parametrize("act", [O.ACT_RELU, O.ACT_GELU_TANH, O.ACT_FAST_GELU, O.ACT_SILU])
+@pytest.mark.parametrize("x_type,override,counts,k,n,must", ACTIVATED)
+def test_activation_on_4_bit_weights(device, x_type, override, counts, k, n, must, act):
+    """int8 x: the activation of the exact float32 value within one output ulp (relu: the same bits).  16-bit x: of the
+    kernel's own plain output within that ulp and the plain output's (the functions are 1.13-Lipschitz)."""
+    rng = np.random.default_rng(n)
+    e, rows = len(counts), sum(counts)
+    w = _weights(rng, 4, e, k, n)
+    if x_type == "i8":
+        x = rng.integers(-128, 128, (rows + 2, k), dtype=np.int8)
+        s, pt = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), rng.uniform(1e-2, 1e-1, rows + 2).astype(np.float32)
+        pre = O.grouped_matmul_w8a8(x, w, np.cumsum(counts), None, s, pt, out_dtype="f32")[:rows]
+        ops = {cabi.IN_SCALE: to_dev(s), cabi.IN_PER_TOKEN_SCALE: to_dev(pt)}
+        got = _run(cabi.DT_I8, 4, x, w, counts, 0, ops, cabi.DT_BF16, override, must, scale_dtype=cabi.DT_F32, scale_per_group=1, per_token_dtype=cabi.DT_F32,
+                   act_type=act)[:rows].view(np.uint16)
+        slack = 0.0
+    else:
+        x, s = O.f32_to_bf16_bits(rng.standard_normal((rows + 2, k)).astype(np.float32)), O.f32_to_bf16_bits(rng.uniform(5e-3, 5e-2, (e, n)).astype(np.float32))
+        run = lambda **f: _run(cabi.DT_BF16, 4, x, w, counts, 0, {cabi.IN_ANTIQUANT_SCALE: to_dev(s)}, cabi.DT_BF16, override, must, antiquant_dtype=cabi.DT_BF16, **f)[:rows].view(np.uint16)
+        pre, got = O.bf16_bits_to_f32(run()), run(act_type=act)
+        slack = 1.13 * 2.0 ** -8
+    assert (pre < -1).any() and (pre > 1).any()
+    ref = O.activation(pre, act)
+    if act == O.ACT_RELU:
+        assert np.array_equal(got, O.f32_to_bf16_bits(ref.astype(np.float32)))
+    else:
+        assert (np.abs(O.bf16_bits_to_f32(got).astype(np.float64) - ref) <= 2.0 ** -7 * np.abs(ref) + slack * np.abs(pre) + 1e-30).all()
