@@ -421,7 +421,9 @@ hipError_t regt_by_strip(const GmmParams &p, int row_blocks, int strip_cols, boo
 
 size_t regt_slice_bytes(int row_blocks, int strip_cols) { return (size_t)row_blocks * (16 * strip_cols / 2 + 8) * 8; }
 
-// row_blocks = 16-row blocks per chunk (1 or 2), strip_cols = columns per strip (256 or 512), shallow: 16-bit x on 8-bit weights only
+// row_blocks = 16-row blocks per chunk (1 or 2), strip_cols = columns per strip (256 or 512), shallow: 16-bit x on 8-bit weights only.
+// The plan takes int8 x on 4-bit weights with 16-row chunks only and int8 x on 8-bit weights never: those forms run under
+// kernel_override (the tests compare them with the oracle).
 hipError_t launch_regt(const GmmParams &p, int weight_bits, int row_blocks, int strip_cols, bool shallow, hipStream_t stream) {
   if (p.m == 0) return hipSuccess;
   if (p.k % 16 != 0 || p.n % 16 != 0) return hipErrorInvalidValue;
