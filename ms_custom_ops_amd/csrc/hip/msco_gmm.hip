@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -148,6 +149,14 @@ int check_desc(const msco_gmm_desc &d) {
   return MSCO_ERR_UNSUPPORTED;
 }
 
+// Groups that hold rows when m rows go to e groups at random: the mean and one standard deviation, at most min(m, e).
+int64_t groups_hit(int64_t m, int64_t e) {
+  if (m < 1 || e < 2) return 1;
+  const double ed = (double)e, q = std::pow(1.0 - 1.0 / ed, (double)m), r = std::pow(1.0 - 2.0 / ed, (double)m);
+  const double var = ed * (ed - 1.0) * r + ed * q - ed * ed * q * q;
+  return std::max<int64_t>(1, std::min<int64_t>(std::min(m, e), (int64_t)std::ceil(ed * (1.0 - q) + std::sqrt(std::max(var, 0.0)))));
+}
+
 // Row-major [E,K,N] weights transposed and converted in registers (gmm_regt.hip).  Called behind choose_plan's own pick:
 // takes the plan over where these kernels are the better ones, and sets up the widening where 4-bit weights go to a
 // kernel that reads int8.
@@ -211,14 +220,30 @@ void plan_regt(msco_gmm_op *op) {
     p.m = (int)m;
     p.e = (int)e;
     const int64_t slots = chunk_slots(p, 16 * blocks);
-    // chunks expected to hold rows (an average group's, not one per group: 8 experts, 40 rows each, K = N = 4096, 4-bit weights: a K
-    // split for 16 chunks instead of 8 and 45.3 -> 37.0 us)
-    const int64_t active = std::max<int64_t>(1, std::min<int64_t>(slots, std::min<int64_t>(m, e) * ((avg + 16 * blocks - 1) / (16 * blocks))));
+    // 16-bit x on 8-bit weights: a form with one K step in flight per wave and four waves per SIMD, for several workgroups per CU
+    const bool can_be_shallow = bits == 8 && is_a16w8(d);
+    // Chunks expected to hold rows (an average group's, not one per group: 8 experts, 40 rows each, K = N = 4096, 4-bit weights: a K
+    // split for 16 chunks instead of 8 and 45.3 -> 37.0 us).  Few rows over many groups: the groups that a random routing hits where
+    // the forms below are chosen by how full the chip is (32 experts, 52 rows, K = 6976, N = 1920, not full: 70.9 -> 65.2 us), as
+    // many as there can be elsewhere (the other estimate there: 110 shapes at 0.98 to 1.13 of the time, 1.003 on average).
+    const int64_t active =
+      std::max<int64_t>(1, std::min<int64_t>(slots, (can_be_shallow ? groups_hit(m, e) : std::min<int64_t>(m, e)) * ((avg + 16 * blocks - 1) / (16 * blocks))));
     const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
     // Strips of 512 columns (eight waves, twice as many neighbouring bytes per K row) while they fill most of the CUs
     // without a K split, strips of 256 (four waves) otherwise.  8 experts, K = 4096, N = 14336, 4 rows per group, 4-bit
     // weights: 44 against 51 us (int8 x), 47 against 52 us (bf16).  One group, N = 11008: 20 against 17 us.
-    int64_t cols = ((n + 511) / 512) * active * 4 >= cus * 3 ? 512 : 256;
+    const int64_t wgs512 = ((n + 511) / 512) * active, wgs256 = ((n + 255) / 256) * active;
+    int64_t cols = wgs512 * 4 >= cus * 3 ? 512 : 256;
+    // 8-bit weights: 512 columns take 0.9 of the time of two strips of 256, but their rounds on the chip are coarser: up to two they are
+    // counted whole, the chip full with 31/32 of the CUs (256 columns: with 34/32, four of them fit a CU and fewer groups may be hit); beyond,
+    // a half for the last one.  Strips of 512 / 256, us, the weights not in the caches: 48 rows over 32 experts, K = 2624, N = 4624 (more than one round): 96.6 / 72.4; 320 over 32, K = 832, N = 4688: 38.8 / 36.4; 288
+    // over 64, K = 1088, N = 4064 (all of two rounds): 73 / 63; 1296 over 128, K = 1248, N = 704 (all of one): 46 / 31; one round: 28 over 8,
+    // K = 2944, N = 13840: 65.9 / 73.5; 24 over 32, K = 3168, N = 4016 (152 workgroups): 57 / 66; many: 198 over 64, K = 704, N = 7824: 71.7 / 80.2.
+    // Fitted to 620 shapes of 1 to 10 rows per group, K = 512 .. 8192, N = 512 .. 14336, random routings.
+    if (can_be_shallow) {
+      auto tenths = [&](int64_t w, int64_t full) { return w <= 2 * cus ? 10 * ((32 * w + full * cus - 1) / (full * cus)) : 10 * w / cus + 5; };
+      cols = wgs512 * 20 >= cus * 11 && 9 * tenths(wgs512, 31) < 5 * tenths(wgs256, 34) ? 512 : 256;
+    }
     if (tuning().regt_cols > 0) cols = tuning().regt_cols;
     const int64_t strips = (n + cols - 1) / cols;
     if (slots <= 65535) {
@@ -236,6 +261,10 @@ void plan_regt(msco_gmm_op *op) {
       int64_t split = 1;
       for (int64_t s = 2; s <= most; ++s)
         if (per_wave(s) + 1 < per_wave(split)) split = s;
+      // A chip that is a little more than half full: two slices would start a second round, three make the shallow form's rounds
+      // (16 experts, K = 7872, N = 2192, 30 rows: 72.6 -> 65.2 us; K = 6368, 40 rows: 60.9 -> 56.8; 8 experts, K = 2720, N = 5120, 10 rows: 26.6 ->
+      // 21; K = 2464, N = 4320, 62 rows: 28.9 -> 29.6; three quarters full, 64 experts, K = 2912, N = 768, 278 rows: 28.5 -> 36.3).
+      if (can_be_shallow && cols == 256 && split == 1 && k >= 1536 && strips * active * 8 <= cus * 5) split = 3;
       if (d.force_split_k > 0) split = std::min<int64_t>(d.force_split_k, steps);
       const size_t tile = (size_t)slots * strips * regt_slice_bytes(blocks, (int)cols);
       while (split > 1 && tile * split > kTileSplitMaxWorkspace) --split;
@@ -245,7 +274,7 @@ void plan_regt(msco_gmm_op *op) {
       // experts, K = 512, N = 14336, 8 rows per group, 224 workgroups: 18.2 -> 15.7 us) and 256 workgroups of 256 (64 experts, K = 4096,
       // N = 1024: 50.9 -> 47.1 us; 8 experts, K = N = 4096, two slices: 31.1 -> 30.2 us); below that three steps (176 workgroups, 8
       // experts, K = 4096, N = 5632: 35.5 against 42.6 us; 224, N = 7168: 43.2 against 44.3 us).
-      op->shallow = bits == 8 && is_a16w8(d) && (cols == 512 || strips * active * split >= cus);
+      op->shallow = can_be_shallow && (cols == 512 || strips * active * split >= cus);
       return;
     }
   }

@@ -205,6 +205,17 @@ def test_long_k_keeps_the_weight_only_decode_kernel():
     assert "widened" in _plan(1, 131072, 131072 // 16, 1, "i8", 4, override=cabi.OV_GENERIC)[1]
 
 
+def test_weight_only_decode_strips_by_how_full_the_chip_is():
+    # [E,K,N], 8-bit weights (no device: K splits are planned but cannot allocate their counters, so only unsplit plans are looked at):
+    # 512 columns where one round of them fills most of the chip or there are many rounds; 256 where they need all of one or two, or a
+    # part of a second; three K steps in flight where the groups that rows go to do not give every CU a workgroup
+    for m, k, n, e, want in ((28, 2944, 13840, 8, "shallow layout=[E,K,N] m=28 k=2944 n=13840 e=8 split_k=1 strips=28"), (198, 704, 7824, 64, "split_k=1 strips=16"),
+                             (36, 5248, 10064, 8, "split_k=1 strips=20"), (24, 3168, 4016, 32, "split_k=1 strips=8"), (36, 4064, 4192, 16, "split_k=1 strips=17"), (48, 2624, 4624, 32, "shallow layout=[E,K,N] m=48 k=2624 n=4624 e=32 split_k=1 strips=19"),
+                             (1296, 1248, 704, 128, "split_k=1 strips=3"), (320, 832, 4688, 32, "split_k=1 strips=19"), (288, 1088, 4064, 64, "split_k=1 strips=16"),
+                             (52, 6976, 1920, 32, "skinny_regt layout=[E,K,N] m=52 k=6976 n=1920 e=32 split_k=1 strips=8")):
+        assert want in _plan(m, k, n, e, "bf16")[1], _plan(m, k, n, e, "bf16")[1]
+
+
 def test_large_a8w4_calls_widen_in_front_of_the_persistent_kernel():
     for m, k, n, e, widened in ((16384, 4096, 14336, 8, False), (32768, 4096, 14336, 8, True), (2048, 4096, 11008, 1, False), (16384, 4096, 11008, 1, True),
                                 (8192, 1024, 1024, 1, False), (32768, 4096, 11008, 16, False)):

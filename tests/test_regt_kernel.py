@@ -116,8 +116,8 @@ def test_16_bit_activations_long_k_exact(device, dtype, bits):
 # (rows per group, K, N, what the plan names): the form with one K step in flight per wave, planned from 256 workgroups on, in
 # strips of 256 columns without and with a K split and in strips of 512; groups of up to 17 rows, the last strip cut at 16 columns
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
-@pytest.mark.parametrize("counts,k,n,must", [([1, 16, 0, 17, 3, 2, 0, 1] * 4, 80, 2320, "split_k=1 strips=10 "), ([3, 0, 1, 2] * 8, 2064, 784, "split_k=2 strips=4 "),
-                                             ([1, 16, 0, 17, 3, 2, 0, 1] * 4, 48, 3600, "split_k=1 strips=8 "), ([1] * 32, 16, 3072 + 16, "split_k=1 strips=7 ")])
+@pytest.mark.parametrize("counts,k,n,must", [([1, 16, 0, 17, 3, 2, 0, 1] * 4, 80, 4112, "split_k=1 strips=17 "), ([3, 0, 1, 2] * 8, 2064, 1040, "split_k=3 strips=5 "),
+                                             ([1, 16, 0, 17, 3, 2, 0, 1] * 4, 48, 3088, "split_k=1 strips=7 "), ([1] * 32, 16, 3072 + 16, "split_k=1 strips=7 ")])
 def test_shallow_form_within_one_rounding(device, counts, k, n, must, dtype):
     """Tolerance as above; the same values given as 4-bit weights take the other form and give the same bits."""
     rng = np.random.default_rng(k + n)
@@ -129,7 +129,7 @@ def test_shallow_form_within_one_rounding(device, counts, k, n, must, dtype):
     o = to_bits(rng.integers(-8, 9, (e, n)).astype(np.float32))
     dt = cabi.DT_BF16 if dtype == "bf16" else cabi.DT_F16
     ops = {cabi.IN_ANTIQUANT_SCALE: to_dev(s), cabi.IN_ANTIQUANT_OFFSET: to_dev(o)}
-    run = lambda bits, w, name: _run(dt, bits, x, w, counts, 0, ops, dt, cabi.OV_AUTO, name, antiquant_dtype=dt, has_antiquant_offset=1).view(np.uint16)
+    run = lambda bits, w, name, split=0: _run(dt, bits, x, w, counts, split, ops, dt, cabi.OV_AUTO, name, antiquant_dtype=dt, has_antiquant_offset=1).view(np.uint16)
     ends, starts = np.cumsum(counts), np.cumsum(counts) - counts
     for bits in (8, 4):
         w = _weights(rng, bits, e, k, n)
@@ -139,7 +139,7 @@ def test_shallow_form_within_one_rounding(device, counts, k, n, must, dtype):
         ulp = 2.0 ** -7 if dtype == "bf16" else 2.0 ** -10
         assert (np.abs(to_f(got[:rows]).astype(np.float64) - exact) <= ulp * np.abs(exact) + 1e-5 * mag).all()
         assert (got[rows:] == 0x7FC0).all()
-    assert np.array_equal(got, run(4, w, "skinny_regt "))
+    assert np.array_equal(got, run(4, w, "skinny_regt ", int(must[8])))   # (the same K slices)
 
 
 def test_large_a8w4_call_widens_first(device):
