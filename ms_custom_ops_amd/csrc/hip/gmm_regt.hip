@@ -266,11 +266,10 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
 #pragma unroll
       for (int j = 0; j < 8; ++j) f[j] = dequant((v[j] >> shift) + load_bias(p, grp, n + j), load_scale(p, grp, n + j), pt);
     }
-    unsigned short o[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = half_out(p, f[j]);
-    const uint4 q = make_uint4(o[0] | ((unsigned)o[1] << 16), o[2] | ((unsigned)o[3] << 16), o[4] | ((unsigned)o[5] << 16), o[6] | ((unsigned)o[7] << 16));
-    *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned short *>(p.out) + (long long)(m0 + row) * p.n + n) = q;
+    unsigned q[4];
+    activate_n(f, p.act_type);
+    pack_half_n(f, p.out_dtype, q);
+    *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned short *>(p.out) + (long long)(m0 + row) * p.n + n) = make_uint4(q[0], q[1], q[2], q[3]);
   };
 
   const long long tile = (long long)blockIdx.z * p.n_strips + strip;

@@ -261,6 +261,7 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
   __syncthreads();
   // out = s * (sum_k x w + o sum_k x)
   constexpr int NV = KN ? 16 : 8, NG = KN ? 1 : 2;   // neighbouring columns per lane, and groups of them
+  auto finish = [&](auto act_c) {
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     // packed: column groups 2 g and 2 g + 1; once the lane rows have been swapped, h & 1 says which and h >> 1 which half of it
@@ -292,21 +293,18 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
       if (live && row < chunk_rows) {
         unsigned q[NV / 2];
 #pragma unroll
-        for (int v = 0; v < NV; v += 2) {
-          float f[2];
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            f[t] = fmaf(of[v + t], xs_row, a[v + t]) * sc[v + t];
-            if (p.act_type != ACT_NONE) f[t] = activate(f[t], p.act_type);
-          }
-          q[v / 2] = BF16 ? pack_bf16x2(f[0], f[1]) : ((unsigned)f32_to_f16_rne(f[0]) | ((unsigned)f32_to_f16_rne(f[1]) << 16));
-        }
+        for (int v = 0; v < NV; ++v) a[v] = fmaf(of[v], xs_row, a[v]) * sc[v];
+        if constexpr (decltype(act_c)::value) activate_n(a, p.act_type);
+        pack_half_n(a, BF16 ? DT_BF16 : DT_F16, q);
         uint4 *dst = reinterpret_cast<uint4 *>(reinterpret_cast<unsigned short *>(p.out) + (long long)(m0 + row) * p.n + n);
 #pragma unroll
         for (int i = 0; i < NV / 8; ++i) dst[i] = uint4{q[4 * i], q[4 * i + 1], q[4 * i + 2], q[4 * i + 3]};
       }
     }
   }
+  };
+  if (p.act_type == ACT_NONE) finish(std::false_type{});
+  else finish(std::true_type{});
 }
 
 template <bool BF16, bool KN>

@@ -233,6 +233,7 @@ __device__ __forceinline__ void rows_run(const GmmParams &p, unsigned char *smem
   for (int cg = 0; cg < XR_CG; ++cg)
     ep_scale[cg] = __uint_as_float((p.scale_dtype == DT_BF16 && p.out_dtype != DT_I32) ? ep_scale_bits[cg] << 16 : ep_scale_bits[cg]);
   __syncthreads();   // every wave is done with the x stages: they become two float32 stages of 16 output rows
+  auto finish = [&](auto act_c) {
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     float(*tile_out)[XR_OUT_PITCH] = reinterpret_cast<float(*)[XR_OUT_PITCH]>(smem + (rb & 1) * S::kOutStage);
@@ -254,21 +255,23 @@ __device__ __forceinline__ void rows_run(const GmmParams &p, unsigned char *smem
         const v4f lo = *reinterpret_cast<const v4f *>(&tile_out[row][c8]);
         const v4f hi = *reinterpret_cast<const v4f *>(&tile_out[row][c8 + 4]);
         float f[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        if (p.act_type != ACT_NONE) {
+        unsigned q[4];
+        if constexpr (RBMAX > 10) {   // (the 256-row form spills with the other kind)
+          if (p.act_type != ACT_NONE) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) f[j] = activate(f[j], p.act_type);
+            for (int j = 0; j < 8; ++j) f[j] = activate(f[j], p.act_type);
+          }
+        } else if constexpr (decltype(act_c)::value) {
+          activate_n(f, p.act_type);
         }
-        uint4 q;
-        if (p.out_dtype == DT_BF16) {
-          q = uint4{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7])};
-        } else {
-          q = uint4{(unsigned)f32_to_f16_rne(f[0]) | ((unsigned)f32_to_f16_rne(f[1]) << 16), (unsigned)f32_to_f16_rne(f[2]) | ((unsigned)f32_to_f16_rne(f[3]) << 16),
-                    (unsigned)f32_to_f16_rne(f[4]) | ((unsigned)f32_to_f16_rne(f[5]) << 16), (unsigned)f32_to_f16_rne(f[6]) | ((unsigned)f32_to_f16_rne(f[7]) << 16)};
-        }
-        *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned short *>(p.out) + (long long)(m0 + 16 * rb + row) * p.n + n) = q;
+        pack_half_n(f, p.out_dtype, q);
+        *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned short *>(p.out) + (long long)(m0 + 16 * rb + row) * p.n + n) = uint4{q[0], q[1], q[2], q[3]};
       }
     }
   }
+  };
+  if (RBMAX <= 10 && p.act_type == ACT_NONE) finish(std::false_type{});
+  else finish(std::true_type{});
 }
 
 // NT: non-temporal weight loads, where a group is one chunk; several chunks of a group share them through the L2 (8 experts,

@@ -191,11 +191,14 @@ __global__ void __launch_bounds__(SK_THREADS, NK ? 3 : 4) gmm_w8a8_skinny_kernel
             reinterpret_cast<int *>(p.out)[(long long)(m0 + 4 * h + r) * p.n + n] = v[e][r] + bias;
       } else {
         const float sc = load_scale(p, grp, n);
+        float f[4];
+        unsigned q[2];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float f = dequant(v[e][r] + bias, sc, pt[r]);
-          tile_out[4 * h + r][cl] = half_out(p, f);
-        }
+        for (int r = 0; r < 4; ++r) f[r] = dequant(v[e][r] + bias, sc, pt[r]);
+        activate_n(f, p.act_type);
+        pack_half_n(f, p.out_dtype, q);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tile_out[4 * h + r][cl] = (unsigned short)(q[r / 2] >> (16 * (r % 2)));
       }
     }
   }
@@ -407,11 +410,14 @@ __global__ void __launch_bounds__(W16_THREADS) gmm_w8a8_skinny16_kernel(const Gm
         if (4 * h + r < chunk_rows)
           reinterpret_cast<int *>(p.out)[(long long)(m0 + 4 * h + r) * p.n + ep_n] = v[r] + ep_bias;
     } else {
+      float f[4];
+      unsigned q[2];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float f = dequant(v[r] + ep_bias, ep_scale, ep_pt[r]);
-        tile_out[4 * h + r][ep_cl] = half_out(p, f);
-      }
+      for (int r = 0; r < 4; ++r) f[r] = dequant(v[r] + ep_bias, ep_scale, ep_pt[r]);
+      activate_n(f, p.act_type);
+      pack_half_n(f, p.out_dtype, q);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tile_out[4 * h + r][ep_cl] = (unsigned short)(q[r / 2] >> (16 * (r % 2)));
     }
   }
   if (p.out_dtype == DT_I32) return;

@@ -284,11 +284,14 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_w8a8_stream_kernel(const Gm
             reinterpret_cast<int *>(p.out)[(long long)(m0 + 4 * h + r) * p.n + n] = v[e][r] + bias;
       } else {
         const float sc = ep_scale[e];
+        float f[4];
+        unsigned q[2];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float f = dequant(v[e][r] + bias, sc, pt[r]);
-          tile_out[4 * h + r][cl] = half_out(p, f);
-        }
+        for (int r = 0; r < 4; ++r) f[r] = dequant(v[e][r] + bias, sc, pt[r]);
+        activate_n(f, p.act_type);
+        pack_half_n(f, p.out_dtype, q);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tile_out[4 * h + r][cl] = (unsigned short)(q[r / 2] >> (16 * (r % 2)));
       }
     }
   }
@@ -500,17 +503,21 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_w8a8_streamm_kernel(const G
     if (cg < cg_count && n < p.n) {
       const int bias = load_bias(p, grp, n);
       const float sc = p.out_dtype == DT_I32 ? 1.0f : load_scale(p, grp, n);
+      if (p.out_dtype == DT_I32) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * t + 4 * h + r;
-        if (row < chunk_rows) {
-          if (p.out_dtype == DT_I32) {
-            reinterpret_cast<int *>(p.out)[(long long)(m0 + row) * p.n + n] = v[j][r] + bias;
-          } else {
-            const float f32 = dequant(v[j][r] + bias, sc, p.per_token ? p.per_token[m0 + row] : 1.0f);
-            tile_out[row][cl] = half_out(p, f32);
-          }
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * t + 4 * h + r;
+          if (row < chunk_rows) reinterpret_cast<int *>(p.out)[(long long)(m0 + row) * p.n + n] = v[j][r] + bias;
         }
+      } else if (16 * t < chunk_rows) {
+        float f[4];
+        unsigned q[2];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f[r] = dequant(v[j][r] + bias, sc, p.per_token ? p.per_token[m0 + min(16 * t + 4 * h + r, chunk_rows - 1)] : 1.0f);
+        activate_n(f, p.act_type);
+        pack_half_n(f, p.out_dtype, q);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tile_out[16 * t + 4 * h + r][cl] = (unsigned short)(q[r / 2] >> (16 * (r % 2)));   // (rows past the chunk are not stored)
       }
     }
   }
@@ -780,11 +787,14 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_a16w8_stream_kernel(const G
       const bool upper = ((long long)grp * p.n + n) & 1;   // which half of its word the element is
       const float s = p.aq_scale ? sa_half_like<BF16>((unsigned short)(upper ? sc_word[e] >> 16 : sc_word[e])) : 1.0f;
       const float o = p.aq_offset ? sa_half_like<BF16>((unsigned short)(upper ? of_word[e] >> 16 : of_word[e])) : 0.0f;
+      float f[4];
+      unsigned q[2];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float f = fmaf(o - 128.0f, xs[r], v[e][r]) * s;
-        tile_out[4 * h + r][cl] = half_out(p, f);
-      }
+      for (int r = 0; r < 4; ++r) f[r] = fmaf(o - 128.0f, xs[r], v[e][r]) * s;
+      activate_n(f, p.act_type);
+      pack_half_n(f, BF16 ? DT_BF16 : DT_F16, q);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tile_out[4 * h + r][cl] = (unsigned short)(q[r / 2] >> (16 * (r % 2)));
     }
   }
   __syncthreads();
@@ -1059,12 +1069,18 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_a16w8_rows_kernel(const Gmm
       const float sc = p.aq_scale ? sa_half_like<BF16>((unsigned short)(upper ? sc_word[cg] >> 16 : sc_word[cg])) : 1.0f;
       const float of = p.aq_offset ? sa_half_like<BF16>((unsigned short)(upper ? of_word[cg] >> 16 : of_word[cg])) : 0.0f;
 #pragma unroll
-      for (int t = 0; t < TCH; ++t)
+      for (int t = 0; t < TCH; ++t) {
+        if (16 * t >= chunk_rows) break;
+        // (rows past the chunk land in the tile as well: the row stores below leave them out)
+        float f[4];
+        unsigned q[2];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 16 * t + 4 * h + r;
-          if (row < chunk_rows) tile_out[row][cl] = half_out(p, fmaf(of - 128.0f, rs[t][r], acc[cg][t][r]) * sc);
-        }
+        for (int r = 0; r < 4; ++r) f[r] = fmaf(of - 128.0f, rs[t][r], acc[cg][t][r]) * sc;
+        activate_n(f, p.act_type);
+        pack_half_n(f, BF16 ? DT_BF16 : DT_F16, q);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tile_out[16 * t + 4 * h + r][cl] = (unsigned short)(q[r / 2] >> (16 * (r % 2)));
+      }
     }
   }
   __syncthreads();
@@ -1433,8 +1449,14 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_a16w8_rows32_kernel(const G
 #pragma unroll
         for (int gp = 0; gp < GP; ++gp) {
           const int cl = 32 * (wave * GP + gp) + c32;
+          float f[4];
+          unsigned q[2];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) tile_out[row0 + r][cl] = half_out(p, fmaf(of[gp], xs4[r], acc[gp][t][4 * j + r]) * sc[gp]);
+          for (int r = 0; r < 4; ++r) f[r] = fmaf(of[gp], xs4[r], acc[gp][t][4 * j + r]) * sc[gp];
+          activate_n(f, p.act_type);
+          pack_half_n(f, BF16 ? DT_BF16 : DT_F16, q);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) tile_out[row0 + r][cl] = (unsigned short)(q[r / 2] >> (16 * (r % 2)));
         }
       }
     }

@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   }
   // int32 rows are 256 bytes: one 32-column block per pass; 16-bit outputs take a single pass
   constexpr int SHIFT = W4 ? 4 : 0;   // the operands were 16 times the nibbles: exact
-  auto run_pass = [&](auto raw_c, auto pass_c) {
+  auto run_pass = [&](auto raw_c, auto pass_c, auto act_c) {
     constexpr bool raw = decltype(raw_c)::value;
     constexpr int pass = decltype(pass_c)::value;
     constexpr int esize = raw ? 4 : 2;
@@ -589,25 +589,14 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
             float v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = dequant((acc[f][i][8 * s2 + j] >> SHIFT) + bi[j], sc[j], pt[i]);
-            if (p.act_type != ACT_NONE) {
-#pragma unroll
-              for (int j = 0; j < 8; ++j) v[j] = activate(v[j], p.act_type);
-            }
-            uint4 q;
-            if (p.out_dtype == DT_BF16) {
-              q.x = pack_bf16x2(v[0], v[1]); q.y = pack_bf16x2(v[2], v[3]);
-              q.z = pack_bf16x2(v[4], v[5]); q.w = pack_bf16x2(v[6], v[7]);
-            } else {
-              q.x = f32_to_f16_rne(v[0]) | ((unsigned)f32_to_f16_rne(v[1]) << 16);
-              q.y = f32_to_f16_rne(v[2]) | ((unsigned)f32_to_f16_rne(v[3]) << 16);
-              q.z = f32_to_f16_rne(v[4]) | ((unsigned)f32_to_f16_rne(v[5]) << 16);
-              q.w = f32_to_f16_rne(v[6]) | ((unsigned)f32_to_f16_rne(v[7]) << 16);
-            }
+            unsigned q[4];
+            if constexpr (decltype(act_c)::value) activate_n(v, p.act_type);
+            pack_half_n(v, p.out_dtype, q);
             if constexpr (KT) {
-              *reinterpret_cast<uint2 *>(dst + cw * 2) = make_uint2(q.x, q.y);
-              *reinterpret_cast<uint2 *>(dst + (cw + RUN2) * 2) = make_uint2(q.z, q.w);
+              *reinterpret_cast<uint2 *>(dst + cw * 2) = make_uint2(q[0], q[1]);
+              *reinterpret_cast<uint2 *>(dst + (cw + RUN2) * 2) = make_uint2(q[2], q[3]);
             } else {
-              *reinterpret_cast<uint4 *>(dst + cw * 2) = q;
+              *reinterpret_cast<uint4 *>(dst + cw * 2) = make_uint4(q[0], q[1], q[2], q[3]);
             }
           }
         }
@@ -631,11 +620,13 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
   if (p.out_dtype == DT_I32) {
-    run_pass(std::true_type{}, std::integral_constant<int, 0>{});
-    if constexpr (FN > 1) run_pass(std::true_type{}, std::integral_constant<int, 1>{});
+    run_pass(std::true_type{}, std::integral_constant<int, 0>{}, std::false_type{});
+    if constexpr (FN > 1) run_pass(std::true_type{}, std::integral_constant<int, 1>{}, std::false_type{});
     static_assert(FN <= 2, "int32 epilogue passes");
+  } else if (p.act_type == ACT_NONE) {
+    run_pass(std::false_type{}, std::integral_constant<int, 0>{}, std::false_type{});
   } else {
-    run_pass(std::false_type{}, std::integral_constant<int, 0>{});
+    run_pass(std::false_type{}, std::integral_constant<int, 0>{}, std::true_type{});
   }
 }
 
