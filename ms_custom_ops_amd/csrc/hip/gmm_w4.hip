@@ -6,15 +6,17 @@
 // (tests/st/test_grouped_matmul_w4.py:100-113; ops/c_api/grouped_matmul_w4/grouped_matmul_w4.cc:50-88.)  The
 // reference's workloads route 5 .. 32 rows to 256 experts: almost every group is empty or holds one row, so this is a
 // batch of matrix-vector products bound by the bytes of the weights of the experts that were hit.  Hence no MFMA:
-//   * one workgroup per (group that holds rows, 16 or more columns): the grid has min(E, M) group slots and a workgroup
+//   * one workgroup per (group that holds rows, share of the columns): the grid has min(E, M) group slots and a workgroup
 //     finds the group of its slot's rank with ballots over group_list; a short K lets several columns share a wavefront's lanes;
-//   * the group's rows (four at a time) sit in LDS, de-interleaved into even-k and odd-k bytes so that they line up
+//   * the group's rows (a few at a time) sit in LDS, de-interleaved into even-k and odd-k bytes so that they line up
 //     with the low and the high nibbles of a weight word;
-//   * a wavefront owns four columns and requests all their weights at once (one memory round trip; they stay in
-//     registers for every block of rows), lane L holding the 16-byte pieces L, L + 64, ... of a column (32
-//     consecutive k, always inside one K group): nibbles are multiplied as u ^ 8 in [0, 15] with v_dot4_i32_i8 and
-//     8 * sum(x) of the piece is subtracted (u ^ 8 = s + 8 for the signed nibble s); the int32 sum of a piece is
-//     exact, is scaled by its K group's float32 scale and added up in float32; lanes are reduced with shuffles.
+//   * a wavefront takes blocks of C neighbouring columns per lane segment, lane L holding the 16-byte pieces L, L + 64, ... of a
+//     column (32 consecutive k, always inside one K group), and requests the next block while it multiplies this one: the
+//     group look-up, the x rows and the first round trip are paid once per workgroup, of which the launch has about four
+//     per CU.  nibbles are multiplied as u ^ 8 in [0, 15] with v_dot4_i32_i8 and 8 * sum(x) of the piece is subtracted
+//     (u ^ 8 = s + 8 for the signed nibble s); the int32 sum of a piece is exact, is scaled by its K group's float32
+//     scale and added up in float32; the lanes' sums of C columns are added in a tree that halves the columns a lane
+//     holds with every step.
 #include "gmm_common.h"
 #include "gmm_kernels.h"
 #include "msco_gmm.h"
@@ -22,20 +24,26 @@
 namespace msco {
 namespace {
 
-constexpr int W4_ROWS = 4;           // rows of a group held in LDS at a time (k bytes each: small, so that many workgroups fit a CU)
-#ifndef MSCO_W4_WAVE_COLS
-#define MSCO_W4_WAVE_COLS 4
-#endif
-constexpr int W4_WAVE_COLS = MSCO_W4_WAVE_COLS;      // columns per lane segment of a wavefront, all in registers at once
 constexpr int W4_MAX_K = 8192;
-constexpr int W4_LANE_PIECES = W4_MAX_K / 32 / 64;   // 16-byte pieces of a column per lane
+constexpr int W4_LDS_BYTES = 32 * 1024;              // x rows in LDS at a time: 32 KiB / K, at most W4_MAX_ROWS
+constexpr int W4_MAX_ROWS = 16;
+constexpr int W4_TARGET_WGS = 1024;                  // four workgroups per CU
+constexpr int w4_cols(int p) { return p == 1 ? 8 : 4; }   // columns of a block per lane segment: 32 weight registers (64 with the longest K)
+inline int w4_rows(int64_t k, int64_t m) {
+  int64_t r = W4_LDS_BYTES / k;
+  r = r > W4_MAX_ROWS ? W4_MAX_ROWS : r < 1 ? 1 : r;
+  return (int)(r < m ? r : m);
+}
 
 __device__ __forceinline__ int dot4(int a, int b, int c) { return __builtin_amdgcn_sdot4(a, b, c, false); }
 
-__global__ void __launch_bounds__(256) gmm_a8w4_kernel(const int8_t *x, const unsigned char *w, const int *group_list,
+// P = 16-byte pieces of a column per lane (K <= 2048 P); VEC: a lane's C scales of a K group are one request (N % C == 0)
+template <int P, bool VEC>
+__global__ void __launch_bounds__(256, VEC ? 3 : 2) gmm_a8w4_kernel(const int8_t *x, const unsigned char *w, const int *group_list,
                                                        const float *x_scale, const float *w_scale, unsigned short *out, int m,
-                                                       int k, int n, int e, int group_size) {
-  extern __shared__ __align__(16) int xs[];   // min(W4_ROWS, m) rows: [row][piece of 32 k]: 4 words of even-k bytes, then 4 of odd-k bytes
+                                                       int k, int n, int e, int group_size, int lds_rows) {
+  constexpr int C = w4_cols(P);
+  extern __shared__ __align__(16) int xs[];   // lds_rows rows: [row][piece of 32 k]: 4 words of even-k bytes, then 4 of odd-k bytes
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // blockIdx.y counts the groups that hold rows (at most min(e, m) of them): find the one with that rank, 64 groups
   // per round of ballots, and leave if there are fewer
@@ -75,121 +83,168 @@ __global__ void __launch_bounds__(256) gmm_a8w4_kernel(const int8_t *x, const un
   }
   if (grp < 0) return;
   const int pieces = k / 32;
-  // a short K leaves lanes over: lanes_per_col lanes share a column, the wavefront works on 64 / lanes_per_col columns side by side
+  // a short K leaves lanes over: lanes_per_col lanes share a column segment, the wavefront works on 64 / lanes_per_col segments side by side
   int lanes_per_col = 64;
-  while (lanes_per_col / 2 >= pieces) lanes_per_col /= 2;
+  if constexpr (P == 1) {
+    while (lanes_per_col > C && lanes_per_col / 2 >= pieces) lanes_per_col /= 2;
+  }
   const int side = 64 / lanes_per_col;
-  const int pl = lane % lanes_per_col, sub = lane / lanes_per_col;
-  const int k_groups = k / group_size;
-  const int pieces_per_group = group_size / 32;
+  const int pl = lane & (lanes_per_col - 1), sub = lane / lanes_per_col;
+  const int pieces_per_group = group_size / 32, k_groups = k / group_size;
+  const int block_cols = 4 * C * side;                       // columns of a workgroup's block
+  const int col_lane = C * (wave * side + sub);               // this lane's first column in it
+  const int blocks = (n + block_cols - 1) / block_cols;
   const unsigned char *wg = w + (long long)grp * n * (k / 2);
   const float *sg = w_scale + (long long)grp * k_groups * n;
-  const int wg_cols = 4 * W4_WAVE_COLS * side;          // columns of this workgroup
-  const int col_base = blockIdx.x * wg_cols;
-  const int col0 = col_base + wave * W4_WAVE_COLS * side + sub;   // this lane's columns: col0 + c * side
 
-  // this wavefront's columns: every piece and its scale requested at once (one memory round trip), nibbles as u ^ 8.
-  // Branch-free, through buffer descriptors over this workgroup's columns of the group's weights and scales: what a
-  // lane has no use for (a piece past K, a column past N) is asked at an offset beyond the descriptor and reads as 0.
-  const int cols_here = min(wg_cols, n - col_base);
-  const __amdgpu_buffer_rsrc_t rs_w = buffer_over(wg + (long long)col_base * (k / 2), (long long)cols_here * (k / 2));
-  const __amdgpu_buffer_rsrc_t rs_s = buffer_over(sg + col_base, 4ll * ((long long)(k_groups - 1) * n + cols_here));
-  // (Staging the scales through LDS with coalesced requests measured slower, 12.4 against 11.4 us: the per-lane form
-  // below repeats cache lines, but it needs no barrier between the scales and the first dot product.)
-  uint4 wv[W4_WAVE_COLS][W4_LANE_PIECES];
-  float sc[W4_WAVE_COLS][W4_LANE_PIECES];
-#pragma unroll
-  for (int c = 0; c < W4_WAVE_COLS; ++c)
-#pragma unroll
-    for (int i = 0; i < W4_LANE_PIECES; ++i) {
-      const int p = pl + lanes_per_col * i, cl = col0 + c * side - col_base;   // column inside the workgroup
-      const bool live = p < pieces && cl < cols_here;
-      const v4i raw = __builtin_amdgcn_raw_buffer_load_b128(rs_w, live ? (unsigned)(cl * (k / 2) + p * 16) : 0xFFFFFFF0u, 0, 0);
-      wv[c][i] = make_uint4((unsigned)raw[0], (unsigned)raw[1], (unsigned)raw[2], (unsigned)raw[3]);
-      sc[c][i] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(
-          rs_s, live ? 4u * (unsigned)((p / pieces_per_group) * n + cl) : 0xFFFFFFFCu, 0, 0));
-    }
-
-  // A block of up to W4_ROWS rows of the group is rows * k consecutive bytes of x: thread t holds the 16-byte pieces
-  // t, t + 256, ... of them (requested through a descriptor over just these bytes, so nothing branches), together with
-  // the rows' activation scales.  The first block is requested right behind the weights -- loads return in order, so
-  // it costs no round trip of its own -- and before anything waits for the weights.
-  constexpr int W4_X_VECS = W4_ROWS * (W4_MAX_K / 16) / 256;   // 16-byte pieces of a block per thread
-  uint4 xr[W4_X_VECS];
-  float xsr[W4_ROWS];
-  const __amdgpu_buffer_rsrc_t rs_xs = buffer_over(x_scale, 4ll * m);
-  auto request_rows = [&](int r0, int rows) {
-    const __amdgpu_buffer_rsrc_t rs_x = buffer_over(x + (long long)r0 * k, (long long)rows * k);
-#pragma unroll
-    for (int u = 0; u < W4_X_VECS; ++u) {
-      const v4i raw = __builtin_amdgcn_raw_buffer_load_b128(rs_x, 16u * (unsigned)(threadIdx.x + 256 * u), 0, 0);
-      xr[u] = make_uint4((unsigned)raw[0], (unsigned)raw[1], (unsigned)raw[2], (unsigned)raw[3]);
-    }
-#pragma unroll
-    for (int r = 0; r < W4_ROWS; ++r)
-      xsr[r] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(rs_xs, r < rows ? 4u * (unsigned)(r0 + r) : 0xFFFFFFFCu, 0, 0));
+  // A block of this lane's columns: every piece and its scale requested at once.  Branch-free, through buffer descriptors over
+  // the block's weights and scales: what a lane has no use for (a piece past K, a column past N) is asked at an offset beyond the
+  // descriptor and reads as 0.
+  struct Block {
+    v4i w[P][C];
+    float s[P][C];
   };
-  request_rows(g_start, min(W4_ROWS, g_end - g_start));
-
-  for (int r0 = g_start; r0 < g_end; r0 += W4_ROWS) {
-    const int rows = min(W4_ROWS, g_end - r0);
-    if (r0 != g_start) request_rows(r0, rows);
-    __syncthreads();   // the previous block of rows is no longer read
+  auto request = [&](Block &b, int block) {
+    const long long n0 = (long long)block * block_cols;
+    const int cols = block < blocks ? min(block_cols, n - (int)n0) : 0;
+    const __amdgpu_buffer_rsrc_t rs_w = buffer_over(wg + n0 * (k / 2), (long long)cols * (k / 2));
+    const __amdgpu_buffer_rsrc_t rs_s = buffer_over(sg + n0, cols > 0 ? 4ll * ((long long)(k_groups - 1) * n + cols) : 0);
 #pragma unroll
-    for (int u = 0; u < W4_X_VECS; ++u) {
-      // 16 bytes (k0 .. k15 of a half piece) -> two words of even-k bytes and two of odd-k bytes
-      const int idx = threadIdx.x + 256 * u;
-      if (idx < rows * pieces * 2) {
-        const uint4 v = xr[u];
-        const int r = idx / (pieces * 2), h = idx - r * pieces * 2;
-        const unsigned e0 = __builtin_amdgcn_perm(v.y, v.x, 0x06040200u), o0 = __builtin_amdgcn_perm(v.y, v.x, 0x07050301u);
-        const unsigned e1 = __builtin_amdgcn_perm(v.w, v.z, 0x06040200u), o1 = __builtin_amdgcn_perm(v.w, v.z, 0x07050301u);
-        int *dst = xs + (r * pieces + (h >> 1)) * 8 + (h & 1) * 2;
-        dst[0] = (int)e0; dst[1] = (int)e1; dst[4] = (int)o0; dst[5] = (int)o1;
+    for (int i = 0; i < P; ++i) {
+      const int p = pl + 64 * i;
+      const bool live = p < pieces;
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        b.w[i][c] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, live && col_lane + c < cols ? (unsigned)(col_lane + c) * (unsigned)(k / 2) + 16u * (unsigned)p : 0xFFFFFFF0u, 0, 0);
+      const unsigned at = 4u * ((unsigned)(p / pieces_per_group) * (unsigned)n + (unsigned)col_lane);
+      if constexpr (VEC && C % 4 == 0) {
+#pragma unroll
+        for (int c = 0; c < C; c += 4) {
+          const v4i v = __builtin_amdgcn_raw_buffer_load_b128(rs_s, live && col_lane < cols ? at + 4u * c : 0xFFFFFFF0u, 0, 0);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) b.s[i][c + q] = __uint_as_float((unsigned)v[q]);
+        }
+      } else if constexpr (VEC) {
+        const unsigned long long v = __builtin_bit_cast(unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(rs_s, live && col_lane < cols ? at : 0xFFFFFFF0u, 0, 0));
+        b.s[i][0] = __uint_as_float((unsigned)v);
+        b.s[i][1] = __uint_as_float((unsigned)(v >> 32));
+      } else {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          b.s[i][c] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(rs_s, live && col_lane + c < cols ? at + 4u * c : 0xFFFFFFFCu, 0, 0));
       }
     }
-    __syncthreads();
+  };
+
+  // rows r0 .. r0 + rows of the block in LDS (piece idx is 16 bytes, k0 .. k15 of half a piece: two words of even-k bytes and two of odd-k bytes)
+  auto stage_rows = [&](int r0, int rows) {
+    const uint4 *src = reinterpret_cast<const uint4 *>(x + (long long)r0 * k);
+    const int total = rows * pieces * 2;
+    for (int idx = threadIdx.x; idx < total; idx += 256) {
+      const uint4 v = src[idx];
+      const int r = idx / (pieces * 2), h = idx - r * pieces * 2;
+      const unsigned e0 = __builtin_amdgcn_perm(v.y, v.x, 0x06040200u), o0 = __builtin_amdgcn_perm(v.y, v.x, 0x07050301u);
+      const unsigned e1 = __builtin_amdgcn_perm(v.w, v.z, 0x06040200u), o1 = __builtin_amdgcn_perm(v.w, v.z, 0x07050301u);
+      int *dst = xs + (r * pieces + (h >> 1)) * 8 + (h & 1) * 2;
+      dst[0] = (int)e0; dst[1] = (int)e1; dst[4] = (int)o0; dst[5] = (int)o1;
+    }
+  };
+
+  auto multiply = [&](const Block &b, int block, int r0, int rows) {
+    const int c0 = block * block_cols + col_lane;
     for (int r = 0; r < rows; ++r) {
-      float acc[W4_WAVE_COLS];
+      unsigned low = 0x0F0F0F0Fu;   // (opaque: split once for all rows, the nibbles would take more registers than there are)
+      asm volatile("" : "+s"(low));
+      float acc[C];
 #pragma unroll
-      for (int c = 0; c < W4_WAVE_COLS; ++c) acc[c] = 0.f;
+      for (int c = 0; c < C; ++c) acc[c] = 0.f;
 #pragma unroll
-      for (int i = 0; i < W4_LANE_PIECES; ++i) {
-        const int p = pl + lanes_per_col * i;
+      for (int i = 0; i < P; ++i) {
+        const int p = pl + 64 * i;
         if (p < pieces) {
           const int4 xe = *reinterpret_cast<const int4 *>(xs + (r * pieces + p) * 8);
           const int4 xo = *reinterpret_cast<const int4 *>(xs + (r * pieces + p) * 8 + 4);
+          const int xev[4] = {xe.x, xe.y, xe.z, xe.w}, xov[4] = {xo.x, xo.y, xo.z, xo.w};
           int sx = 0;
-          sx = dot4(xe.x, 0x01010101, sx); sx = dot4(xo.x, 0x01010101, sx); sx = dot4(xe.y, 0x01010101, sx);
-          sx = dot4(xo.y, 0x01010101, sx); sx = dot4(xe.z, 0x01010101, sx); sx = dot4(xo.z, 0x01010101, sx);
-          sx = dot4(xe.w, 0x01010101, sx); sx = dot4(xo.w, 0x01010101, sx);
 #pragma unroll
-          for (int c = 0; c < W4_WAVE_COLS; ++c) {
-            const unsigned t[4] = {wv[c][i].x ^ 0x88888888u, wv[c][i].y ^ 0x88888888u, wv[c][i].z ^ 0x88888888u, wv[c][i].w ^ 0x88888888u};
-            const int xev[4] = {xe.x, xe.y, xe.z, xe.w}, xov[4] = {xo.x, xo.y, xo.z, xo.w};
+          for (int j = 0; j < 4; ++j) sx = dot4(xov[j], 0x01010101, dot4(xev[j], 0x01010101, sx));
+#pragma unroll
+          for (int c = 0; c < C; ++c) {
             int d = 0;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              d = dot4(xev[j], (int)(t[j] & 0x0F0F0F0Fu), d);           // k = 8 j + 0, 2, 4, 6
-              d = dot4(xov[j], (int)((t[j] >> 4) & 0x0F0F0F0Fu), d);    // k = 8 j + 1, 3, 5, 7
+              const unsigned t = (unsigned)b.w[i][c][j] ^ 0x88888888u;
+              d = dot4(xev[j], (int)(t & low), d);           // k = 8 j + 0, 2, 4, 6
+              d = dot4(xov[j], (int)((t >> 4) & low), d);    // k = 8 j + 1, 3, 5, 7
             }
-            acc[c] += (float)(d - 8 * sx) * sc[c][i];
+            acc[c] += (float)(d - 8 * sx) * b.s[i][c];
           }
         }
       }
-      float xs_r = xsr[0];   // (selected, not indexed: the array stays in registers)
+      // lanes pl of a segment: the sums of columns c and c + half change sides, so that a lane is left with the column its low bits name
 #pragma unroll
-      for (int q = 1; q < W4_ROWS; ++q) xs_r = r == q ? xsr[q] : xs_r;
+      for (int half = C / 2, bit = 1; half > 0; half /= 2, bit *= 2) {
+        const bool up = (lane & bit) != 0;
 #pragma unroll
-      for (int c = 0; c < W4_WAVE_COLS; ++c) {
-        float v = acc[c];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-          if (o < lanes_per_col) v += __shfl_xor(v, o);   // wave-uniform
-        if (pl == 0 && col0 + c * side < n) out[(long long)(r0 + r) * n + col0 + c * side] = f32_to_f16_rne(v * xs_r);
+        for (int c = 0; c < half; ++c) {
+          const float give = up ? acc[c] : acc[c + half], keep = up ? acc[c + half] : acc[c];
+          acc[c] = keep + __shfl_xor(give, bit);
+        }
       }
+      float v = acc[0];
+      for (int o = C; o < lanes_per_col; o *= 2) v += __shfl_xor(v, o);   // wave-uniform
+      // bit 0 of the lane chose between halves C / 2 apart, bit 1 between quarters, ..
+      int col = 0;
+#pragma unroll
+      for (int half = C / 2, bit = 1; half > 0; half /= 2, bit *= 2) col += (lane & bit) ? half : 0;
+      if (pl < C && c0 + col < n) out[(long long)(r0 + r) * n + c0 + col] = f32_to_f16_rne(v * x_scale[r0 + r]);
+    }
+  };
+
+  Block even, odd;   // (the longest K has one block in flight: with half as many columns each, or both blocks, slower, 14.5 against 12.4 us)
+  const int stride = (int)gridDim.x;
+  for (int r0 = g_start; r0 < g_end; r0 += lds_rows) {
+    const int rows = min(lds_rows, g_end - r0);
+    int block = (int)blockIdx.x;
+    request(even, block);
+    if (r0 != g_start) __syncthreads();   // the rows before are no longer read
+    stage_rows(r0, rows);
+    __syncthreads();
+    if constexpr (P == 4) {
+      for (; block < blocks; block += stride) {
+        multiply(even, block, r0, rows);
+        request(even, block + stride);
+      }
+      continue;
+    }
+    for (; block < blocks; block += 2 * stride) {
+      request(odd, block + stride);
+      multiply(even, block, r0, rows);
+      if (block + stride >= blocks) break;
+      request(even, block + 2 * stride);
+      multiply(odd, block + stride, r0, rows);
     }
   }
+}
+
+template <int P>
+hipError_t launch_a8w4(const int8_t *x, const unsigned char *w, const int *group_list, const float *x_scale, const float *w_scale,
+                       unsigned short *out, int m, int k, int n, int e, int group_size, hipStream_t stream) {
+  constexpr int C = w4_cols(P);
+  int lanes_per_col = 64;
+  while (P == 1 && lanes_per_col > C && lanes_per_col / 2 >= k / 32) lanes_per_col /= 2;
+  const int block_cols = 4 * C * (64 / lanes_per_col), blocks = (n + block_cols - 1) / block_cols;
+  const int slots = e < m ? e : m;
+  // (slots past the last group that holds rows leave at once: counting them all makes the shares of the columns larger, not smaller)
+  int shares = (W4_TARGET_WGS + slots - 1) / slots;
+  shares = shares < blocks ? shares : blocks;
+  const int steps = (blocks + shares - 1) / shares;
+  const dim3 grid((unsigned)((blocks + steps - 1) / steps), (unsigned)slots);
+  const int rows = w4_rows(k, m);
+  const size_t lds = (size_t)rows * (size_t)k;
+  auto kern = n % (C < 4 ? C : 4) == 0 ? gmm_a8w4_kernel<P, true> : gmm_a8w4_kernel<P, false>;
+  hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, x, w, group_list, x_scale, w_scale, out, m, k, n, e, group_size, rows);
+  return hipGetLastError();
 }
 
 // 4-bit values widened to int8: 16 source bytes (32 nibbles) -> 32 bytes per thread, low nibble first, sign extended
@@ -258,13 +313,9 @@ extern "C" int msco_gmm_a8w4(const int8_t *x, const void *weight, const int32_t 
   if (m == 0) return MSCO_OK;
   if (x == nullptr || weight == nullptr || group_list == nullptr || x_scale == nullptr || weight_scale == nullptr || out == nullptr)
     return MSCO_ERR_INVALID_ARG;
-  int lanes_per_col = 64;
-  while (lanes_per_col / 2 >= k / 32) lanes_per_col /= 2;
-  const long long wg_cols = 4ll * W4_WAVE_COLS * (64 / lanes_per_col);
-  const dim3 grid((unsigned)((n + wg_cols - 1) / wg_cols), (unsigned)(e < m ? e : m));
-  const size_t lds = (size_t)(m < W4_ROWS ? m : W4_ROWS) * (size_t)k;
-  hipLaunchKernelGGL(gmm_a8w4_kernel, grid, dim3(256), lds, static_cast<hipStream_t>(stream), x,
-                     static_cast<const unsigned char *>(weight), group_list, x_scale, weight_scale,
-                     static_cast<unsigned short *>(out), (int)m, (int)k, (int)n, (int)e, (int)group_size);
-  return hipGetLastError() == hipSuccess ? MSCO_OK : MSCO_ERR_DEVICE;
+  auto launch = k <= 2048 ? launch_a8w4<1> : k <= 4096 ? launch_a8w4<2> : launch_a8w4<4>;
+  return launch(x, static_cast<const unsigned char *>(weight), group_list, x_scale, weight_scale, static_cast<unsigned short *>(out),
+                (int)m, (int)k, (int)n, (int)e, (int)group_size, static_cast<hipStream_t>(stream)) == hipSuccess
+           ? MSCO_OK
+           : MSCO_ERR_DEVICE;
 }

@@ -148,3 +148,28 @@ def test_a8w4_malformed_group_list_is_clamped_like_the_other_kernels():
     b = _run(*case_good, g)
     assert np.array_equal(a.view(np.uint16), b.view(np.uint16))
     _check(b, *case_good, g)
+
+
+@pytest.mark.parametrize("m,k,n,e,g,gl", [
+    (5, 2048, 2088, 2, 128, [0, 5]),                 # one piece per lane, several column blocks per workgroup, a last block that is not full
+    (70, 4096, 1028, 64, 256, None),                 # two pieces per lane, 65 blocks over 15 shares
+    (9, 4096, 67, 1, 64, [9]),                       # scales one by one (N % 4 != 0), more rows than LDS holds
+    (66, 8192, 331, 2, 256, [33, 66]),               # four pieces per lane, N odd, several row blocks, column blocks read again
+    (65, 96, 24, 3, 32, [65, 65, 65]),               # more than sixteen rows, three pieces: lanes shared by column segments
+])
+def test_a8w4_column_shares_and_row_blocks(m, k, n, e, g, gl):
+    """One float16 rounding (2^-11, or half its smallest step) of the exact value and at most 16 float32 roundings (a product with
+    the scale, the additions of a lane's pieces and of the lanes, the row's scale) of sums no larger than the terms' magnitudes."""
+    x, xs, wp, ws, gl = _case(m + n, m, k, n, e, g, gl)
+    out = _run(x, xs, wp, ws, gl, g)
+    rows = int(gl[-1])
+    exact = O.grouped_a8w4_f64(x, wp, gl, xs, ws, g)[:rows]
+    mag = np.empty_like(exact)
+    for i in range(e):
+        a, b = (int(gl[i - 1]) if i else 0), int(gl[i])
+        if b > a:
+            w = np.abs(O.unpack_int4(wp[i:i + 1])[0].astype(np.float64)).T * np.repeat(ws[i].astype(np.float64), g, axis=0)
+            mag[a:b] = (np.abs(x[a:b].astype(np.float64)) @ w) * xs[a:b, None]
+    got = out[:rows].astype(np.float64)
+    assert (np.abs(got - exact) <= np.abs(exact) * 2.0 ** -11 + 2.0 ** -25 + 16 * 2.0 ** -24 * mag).all()
+    assert np.isnan(out[rows:].astype(np.float32)).all()
