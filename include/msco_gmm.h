@@ -138,7 +138,8 @@ typedef struct msco_gmm_desc {
                               * 9 / 10 / 11 packed weights: chunks of up to 128 / 256 / 160 rows through LDS and weights
                               * straight into MFMA operands, 12 [E,K,N] weights transposed in registers, 13 tiles on 4-bit
                               * weights (4-bit weights: every other value widens them to int8 first and forces the family on the result),
-                              * 14 weight-only: equal chunks of up to 128 rows x strips of 512 columns
+                              * 14 weight-only: equal chunks of up to 128 rows x strips of 512 columns, 15 x strips of 256,
+                              * 16 the same with two sets of waves that take turns at the K blocks
                               * (msco_gmm_plan_info names what was planned) */
   int32_t weight_layout;     /* MSCO_WL_ROW_MAJOR: as transpose_b says; MSCO_WL_PACKED: written by msco_pack_weight */
   int32_t act_type;          /* msco_act: activation applied to the dequantised float32 value before the output cast */

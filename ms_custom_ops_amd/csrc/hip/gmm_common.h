@@ -172,12 +172,12 @@ __device__ __forceinline__ bool chunk_of_slot(const GmmParams &p, int slot, int 
 // groups that hold rows are numbered; strip s of the r-th is unit r p.n_strips + s and belongs to XCD unit % 8 (workgroups are dealt
 // to the XCDs in turn), where all chunks of a unit follow one another: its weights come into one L2 once.  A group's rows
 // are cut into equal chunks of whole 16-row blocks (a group of 270 rows: 144 + 126, not 160 + 110).  False past an XCD's last
-// one; the grid is xcd_slots workgroups.  Every lane of the wave calls it.
+// one; the grid is xcd_slots workgroups.  `chunk` numbers the chunks of all groups in order (below chunk_slots).  Every lane of the wave calls it.
 __device__ __forceinline__ int units_on_xcd(int y, int xcd) { return (y - xcd + kNumXcd - 1) / kNumXcd; }   // units u < y with u % 8 == xcd
 __device__ __forceinline__ bool chunk_of_xcd_slot(const GmmParams &p, int rows_per_chunk, int wg, int lane, int &grp, int &strip, int &m0,
-                                                  int &chunk_rows) {
+                                                  int &chunk_rows, int &chunk) {
   const int xcd = wg % kNumXcd, pos = wg / kNumXcd;
-  int carry = 0, seen = 0, rank0 = 0;
+  int carry = 0, seen = 0, rank0 = 0, chunks0 = 0;
   for (int g0 = 0; g0 < p.e; g0 += 64) {
     int start, end;
     group_rows_chunk(p, g0, lane, carry, start, end);
@@ -186,6 +186,7 @@ __device__ __forceinline__ bool chunk_of_xcd_slot(const GmmParams &p, int rows_p
     const int first = (rank0 + __popcll(held & ((1ull << lane) - 1ull))) * p.n_strips;
     const int mine = (units_on_xcd(first + p.n_strips, xcd) - units_on_xcd(first, xcd)) * chunks;
     const int upto = seen + wave_scan_add(mine, lane);
+    const int numbered = chunks0 + wave_scan_add(chunks, lane);
     const unsigned long long beyond = __ballot(upto > pos);
     if (beyond != 0) {
       const int l = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(beyond));
@@ -197,9 +198,11 @@ __device__ __forceinline__ bool chunk_of_xcd_slot(const GmmParams &p, int rows_p
       const int blocks = (r + 15) / 16, b0 = (int)((long long)i * blocks / c), b1 = (int)((long long)(i + 1) * blocks / c);
       m0 = wave_bcast(start, l) + 16 * b0;
       chunk_rows = min(16 * (b1 - b0), r - 16 * b0);
+      chunk = wave_bcast(numbered, l) - c + i;
       return true;
     }
     seen = wave_bcast(upto, 63);
+    chunks0 = wave_bcast(numbered, 63);
     rank0 += __popcll(held);
   }
   return false;

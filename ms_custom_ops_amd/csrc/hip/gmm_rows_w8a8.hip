@@ -280,8 +280,8 @@ template <int RBMAX, bool NT>
 __global__ void __launch_bounds__(XR_THREADS, RBMAX <= 10 ? 2 : 1) gmm_w8a8_rows_kernel(const GmmParams p) {
   extern __shared__ __align__(16) unsigned char xr_smem[];
   const int lane = threadIdx.x & 63;
-  int grp, strip, m0, chunk_rows;
-  if (!chunk_of_xcd_slot(p, 16 * RBMAX, (int)blockIdx.x, lane, grp, strip, m0, chunk_rows)) return;
+  int grp, strip, m0, chunk_rows, chunk;
+  if (!chunk_of_xcd_slot(p, 16 * RBMAX, (int)blockIdx.x, lane, grp, strip, m0, chunk_rows, chunk)) return;
   const int rb = (chunk_rows + 15) / 16;
   // one copy of the K loop per number of live 32-row block pairs
   bool done = false;

@@ -32,7 +32,9 @@ enum Override : int {
   OV_ROWS160 = 11,  // ... of up to 160 rows (other layouts: the persistent kernel)
   OV_REGT = 12,     // [E,K,N] weights transposed and converted in registers (other layouts: as planned)
   OV_TILE_4BIT = 13,  // 4-bit weights, int8 x: 64 x 256 or 128 x 256 tiles that read the nibbles (else: as planned)
-  OV_ROWS16 = 14      // weight-only: equal chunks of up to 128 rows x strips of 512 columns (else: as planned)
+  OV_ROWS16 = 14,     // weight-only: equal chunks of up to 128 rows x strips of 512 columns (else: as planned)
+  OV_ROWS16_256 = 15,  // the same with strips of 256 columns
+  OV_ROWS16_256X2 = 16 // ... and two sets of waves that take turns at the K blocks
 };
 
 constexpr int64_t kSkinnyMaxRows = 64;   // total rows up to which the weight-streaming kernel is planned
@@ -94,7 +96,8 @@ struct msco_gmm_op {
   int w_nontemporal = 0;     // small tile kernels on packed weights: non-temporal weight loads
   int small_group_rows = 0;  // > 0: the persistent kernel takes the groups with more rows, a second launch of 64 x 128 tiles the others
   int row_blocks = 1;        // register-transpose kernels: 16-row blocks per chunk
-  int strip_cols = 256;      // ... and columns per strip
+  int strip_cols = 256;      // ... and columns per strip (also of the weight-only 128-row kernel)
+  int wave_sets = 1;         // weight-only 128-row kernel: sets of waves that take turns at the K blocks
   bool shallow = false;      // ... and the form with one K step in flight per wave (several workgroups per CU)
   int64_t widen_bytes = 0;   // 4-bit weights without a kernel of their own for the shape: int8 copy of them at the front of the workspace
   size_t workspace_bytes = 0;
@@ -121,7 +124,7 @@ int check_desc(const msco_gmm_desc &d) {
   if (d.group_list_dtype != MSCO_DT_NONE && d.group_list_dtype != MSCO_DT_I32 && d.group_list_dtype != MSCO_DT_I64)
     return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_type != 0 && d.group_list_type != 1) return MSCO_ERR_INVALID_ARG;
-  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_ROWS16) return MSCO_ERR_INVALID_ARG;
+  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_ROWS16_256X2) return MSCO_ERR_INVALID_ARG;
   if (d.weight_layout != MSCO_WL_ROW_MAJOR && d.weight_layout != MSCO_WL_PACKED) return MSCO_ERR_INVALID_ARG;
   if (d.force_split_k < 0) return MSCO_ERR_INVALID_ARG;
   if (d.act_type < MSCO_ACT_NONE || d.act_type > MSCO_ACT_SILU) return MSCO_ERR_INVALID_ARG;
@@ -288,31 +291,101 @@ void plan_regt(msco_gmm_op *op) {
   }
 }
 
-// Weight-only on packed or [E,K,N] weights: tiles of 128 rows x 512 columns (gmm_rows_a16w8.hip) where they fill the chip.  One
-// workgroup per CU, and a tile takes about 19 us + 1.2 .. 1.4 us per 64 K, so what counts is how full the rounds are and that a
-// tile has rows enough; otherwise the 32- to 128-row kernels with their narrower strips and K split stay (us, before -> this,
-// packed / [E,K,N]):
-//   8 experts, K = 4096, N = 14336, 32 / 48 / 96 / 192 / 512 rows per group: 91 -> 96, 117 -> 101, 139 -> 118, 270 -> 197, 572 -> 435 /
-//   95 -> 93, 111 -> 95, 142 -> 122, 270 -> 222, 577 -> 456; 64 experts, K = 2048, N = 1408, 64 / 160 rows: 65 -> 53, 137 -> 106 / 63 -> 59,
-//   139 -> 118; one group, N = 11008, 512 (88 tiles) / 1024 (176) / 4096 rows: 91 -> 113, 158 -> 108, 444 -> 327 / 90 -> 107, 141 -> 116, 464 -> 347;
-//   128 tiles (8 experts, 4096 x 4096, 160 rows): 92 -> 89 / 95 -> 102; 288 tiles (16 experts, 2048 x 2816, 320 rows): 123 -> 113 / 112 -> 124;
-//   a strip and a half (128 experts, 1024 x 768, 100 rows): 53 -> 72 / 50 -> 81.  Short K, 64 experts x 64 rows, N = 2048, K = 512 / 768 / 1408: 32 -> 37,
-//   38.5 -> 36.5, 57 -> 53 / 31.5 -> 34.5, 38.2 -> 38.8, 57 -> 56 (the weights not in the caches 52 -> 54); x 150 rows, K = 512: 66 -> 60 / 62 -> 61.
-//   [E,K,N], 64 experts, N = 4096: K = 768 x 200 rows 161 -> 152, three tiles per group (270 rows) K = 576 / 1024: 181 -> 189, 253 -> 255.
-void plan_rows16(msco_gmm_op *op) {
+// Weight-only on packed or [E,K,N] weights beyond one 16-row chunk per group: the forms of the 128-row kernel
+// (gmm_rows_a16w8_kernel.h) -- strips of 512 columns, strips of 256 with two workgroups per CU, strips of 256 whose K blocks two
+// sets of waves share, the last two with a K split -- against the 32- and 64-row kernels, by a model of the time in us.  All
+// of them take as long as their rounds on the chip are many; a round has ends of its own and a part per K block, larger with more
+// rows, and the weights and rows have to be read.  Fitted to 460 random shapes (8 to 128 experts, 10 to 3200 rows per group,
+// K = 512 .. 8192, N = 512 .. 14336, random routings), every form measured on all of them: off by 8 .. 10 % (rms), and what it picks takes
+// 1.03 of the time of the best form and 0.83 of what the rules before it picked.  us, before -> now: 8 experts, K = 5056,
+// N = 3984, 145 rows per group, [E,K,N] 136 -> 71 (two sets; strips of 512: 107, of 256: 81); K = 6176, N = 688, 2485 rows, packed 318 -> 185
+// (256; 512: 271); 16 experts, K = 6336, N = 544, 51 rows 78 -> 38 (two sets, two slices; one set, one slice: 63); 64 experts, K = 928,
+// N = 2000, 282 rows, [E,K,N] 150 -> 104; 8 experts, K = 4096, N = 14336, 512 rows stays with 512: 437 (256: 445).
+struct Rows16Form { int cols, sets, split; };
+// fixed, per round, per K block and round, the same per 16 rows, per us of reading; K split: fixed, per slice, 16 rows and round
+struct Rows16Cost { double fixed, round, block, rows, stream, split, slice; };
+constexpr Rows16Cost kRows16[2][4] = {   // [packed][strips of 512; of 256 alone on their CUs; of 256 two per CU; two sets]
+  {{2.6, 8.15, 0.632, 0.075, 0.54, 0, 0}, {8.75, 0, 0.337, 0.063, 0.67, 4.0, 0.74}, {8.75, 1.57, 0.533, 0.100, 0.67, 4.0, 0.74}, {4.73, 6.91, 0.428, 0.103, 0.75, 4.2, 0.20}},
+  {{2.4, 5.81, 0.357, 0.095, 0.68, 0, 0}, {7.05, 0, 0.181, 0.068, 0.74, 3.1, 0.74}, {7.05, 1.47, 0.320, 0.101, 0.74, 3.1, 0.74}, {3.11, 6.09, 0.182, 0.123, 0.77, 3.8, 0.22}}};
+constexpr Rows16Cost kRowsSmall[2][2] = {   // [packed][32- and 64-row chunks], strips of 256 columns
+  {{6.2, 0, 0.665, 0.079, 0.84, 0, 0}, {7.8, 0, 0.803, 0.071, 0.84, 0, 0}}, {{5.9, 0, 0.860, 0.034, 0.50, 0, 0}, {5.8, 0, 0.747, 0.173, 0.50, 0, 0}}};
+
+double chip_rounds(double workgroups, double slots) { return workgroups <= slots ? 1.0 : workgroups / slots + 0.5; }
+
+double rows_stream_us(int64_t m, int64_t k, int64_t n, int64_t e) {   // at the rate of a read-only launch
+  return ((double)std::max<int64_t>(1, std::min(e, m)) * (double)(k * n) + 2.0 * (double)m * (double)(k + n)) / 6.7e6;
+}
+
+double rows16_us(int64_t m, int64_t k, int64_t n, int64_t e, int64_t cus, bool packed, const Rows16Form &f) {
+  const int64_t avg = (m + e - 1) / e, rows = e == 1 ? m : avg + avg / 10;   // (real routings are uneven)
+  const int64_t groups = std::max<int64_t>(1, std::min(e, m)), chunks = (rows + 127) / 128;
+  const double rb = (double)std::min<int64_t>(8, ((rows + chunks - 1) / chunks + 15) / 16);
+  const int depth = rb <= 2 ? 6 : rb <= 4 ? 4 : 3;   // K blocks per unrolled round of the kernel
+  const int64_t slice = ((k + 63) / 64 + f.split - 1) / f.split, own = (slice + f.sets - 1) / f.sets;
+  const double blocks = (double)((own + depth - 1) / depth * depth);
+  const double wgs = (double)((n + f.cols - 1) / f.cols) * (double)(groups * chunks * f.split);
+  const bool pairs = f.cols == 256 && f.sets == 1 && wgs > (double)cus;
+  const Rows16Cost &c = kRows16[packed][f.cols == 512 ? 0 : f.sets == 2 ? 3 : pairs ? 2 : 1];
+  const double r = chip_rounds(wgs, pairs ? 2.0 * (double)cus : (double)cus);
+  const double us = c.fixed + r * (c.round + blocks * (c.block + c.rows * rb)) + c.stream * rows_stream_us(m, k, n, e) + (f.split > 1 ? c.split + c.slice * rb * r * (f.split - 1) : 0.0);
+  return pairs && r > 3 && rb >= 6 ? 1.07 * us : us;   // (what the fit is off by there: x comes in twice per CU)
+}
+
+// the kernels with 32- and 64-row chunks (tch = 2, 4)
+double rows_small_us(int64_t m, int64_t k, int64_t n, int64_t e, int64_t cus, int tch, bool packed) {
+  const int64_t avg = (m + e - 1) / e, chunk = 16 * tch, groups = std::max<int64_t>(1, std::min(e, m)), col_groups = (n + 15) / 16;
+  const int64_t active = std::max<int64_t>(1, std::min<int64_t>(e * ((m + chunk - 1) / chunk), groups + m / chunk));
+  const int wide = ((col_groups + 15) / 16) * active >= 2 * cus ? 16 : 8;   // column groups per strip (as planned below)
+  const double wgs = (double)((col_groups + wide - 1) / wide) * (double)(groups * ((avg + avg / 10 + chunk - 1) / chunk));
+  const double live = (double)std::min<int64_t>(tch, (avg + 15) / 16), blocks = (double)((k + 63) / 64) * wide / 16;
+  const Rows16Cost &c = kRowsSmall[packed][tch == 4];
+  return c.fixed + chip_rounds(wgs, 2.0 * (double)cus) * blocks * (c.block + c.rows * live) + c.stream * rows_stream_us(m, k, n, e);
+}
+
+// `family_fits`: the kernels planned so far can take the shape (their grids are bounded; the 128-row kernel's is not)
+void plan_rows16(msco_gmm_op *op, bool family_fits) {
   const msco_gmm_desc &d = op->desc;
-  if (op->family != FAM_SKINNY || !is_a16w8(d) || layout_of(d) == 1 || op->k >= ((int64_t)1 << 22)) return;   // (128 rows of x through 32-bit offsets)
-  const int64_t m = op->m, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
-  const int64_t strips = (n + 511) / 512, groups = std::max<int64_t>(1, std::min<int64_t>(e, m)), avg = (m + e - 1) / e;
-  const int64_t rows = e == 1 ? m : avg + avg / 10;   // (real routings are uneven)
-  const int64_t tiles = strips * groups * ((rows + 127) / 128), rounds = (tiles + cus - 1) / cus;
-  const bool full = tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65;
-  const int64_t k_min = rows <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : rows <= 256 ? 768 : 1280;
-  if (d.kernel_override != OV_ROWS16 && !(d.kernel_override == OV_AUTO && d.force_split_k == 0 && op->k >= k_min && avg >= 48 && full && n * 100 >= strips * 512 * 85)) return;
+  if ((op->family != FAM_SKINNY && family_fits) || !is_a16w8(d) || layout_of(d) == 1 || op->k >= ((int64_t)1 << 22)) return;   // (128 rows of x through 32-bit offsets)
+  const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
+  GmmParams p{};
+  p.m = (int)m;
+  p.e = (int)e;
+  auto workspace = [&](const Rows16Form &f) {
+    return f.split > 1 ? (size_t)chunk_slots(p, 128) * ((n + f.cols - 1) / f.cols) * f.split * rows_a16w8_slice_bytes() : (size_t)0;
+  };
+  Rows16Form best{512, 1, 1};
+  if (d.kernel_override == OV_ROWS16 || d.kernel_override == OV_ROWS16_256 || d.kernel_override == OV_ROWS16_256X2) {
+    if (d.kernel_override != OV_ROWS16) best = Rows16Form{256, d.kernel_override == OV_ROWS16_256X2 ? 2 : 1, (int)std::min<int64_t>(std::max(d.force_split_k, 1), (k + 63) / 64)};
+    while (best.split > 1 && workspace(best) > kTileSplitMaxWorkspace) --best.split;
+  } else if (d.kernel_override != OV_AUTO || d.force_split_k != 0 || (family_fits && op->stream_tch == 1)) {
+    return;
+  } else if (e == 1) {
+    // One group, where these kernels have a K split of their own: strips of 512 once they fill most of the chip.  N = 11008, K = 4096, 512
+    // (88 tiles) / 1024 (176) / 4096 rows: 91 -> 113, 158 -> 108, 444 -> 327 us packed, 90 -> 107, 141 -> 116, 464 -> 347 us [E,K,N].
+    const int64_t strips = (n + 511) / 512, tiles = strips * ((m + 127) / 128), rounds = (tiles + cus - 1) / cus;
+    const int64_t k_min = m <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : m <= 256 ? 768 : 1280;
+    if (!(k >= k_min && m >= 48 && (tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65) && n * 100 >= strips * 512 * 85)) return;
+  } else {
+    double us = rows16_us(m, k, n, e, cus, is_packed(d), best);
+    for (int sets = 1; sets <= 2; ++sets)
+      for (int split = 1; split <= 4 && split <= (k + 63) / 64; ++split) {
+        const Rows16Form f{256, sets, split};
+        if (workspace(f) > (size_t)MSCO_GMM_STATIC_WORKSPACE_BYTES) break;   // (msco_gmm_launch_static takes what it took without a split)
+        const double t = rows16_us(m, k, n, e, cus, is_packed(d), f);
+        if (t < us) {
+          us = t;
+          best = f;
+        }
+      }
+    // (the kernels for smaller chunks keep what is not clearly better here; 128-row chunks are always better off)
+    if (family_fits && op->stream_tch <= 4 && 0.9 * rows_small_us(m, k, n, e, cus, op->stream_tch, is_packed(d)) < us) return;
+  }
   op->family = FAM_ROWS16;
-  op->n_strips = (int)strips;
-  op->split_k = 1;
-  op->workspace_bytes = 0;
+  op->strip_cols = best.cols;
+  op->wave_sets = best.sets;
+  op->n_strips = (int)((n + best.cols - 1) / best.cols);
+  op->split_k = best.split;
+  op->workspace_bytes = workspace(best);
 }
 
 void choose_plan(msco_gmm_op *op) {
@@ -569,6 +642,7 @@ void choose_plan(msco_gmm_op *op) {
       (d.kernel_override == OV_AUTO || d.kernel_override == OV_TILE_256_W4) && tuning().two_level != 0)
     op->small_group_rows = 64;
   op->stream_tch = 1;
+  bool rows16_fits = false;   // more (expert, chunk) pairs than the other weight-only kernels' grids hold
   if (family == FAM_SKINNY && is_packed(d) && is_w8a8(d)) {
     // rows a group is expected to hold (shapes only): 16-row chunks up to 16 rows, else chunks of 32 / 64 / 128 rows
     // (several groups: 1.5 x the average, real routings are uneven and a group that overflows its chunk streams its
@@ -602,7 +676,10 @@ void choose_plan(msco_gmm_op *op) {
     const int64_t chunk_rows = (int64_t)kSkinnyRows * op->stream_tch;
     op->max_chunks = (int)((m + chunk_rows - 1) / chunk_rows);
     if (op->max_chunks < 1) op->max_chunks = 1;
-    if (e * op->max_chunks > 65535) family = FAM_GENERIC;
+    if (e * op->max_chunks > 65535) {
+      family = FAM_GENERIC;
+      rows16_fits = is_a16w8(d);
+    }
   }
   if (family == FAM_SKINNY) {
     // Only shapes enter: the number of (group, chunk) pairs that can hold rows is estimated from M and E.
@@ -699,12 +776,12 @@ void choose_plan(msco_gmm_op *op) {
   }
   op->family = family;
   op->widen_bytes = 0;
-  plan_rows16(op);
+  plan_rows16(op, !rows16_fits);
   plan_regt(op);
 
   family = op->family;
   char buf[320];
-  const char *fam = family == FAM_REGT ? (op->shallow ? "skinny_regt_shallow" : "skinny_regt") : family == FAM_ROWS16 ? "rows128" : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
+  const char *fam = family == FAM_REGT ? (op->shallow ? "skinny_regt_shallow" : "skinny_regt") : family == FAM_ROWS16 ? (op->strip_cols == 512 ? "rows128" : op->wave_sets == 2 ? "rows128x256_2" : "rows128x256") : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
   std::snprintf(buf, sizeof(buf),
                 "msco_gmm plan: kernel=%s%s%s%s layout=%s m=%lld k=%lld n=%lld e=%lld split_k=%d strips=%d "
                 "workspace=%zu%s",
@@ -769,7 +846,8 @@ int msco_gmm_plan(msco_gmm_handle h, int64_t m, int64_t k, int64_t n, int64_t e,
     GmmParams p{};
     p.m = (int)m;
     p.e = (int)e;
-    const size_t need = h->family == FAM_REGT ? (size_t)chunk_slots(p, 16 * h->row_blocks) * h->n_strips
+    const size_t need = h->family == FAM_ROWS16 ? (size_t)chunk_slots(p, 128) * h->n_strips
+                        : h->family == FAM_REGT ? (size_t)chunk_slots(p, 16 * h->row_blocks) * h->n_strips
                         : h->family == FAM_TILE ? tile_count_bound(h->tile_cfg, m, n, e)
                                               : skinny_counter_count(m, n, e, h->skinny_cols);
     if (need > h->counters_cap) {
@@ -874,7 +952,7 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   if (h->family == FAM_REGT) {
     err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, h->shallow, s);
   } else if (h->family == FAM_ROWS16) {
-    err = launch_rows_a16w8(p, layout == 2, s);
+    err = launch_rows_a16w8(p, layout == 2, h->strip_cols, h->wave_sets, s);
   } else if (is_w8a8(d)) {
     if (h->family == FAM_TILE && h->small_group_rows > 0) {
       GmmParams big = p, small = p;

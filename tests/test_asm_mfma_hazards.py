@@ -73,3 +73,9 @@ def test_inline_mfmas_keep_their_wait_states(tmp_path):
         seen += sum(name.startswith("v_mfma") for name, _ in lines)
         assert _violations(lines) == [], kernel[:80]
     assert seen >= 1000
+
+
+@pytest.mark.parametrize("unit", ["bf16_kn", "f16_packed", "f16_kn"])
+def test_the_other_types_and_layouts_keep_them_too(unit, tmp_path, monkeypatch):
+    monkeypatch.setitem(globals(), "OBJ", OBJ.replace("a16w8.o", "a16w8_%s.o" % unit))
+    test_inline_mfmas_keep_their_wait_states(tmp_path)
