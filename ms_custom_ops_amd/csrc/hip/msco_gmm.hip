@@ -359,12 +359,14 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     while (best.split > 1 && workspace(best) > kTileSplitMaxWorkspace) --best.split;
   } else if (d.kernel_override != OV_AUTO || d.force_split_k != 0 || (family_fits && op->stream_tch == 1)) {
     return;
-  } else if (e == 1) {
-    // One group, where these kernels have a K split of their own: strips of 512 once they fill most of the chip.  N = 11008, K = 4096, 512
-    // (88 tiles) / 1024 (176) / 4096 rows: 91 -> 113, 158 -> 108, 444 -> 327 us packed, 90 -> 107, 141 -> 116, 464 -> 347 us [E,K,N].
-    const int64_t strips = (n + 511) / 512, tiles = strips * ((m + 127) / 128), rounds = (tiles + cus - 1) / cus;
-    const int64_t k_min = m <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : m <= 256 ? 768 : 1280;
-    if (!(k >= k_min && m >= 48 && (tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65) && n * 100 >= strips * 512 * 85)) return;
+  } else if (e < 8 || k < 512) {
+    // Outside what the model was fitted to (one group has kernels with a K split of its own): strips of 512 where they fill the chip and
+    // a tile has rows enough.  One group, N = 11008, K = 4096, 512 (88 tiles) / 1024 (176) / 4096 rows: 91 -> 113, 158 -> 108, 444 -> 327 us
+    // packed, 90 -> 107, 141 -> 116, 464 -> 347 us [E,K,N].
+    const int64_t strips = (n + 511) / 512, avg = (m + e - 1) / e, rows = e == 1 ? m : avg + avg / 10;
+    const int64_t tiles = strips * std::max<int64_t>(1, std::min<int64_t>(e, m)) * ((rows + 127) / 128), rounds = (tiles + cus - 1) / cus;
+    const int64_t k_min = rows <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : rows <= 256 ? 768 : 1280;
+    if (!(k >= k_min && avg >= 48 && (tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65) && n * 100 >= strips * 512 * 85)) return;
   } else {
     double us = rows16_us(m, k, n, e, cus, is_packed(d), best);
     for (int sets = 1; sets <= 2; ++sets)
