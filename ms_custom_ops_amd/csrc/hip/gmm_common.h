@@ -79,32 +79,35 @@ __device__ __forceinline__ int group_end(const GmmParams &p, int g, int prev) {
 // group_end() has closed forms, so a wave computes it with prefix scans instead of E dependent loads:
 //   cumulative ends: end_g = min(max(carry, v_0..v_g), M)            (prefix maximum)
 //   counts:          end_g = min(carry + max(v_0,0) + .. + max(v_g,0), M)   (saturating prefix sum)
-__device__ __forceinline__ int wave_scan_max(int v, int lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int t = __shfl_up(v, d);
-    if (lane >= d) v = max(v, t);
-  }
+// Scans over the lanes with data-parallel moves, a few cycles a step (through LDS permutes a step is a hundred: look-ups of
+// a group list 3.5 k cycles, 2.1 k this way, of which the load of the list is most).  Values from lanes that do not exist are 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int lane_move(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+template <typename F>
+__device__ __forceinline__ int wave_scan(int v, F &&op) {
+  v = op(v, lane_move<0x111, 0xF>(v));   // lanes 1, 2, 4 and 8 below in a row of 16
+  v = op(v, lane_move<0x112, 0xF>(v));
+  v = op(v, lane_move<0x114, 0xF>(v));
+  v = op(v, lane_move<0x118, 0xF>(v));
+  v = op(v, lane_move<0x142, 0xA>(v));   // the last lane of rows 0 and 2 to rows 1 and 3
+  v = op(v, lane_move<0x143, 0xC>(v));   // lane 31 to rows 2 and 3
   return v;
 }
-__device__ __forceinline__ int wave_scan_add_sat(int v, int lane, int cap) {   // operands in [0, cap], cap < 2^30
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int t = __shfl_up(v, d);
-    if (lane >= d) v = min(v + t, cap);
-  }
-  return v;
+__device__ __forceinline__ int wave_scan_max(int v) {   // operands >= 0
+  return wave_scan(v, [](int a, int b) { return max(a, b); });
 }
-__device__ __forceinline__ int wave_scan_add(int v, int lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int t = __shfl_up(v, d);
-    if (lane >= d) v += t;
-  }
-  return v;
+__device__ __forceinline__ int wave_scan_add_sat(int v, int cap) {   // operands in [0, cap], cap < 2^30
+  return wave_scan(v, [=](int a, int b) { return min(a + b, cap); });
 }
-__device__ __forceinline__ int wave_bcast(int v, int src_lane) {
-  return __builtin_amdgcn_readfirstlane(__shfl(v, src_lane));
+__device__ __forceinline__ int wave_scan_add(int v) {
+  return wave_scan(v, [](int a, int b) { return a + b; });
+}
+// lane l receives v of lane l - 1, lane 0 `first`
+__device__ __forceinline__ int wave_from_below(int v, int first) { return __builtin_amdgcn_update_dpp(first, v, 0x138, 0xF, 0xF, false); }
+__device__ __forceinline__ int wave_bcast(int v, int src_lane) {   // src_lane is wave-uniform
+  return __builtin_amdgcn_readlane(v, src_lane);
 }
 
 // Lane l receives [start, end) of group g0 + l (empty for lanes past E); `carry` is the row end of
@@ -120,10 +123,9 @@ __device__ __forceinline__ void group_rows_chunk(const GmmParams &p, int g0, int
   }
   const int c = (int)(v < 0 ? 0 : (v > p.m ? p.m : v));   // clamping the operands first changes neither closed form
   int e_l;
-  if (p.gl_type == 1 && p.gl_dtype != DT_NONE) e_l = min(carry + wave_scan_add_sat(valid ? c : 0, lane, p.m), p.m);
-  else e_l = max(carry, wave_scan_max(valid ? c : 0, lane));
-  const int prev = __shfl_up(e_l, 1);
-  start = lane == 0 ? carry : prev;
+  if (p.gl_type == 1 && p.gl_dtype != DT_NONE) e_l = min(carry + wave_scan_add_sat(valid ? c : 0, p.m), p.m);
+  else e_l = max(carry, wave_scan_max(valid ? c : 0));
+  start = wave_from_below(e_l, carry);
   end = e_l;
   carry = wave_bcast(e_l, 63);
 }
@@ -153,7 +155,7 @@ __device__ __forceinline__ bool chunk_of_slot(const GmmParams &p, int slot, int 
     int s0, e0;
     group_rows_chunk(p, g0, lane, carry, s0, e0);
     const int chunks = (e0 - s0 + rows_per_chunk - 1) / rows_per_chunk;   // 0 for empty groups and for lanes past E
-    const int upto = seen + wave_scan_add(chunks, lane);                  // chunks up to and including this lane's group
+    const int upto = seen + wave_scan_add(chunks);                  // chunks up to and including this lane's group
     const unsigned long long beyond = __ballot(upto > slot);               // `upto` is non-decreasing
     if (beyond != 0) {
       const int first = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(beyond));
@@ -185,8 +187,8 @@ __device__ __forceinline__ bool chunk_of_xcd_slot(const GmmParams &p, int rows_p
     const unsigned long long held = __ballot(rows > 0);
     const int first = (rank0 + __popcll(held & ((1ull << lane) - 1ull))) * p.n_strips;
     const int mine = (units_on_xcd(first + p.n_strips, xcd) - units_on_xcd(first, xcd)) * chunks;
-    const int upto = seen + wave_scan_add(mine, lane);
-    const int numbered = chunks0 + wave_scan_add(chunks, lane);
+    const int upto = seen + wave_scan_add(mine);
+    const int numbered = chunks0 + wave_scan_add(chunks);
     const unsigned long long beyond = __ballot(upto > pos);
     if (beyond != 0) {
       const int l = __builtin_amdgcn_readfirstlane((int)__builtin_ctzll(beyond));

@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(T4_NW * 64, 1) gmm_w8a8_tile4_nk_kernel(const 
     group_rows_chunk(p, g0, lane, carry, s0, e0);
     // (groups outside (rows_lo, rows_hi] have no tiles here: a second launch of the small tile kernel takes them)
     const int rows_g = e0 - s0;
-    const int upto = total + wave_scan_add((rows_g > p.rows_lo && rows_g <= p.rows_hi) ? ((rows_g + T4_BM - 1) / T4_BM) * n_tiles : 0, lane);
+    const int upto = total + wave_scan_add((rows_g > p.rows_lo && rows_g <= p.rows_hi) ? ((rows_g + T4_BM - 1) / T4_BM) * n_tiles : 0);
     if (wave == 0 && g0 + lane < p.e) {
       meta_end[g0 + lane] = e0;
       meta_upto[g0 + lane] = upto;

@@ -175,17 +175,19 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
   const int l32 = lane & 31, hh = lane >> 5;
 
-  // ---- tile lookup: two wave-parallel passes over group_list (count, then locate) -------------
-  // 64 groups per step with prefix scans, so the cost does not grow with the number of experts;
-  // every wave does the same work, no LDS or barrier is involved.
+  // ---- tile lookup: a wave-parallel pass over group_list counts the tiles; up to 64 groups are still in registers when the
+  // tile is located, more take a second pass.  Every wave does the same work, no LDS or barrier is involved.
   const int n_tiles = (p.n + BN - 1) / BN;
-  int total = 0;
+  int total = 0, s0 = 0, e0 = 0, tiles = 0, upto = 0;
+  auto group_tiles = [&]() {   // (groups outside (rows_lo, rows_hi] have no tiles in this launch)
+    const int rows_g = e0 - s0;
+    return (rows_g > p.rows_lo && rows_g <= p.rows_hi) ? ((rows_g + BM - 1) / BM) * n_tiles : 0;
+  };
   for (int g0 = 0, carry = 0; g0 < p.e; g0 += 64) {
-    int s0, e0;
     group_rows_chunk(p, g0, lane, carry, s0, e0);
-    const int rows_g = e0 - s0;   // (groups outside (rows_lo, rows_hi] have no tiles in this launch)
-    const int t = wave_scan_add((rows_g > p.rows_lo && rows_g <= p.rows_hi) ? ((rows_g + BM - 1) / BM) * n_tiles : 0, lane);
-    total += wave_bcast(t, 63);
+    tiles = group_tiles();
+    upto = wave_scan_add(tiles);
+    total += wave_bcast(upto, 63);
   }
   // K split across workgroups (small problems): the slices of one tile sit next to each other in the
   // grid, on the same XCD
@@ -193,36 +195,43 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   const int split = (CAN_SPLIT && p.split_k > 1) ? p.split_k : 1;
   const int per_xcd = (total + kNumXcd - 1) / kNumXcd;
   const int slot = blockIdx.x / kNumXcd;
-  const int local = slot / split, ks = slot - local * split;
+  const int local = split == 1 ? slot : slot / split, ks = slot - local * split;
   if (local >= per_xcd) return;
   const int lid = (blockIdx.x % kNumXcd) * per_xcd + local;
   if (lid >= total) return;
 
   int grp = 0, g_start = 0, g_end = 0, t_in_group = 0;
-  for (int g0 = 0, carry = 0, tiles_before = 0; g0 < p.e; g0 += 64) {
-    int s0, e0;
-    group_rows_chunk(p, g0, lane, carry, s0, e0);
-    const int rows_g = e0 - s0;
-    const int tiles = (rows_g > p.rows_lo && rows_g <= p.rows_hi) ? ((rows_g + BM - 1) / BM) * n_tiles : 0;
-    const int upto = tiles_before + wave_scan_add(tiles, lane);      // tiles of groups 0 .. g0 + lane
-    const int first = __popcll(__ballot(upto <= lid));              // `upto` is non-decreasing: first lane beyond lid
-    if (first < 64) {
-      grp = g0 + first;
-      g_start = wave_bcast(s0, first);
-      g_end = wave_bcast(e0, first);
-      t_in_group = lid - (wave_bcast(upto, first) - wave_bcast(tiles, first));
-      break;
+  auto locate = [&](int g0, int before) {   // upto: tiles of groups 0 .. g0 + lane
+    const int first = __popcll(__ballot(before + upto <= lid));   // `upto` is non-decreasing: first lane beyond lid
+    if (first == 64) return false;
+    grp = g0 + first;
+    g_start = wave_bcast(s0, first);
+    g_end = wave_bcast(e0, first);
+    t_in_group = lid - (before + wave_bcast(upto, first) - wave_bcast(tiles, first));
+    return true;
+  };
+  if (p.e <= 64) {
+    locate(0, 0);
+  } else {
+    for (int g0 = 0, carry = 0, before = 0; g0 < p.e; g0 += 64) {
+      group_rows_chunk(p, g0, lane, carry, s0, e0);
+      tiles = group_tiles();
+      upto = wave_scan_add(tiles);
+      if (locate(g0, before)) break;
+      before += wave_bcast(upto, 63);
     }
-    tiles_before = wave_bcast(upto, 63);
   }
   // order inside a group: panel of PANEL m-tiles, then n-tile, then m-tile inside the panel
   const int m_tiles = (g_end - g_start + BM - 1) / BM;
-  const int panel_tiles = PANEL * n_tiles;
-  const int panel = t_in_group / panel_tiles;
-  const int in_panel = t_in_group - panel * panel_tiles;
-  const int panel_m = min(PANEL, m_tiles - panel * PANEL);
-  const int nt = in_panel / panel_m;
-  const int mt = panel * PANEL + in_panel % panel_m;
+  int nt = t_in_group, mt = 0;
+  if (m_tiles > 1) {   // (three divisions, a hundred instructions on a cold instruction cache)
+    const int panel_tiles = PANEL * n_tiles;
+    const int panel = t_in_group / panel_tiles;
+    const int in_panel = t_in_group - panel * panel_tiles;
+    const int panel_m = min(PANEL, m_tiles - panel * PANEL);
+    nt = in_panel / panel_m;
+    mt = panel * PANEL + in_panel - nt * panel_m;
+  }
 
   const int m0 = g_start + mt * BM;
   const int n0 = nt * BN;
@@ -304,14 +313,15 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
       else b_voff[u] = (unsigned)((rho & ~31) + col_of_q(rho & 31)) * (unsigned)p.k + b_chunk[u] * 16;
     }
   }
-  auto issue_direct = [&](int kt) {
-    const int stage = kt % NSTAGE;
+  // INSIDE: the slab lies inside K, nothing has to be masked
+  auto issue_direct = [&](int kt, int stage, auto inside_c) {
+    constexpr bool INSIDE = decltype(inside_c)::value;
     const unsigned kbase = (k_first + kt) * BKT;
     // K tail, and whole slabs past K (requested by the last steps of the branch-free loop): read as zero
 #pragma unroll
     for (int u = 0; u < A_LD; ++u) {
       const int blk = wave * A_LD + u;
-      const unsigned kill_a = (kbase + a_chunk[u] * 16 >= (unsigned)p.k) ? OOB : 0u;
+      const unsigned kill_a = (!INSIDE && kbase + a_chunk[u] * 16 >= (unsigned)p.k) ? OOB : 0u;
       buffer_load_lds_b128(rx, lds_a + stage * A_STAGE + blk * 1024, a_voff[u] | kill_a, kbase);
     }
 #pragma unroll
@@ -321,13 +331,13 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
         // K block (k_first + kt) KB_PER_SLAB + blk % KB_PER_SLAB of the column group; blocks past K do not exist
         // (the last one is zero padded)
         const int kblock = (k_first + kt) * KB_PER_SLAB + blk % KB_PER_SLAB;
-        const unsigned kill_w = (kblock >= pk_blocks) ? OOB : 0u;
+        const unsigned kill_w = (!INSIDE && kblock >= pk_blocks) ? OOB : 0u;
         buffer_load_lds_b128<WNT ? 2 : 0>(rw, lds_b + stage * B_STAGE + blk * 1024, b_voff[u] | kill_w, kblock * 1024);
       } else if constexpr (KT) {
-        const unsigned kill_b = (kbase + (unsigned)b_chunk[u] >= (unsigned)p.k) ? OOB : 0u;   // K rows past K
+        const unsigned kill_b = (!INSIDE && kbase + (unsigned)b_chunk[u] >= (unsigned)p.k) ? OOB : 0u;   // K rows past K
         buffer_load_lds_b128<WNT ? 2 : 0>(rw, lds_b + stage * B_STAGE + blk * 1024, b_voff[u] | kill_b, kbase * (unsigned)(p.n / WPB));
       } else {
-        const unsigned kill_b = (kbase + b_chunk[u] * 16 >= (unsigned)p.k) ? OOB : 0u;
+        const unsigned kill_b = (!INSIDE && kbase + b_chunk[u] * 16 >= (unsigned)p.k) ? OOB : 0u;
         buffer_load_lds_b128(rw, lds_b + stage * B_STAGE + blk * 1024, b_voff[u] | kill_b, kbase);
       }
     }
@@ -335,15 +345,15 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
 
   // ---- fragment reads (one 16-byte LDS read per lane and fragment) ----------------------------
   // lane (l32, hh) of k-half kk reads row l32 of its 32-row block, 16-byte chunk c = 2 kk + hh
-  auto read_x = [&](int kt, int i, int kk) -> v4i {
-    const unsigned char *a = lds_a + (kt % NSTAGE) * A_STAGE;
+  auto read_x = [&](int stage, int i, int kk) -> v4i {
+    const unsigned char *a = lds_a + stage * A_STAGE;
     const int row = wave_m * WTM + 32 * i + l32;
     return *reinterpret_cast<const v4i *>(a + row * BKT + (((2 * kk + hh) ^ swz<BKT>(row)) << 4));
   };
-  auto read_w = [&](int kt, int f, int kk) -> v4i {
+  auto read_w = [&](int stage, int f, int kk) -> v4i {
     const int rho = wave_n * WTN + 32 * f + l32;
     if constexpr (PK) {
-      const unsigned char *b = lds_b + (kt % NSTAGE) * B_STAGE;
+      const unsigned char *b = lds_b + stage * B_STAGE;
       const int col = wave_n * WTN + 32 * f + col_of_q(l32);   // MFMA row l32 of block f is this column of the tile
       // chunk 2 kk + hh of the slab: block (2 kk + hh) / 4 of the column group's blocks in this slab, chunk % 4 inside it
       return *reinterpret_cast<const v4i *>(b + ((col >> 4) * KB_PER_SLAB + ((2 * kk + hh) >> 2)) * 1024 +
@@ -354,24 +364,24 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
       const int i = lane & 15;
       const int krow = 32 * kk + 16 * hh + (i >> 1);
       const int chunk = (wave_n * WTN + 32 * f) / 16 + ((lane >> 4) & 1);
-      const unsigned char *b = lds_b + (kt % NSTAGE) * B_STAGE + krow * BN + ((chunk ^ swz_kt<BN>(krow)) << 4) + (i & 1) * 8;
+      const unsigned char *b = lds_b + stage * B_STAGE + krow * BN + ((chunk ^ swz_kt<BN>(krow)) << 4) + (i & 1) * 8;
       uint2 lo, hi;
       lds_read_tr8_pair<8 * BN>(b, lo, hi);   // (the caller orders these reads before its own and waits for them)
       return v4i{(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
     } else {
-      const unsigned char *b = lds_b + (kt % NSTAGE) * B_STAGE;
+      const unsigned char *b = lds_b + stage * B_STAGE;
       return *reinterpret_cast<const v4i *>(b + rho * BKT + (((2 * kk + hh) ^ swz<BKT>(rho)) << 4));
     }
   };
 
   // 4-bit weights: lane i of a block of 16 names the K row whose nibble lands at position i.  Even positions become the low
   // operand words, odd ones the high ones, so positions 0, 2, 4, 6, 1, 3, 5, 7 (and 8 more) are K rows 0 .. 7 (8 .. 15).
-  auto read_w4 = [&](int kt, int f, int kk, uint2 &v) {
+  auto read_w4 = [&](int stage, int f, int kk, uint2 &v) {
     const int i = lane & 15;
     const int krow = 32 * kk + 16 * hh + (i & 8) + 4 * (i & 1) + ((i & 7) >> 1);
     const int chunk = (wave_n * WTN + 32 * f) / 32;
     const int half = w4_half_offset(krow, n0 + 32 * chunk, p.n, (lane >> 4) & 1);   // (the same for every kk)
-    lds_read_tr4(lds_b + (kt % NSTAGE) * B_STAGE + krow * (BN / WPB) + ((chunk ^ kt_swz(krow)) << 4) + half, v);
+    lds_read_tr4(lds_b + stage * B_STAGE + krow * (BN / WPB) + ((chunk ^ kt_swz(krow)) << 4) + half, v);
   };
 
   v16i acc[FN][FM];
@@ -404,21 +414,27 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   // the loop then issues the same number of loads, which keeps the vmcnt waits exact -- with
   // conditional requests the compiler has to assume the shortest path and waits for the loads it has
   // just issued.
-  auto step = [&](int kt) {
-    issue_direct(kt + AHEAD);
+  auto step = [&](int kt, int stage, auto inside_c) {
+    if constexpr (PINGPONG) issue_direct(kt + AHEAD, stage == 0 ? AHEAD : stage - 1, inside_c);
     v4i xf[KS][FM], wf[KS][FN];
     uint2 w4[KS][FN];
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
       for (int f = 0; f < FN; ++f) {
-        if constexpr (W4) read_w4(kt, f, kk, w4[kk][f]);
-        else wf[kk][f] = read_w(kt, f, kk);
+        if constexpr (W4) read_w4(stage, f, kk, w4[kk][f]);
+        else wf[kk][f] = read_w(stage, f, kk);
       }
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-      for (int i = 0; i < FM; ++i) xf[kk][i] = read_x(kt, i, kk);
+      for (int i = 0; i < FM; ++i) xf[kk][i] = read_x(stage, i, kk);
+    if constexpr (!PINGPONG) {
+      // (all fragment reads at once, then the requests, which the wave issues while the first fragments are on their way)
+      __builtin_amdgcn_sched_barrier(0);
+      issue_direct(kt + AHEAD, stage == 0 ? AHEAD : stage - 1, inside_c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if constexpr (KT) {
       // hand-issued weight reads: older than every x read, so one wait covers them
 #pragma unroll
@@ -462,14 +478,20 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64, 2) gmm_w8a8_tile_kernel
   };
 
   // prologue: slabs 0, 1, 2 requested; slab 0 published
-  issue_direct(0);
-  issue_direct(1);
-  if constexpr (AHEAD > 2) issue_direct(2);
+  static_for<AHEAD>([&](auto s_c) { issue_direct(decltype(s_c)::value, decltype(s_c)::value, std::false_type{}); });
   wait_vmcnt<(AHEAD - 1) * VM_PER_SLAB>();
   lds_barrier();
   if (behind) phase_barrier();
 
-  for (int kt = 0; kt < k_slabs; ++kt) step(kt);
+  // Whole turns of the ring while even the slab requested lies inside K: stages are constants, nothing is masked, 40
+  // instructions a slab in place of 150 (64 x 128 tile; a wave alone on its SIMD issues one per six cycles, and its MFMAs take 256).
+  // With the shorter look-up, us: one group, 297 rows, 8032 x 4304 31.4 -> 25.2; 158 rows, 1504 x 1600 10.9 -> 8.6; 801 rows, 7584 x 3760 45.2 -> 39.8;
+  // 150 shapes of 17 .. 4096 rows 0.84 .. 0.90 of the time.  What is left per slab is LDS traffic: 48 KiB of fragment reads and 24 KiB of
+  // slab writes at 128 bytes per cycle are 576 of about 730 cycles.
+  int kt = 0;
+  for (const int inside = min(k_slabs, p.k / BKT - AHEAD - k_first); kt + NSTAGE <= inside; kt += NSTAGE)
+    static_for<NSTAGE>([&](auto s_c) { step(kt + decltype(s_c)::value, decltype(s_c)::value, std::true_type{}); });
+  for (int stage = 0; kt < k_slabs; ++kt, stage = stage == NSTAGE - 1 ? 0 : stage + 1) step(kt, stage, std::false_type{});
   if (PINGPONG && !behind) phase_barrier();
 
   // ---- K split: partial tiles meet in the workspace, the last slice to arrive adds them up ----------

@@ -62,9 +62,8 @@ __global__ void __launch_bounds__(256, VEC ? 3 : 2) gmm_a8w4_kernel(const int8_t
     // never make two groups overlap); `carry` is the end of the last group of the round before
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      hi[u] = max(carry, wave_scan_max(hi[u], lane));
-      const int prev = __shfl_up(hi[u], 1);
-      lo[u] = lane == 0 ? carry : prev;
+      hi[u] = max(carry, wave_scan_max(hi[u]));
+      lo[u] = wave_from_below(hi[u], carry);
       carry = wave_bcast(hi[u], 63);
     }
 #pragma unroll
@@ -73,10 +72,10 @@ __global__ void __launch_bounds__(256, VEC ? 3 : 2) gmm_a8w4_kernel(const int8_t
       const int here = __popcll(holds);
       if (grp < 0 && seen + here > (int)blockIdx.y) {
         for (int skip = (int)blockIdx.y - seen; skip > 0; --skip) holds &= holds - 1;
-        const int src = __ffsll((long long)holds) - 1;
+        const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)holds) - 1);
         grp = g0 + 64 * u + src;
-        g_start = __shfl(lo[u], src);
-        g_end = __shfl(hi[u], src);
+        g_start = wave_bcast(lo[u], src);
+        g_end = wave_bcast(hi[u], src);
       }
       seen += here;
     }

@@ -94,7 +94,7 @@ __global__ void __launch_bounds__(1024) route_scan_kernel(int *block_hist, int *
       total += v;
     }
   }
-  const int incl = wave_scan_add(total, lane);
+  const int incl = wave_scan_add(total);
   if (lane == 63) wave_sum[wave] = incl;
   __syncthreads();
   if (tid < expert_num) {
@@ -403,7 +403,7 @@ __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsign
     }
     before[tid] = bsum;   // copy 0 now holds the folded value (a thread touches only its own expert)
   }
-  const int incl = wave_scan_add(tsum, lane);
+  const int incl = wave_scan_add(tsum);
   if (lane == 63) wave_sum[wave] = incl;
   __syncthreads();
   int offset = incl - tsum;
