@@ -35,7 +35,7 @@ from __future__ import annotations
 
 import contextlib
 import os
-from typing import List, Optional, Sequence
+from typing import List, Optional
 
 import torch
 
@@ -141,6 +141,7 @@ def widen_qint4x2(weight) -> torch.Tensor:
 
 
 # ---- framework hooks: PyTorch owns device memory and streams -------------------------------------
+# (the operators read torch tensors, allocate their results and return them in C++; graph mode's argument lists are wrapped here)
 def _wrap(t: Optional[torch.Tensor]):
     if t is None:
         return None
@@ -164,26 +165,15 @@ def _wrap_list(ts):
     return [_wrap(t) for t in ts]
 
 
-_CUDA = torch.device("cuda")
-
-
-def _allocate(type_id: int, shape: Sequence[int]):
-    # (called once or twice per operator call from the C++ layer: kept free of argument checks and string parsing)
-    t = torch.empty(tuple(shape), dtype=_DTYPES[type_id], device=_CUDA)
-    return _C.Tensor(t.data_ptr(), type_id, list(shape), list(t.stride()), t)
-
-
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _current_stream() -> int:
-    # the raw getter skips the construction of a torch.cuda.Stream object (a few microseconds per operator call)
-    if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
     return torch.cuda.current_stream().cuda_stream
 
 
-_C._set_framework_hooks(_allocate, _current_stream)
+# the raw getter skips this function and the construction of a torch.cuda.Stream object
+_C._set_framework_hooks(_current_stream, _raw_stream, QInt4x2)
 
 
 def plan_cache_stats():
@@ -200,10 +190,9 @@ def grouped_matmul(x, weight, group_list, bias=None, scale=None, per_token_scale
     if _mode == GRAPH_MODE:
         args = [_wrap(x), _wrap(weight), _wrap(group_list), _wrap(bias), _wrap(scale), _wrap(per_token_scale),
                 _wrap(antiquant_scale), bool(transpose_a), bool(transpose_b), int(x_format), od]
-        return _C._graph_run("grouped_matmul", args)[0].owner
-    return _C.grouped_matmul(_wrap(x), _wrap(weight), _wrap(group_list), _wrap(bias), _wrap(scale),
-                             _wrap(per_token_scale), _wrap(antiquant_scale), bool(transpose_a), bool(transpose_b),
-                             int(x_format), od).owner
+        return _C._graph_run("grouped_matmul", args)[0]
+    return _C.grouped_matmul(x, weight, group_list, bias, scale, per_token_scale, antiquant_scale, bool(transpose_a),
+                             bool(transpose_b), int(x_format), od)
 
 
 def grouped_matmul_v4_cops(x, weight, bias=None, scale=None, offset=None, antiquant_scale=None, antiquant_offset=None,
@@ -212,18 +201,15 @@ def grouped_matmul_v4_cops(x, weight, bias=None, scale=None, offset=None, antiqu
                            weight_format="ND", output_dtype=None) -> List[torch.Tensor]:
     """List-of-tensor grouped matmul (GMM V4); returns a list of tensors."""
     od = dtype_to_type_id(output_dtype)
-    lists = [_wrap_list(v) for v in (x, weight, bias, scale, offset, antiquant_scale, antiquant_offset,
-                                     per_token_scale)]
-    acts = [_wrap_list(v) for v in (activation_input, activation_quant_scale, activation_quant_offset)]
-    gl = _wrap(group_list)
     if _mode == GRAPH_MODE:
-        args = lists + [gl] + acts + [int(split_item), int(group_type), int(group_list_type), int(act_type),
-                                      str(weight_format), od]
-        outs = _C._graph_run("grouped_matmul_v4_cops", args)
-    else:
-        outs = _C.grouped_matmul_v4_cops(*lists, gl, *acts, int(split_item), int(group_type), int(group_list_type),
-                                         int(act_type), str(weight_format), od)
-    return [o.owner for o in outs]
+        lists = [_wrap_list(v) for v in (x, weight, bias, scale, offset, antiquant_scale, antiquant_offset,
+                                         per_token_scale)]
+        acts = [_wrap_list(v) for v in (activation_input, activation_quant_scale, activation_quant_offset)]
+        return _C._graph_run("grouped_matmul_v4_cops", lists + [_wrap(group_list)] + acts +
+                             [int(split_item), int(group_type), int(group_list_type), int(act_type), str(weight_format), od])
+    return _C.grouped_matmul_v4_cops(x, weight, bias, scale, offset, antiquant_scale, antiquant_offset, per_token_scale, group_list,
+                                     activation_input, activation_quant_scale, activation_quant_offset, int(split_item),
+                                     int(group_type), int(group_list_type), int(act_type), str(weight_format), od)
 
 
 def quant_batch_matmul(x1, x2, scale, offset=None, bias=None, pertoken_scale=None, transpose_x1=False,
@@ -233,9 +219,9 @@ def quant_batch_matmul(x1, x2, scale, offset=None, bias=None, pertoken_scale=Non
     if _mode == GRAPH_MODE:
         args = [_wrap(x1), _wrap(x2), _wrap(scale), _wrap(offset), _wrap(bias), _wrap(pertoken_scale),
                 bool(transpose_x1), bool(transpose_x2), str(x2_format), od]
-        return _C._graph_run("quant_batch_matmul", args)[0].owner
-    return _C.quant_batch_matmul(_wrap(x1), _wrap(x2), _wrap(scale), _wrap(offset), _wrap(bias), _wrap(pertoken_scale),
-                                 bool(transpose_x1), bool(transpose_x2), str(x2_format), od).owner
+        return _C._graph_run("quant_batch_matmul", args)[0]
+    return _C.quant_batch_matmul(x1, x2, scale, offset, bias, pertoken_scale, bool(transpose_x1), bool(transpose_x2),
+                                 str(x2_format), od)
 
 
 def grouped_matmul_w4(x, weight, group_list, bias, x_scale, weight_scale):
@@ -246,10 +232,10 @@ def grouped_matmul_w4(x, weight, group_list, bias, x_scale, weight_scale):
     tensor (torch has no 4-bit type); group_list int32 [e], cumulative; bias float32 [e, n] (the reference kernel's
     compensation term 8 * column sums of the dequantised weight: checked, not read, the nibbles are multiplied signed
     here); x_scale float32 [m]; weight_scale float32 [e, k/group_size, n]."""
-    args = [_wrap(x), _wrap(weight), _wrap(group_list), _wrap(bias), _wrap(x_scale), _wrap(weight_scale)]
     if _mode == GRAPH_MODE:
-        return _C._graph_run("grouped_matmul_w4", args)[0].owner
-    return _C.grouped_matmul_w4(*args).owner
+        return _C._graph_run("grouped_matmul_w4", [_wrap(x), _wrap(weight), _wrap(group_list), _wrap(bias), _wrap(x_scale),
+                                                   _wrap(weight_scale)])[0]
+    return _C.grouped_matmul_w4(x, weight, group_list, bias, x_scale, weight_scale)
 
 
 def moe_init_routing_v2(x, expert_idx, active_num, expert_capacity, expert_num, drop_pad_mode,
@@ -261,10 +247,10 @@ def moe_init_routing_v2(x, expert_idx, active_num, expert_capacity, expert_num, 
                 int(expert_tokens_count_or_cumsum_flag), bool(expert_tokens_before_capacity_flag)]
         outs = _C._graph_run("moe_init_routing_v2", args)
     else:
-        outs = _C.moe_init_routing_v2(_wrap(x), _wrap(expert_idx), int(active_num), int(expert_capacity), int(expert_num),
+        outs = _C.moe_init_routing_v2(x, expert_idx, int(active_num), int(expert_capacity), int(expert_num),
                                       int(drop_pad_mode), int(expert_tokens_count_or_cumsum_flag),
                                       bool(expert_tokens_before_capacity_flag))
-    return tuple(o.owner for o in outs)
+    return tuple(outs)
 
 
 def moe_init_routing_quant(x, expert_idx, expert_num, expert_tokens_count_or_cumsum_flag=1):
@@ -279,8 +265,8 @@ def moe_init_routing_quant(x, expert_idx, expert_num, expert_tokens_count_or_cum
         outs = _C._graph_run("moe_init_routing_quant", [_wrap(x), _wrap(expert_idx), int(expert_num),
                                                         int(expert_tokens_count_or_cumsum_flag)])
     else:
-        outs = _C.moe_init_routing_quant(_wrap(x), _wrap(expert_idx), int(expert_num), int(expert_tokens_count_or_cumsum_flag))
-    return tuple(o.owner for o in outs)
+        outs = _C.moe_init_routing_quant(x, expert_idx, int(expert_num), int(expert_tokens_count_or_cumsum_flag))
+    return tuple(outs)
 
 
 def moe_token_unpermute(permuted_tokens, sorted_indices, probs, padded_mode=False, restore_shape=None):
@@ -289,9 +275,9 @@ def moe_token_unpermute(permuted_tokens, sorted_indices, probs, padded_mode=Fals
     if _mode == GRAPH_MODE:
         args = [_wrap(permuted_tokens), _wrap(sorted_indices), _wrap(probs), bool(padded_mode),
                 None if restore_shape is None else str(tuple(restore_shape))]
-        return _C._graph_run("moe_token_unpermute", args)[0].owner
-    return _C.moe_token_unpermute(_wrap(permuted_tokens), _wrap(sorted_indices), _wrap(probs), bool(padded_mode),
-                                  None if restore_shape is None else [int(v) for v in restore_shape]).owner
+        return _C._graph_run("moe_token_unpermute", args)[0]
+    return _C.moe_token_unpermute(permuted_tokens, sorted_indices, probs, bool(padded_mode),
+                                  None if restore_shape is None else [int(v) for v in restore_shape])
 
 
 def trans_data(tensor, transdata_type=1, nd_shape=None, transposed=False):

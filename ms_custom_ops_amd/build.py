@@ -111,7 +111,9 @@ def build_pybind(verbose: bool = False) -> str:
     """Compile the C++ operator layer (framework + one translation unit per op) into a pybind11
     module that links against libmsco_gmm.so."""
     import pybind11
+    import torch
 
+    torch_dir = os.path.dirname(torch.__file__)
     cxx = shutil.which("g++") or "g++"
     srcs = []
     for root, _, files in os.walk(os.path.join(CSRC, "ops")):
@@ -124,7 +126,10 @@ def build_pybind(verbose: bool = False) -> str:
 
     def compile_one(src):
         obj = os.path.join(OBJ_DIR, os.path.relpath(src, CSRC).replace(os.sep, "_").replace(".cc", ".o"))
-        out = _run([cxx] + flags + ["-c", src, "-o", obj])
+        # (torch's headers are read by one file; its directory's own pybind11 must not be found by the others)
+        extra = ["-I", os.path.join(torch_dir, "include"), "-I", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+                 "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch.compiled_with_cxx11_abi())] if src.endswith("torch_bridge.cc") else []
+        out = _run([cxx] + flags + extra + ["-c", src, "-o", obj])
         if verbose and out.strip():
             print(out)
         return obj
@@ -132,7 +137,9 @@ def build_pybind(verbose: bool = False) -> str:
     with cf.ThreadPoolExecutor(max_workers=8) as pool:
         objs = list(pool.map(compile_one, srcs))
     target = pybind_module_path()
-    _run([cxx, "-shared", "-o", target] + objs + ["-L", LIB_DIR, "-lmsco_gmm", "-Wl,-rpath,$ORIGIN/lib"])
+    _run([cxx, "-shared", "-o", target] + objs + ["-L", LIB_DIR, "-lmsco_gmm", "-Wl,-rpath,$ORIGIN/lib",
+                                                  "-L", os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+                                                  "-Wl,-rpath," + os.path.join(torch_dir, "lib")])
     return target
 
 

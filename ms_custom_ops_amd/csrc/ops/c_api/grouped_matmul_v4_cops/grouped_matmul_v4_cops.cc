@@ -340,20 +340,20 @@ REG_GRAPH_MODE_OP(grouped_matmul_v4_cops, ms_custom_ops::GroupedMatmulV4CopsFunc
 // PYBOOST MODE IMPLEMENTATION
 // =============================================================================
 namespace ms_custom_ops {
-static TensorVec GetOptionalTensorList(const std::optional<TensorVec> &tensor_list) {
-  return tensor_list.has_value() ? tensor_list.value() : TensorVec();
+static std::optional<TensorVec> OptionalList(const TensorListArg &arg) {
+  return arg.given ? std::optional<TensorVec>(arg.list) : std::nullopt;
 }
 
 std::vector<ms::Tensor> grouped_matmul_v4_cops_custom(
-  const TensorVec &x, const TensorVec &weight, const std::optional<TensorVec> &bias,
-  const std::optional<TensorVec> &scale, const std::optional<TensorVec> &offset,
-  const std::optional<TensorVec> &antiquant_scale, const std::optional<TensorVec> &antiquant_offset,
-  const std::optional<TensorVec> &per_token_scale, const std::optional<ms::Tensor> &group_list,
-  const std::optional<TensorVec> &activation_input, const std::optional<TensorVec> &activation_quant_scale,
-  const std::optional<TensorVec> &activation_quant_offset, const int64_t &split_item, const int64_t &group_type,
+  const TensorListArg &x_arg, const TensorListArg &weight_arg, const TensorListArg &bias, const TensorListArg &scale, const TensorListArg &offset,
+  const TensorListArg &antiquant_scale, const TensorListArg &antiquant_offset, const TensorListArg &per_token_scale,
+  const std::optional<ms::Tensor> &group_list, const TensorListArg &activation_input, const TensorListArg &activation_quant_scale,
+  const TensorListArg &activation_quant_offset, const int64_t &split_item, const int64_t &group_type,
   const int64_t &group_list_type, const int64_t &act_type, const std::string &weight_format,
   const std::optional<int64_t> &output_dtype) {
-  auto output_types = InferOutputTypes(x, weight, scale, output_dtype);
+  if (!x_arg.given || !weight_arg.given) MS_EXCEPTION_TYPE << "For " << kGroupedMatmulV4CopsName << ", 'x' and 'weight' must be lists of tensors.";
+  const TensorVec &x = x_arg.list, &weight = weight_arg.list;
+  auto output_types = InferOutputTypes(x, weight, OptionalList(scale), output_dtype);
   auto output_shapes = InferOutputShapes(x, weight, group_list, group_type, weight_format);
   if (output_types.size() != output_shapes.size()) {
     MS_EXCEPTION_VALUE << "For " << kGroupedMatmulV4CopsName
@@ -364,16 +364,16 @@ std::vector<ms::Tensor> grouped_matmul_v4_cops_custom(
   V4Args args;
   args.x = x;
   args.weight = weight;
-  args.bias = GetOptionalTensorList(bias);
-  args.scale = GetOptionalTensorList(scale);
-  args.offset = GetOptionalTensorList(offset);
-  args.antiquant_scale = GetOptionalTensorList(antiquant_scale);
-  args.antiquant_offset = GetOptionalTensorList(antiquant_offset);
-  args.per_token_scale = GetOptionalTensorList(per_token_scale);
+  args.bias = bias.list;
+  args.scale = scale.list;
+  args.offset = offset.list;
+  args.antiquant_scale = antiquant_scale.list;
+  args.antiquant_offset = antiquant_offset.list;
+  args.per_token_scale = per_token_scale.list;
   args.group_list = GetTensorOrEmpty(group_list);
-  args.activation_input = GetOptionalTensorList(activation_input);
-  args.activation_quant_scale = GetOptionalTensorList(activation_quant_scale);
-  args.activation_quant_offset = GetOptionalTensorList(activation_quant_offset);
+  args.activation_input = activation_input.list;
+  args.activation_quant_scale = activation_quant_scale.list;
+  args.activation_quant_offset = activation_quant_offset.list;
   args.split_item = split_item;
   args.group_type = group_type;
   args.group_list_type = group_list_type;
@@ -393,11 +393,11 @@ std::vector<ms::Tensor> grouped_matmul_v4_cops_custom(
 
 MS_CUSTOM_OPS_EXTENSION_MODULE(m) {
   m.def("grouped_matmul_v4_cops", &ms_custom_ops::grouped_matmul_v4_cops_custom, "GroupedMatmulV4", pybind11::arg("x"),
-        pybind11::arg("weight"), pybind11::arg("bias") = std::nullopt, pybind11::arg("scale") = std::nullopt,
-        pybind11::arg("offset") = std::nullopt, pybind11::arg("antiquant_scale") = std::nullopt,
-        pybind11::arg("antiquant_offset") = std::nullopt, pybind11::arg("per_token_scale") = std::nullopt,
-        pybind11::arg("group_list") = std::nullopt, pybind11::arg("activation_input") = std::nullopt,
-        pybind11::arg("activation_quant_scale") = std::nullopt, pybind11::arg("activation_quant_offset") = std::nullopt,
+        pybind11::arg("weight"), pybind11::arg("bias") = pybind11::none(), pybind11::arg("scale") = pybind11::none(),
+        pybind11::arg("offset") = pybind11::none(), pybind11::arg("antiquant_scale") = pybind11::none(),
+        pybind11::arg("antiquant_offset") = pybind11::none(), pybind11::arg("per_token_scale") = pybind11::none(),
+        pybind11::arg("group_list") = std::nullopt, pybind11::arg("activation_input") = pybind11::none(),
+        pybind11::arg("activation_quant_scale") = pybind11::none(), pybind11::arg("activation_quant_offset") = pybind11::none(),
         pybind11::arg("split_item") = 0, pybind11::arg("group_type") = -1, pybind11::arg("group_list_type") = 0,
         pybind11::arg("act_type") = 0, pybind11::arg("weight_format") = std::string("ND"),
         pybind11::arg("output_dtype") = std::nullopt);

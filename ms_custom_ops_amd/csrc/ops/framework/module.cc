@@ -9,18 +9,61 @@
 #include <sstream>
 
 #include "ops/framework/hip_backend/hip_gmm_runner.h"
+#include "ops/framework/torch_bridge.h"
 
 namespace py = pybind11;
 
 namespace ms_custom_ops {
 ms::Tensor AllocateTensor(TypeId type, const ShapeVector &shape) {
-  auto &hooks = FrameworkHooks::Get();
-  if (hooks.allocate.is_none() || !hooks.allocate) {
-    MS_LOG_EXCEPTION << "No device allocator is registered: import the ms_custom_ops_amd package (it registers the "
-                        "host framework's allocator) before calling an operator.";
-  }
   py::gil_scoped_acquire gil;
-  return hooks.allocate(static_cast<int>(type), shape).cast<ms::Tensor>();
+  void *data = nullptr;
+  PyObject *tensor = NewTorchTensor(static_cast<int>(type), shape.data(), shape.size(), &data);
+  if (tensor == nullptr) throw py::error_already_set();
+  return ms::Tensor(reinterpret_cast<uintptr_t>(data), static_cast<int>(type), shape, ShapeVector(), py::reinterpret_steal<py::object>(tensor));
+}
+
+bool TensorFromObject(py::handle object, ms::Tensor *tensor) {
+  if (!object || object.is_none()) return false;
+  TorchTensorView view;
+  py::object held = py::reinterpret_borrow<py::object>(object);
+  int found = ViewTorchTensor(object.ptr(), &view);
+  const auto &hooks = FrameworkHooks::Get();
+  const bool nibbles = found == 0 && hooks.qint4x2 && py::isinstance(object, hooks.qint4x2);
+  if (nibbles) {
+    held = object.attr("tensor");
+    found = ViewTorchTensor(held.ptr(), &view);
+  }
+  if (found < 0) throw py::error_already_set();
+  if (found == 0) {
+    if (py::type::handle_of(object).is(py::type::of<ms::Tensor>())) return false;
+    throw py::type_error("expected a torch.Tensor, got " + std::string(py::str(py::type::handle_of(object).attr("__name__"))));
+  }
+  if (!view.on_gpu) {
+    throw py::value_error("ms_custom_ops_amd operators take GPU tensors; got a tensor on " + std::string(py::str(held.attr("device"))));
+  }
+  const int type_id = nibbles ? static_cast<int>(kNumberTypeInt4) : view.type_id;
+  if (type_id == 0) throw py::type_error("unsupported dtype " + std::string(py::str(held.attr("dtype"))));
+  ShapeVector shape(view.sizes, view.sizes + view.dims), strides;
+  if (!ms::Tensor::ContiguousStrides(view.sizes, view.strides, view.dims)) strides.assign(view.strides, view.strides + view.dims);
+  *tensor = ms::Tensor(reinterpret_cast<uintptr_t>(view.data), type_id, std::move(shape), std::move(strides), std::move(held));
+  return true;
+}
+
+TensorListArg TensorListFromObject(py::handle object) {
+  TensorListArg arg;
+  if (object.is_none()) return arg;
+  TorchTensorView view;
+  const int found = ViewTorchTensor(object.ptr(), &view);
+  if (found < 0) throw py::error_already_set();
+  if (found > 0) throw py::type_error("expected a list of tensors");
+  arg.given = true;
+  for (py::handle item : py::iter(object)) {
+    arg.list.emplace_back();
+    if (TensorFromObject(item, &arg.list.back())) continue;
+    if (item.is_none()) throw py::type_error("expected a list of tensors, got a list with None in it");
+    arg.list.back() = item.cast<ms::Tensor>();
+  }
+  return arg;
 }
 
 namespace {
@@ -42,6 +85,11 @@ void *CurrentStream() {
   auto &hooks = FrameworkHooks::Get();
   if (hooks.current_stream.is_none() || !hooks.current_stream) return nullptr;
   py::gil_scoped_acquire gil;
+  if (hooks.raw_stream && !hooks.raw_stream.is_none()) {
+    const int device = CurrentTorchDevice();
+    if (device < 0) throw py::error_already_set();
+    return reinterpret_cast<void *>(hooks.raw_stream(device).cast<uintptr_t>());
+  }
   return reinterpret_cast<void *>(hooks.current_stream().cast<uintptr_t>());
 }
 
@@ -50,7 +98,7 @@ KernelTensor ToKernelTensor(const py::handle &obj) {
   KernelTensor kt;
   if (obj.is_none()) return kt;
   kt.is_none = false;
-  if (py::isinstance<ms::Tensor>(obj)) {
+  if (py::type::handle_of(obj).is(py::type::of<ms::Tensor>())) {
     kt.tensor = obj.cast<ms::Tensor>();
   } else if (py::isinstance<py::bool_>(obj)) {
     kt.value = obj.cast<bool>();
@@ -198,10 +246,11 @@ PYBIND11_MODULE(MS_EXTENSION_NAME, m) {
     .def("is_defined", &ms::Tensor::is_defined)
     .def("is_contiguous", &ms::Tensor::is_contiguous);
 
-  m.def("_set_framework_hooks", [](py::object allocate, py::object current_stream) {
+  m.def("_set_framework_hooks", [](py::object current_stream, py::object raw_stream, py::object qint4x2) {
     auto &hooks = ms_custom_ops::FrameworkHooks::Get();
-    hooks.allocate = std::move(allocate);
     hooks.current_stream = std::move(current_stream);
+    hooks.raw_stream = std::move(raw_stream);
+    hooks.qint4x2 = std::move(qint4x2);
   });
   m.def("_graph_run", &ms_custom_ops::GraphRun, "Run a registered op through the graph-mode kernel module");
   m.def("_graph_infer", &ms_custom_ops::GraphInfer, "InferShape / InferType of a registered op");

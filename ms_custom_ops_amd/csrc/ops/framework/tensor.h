@@ -3,13 +3,15 @@
 // The reference's operator glue is written against MindSpore's ms::Tensor / TypeId
 // (ops/framework/utils.h:24, ops/framework/module.h:24).  This backend has no MindSpore: a tensor is
 // a device pointer plus dtype, shape and strides, handed over by the host framework (PyTorch-ROCm
-// tensors are converted by the Python package), and `owner` keeps the framework object alive.
+// tensors are converted as an operator's arguments are read, torch_bridge.h), and `owner` keeps the framework object alive.
 #ifndef MS_CUSTOM_OPS_FRAMEWORK_TENSOR_H_
 #define MS_CUSTOM_OPS_FRAMEWORK_TENSOR_H_
 
 #include <pybind11/pybind11.h>
+#include <pybind11/stl.h>
 
 #include <cstdint>
+#include <memory>
 #include <numeric>
 #include <optional>
 #include <string>
@@ -75,52 +77,102 @@ namespace ms {
 using mindspore::ShapeVector;
 using mindspore::TypeId;
 
+// Copies share one description (an operator hands its tensors on several times per call).
 class Tensor {
  public:
   Tensor() = default;
   Tensor(uintptr_t data, int type_id, ShapeVector shape, ShapeVector strides, pybind11::object owner)
-      : data_(reinterpret_cast<void *>(data)),
-        dtype_(static_cast<TypeId>(type_id)),
-        shape_(std::move(shape)),
-        strides_(std::move(strides)),
-        owner_(std::move(owner)),
-        defined_(true) {}
+      : d_(std::make_shared<Description>(Description{reinterpret_cast<void *>(data), static_cast<TypeId>(type_id), std::move(shape),
+                                                     std::move(strides), std::move(owner)})) {}
 
-  bool is_defined() const { return defined_; }
-  void *GetDataPtr() const { return data_; }
-  TypeId data_type() const { return dtype_; }
-  const ShapeVector &shape() const { return shape_; }
-  const ShapeVector &strides() const { return strides_; }
-  const pybind11::object &owner() const { return owner_; }
+  bool is_defined() const { return d_ != nullptr; }
+  void *GetDataPtr() const { return d_ ? d_->data : nullptr; }
+  TypeId data_type() const { return d_ ? d_->dtype : mindspore::kMetaTypeNone; }
+  const ShapeVector &shape() const { return d_ ? d_->shape : Nothing(); }
+  const ShapeVector &strides() const { return d_ ? d_->strides : Nothing(); }   // may be empty where contiguous
+  pybind11::object owner() const { return d_ ? d_->owner : pybind11::object(); }
   int64_t numel() const {
-    return std::accumulate(shape_.begin(), shape_.end(), static_cast<int64_t>(1), std::multiplies<int64_t>());
+    return std::accumulate(shape().begin(), shape().end(), static_cast<int64_t>(1), std::multiplies<int64_t>());
   }
-  size_t nbytes() const { return static_cast<size_t>(numel()) * mindspore::TypeIdSize(dtype_); }
-  bool is_contiguous() const {
-    if (strides_.empty()) return true;
+  size_t nbytes() const { return static_cast<size_t>(numel()) * mindspore::TypeIdSize(data_type()); }
+  bool is_contiguous() const { return strides().empty() || ContiguousStrides(shape().data(), strides().data(), shape().size()); }
+  static bool ContiguousStrides(const int64_t *shape, const int64_t *strides, size_t dims) {
     int64_t expect = 1;
-    for (int i = static_cast<int>(shape_.size()) - 1; i >= 0; --i) {
-      if (shape_[i] != 1 && strides_[i] != expect) return false;
-      expect *= shape_[i];
+    for (size_t i = dims; i-- > 0;) {
+      if (shape[i] != 1 && strides[i] != expect) return false;
+      expect *= shape[i];
     }
     return true;
   }
   // A view on a sub-range of the same buffer (used to walk batches).
   Tensor Slice(int64_t elem_offset, ShapeVector shape) const {
-    Tensor t = *this;
-    t.data_ = static_cast<char *>(data_) + elem_offset * static_cast<int64_t>(mindspore::TypeIdSize(dtype_));
-    t.shape_ = std::move(shape);
-    t.strides_.clear();
-    return t;
+    char *at = static_cast<char *>(GetDataPtr()) + elem_offset * static_cast<int64_t>(mindspore::TypeIdSize(data_type()));
+    return Tensor(reinterpret_cast<uintptr_t>(at), data_type(), std::move(shape), ShapeVector(), owner());
   }
 
  private:
-  void *data_{nullptr};
-  TypeId dtype_{mindspore::kMetaTypeNone};
-  ShapeVector shape_;
-  ShapeVector strides_;
-  pybind11::object owner_;
-  bool defined_{false};
+  struct Description {
+    void *data;
+    TypeId dtype;
+    ShapeVector shape;
+    ShapeVector strides;
+    pybind11::object owner;
+  };
+  static const ShapeVector &Nothing() {
+    static const ShapeVector nothing;
+    return nothing;
+  }
+  std::shared_ptr<const Description> d_;
 };
 }  // namespace ms
+
+namespace ms_custom_ops {
+// A torch.Tensor or a QInt4x2 as an operator sees it.  False for None and for objects of the compiled Tensor class; a tensor that is not
+// on the GPU or has a dtype without a TypeId raises, and so does anything else.
+bool TensorFromObject(pybind11::handle object, ms::Tensor *tensor);
+// an operator's list argument: None, or any iterable of tensors but a tensor itself
+struct TensorListArg {
+  bool given{false};
+  std::vector<ms::Tensor> list;
+};
+TensorListArg TensorListFromObject(pybind11::handle object);
+}  // namespace ms_custom_ops
+
+// Operators take the host framework's tensors and return them: no Python object stands between.
+namespace pybind11 {
+namespace detail {
+template <>
+class type_caster<ms::Tensor> : public type_caster_base<ms::Tensor> {
+  using Base = type_caster_base<ms::Tensor>;
+
+ public:
+  bool load(handle src, bool convert) {
+    if (!ms_custom_ops::TensorFromObject(src, &local_)) return Base::load(src, convert);
+    this->value = &local_;
+    return true;
+  }
+  static handle cast(const ms::Tensor &src, return_value_policy policy, handle parent) {
+    const object owner = src.owner();
+    return owner && !owner.is_none() ? owner.inc_ref() : Base::cast(src, policy, parent);
+  }
+  static handle cast(ms::Tensor &&src, return_value_policy policy, handle parent) { return cast(static_cast<const ms::Tensor &>(src), policy == return_value_policy::move ? return_value_policy::copy : policy, parent); }
+  static handle cast(const ms::Tensor *src, return_value_policy policy, handle parent) { return src ? cast(*src, policy, parent) : none().release(); }
+
+ private:
+  ms::Tensor local_;
+};
+template <>
+class type_caster<ms_custom_ops::TensorListArg> {
+ public:
+  PYBIND11_TYPE_CASTER(ms_custom_ops::TensorListArg, const_name("list"));
+  bool load(handle src, bool) {
+    value = ms_custom_ops::TensorListFromObject(src);
+    return true;
+  }
+  static handle cast(const ms_custom_ops::TensorListArg &src, return_value_policy policy, handle parent) {
+    return src.given ? make_caster<std::vector<ms::Tensor>>::cast(src.list, policy, parent) : none().release();
+  }
+};
+}  // namespace detail
+}  // namespace pybind11
 #endif  // MS_CUSTOM_OPS_FRAMEWORK_TENSOR_H_

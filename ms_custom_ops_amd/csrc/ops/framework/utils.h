@@ -79,10 +79,11 @@ struct ExceptionThrower {
 
 // ---- host-framework hooks -----------------------------------------------------------------------
 // The host framework (the Python package on top of PyTorch-ROCm) owns device memory and streams:
-// it registers an allocator and a current-stream getter once at import.
+// it registers a current-stream getter and its 4-bit marker class once at import.
 struct FrameworkHooks {
-  pybind11::object allocate;        // (type_id:int, shape:list[int]) -> ms::Tensor
   pybind11::object current_stream;  // () -> int (hipStream_t)
+  pybind11::object raw_stream;      // (device:int) -> int, or None: the same without a Python function around it
+  pybind11::object qint4x2;         // class whose objects carry 4-bit data in `.tensor`
   static FrameworkHooks &Get() {
     static FrameworkHooks *hooks = new FrameworkHooks();  // leaked on purpose: outlives the interpreter
     return *hooks;
