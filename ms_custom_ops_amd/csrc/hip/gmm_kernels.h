@@ -16,7 +16,9 @@ enum TileCfg : int {
   TILE_ROWS160 = 8,   // ... of up to 160 rows, two workgroups per CU, two K blocks of weights in flight
   TILE_64x256_W4B = 9,    // 4-bit weights [E,K,N/2]
   TILE_128x256_W4B = 10,
-  TILE_CFG_COUNT = 11
+  TILE_32x128 = 11,   // a few rows on [E,K,N] and [E,N,K] weights, two waves side by side, two workgroups per CU
+  TILE_32x256 = 12,   // ... on [E,K,N] weights, four waves side by side
+  TILE_CFG_COUNT = 13
 };
 
 // MFMA tile kernel for W8A8 (prefill shapes).  nk: weights stored [E,N,K]; packed: the packed layout (nk is ignored).

@@ -668,9 +668,10 @@ static hipError_t launch_cfg(const GmmParams &p, hipStream_t stream) {
     attr_set = true;
   }
   const long long n_tiles = (p.n + BN - 1) / BN;
-  // every non-empty group adds at most one partial tile; a launch for the small groups only: that many tiles per group
-  const long long m_tiles_ub = p.rows_hi < p.m ? std::min<long long>((p.m + BM - 1) / BM + p.e, (long long)p.e * ((p.rows_hi + BM - 1) / BM))
-                                               : (p.m + BM - 1) / BM + p.e;
+  // every group that holds rows adds at most one partial tile, and at most min(E, M) groups do (34 rows over 128 experts: the
+  // workgroups of the other 94 would take a slot on a CU each to find that out); a launch for the small groups only: that many tiles per group
+  const long long with_rows = (p.m + BM - 1) / BM + std::min(p.e, p.m);
+  const long long m_tiles_ub = p.rows_hi < p.m ? std::min<long long>(with_rows, (long long)p.e * ((p.rows_hi + BM - 1) / BM)) : with_rows;
   const long long total_ub = m_tiles_ub * n_tiles;
   const long long grid = ((total_ub + kNumXcd - 1) / kNumXcd) * kNumXcd * (p.split_k > 1 ? p.split_k : 1);
   if (grid <= 0) return hipSuccess;
@@ -694,6 +695,22 @@ static hipError_t launch_small(const GmmParams &p, int layout, hipStream_t strea
                         : launch_cfg<BM, BN, 2, 2, 4, false, 2, false, true>(p, stream);
 }
 
+// A few rows: 32-row tiles, 128-byte K slabs in a 3-stage ring.  The waves sit side by side in columns, so no fragment of the
+// weights is read twice: 44 KiB of LDS traffic per slab of 128 columns (16 KiB of weight and 8 KiB of x
+// fragments read, 20 KiB written) in place of the 72 KiB of a 64 x 128 tile, and 63 KB of LDS, so two workgroups share a CU.  With a K
+// split, us, 64 x 128 -> 32 x 128: one group, 9 rows, 2752 x 5024, [E,K,N] 12.4 -> 10.9; 24 rows, 4032 x 8800 14.6 -> 13.7; [E,N,K], 4 rows,
+// 3712 x 1264 10.4 -> 9.1.  (Four stages, one workgroup per CU: within 3 % with one group, 7 % slower with many.)  A workgroup of
+// four waves and 256 columns halves the x traffic once more (84 KiB per 256 columns) and has 72 KiB of slabs in flight: 8
+// experts, 6 rows, 3296 x 8480 35.8 -> 30.3; 64 experts, 48 rows, 4768 x 1568 57.9 -> 46.1.  (Two stages and two workgroups per CU: 62
+// there, and 67 against 72 only where workgroups are many: 280 rows over 32 experts, 1568 x 8400.)
+static hipError_t launch_32_rows(const GmmParams &p, int bn, int layout, hipStream_t stream) {
+  if (layout == 0 && bn == 128) return launch_cfg<32, 128, 1, 2, 3, false, 4>(p, stream);
+  if (layout != 2) return hipErrorInvalidValue;   // (packed weights have streaming kernels of their own)
+  if (bn == 128)
+    return p.w_nontemporal ? launch_cfg<32, 128, 1, 2, 3, false, 4, true, true>(p, stream) : launch_cfg<32, 128, 1, 2, 3, false, 4, false, true>(p, stream);
+  return p.w_nontemporal ? launch_cfg<32, 256, 1, 4, 3, false, 4, true, true>(p, stream) : launch_cfg<32, 256, 1, 4, 3, false, 4, false, true>(p, stream);
+}
+
 // nk: weights stored [E,N,K]; packed: the blocked layout; neither: [E,K,N] (N a multiple of 16, which the plan's
 // alignment rule guarantees for every MFMA kernel)
 hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool packed, hipStream_t stream) {
@@ -711,6 +728,8 @@ hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool pack
   switch (tile_cfg) {
     case TILE_128x128: return launch_small<128, 128>(p, layout, stream);
     case TILE_64x128: return launch_small<64, 128>(p, layout, stream);
+    case TILE_32x128: return launch_32_rows(p, 128, layout, stream);
+    case TILE_32x256: return launch_32_rows(p, 256, layout, stream);
     case TILE_256x256:   // eight waves, two per SIMD
       return layout == 1 ? launch_cfg<256, 256, 2, 4, 4, true>(p, stream)
            : layout == 0 ? launch_cfg<256, 256, 2, 4>(p, stream)
@@ -751,6 +770,8 @@ const char *tile_cfg_name(int tile_cfg) {
     case TILE_ROWS256: return "rows256";
     case TILE_ROWS128: return "rows128";
     case TILE_ROWS160: return "rows160";
+    case TILE_32x128: return "32x128";
+    case TILE_32x256: return "32x256";
     case TILE_64x256_W4B: return "64x256_4bit";
     case TILE_128x256_W4B: return "128x256_4bit";
     default: return "?";
@@ -777,6 +798,8 @@ void tile_cfg_dims(int tile_cfg, int *bm, int *bn) {
     case TILE_256x256: case TILE_256x256_W4: case TILE_256x256_W4_MFMA32: case TILE_ROWS256: case TILE_ROWS160: *bm = 256; *bn = 256; break;
     case TILE_128x128: *bm = 128; *bn = 128; break;
     case TILE_128x256: case TILE_ROWS128: case TILE_128x256_W4B: *bm = 128; *bn = 256; break;
+    case TILE_32x128: *bm = 32; *bn = 128; break;
+    case TILE_32x256: *bm = 32; *bn = 256; break;
     case TILE_64x256_W4B: *bm = 64; *bn = 256; break;
     default: *bm = 64; *bn = 128; break;
   }

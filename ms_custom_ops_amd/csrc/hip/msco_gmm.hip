@@ -34,7 +34,9 @@ enum Override : int {
   OV_TILE_4BIT = 13,  // 4-bit weights, int8 x: 64 x 256 or 128 x 256 tiles that read the nibbles (else: as planned)
   OV_ROWS16 = 14,     // weight-only: equal chunks of up to 128 rows x strips of 512 columns (else: as planned)
   OV_ROWS16_256 = 15,  // the same with strips of 256 columns
-  OV_ROWS16_256X2 = 16 // ... and two sets of waves that take turns at the K blocks
+  OV_ROWS16_256X2 = 16, // ... and two sets of waves that take turns at the K blocks
+  OV_TILE_32x128 = 17,  // a few rows on [E,K,N] and [E,N,K] weights (packed: 64 x 128 tiles)
+  OV_TILE_32x256 = 18   // ... on [E,K,N] weights ([E,N,K]: as 17)
 };
 
 constexpr int64_t kSkinnyMaxRows = 64;   // total rows up to which the weight-streaming kernel is planned
@@ -124,7 +126,7 @@ int check_desc(const msco_gmm_desc &d) {
   if (d.group_list_dtype != MSCO_DT_NONE && d.group_list_dtype != MSCO_DT_I32 && d.group_list_dtype != MSCO_DT_I64)
     return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_type != 0 && d.group_list_type != 1) return MSCO_ERR_INVALID_ARG;
-  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_ROWS16_256X2) return MSCO_ERR_INVALID_ARG;
+  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_TILE_32x256) return MSCO_ERR_INVALID_ARG;
   if (d.weight_layout != MSCO_WL_ROW_MAJOR && d.weight_layout != MSCO_WL_PACKED) return MSCO_ERR_INVALID_ARG;
   if (d.force_split_k < 0) return MSCO_ERR_INVALID_ARG;
   if (d.act_type < MSCO_ACT_NONE || d.act_type > MSCO_ACT_SILU) return MSCO_ERR_INVALID_ARG;
@@ -390,6 +392,34 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
   op->workspace_bytes = workspace(best);
 }
 
+// 128-column tiles a launch is expected to have when no group has more rows than a tile
+int64_t few_row_tiles(int64_t m, int64_t n, int64_t e) { return groups_hit(m, e) * ((n + 127) / 128); }
+
+// int8 x on [E,K,N] or [E,N,K] weights, groups that a 32-row tile holds (gmm_tile_w8a8.hip): all the rows of one group, or 16 a
+// group on average -- real routings are uneven.  Everything is us, the plan before -> the 32-row tile, 160 [E,K,N] and 100 [E,N,K] shapes of 1 to
+// 800 rows, 1 to 128 experts, K = 512 .. 8192, N = 512 .. 14336, random routings (popularity even or falling as 1 / rank^0.6 or 1 / rank^1.2),
+// each form measured on all of them: 0.80 of the time on [E,K,N], 0.93 with one group; four of 122 grouped shapes slower by 4 to 16 %.
+//   up to 9/8 tiles of 128 columns per CU: 32 x 128.  16 experts, 18 rows, 3392 x 1168 24.6 -> 14.3; 32 experts, 18 rows, 640 x 2208 13.7 ->
+//   9.0; one group, 13 rows, 7968 x 5392 20.2 -> 16.8; 64 experts, 76 rows, 7008 x 720 77.5 -> 55.9.
+//   more: 32 x 256 (8 experts, 32 rows, 5632 x 5120 60.4 -> 48.7, 32 x 128: 62.4), or, where K below 1024 leaves its three-slab ring too
+//   little to walk, 64 x 128 with 64-byte slabs and three workgroups per CU (16 experts, 162 rows, 864 x 4112 22.7 -> 15.3, 32 x 256: 18.8).
+// The decode kernels keep what leaves most CUs idle whatever the tile, because their 16 waves split K inside a workgroup: a handful of
+// rows over dozens of experts (64 experts, 1 row, 2272 x 800: 8.3 against 9.9; 5 rows, 800 x 1824: 8.0 against 8.8) and one group of ten
+// tiles and a long K (1 row, 3744 x 1120: 9.5 against 10.4).  They also keep K below 512 (not measured).  On [E,N,K] weights several groups take 64 x 128
+// tiles already, which are as fast (60 shapes: 0.98), but for more than 32 experts and up to 64 rows (41 rows over 64 experts, 4352 x 688: 27.9 ->
+// 20.3; 52 rows, 544 x 10576: 17.2 -> 15.3 with 64 x 128 tiles), where the decode kernels' plan dates from launches with workgroups for experts
+// without rows.
+void plan_few_rows(msco_gmm_op *op, int &family) {
+  const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
+  const bool nk = op->desc.transpose_b != 0;
+  if (is_packed(op->desc) || k < 512 || (e == 1 ? m > 32 : m > 16 * e)) return;
+  const int64_t tiles = few_row_tiles(m, n, e);
+  if (e == 1 && !nk && m <= kSkinnyRows && tiles <= 10 && k >= 2048) return;
+  if (e > 1 && ((nk && family != FAM_SKINNY) || tiles <= 10 || (e >= 32 && m <= 5))) return;
+  family = FAM_TILE;
+  op->tile_cfg = tiles * 8 <= cus * 9 ? TILE_32x128 : nk || k < 1024 ? TILE_64x128 : TILE_32x256;
+}
+
 void choose_plan(msco_gmm_op *op) {
   const msco_gmm_desc &d = op->desc;
   const int num_cus = op->num_cus;
@@ -529,6 +559,7 @@ void choose_plan(msco_gmm_op *op) {
       op->tile_cfg = TILE_64x128;
     }
   }
+  if (d.kernel_override == OV_AUTO && aligned && is_w8a8(d) && !is_w4(d)) plan_few_rows(op, family);
   switch (d.kernel_override) {
     case OV_TILE_256: family = FAM_TILE; op->tile_cfg = TILE_256x256; break;
     case OV_TILE_256_W4: family = FAM_TILE; op->tile_cfg = TILE_256x256_W4; break;
@@ -539,6 +570,8 @@ void choose_plan(msco_gmm_op *op) {
     case OV_ROWS128: family = FAM_TILE; op->tile_cfg = is_packed(d) ? TILE_ROWS128 : TILE_128x256; break;
     case OV_ROWS256: family = FAM_TILE; op->tile_cfg = is_packed(d) ? TILE_ROWS256 : TILE_256x256_W4; break;
     case OV_ROWS160: family = FAM_TILE; op->tile_cfg = is_packed(d) ? TILE_ROWS160 : TILE_256x256_W4; break;
+    case OV_TILE_32x128: family = FAM_TILE; op->tile_cfg = is_packed(d) ? TILE_64x128 : TILE_32x128; break;
+    case OV_TILE_32x256: family = FAM_TILE; op->tile_cfg = is_packed(d) ? TILE_64x128 : d.transpose_b ? TILE_32x128 : TILE_32x256; break;
     case OV_SKINNY: family = FAM_SKINNY; break;
     case OV_GENERIC: family = FAM_GENERIC; break;
     default: break;
@@ -558,28 +591,32 @@ void choose_plan(msco_gmm_op *op) {
     if (op->tile_cfg == TILE_ROWS128 && !is_packed(d)) op->tile_cfg = TILE_128x256;
     // Few tiles (M of a few hundred rows): split K across workgroups until about kTileTargetWorkgroups of them
     // stream operands; every slice keeps at least kTileMinSlabs 64-byte K slabs.  Small tile shapes only.
-    if (op->tile_cfg == TILE_128x128 || op->tile_cfg == TILE_64x128) {
+    const bool few = op->tile_cfg == TILE_32x128;
+    if (op->tile_cfg == TILE_128x128 || op->tile_cfg == TILE_64x128 || few || op->tile_cfg == TILE_32x256) {
       int bm, bn;
       tile_cfg_dims(op->tile_cfg, &bm, &bn);
       // tiles the launch is expected to have: every group that holds rows has at least one m-tile
       const int64_t groups_with_rows = std::min<int64_t>(e, m);
-      const int64_t t = std::max<int64_t>((m + bm - 1) / bm, groups_with_rows) * ((n + bn - 1) / bn);
+      const int64_t t = few ? few_row_tiles(m, n, e) : std::max<int64_t>((m + bm - 1) / bm, groups_with_rows) * ((n + bn - 1) / bn);
       // t tiles x s slices run in ceil(t s / CUs) rounds (the operand ring takes most of a CU's LDS: one workgroup per
       // CU).  In units of one 64-byte K slab of a tile (0.2 us): a round costs its slabs plus 10 (prologue, epilogue),
       // a split adds 8 per slice for 64 x 128 tiles and 12 for 128 x 128 (its partial tile out and in, one round trip of
       // the last arriver), less 2.  The cheapest s wins, the smaller one on a tie.  Fitted to M = 128, K = N = 4096
       // (64 tiles; s = 1 / 2 / 3 / 4 / 6: 18.7 / 15.2 / 14.5 / 15.3 / 21.3 us) and M = 64, K = 4096, N = 11008 (86 tiles;
-      // s = 1 / 2 / 3: 20.9 / 18.0 / 24.3 us, the third slice starting a second round).
+      // s = 1 / 2 / 3: 20.9 / 18.0 / 24.3 us, the third slice starting a second round).  Of the 32 x 128 tiles two share a CU, in a
+      // fifth more time than one alone, and the exchange is half as large: 128 experts, 24 rows, 3264 x 976, s = 1 / 2: 21.7 / 16.9; 16 experts,
+      // 18 rows, 3392 x 1168: 16.0 / 14.3; 8 experts, 16 rows, 6400 x 2304: 32.6 / 30.3; 16 experts, 12 rows, 608 x 2096: 7.8 / 9.7.
       const int cus = or_default(tuning().tile_target_wgs, num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       const int cap = (int)std::max<int64_t>(1, ((k + 63) / 64) / kTileMinSlabs);
       auto split_cost = [&](int sl) {
         const int64_t slabs = ((k + 63) / 64 + sl - 1) / sl;
         const int64_t rounds = (t * sl + cus - 1) / cus;
+        const int64_t fifths = few && rounds > 1 ? (rounds + 1) / 2 * 6 : rounds * 5;
         const int64_t exchange = sl > 1 ? (int64_t)(4 + bm * bn / 2048) * sl - 2 : 0;
-        return rounds * (slabs + 10 + exchange);
+        return fifths * (slabs + 10 + exchange);
       };
       int want = 1;
-      if (t <= kTileSplitMaxTiles) {
+      if (t <= (few ? 2 * kTileSplitMaxTiles : kTileSplitMaxTiles)) {
         for (int sl = 2; sl <= std::min(kMaxSplitK, cap); ++sl)
           if (split_cost(sl) < split_cost(want)) want = sl;
       }
@@ -587,7 +624,9 @@ void choose_plan(msco_gmm_op *op) {
       if (forced_split > 0) want = std::min(forced_split, cap);
       // the partial tiles of a K split are sized for the worst group_list (one partial m-tile per group): with many
       // groups that bound dwarfs the problem, so the split is halved until the workspace fits under the cap
-      while (want > 1 && tile_workspace_bytes(op->tile_cfg, m, n, e, want) > kTileSplitMaxWorkspace) want /= 2;
+      // (few rows: no more than a launch without a workspace of the caller's has)
+      const size_t most_bytes = few && d.force_split_k <= 0 ? (size_t)MSCO_GMM_STATIC_WORKSPACE_BYTES : kTileSplitMaxWorkspace;
+      while (want > 1 && tile_workspace_bytes(op->tile_cfg, m, n, e, want) > most_bytes) want /= 2;
       op->split_k = want;
       op->workspace_bytes = tile_workspace_bytes(op->tile_cfg, m, n, e, op->split_k);
       // 128-byte K slabs (a 4-stage ring of them takes most of a CU's LDS: one workgroup per CU) when the workgroups
@@ -596,7 +635,7 @@ void choose_plan(msco_gmm_op *op) {
       op->wide_k_slabs = t * want <= (num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       if (tuning().tile_wide_k >= 0) op->wide_k_slabs = tuning().tile_wide_k != 0;
     }
-    if (op->tile_cfg == TILE_128x128 || op->tile_cfg == TILE_64x128 || op->tile_cfg == TILE_128x256) {
+    if (op->tile_cfg == TILE_128x128 || op->tile_cfg == TILE_64x128 || op->tile_cfg == TILE_128x256 || few || op->tile_cfg == TILE_32x256) {
       // Non-temporal weight loads: a weight stream of tens of megabytes that at most two m-tiles read should not push x
       // out of the caches (E = 8 x 32 rows, 470 MB: 87.7 -> 79.4 us; M = 128, 45 MB: 20.8 -> 19.6 us); three m-tiles
       // re-read it from the cache and lose badly without it there (M = 384: 35 -> 47 us), and a weight set the caches
@@ -783,7 +822,7 @@ void choose_plan(msco_gmm_op *op) {
 
   family = op->family;
   char buf[320];
-  const char *fam = family == FAM_REGT ? (op->shallow ? "skinny_regt_shallow" : "skinny_regt") : family == FAM_ROWS16 ? (op->strip_cols == 512 ? "rows128" : op->wave_sets == 2 ? "rows128x256_2" : "rows128x256") : family == FAM_TILE ? "tile" : family == FAM_SKINNY ? "skinny" : "generic";
+  const char *fam = family == FAM_REGT ? (op->shallow ? "skinny_regt_shallow" : "skinny_regt") : family == FAM_ROWS16 ? (op->strip_cols == 512 ? "rows128" : op->wave_sets == 2 ? "rows128x256_2" : "rows128x256") : family == FAM_TILE ? (op->tile_cfg >= TILE_32x128 ? "skinny_tile" : "tile") : family == FAM_SKINNY ? "skinny" : "generic";
   std::snprintf(buf, sizeof(buf),
                 "msco_gmm plan: kernel=%s%s%s%s layout=%s m=%lld k=%lld n=%lld e=%lld split_k=%d strips=%d "
                 "workspace=%zu%s",
