@@ -65,7 +65,7 @@ hipError_t launch_stream_a16w8(const GmmParams &p, hipStream_t stream);   // K s
 hipError_t launch_streamm_w8a8(const GmmParams &p, int tch, hipStream_t stream);
 hipError_t launch_streamm_a16w8(const GmmParams &p, int tch, bool packed, hipStream_t stream);   // weight-only, 32 / 64 / 128 rows per chunk (tch = 2, 4, 8), packed or [E,K,N] weights, no K split
 // weight-only, packed or [E,K,N] weights: equal chunks of up to 128 rows x strips of 512 or 256 columns, p.split_k slices of K, one or two sets of waves (gmm_rows_a16w8_kernel.h)
-hipError_t launch_rows_a16w8(const GmmParams &p, bool packed, int strip_cols, int sets, hipStream_t stream);
+hipError_t launch_rows_a16w8(const GmmParams &p, bool packed, bool w4, int strip_cols, int sets, hipStream_t stream);
 size_t rows_a16w8_slice_bytes();   // workspace bytes of one (chunk, strip, K slice) partial tile
 size_t streamm_tile_bytes(int tch);   // workspace bytes of one (chunk, strip, K slice) partial tile
 size_t rows32_a16w8_slice_bytes(int strip_groups);   // workspace bytes of one (chunk, strip, K slice) partial tile of the 128-row weight-only kernel

@@ -1,4 +1,4 @@
-// Grouped weight-only matmul (16-bit x, 8-bit weights) for groups of a few dozen rows and more (gfx950): packed or row-major
+// Grouped weight-only matmul (16-bit x, 8-bit weights, or 4-bit ones as [E,K,N]) for groups of a few dozen rows and more (gfx950): packed or row-major
 // [E,K,N] weights go from memory into registers, are converted there once and meet up to 128 rows of x from LDS.
 //
 // The matrix pipe wants a 16 x 16 x 32 MFMA every 16 cycles from every SIMD.  What stands in its way is the conversion (one
@@ -14,6 +14,9 @@
 //     [E,K,N]: a lane requests four neighbouring columns of its 16 K rows; column j of two rows is converted and packed by
 //     the same instructions (byte select), so the turn costs nothing.  The output column of MFMA column c of word position j
 //     then is 4 c + j.
+//     4-bit [E,K,N]: two bytes hold the lane's four columns of a row; four instructions make signed bytes of two rows, at 16 times
+//     their value (exact in either type, taken out of the sums again), and the rest is the same: bit for bit what the int8 copy of
+//     the weights gives, without the launch that writes it (1.5 bytes per weight) and the second byte of every later read.
 //   * the weights are the MFMA's first operand: a lane ends up with neighbouring columns of one row ([E,K,N]: 16; packed: 8,
 //     once two lane rows have changed places), stored straight from the accumulators.
 //   * x goes straight into a ring of LDS stages of 64 K positions (128 bytes) per row; 16-byte piece q of row r sits at piece
@@ -110,8 +113,9 @@ __device__ __forceinline__ void xa_load_lds(__amdgpu_buffer_rsrc_t rsrc, unsigne
 
 // RB = 16-row blocks of the chunk; NW = waves side by side, 64 columns each; KS = sets of them that take turns at the K blocks;
 // tile = number of the (chunk, strip) pair
-template <bool BF16, bool KN, int RB, int NW, int KS>
+template <bool BF16, bool KN, bool W4, int RB, int NW, int KS>
 __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char *smem, int grp, int strip, int m0, int chunk_rows, long long tile) {
+  static_assert(KN || !W4);
   constexpr bool SPLIT = NW == 4;   // (wide strips are planned where they fill the chip)
   constexpr int XA_WAVES = NW, XA_COLS = 64 * NW;
   constexpr int DEPTH = RB <= 2 ? 6 : RB <= 4 ? 4 : 3;   // register sets for the weights of a K block; x stages
@@ -133,7 +137,8 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
   // ---- weights: a wave's four blocks of 16 columns x 64 K bytes, 16 registers per lane and K block.  Packed: one descriptor
   // per column group over exactly its K blocks; [E,K,N]: one over the expert's matrix, a lane outside N x K out of its range.
   // (K % 16 == 0: a lane's 16 K rows are all inside or all outside; only the vector offset is range-checked)
-  const long long group_bytes = KN ? (long long)p.k * p.n : (long long)col_groups * k_blocks * 1024;
+  const unsigned row_bytes = W4 ? (unsigned)p.n / 2 : (unsigned)p.n;   // [E,K,N]
+  const long long group_bytes = KN ? (long long)p.k * row_bytes : (long long)col_groups * k_blocks * 1024;
   __amdgpu_buffer_rsrc_t rw[4];
   if constexpr (KN) {
     rw[0] = buffer_over(p.w + (long long)grp * group_bytes, group_bytes);
@@ -144,14 +149,16 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
       rw[cg] = buffer_over(p.w + (long long)grp * group_bytes + (long long)min(g, col_groups - 1) * k_blocks * 1024, g < col_groups ? (long long)kb_end * 1024 : 0);
     }
   }
-  const unsigned w_lane = KN ? (n_wave + 4 * c16 < p.n ? (unsigned)(16 * h) * (unsigned)p.n + (unsigned)(n_wave + 4 * c16) : kBufferOob) : (unsigned)lane * 16u;
+  const unsigned w_lane = KN ? (n_wave + 4 * c16 < p.n ? (unsigned)(16 * h) * row_bytes + (unsigned)(n_wave + 4 * c16) / (W4 ? 2 : 1) : kBufferOob) : (unsigned)lane * 16u;
   int raw[DEPTH][4][4];   // packed: [column group][dword]; [E,K,N]: K row 4 i + j in [i][j]
   constexpr int WL = KN ? 16 : 4;   // requests per K block
   auto wload1 = [&](auto set_c, auto i_c, int kb) {
     constexpr int SET = decltype(set_c)::value, I = decltype(i_c)::value;
     if constexpr (KN) {
       const unsigned vo = 64 * kb + 16 * h < k_end ? w_lane : kBufferOob;
-      raw[SET][I / 4][I % 4] = (int)__builtin_amdgcn_raw_buffer_load_b32(rw[0], vo, (unsigned)(64 * kb + I) * (unsigned)p.n, 0);
+      const unsigned so = (unsigned)(64 * kb + I) * row_bytes;
+      if constexpr (W4) raw[SET][I / 4][I % 4] = (int)__builtin_amdgcn_raw_buffer_load_b16(rw[0], vo, so, 0);
+      else raw[SET][I / 4][I % 4] = (int)__builtin_amdgcn_raw_buffer_load_b32(rw[0], vo, so, 0);
     } else {
       const v4i v = __builtin_amdgcn_raw_buffer_load_b128(rw[I], (unsigned)kb * 1024u + w_lane, 0, 0);
 #pragma unroll
@@ -165,7 +172,16 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
     constexpr int J = KN ? I % 4 : I / 4, D = KN ? I / 4 : I % 4;
     if constexpr (KN) {
       constexpr int R = 8 * HALF + 2 * D;
-      f[J][D] = xa_pair<BF16, J, J>((unsigned)raw[SET][R / 4][R % 4], (unsigned)raw[SET][(R + 1) / 4][(R + 1) % 4]);
+      if constexpr (W4) {
+        // four columns of two rows: 16 times their values as signed bytes, the even columns in one word and the odd ones in the other
+        int &even = raw[SET][R / 4][R % 4], &odd = raw[SET][(R + 1) / 4][(R + 1) % 4];
+        if constexpr (J == 0) {
+          const unsigned both = (unsigned)even | (unsigned)odd << 16;
+          even = (int)((both << 4) & 0xF0F0F0F0u);
+          odd = (int)(both & 0xF0F0F0F0u);
+        }
+        f[J][D] = xa_pair<BF16, J / 2, 2 + J / 2>((unsigned)(J % 2 == 0 ? even : odd), (unsigned)(J % 2 == 0 ? even : odd));
+      } else f[J][D] = xa_pair<BF16, J, J>((unsigned)raw[SET][R / 4][R % 4], (unsigned)raw[SET][(R + 1) / 4][(R + 1) % 4]);
     } else {
       constexpr int W = 2 * HALF + D / 2;
       f[J][D] = xa_pair<BF16, 2 * (D % 2), 2 * (D % 2) + 1>((unsigned)raw[SET][J][W], (unsigned)raw[SET][J][W]);
@@ -403,7 +419,7 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
       if (live && row < chunk_rows) {
         unsigned q[NV / 2];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) a[v] = fmaf(of[v], xs_row, a[v]) * sc[v];
+        for (int v = 0; v < NV; ++v) a[v] = fmaf(of[v], xs_row, W4 ? a[v] * 0.0625f : a[v]) * sc[v];
         if constexpr (decltype(act_c)::value) activate_n(a, p.act_type);
         pack_half_n(a, BF16 ? DT_BF16 : DT_F16, q);
         uint4 *dst = reinterpret_cast<uint4 *>(reinterpret_cast<unsigned short *>(p.out) + (long long)(m0 + row) * p.n + n);
@@ -417,7 +433,7 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
   else finish(std::true_type{});
 }
 
-template <bool BF16, bool KN, int NW, int KS>
+template <bool BF16, bool KN, bool W4, int NW, int KS>
 __global__ void __launch_bounds__(64 * NW * KS, 2) gmm_a16w8_rows128_kernel(const GmmParams p) {
   extern __shared__ __align__(16) unsigned char xa_smem[];
   const int lane = threadIdx.x & 63;
@@ -428,15 +444,15 @@ __global__ void __launch_bounds__(64 * NW * KS, 2) gmm_a16w8_rows128_kernel(cons
   static_for<XA_RB>([&](auto i_c) {   // one copy of the K loop per number of 16-row blocks
     constexpr int RB = decltype(i_c)::value + 1;
     if (!done && rb == RB) {
-      rows_a16w8_run<BF16, KN, RB, NW, KS>(p, xa_smem, grp, strip, m0, chunk_rows, (long long)chunk * p.n_strips + strip);
+      rows_a16w8_run<BF16, KN, W4, RB, NW, KS>(p, xa_smem, grp, strip, m0, chunk_rows, (long long)chunk * p.n_strips + strip);
       done = true;
     }
   });
 }
 
-template <bool BF16, bool KN, int NW, int KS>
+template <bool BF16, bool KN, bool W4, int NW, int KS>
 static hipError_t rows_a16w8_form(const GmmParams &p, dim3 grid, hipStream_t stream) {
-  auto kern = gmm_a16w8_rows128_kernel<BF16, KN, NW, KS>;
+  auto kern = gmm_a16w8_rows128_kernel<BF16, KN, W4, NW, KS>;
   constexpr int lds = xa_lds(KS);
   if (lds > 64 * 1024) {
     static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race between first launches repeats it at worst
@@ -451,11 +467,11 @@ static hipError_t rows_a16w8_form(const GmmParams &p, dim3 grid, hipStream_t str
 }
 
 // wave sets: 1, or 2 with strips of 256 columns
-template <bool BF16, bool KN>
+template <bool BF16, bool KN, bool W4 = false>
 static hipError_t rows_a16w8_pick(const GmmParams &p, int strip_cols, int sets, dim3 grid, hipStream_t stream) {
-  if (strip_cols == 512 && sets == 1) return rows_a16w8_form<BF16, KN, 8, 1>(p, grid, stream);
-  if (strip_cols == 256 && sets == 1) return rows_a16w8_form<BF16, KN, 4, 1>(p, grid, stream);
-  if (strip_cols == 256 && sets == 2) return rows_a16w8_form<BF16, KN, 4, 2>(p, grid, stream);
+  if (strip_cols == 512 && sets == 1) return rows_a16w8_form<BF16, KN, W4, 8, 1>(p, grid, stream);
+  if (strip_cols == 256 && sets == 1) return rows_a16w8_form<BF16, KN, W4, 4, 1>(p, grid, stream);
+  if (strip_cols == 256 && sets == 2) return rows_a16w8_form<BF16, KN, W4, 4, 2>(p, grid, stream);
   return hipErrorInvalidValue;
 }
 

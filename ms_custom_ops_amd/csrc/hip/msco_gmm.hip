@@ -181,7 +181,7 @@ void plan_regt(msco_gmm_op *op) {
   // more than a second and third pass over the nibbles (4 / 32 rows per group: 47 / 95 us in all).
   // Weight-only on 8-bit weights, one 16-row chunk per group: the decode form.
   const bool want = d.kernel_override == OV_REGT ||
-                    (d.kernel_override == OV_AUTO && bits == 4 && rows <= 64) ||
+                    (d.kernel_override == OV_AUTO && bits == 4 && rows <= 64 && op->family != FAM_ROWS16) ||
                     (op->family == FAM_SKINNY && bits == 8 && is_a16w8(d) && op->stream_tch == 1);
   // 4-bit weights, int8 x, more than one 16-row chunk per group: tiles that read the nibbles through LDS (4 / 16 / 32 rows
   // per group 52 / 53 / 58 us against 44 / 53 / 82 us in 32-row chunks)
@@ -287,7 +287,7 @@ void plan_regt(msco_gmm_op *op) {
     op->family = FAM_GENERIC;
     op->split_k = 1;
   }
-  if (bits == 4) {
+  if (bits == 4 && op->family != FAM_ROWS16) {   // (the 128-row weight-only kernel reads the nibbles)
     op->widen_bytes = (e * k * n + 255) / 256 * 256;
     op->workspace_bytes += (size_t)op->widen_bytes;
   }
@@ -314,11 +314,11 @@ constexpr Rows16Cost kRowsSmall[2][2] = {   // [packed][32- and 64-row chunks], 
 
 double chip_rounds(double workgroups, double slots) { return workgroups <= slots ? 1.0 : workgroups / slots + 0.5; }
 
-double rows_stream_us(int64_t m, int64_t k, int64_t n, int64_t e) {   // at the rate of a read-only launch
-  return ((double)std::max<int64_t>(1, std::min(e, m)) * (double)(k * n) + 2.0 * (double)m * (double)(k + n)) / 6.7e6;
+double rows_stream_us(int64_t m, int64_t k, int64_t n, int64_t e, int bits) {   // at the rate of a read-only launch
+  return ((double)std::max<int64_t>(1, std::min(e, m)) * (double)(k * n) * bits / 8 + 2.0 * (double)m * (double)(k + n)) / 6.7e6;
 }
 
-double rows16_us(int64_t m, int64_t k, int64_t n, int64_t e, int64_t cus, bool packed, const Rows16Form &f) {
+double rows16_us(int64_t m, int64_t k, int64_t n, int64_t e, int64_t cus, bool packed, int bits, const Rows16Form &f) {
   const int64_t avg = (m + e - 1) / e, rows = e == 1 ? m : avg + avg / 10;   // (real routings are uneven)
   const int64_t groups = std::max<int64_t>(1, std::min(e, m)), chunks = (rows + 127) / 128;
   const double rb = (double)std::min<int64_t>(8, ((rows + chunks - 1) / chunks + 15) / 16);
@@ -329,7 +329,7 @@ double rows16_us(int64_t m, int64_t k, int64_t n, int64_t e, int64_t cus, bool p
   const bool pairs = f.cols == 256 && f.sets == 1 && wgs > (double)cus;
   const Rows16Cost &c = kRows16[packed][f.cols == 512 ? 0 : f.sets == 2 ? 3 : pairs ? 2 : 1];
   const double r = chip_rounds(wgs, pairs ? 2.0 * (double)cus : (double)cus);
-  const double us = c.fixed + r * (c.round + blocks * (c.block + c.rows * rb)) + c.stream * rows_stream_us(m, k, n, e) + (f.split > 1 ? c.split + c.slice * rb * r * (f.split - 1) : 0.0);
+  const double us = c.fixed + r * (c.round + blocks * (c.block + c.rows * rb)) + c.stream * rows_stream_us(m, k, n, e, bits) + (f.split > 1 ? c.split + c.slice * rb * r * (f.split - 1) : 0.0);
   return pairs && r > 3 && rb >= 6 ? 1.07 * us : us;   // (what the fit is off by there: x comes in twice per CU)
 }
 
@@ -341,14 +341,21 @@ double rows_small_us(int64_t m, int64_t k, int64_t n, int64_t e, int64_t cus, in
   const double wgs = (double)((col_groups + wide - 1) / wide) * (double)(groups * ((avg + avg / 10 + chunk - 1) / chunk));
   const double live = (double)std::min<int64_t>(tch, (avg + 15) / 16), blocks = (double)((k + 63) / 64) * wide / 16;
   const Rows16Cost &c = kRowsSmall[packed][tch == 4];
-  return c.fixed + chip_rounds(wgs, 2.0 * (double)cus) * blocks * (c.block + c.rows * live) + c.stream * rows_stream_us(m, k, n, e);
+  return c.fixed + chip_rounds(wgs, 2.0 * (double)cus) * blocks * (c.block + c.rows * live) + c.stream * rows_stream_us(m, k, n, e, 8);
 }
 
+// 4-bit weights: these kernels read the nibbles; the model with their bytes picks forms that take 1.035 of the time of the best one (87
+// shapes).  Beyond 30 rows per group on average they beat the 32-row chunks of the register-transpose kernels (us, those -> these: 33 rows, 64
+// experts, 1376 x 1120 50 -> 37; 128 experts, 1696 x 1712 132 -> 91; 35 rows, 64 experts, 544 x 6032 93 -> 65; 37 rows, 32 experts, 3424 x
+// 2608 112 -> 74; up to there 54 against 62 and 58 against 67, one group at most 128 rows either way), and what they replace beyond: the weights
+// widened into the workspace first, then the kernels for int8 weights (64 experts, 6336 x 896, 89 rows 205 -> 113; 128 experts,
+// 1536 x 1856, 76 rows 209 -> 98).
 // `family_fits`: the kernels planned so far can take the shape (their grids are bounded; the 128-row kernel's is not)
 void plan_rows16(msco_gmm_op *op, bool family_fits) {
   const msco_gmm_desc &d = op->desc;
   if ((op->family != FAM_SKINNY && family_fits) || !is_a16w8(d) || layout_of(d) == 1 || op->k >= ((int64_t)1 << 22)) return;   // (128 rows of x through 32-bit offsets)
   const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
+  const int bits = is_w4(d) ? 4 : 8;
   GmmParams p{};
   p.m = (int)m;
   p.e = (int)e;
@@ -361,6 +368,8 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     while (best.split > 1 && workspace(best) > kTileSplitMaxWorkspace) --best.split;
   } else if (d.kernel_override != OV_AUTO || d.force_split_k != 0 || (family_fits && op->stream_tch == 1)) {
     return;
+  } else if (bits == 4 && e >= 8 && k >= 512 && m <= 30 * e) {
+    return;   // (the register-transpose kernels)
   } else if (e < 8 || k < 512) {
     // Outside what the model was fitted to (one group has kernels with a K split of its own): strips of 512 where they fill the chip and
     // a tile has rows enough.  One group, N = 11008, K = 4096, 512 (88 tiles) / 1024 (176) / 4096 rows: 91 -> 113, 158 -> 108, 444 -> 327 us
@@ -370,19 +379,19 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     const int64_t k_min = rows <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : rows <= 256 ? 768 : 1280;
     if (!(k >= k_min && avg >= 48 && (tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65) && n * 100 >= strips * 512 * 85)) return;
   } else {
-    double us = rows16_us(m, k, n, e, cus, is_packed(d), best);
+    double us = rows16_us(m, k, n, e, cus, is_packed(d), bits, best);
     for (int sets = 1; sets <= 2; ++sets)
       for (int split = 1; split <= 4 && split <= (k + 63) / 64; ++split) {
         const Rows16Form f{256, sets, split};
         if (workspace(f) > (size_t)MSCO_GMM_STATIC_WORKSPACE_BYTES) break;   // (msco_gmm_launch_static takes what it took without a split)
-        const double t = rows16_us(m, k, n, e, cus, is_packed(d), f);
+        const double t = rows16_us(m, k, n, e, cus, is_packed(d), bits, f);
         if (t < us) {
           us = t;
           best = f;
         }
       }
     // (the kernels for smaller chunks keep what is not clearly better here; 128-row chunks are always better off)
-    if (family_fits && op->stream_tch <= 4 && 0.9 * rows_small_us(m, k, n, e, cus, op->stream_tch, is_packed(d)) < us) return;
+    if (bits == 8 && family_fits && op->stream_tch <= 4 && 0.9 * rows_small_us(m, k, n, e, cus, op->stream_tch, is_packed(d)) < us) return;
   }
   op->family = FAM_ROWS16;
   op->strip_cols = best.cols;
@@ -993,7 +1002,7 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   if (h->family == FAM_REGT) {
     err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, h->shallow, s);
   } else if (h->family == FAM_ROWS16) {
-    err = launch_rows_a16w8(p, layout == 2, h->strip_cols, h->wave_sets, s);
+    err = launch_rows_a16w8(p, layout == 2, is_w4(d), h->strip_cols, h->wave_sets, s);
   } else if (is_w8a8(d)) {
     if (h->family == FAM_TILE && h->small_group_rows > 0) {
       GmmParams big = p, small = p;

@@ -75,7 +75,7 @@ def test_inline_mfmas_keep_their_wait_states(tmp_path):
     assert seen >= 1000
 
 
-@pytest.mark.parametrize("unit", ["bf16_kn", "f16_packed", "f16_kn"])
+@pytest.mark.parametrize("unit", ["a16w8_bf16_kn", "a16w8_f16_packed", "a16w8_f16_kn", "a16w4_bf16", "a16w4_f16"])
 def test_the_other_types_and_layouts_keep_them_too(unit, tmp_path, monkeypatch):
-    monkeypatch.setitem(globals(), "OBJ", OBJ.replace("a16w8.o", "a16w8_%s.o" % unit))
+    monkeypatch.setitem(globals(), "OBJ", OBJ.replace("a16w8.o", unit + ".o"))
     test_inline_mfmas_keep_their_wait_states(tmp_path)
