@@ -2,9 +2,8 @@
 // un-permutation for gfx950.  Both are HBM-bound row copies around a small integer problem:
 //
 //   init_routing   up to 16384 entries: ONE launch (route_fused_kernel): every workgroup counts all expert ids itself,
-//                  places its own 32 entries and moves their rows (plain copy, or per-row dynamic int8 quantisation);
-//                  a wavefront owns consecutive entries, so the k entries of a token cost one read (and one
-//                  quantisation) of its row.  More entries take four launches:
+//                  places the entries of a few tokens and moves their rows (plain copy, or per-row dynamic int8 quantisation);
+//                  the k entries of a token cost one read (and one quantisation) of its row.  More entries take four launches:
 //                  1. per block of 1024 entries: histogram of the expert ids (LDS atomics)
 //                  2. one workgroup: per expert, exclusive scan over the blocks (runs of blocks in parallel), then over
 //                     the experts; writes the count / cumulative-count output
@@ -16,6 +15,8 @@
 #include "msco_moe.h"
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "gmm_common.h"
 
@@ -160,18 +161,28 @@ __global__ void __launch_bounds__(1024) route_rank_kernel(const int *expert_idx,
 // |x| is ordered like its bit pattern without the sign, so the maximum is taken on 15-bit integers and converted once.
 template <bool BF16>
 __device__ __forceinline__ float rq_widen(unsigned short b) { return BF16 ? bf16_bits_to_f32(b) : f16_bits_to_f32(b); }
-__device__ __forceinline__ void rq_fold(unsigned &mx, const uint4 &v) {
+typedef unsigned short rq_v2s __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void rq_fold(rq_v2s &mx, const uint4 &v) {   // even and odd elements
   const unsigned w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    mx = max(mx, w[i] & 0x7FFFu);
-    mx = max(mx, (w[i] >> 16) & 0x7FFFu);
-  }
+  for (int i = 0; i < 4; ++i) mx = __builtin_elementwise_max(mx, __builtin_bit_cast(rq_v2s, w[i] & 0x7FFF7FFFu));
+}
+// over the wavefront: within rows of 16 lanes by lane moves, then the four rows
+__device__ __forceinline__ unsigned rq_wave_max(rq_v2s v) {
+  unsigned m = max((unsigned)v.x, (unsigned)v.y);
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xF, 0xF, true));   // row_half_mirror
+  m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x140, 0xF, 0xF, true));   // row_mirror
+  unsigned all = 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) all = max(all, (unsigned)__builtin_amdgcn_readlane((int)m, 16 * r));
+  return all;
 }
 // The golden rounds the correctly rounded quotient x / scale to an integer.  A correctly rounded division costs a
-// dozen instructions per element.  r = x * (1 / scale) differs from that quotient by at most 1.5 * 2^-23 * 127.5 < 2.3e-5
-// (two roundings here, one there), so unless r lies within kRqMargin = 5e-5 of a half-integer both round to the same
-// integer.  Adding 1.5 * 2^23 rounds r to that integer (nearest, ties to even, like rint) in the low mantissa bits: its
+// dozen instructions per element.  r = x * (1 / scale), not rounded, differs from that quotient by at most 1.5 * 2^-23 * 127.5 < 2.3e-5
+// (the reciprocal's rounding here, the quotient's there), so unless r lies within kRqMargin = 5e-5 of a half-integer both round to the same
+// integer.  Adding 1.5 * 2^23 in one multiply-add rounds r to that integer (nearest, ties to even, like rint) in the low mantissa bits: its
 // low byte is the int8.  Elements too close to a half-integer (1e-4 of them) are done again with the division.
 // eight elements -> eight int8; `nonzero`: the row's maximum is not zero (a row of zeros has scale 0: the golden divides
 // 0 by 0 there; it gets zeros)
@@ -190,12 +201,11 @@ __device__ __forceinline__ uint2 rq_quantise(const uint4 &v, float scale, float 
   }
 #pragma unroll
   for (int e = 0; e < 8; e += 2) {
-    const float r0 = f[e] * inv, r1 = f[e + 1] * inv;
-    const float t0 = r0 + kRound, t1 = r1 + kRound;
+    const float t0 = fmaf(f[e], inv, kRound), t1 = fmaf(f[e + 1], inv, kRound);
     b[e] = __float_as_uint(t0);
     b[e + 1] = __float_as_uint(t1);
-    d[e] = r0 - (t0 - kRound);
-    d[e + 1] = r1 - (t1 - kRound);
+    d[e] = fmaf(f[e], inv, kRound - t0);
+    d[e + 1] = fmaf(f[e + 1], inv, kRound - t1);
     worst = fmaxf(fmaxf(fabsf(d[e]), fabsf(d[e + 1])), worst);
   }
   if (!(worst <= 0.5f - kRqMargin)) {
@@ -240,216 +250,266 @@ __device__ __forceinline__ void row_store8(__amdgpu_buffer_rsrc_t rs, long long 
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(rq_v2i, rq_v2u{v.x, v.y}), rs, off, 0, 0);
 }
 
-// the first KV vectors per lane of a row (lane + 64 u), requested together; zeros past the row's end
+// A row is moved by 1 << shift waves, of which this is number `sub`; they take turns at pieces of 2 KiB (two vectors of 16 bytes
+// per lane).  First byte of the u-th vector that a wave takes, lane 0:
+struct WaveShare {
+  int sub = 0, shift = 0;
+  __device__ __forceinline__ long long at(int u) const { return 1024ll * ((((u >> 1) << shift | sub) << 1) | (u & 1)); }
+  __device__ __forceinline__ long long pass_bytes(int kv) const { return 1024ll * kv << shift; }   // of the row that all of them take with kv vectors each
+};
+
+// the first KV vectors per lane of a wave's share of a row, requested together; zeros past the row's end
 template <int KV>
-__device__ __forceinline__ void wave_load_row(uint4 (&kept)[KV], __amdgpu_buffer_rsrc_t src, int lane, long long first_byte = 0) {
+__device__ __forceinline__ void wave_load_row(uint4 (&kept)[KV], __amdgpu_buffer_rsrc_t src, int lane, const WaveShare &share, long long first_byte = 0) {
   static_for<KV>([&](auto u_c) {
     constexpr int U = decltype(u_c)::value;
-    kept[U] = row_load16(src, first_byte + 16ll * (lane + 64 * U));
+    kept[U] = row_load16(src, first_byte + share.at(U) + 16 * lane);
   });
 }
 
 // `first`: what wave_load_row brought of this row; dest_row(j): the j-th destination row
 template <int KV, typename DestFn>
-__device__ __forceinline__ void wave_copy_row(const uint4 (&first)[KV], __amdgpu_buffer_rsrc_t src, int lane, int copies,
+__device__ __forceinline__ void wave_copy_row(const uint4 (&first)[KV], __amdgpu_buffer_rsrc_t src, int lane, const WaveShare &share, int copies,
                                               DestFn dest_row, unsigned char *expanded_x, long long row_bytes) {
   for (int j = 0; j < copies; ++j) {
     const __amdgpu_buffer_rsrc_t dst = buffer_over(expanded_x + (long long)dest_row(j) * row_bytes, row_bytes);
     static_for<KV>([&](auto u_c) {
       constexpr int U = decltype(u_c)::value;
-      row_store16(dst, 16ll * (lane + 64 * U), first[U]);   // kept cacheable: the matmul reads it next
+      row_store16(dst, share.at(U) + 16 * lane, first[U]);   // kept cacheable: the matmul reads it next
     });
   }
-  for (long long b0 = 1024ll * KV; b0 < row_bytes; b0 += 1024ll * KV) {
+  for (long long b0 = share.pass_bytes(KV); b0 < row_bytes; b0 += share.pass_bytes(KV)) {
     uint4 buf[KV];
-    wave_load_row(buf, src, lane, b0);
+    wave_load_row(buf, src, lane, share, b0);
     for (int j = 0; j < copies; ++j) {
       const __amdgpu_buffer_rsrc_t dst = buffer_over(expanded_x + (long long)dest_row(j) * row_bytes, row_bytes);
       static_for<KV>([&](auto u_c) {
         constexpr int U = decltype(u_c)::value;
-        row_store16(dst, b0 + 16ll * (lane + 64 * U), buf[U]);
+        row_store16(dst, b0 + share.at(U) + 16 * lane, buf[U]);
       });
     }
   }
 }
 
-// The same with the per-row dynamic int8 quantisation on the way: the row's maximum needs no LDS (one wavefront holds
-// the whole row); a lane keeps KEEP vectors of the row in registers (64 lanes x KEEP x 16 bytes in one pass), what lies
-// beyond is read again for the division (L2 hits).  Zeros past the row's end change neither the maximum nor anything
-// that is stored.
-template <bool BF16, int KEEP, typename DestFn>
-__device__ __forceinline__ void wave_quantise_row(const uint4 (&kept)[KEEP], __amdgpu_buffer_rsrc_t src, int lane, int copies,
-                                                  DestFn dest_row, signed char *expanded_x, float *expanded_scale,
-                                                  long long hidden) {
-  const long long row_bytes = 2 * hidden;
-  unsigned mx = 0;
+// The same with the per-row dynamic int8 quantisation on the way, in two steps.  The maximum over a wave's share of the row: a lane
+// keeps KEEP vectors in registers, what lies beyond is read again for the division (L2 hits).  Zeros past the row's end change
+// neither the maximum nor anything that is stored.
+template <int KEEP>
+__device__ __forceinline__ unsigned wave_row_max(const uint4 (&kept)[KEEP], __amdgpu_buffer_rsrc_t src, int lane, const WaveShare &share, long long row_bytes) {
+  rq_v2s mx = {0, 0};
   static_for<KEEP>([&](auto u_c) { rq_fold(mx, kept[decltype(u_c)::value]); });
-  for (long long b = 1024ll * KEEP; b < row_bytes; b += 1024) rq_fold(mx, row_load16(src, b + 16 * lane));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
+  for (long long b0 = share.pass_bytes(KEEP); b0 < row_bytes; b0 += share.pass_bytes(2)) {
+    rq_fold(mx, row_load16(src, b0 + share.at(0) + 16 * lane));
+    rq_fold(mx, row_load16(src, b0 + share.at(1) + 16 * lane));
+  }
+  return rq_wave_max(mx);
+}
+
+// mx: the maximum over the whole row
+template <bool BF16, int KEEP, typename DestFn>
+__device__ __forceinline__ void wave_quantise_row(uint4 (&kept)[KEEP], unsigned mx, __amdgpu_buffer_rsrc_t src, int lane, const WaveShare &share,
+                                                  int copies, DestFn dest_row, signed char *expanded_x, float *expanded_scale, long long hidden) {
+  const long long row_bytes = 2 * hidden;
   const float scale = rq_widen<BF16>((unsigned short)mx) / 127.0f;
   const float inv = 1.0f / scale;
-  if (lane == 0) {
-    for (int j = 0; j < copies; ++j) expanded_scale[dest_row(j)] = scale;
+  if (share.sub == 0) {
+    for (int j = 0; j < copies; ++j) {
+      const int row = dest_row(j);   // (read by the whole wave)
+      if (lane == 0) expanded_scale[row] = scale;
+    }
   }
   // two vectors at a time, to every copy (the quantised row never exists as a whole in registers).  A lane's eight
   // bytes and its neighbour's are consecutive in the row: the even lane of a pair takes both lanes' bytes of the first
   // vector and the odd lane both of the second, so that every lane stores 16 bytes (rows of a multiple of 16 bytes).
   const bool wide = (hidden & 15) == 0;
   const long long pair_byte = 512 * (lane & 1) + 16 * (lane >> 1);
-  static_for<KEEP / 2>([&](auto p_c) {
-    constexpr int P = decltype(p_c)::value;
-    const uint2 qa = rq_quantise<BF16>(kept[2 * P], scale, inv, mx != 0);
-    const uint2 qb = rq_quantise<BF16>(kept[2 * P + 1], scale, inv, mx != 0);
-    if (wide) {
-      const bool odd = lane & 1;
-      const unsigned sx = odd ? qa.x : qb.x, sy = odd ? qa.y : qb.y;
-      const unsigned rx = (unsigned)__builtin_amdgcn_update_dpp(0, (int)sx, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
-      const unsigned ry = (unsigned)__builtin_amdgcn_update_dpp(0, (int)sy, 0xB1, 0xF, 0xF, true);
-      const uint4 out = odd ? make_uint4(rx, ry, qb.x, qb.y) : make_uint4(qa.x, qa.y, rx, ry);
-      for (int j = 0; j < copies; ++j)
-        row_store16(buffer_over(expanded_x + (long long)dest_row(j) * hidden, hidden), 1024ll * P + pair_byte, out);
-    } else {
-      for (int j = 0; j < copies; ++j) {
-        const __amdgpu_buffer_rsrc_t dst = buffer_over(expanded_x + (long long)dest_row(j) * hidden, hidden);
-        row_store8(dst, 8ll * (lane + 128 * P), qa);
-        row_store8(dst, 8ll * (lane + 128 * P + 64), qb);
+  // (a loop whose registers move up by a few pairs each time: a third of the code of KEEP / 2 copies, in the same time)
+  constexpr int STEP = KEEP / 4;
+#pragma unroll 1
+  for (int pair0 = 0; pair0 < KEEP / 2 && share.at(2 * pair0) < row_bytes; pair0 += STEP) {
+    static_for<STEP>([&](auto p_c) {
+      constexpr int P = decltype(p_c)::value;
+      const int pair = pair0 + P;
+      if (P > 0 && share.at(2 * pair) >= row_bytes) return;
+      const uint2 qa = rq_quantise<BF16>(kept[2 * P], scale, inv, mx != 0);
+      const uint2 qb = rq_quantise<BF16>(kept[2 * P + 1], scale, inv, mx != 0);
+      if (wide) {
+        const bool odd = lane & 1;
+        const unsigned sx = odd ? qa.x : qb.x, sy = odd ? qa.y : qb.y;
+        const unsigned rx = (unsigned)__builtin_amdgcn_update_dpp(0, (int)sx, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
+        const unsigned ry = (unsigned)__builtin_amdgcn_update_dpp(0, (int)sy, 0xB1, 0xF, 0xF, true);
+        const uint4 out = odd ? make_uint4(rx, ry, qb.x, qb.y) : make_uint4(qa.x, qa.y, rx, ry);
+        for (int j = 0; j < copies; ++j)
+          row_store16(buffer_over(expanded_x + (long long)dest_row(j) * hidden, hidden), share.at(2 * pair) / 2 + pair_byte, out);
+      } else {
+        for (int j = 0; j < copies; ++j) {
+          const __amdgpu_buffer_rsrc_t dst = buffer_over(expanded_x + (long long)dest_row(j) * hidden, hidden);
+          row_store8(dst, share.at(2 * pair) / 2 + 8 * lane, qa);
+          row_store8(dst, share.at(2 * pair + 1) / 2 + 8 * lane, qb);
+        }
       }
+    });
+#pragma unroll
+    for (int i = 0; i < KEEP - 2 * STEP; ++i) kept[i] = kept[i + 2 * STEP];
+  }
+  for (long long b0 = share.pass_bytes(KEEP); b0 < row_bytes; b0 += share.pass_bytes(2)) {
+    const uint4 va = row_load16(src, b0 + share.at(0) + 16 * lane), vb = row_load16(src, b0 + share.at(1) + 16 * lane);
+    const uint2 qa = rq_quantise<BF16>(va, scale, inv, mx != 0), qb = rq_quantise<BF16>(vb, scale, inv, mx != 0);
+    for (int j = 0; j < copies; ++j) {
+      const __amdgpu_buffer_rsrc_t dst = buffer_over(expanded_x + (long long)dest_row(j) * hidden, hidden);
+      row_store8(dst, (b0 + share.at(0)) / 2 + 8 * lane, qa);
+      row_store8(dst, (b0 + share.at(1)) / 2 + 8 * lane, qb);
     }
-  });
-  for (long long b = 1024ll * KEEP; b < row_bytes; b += 1024) {
-    const uint2 q = rq_quantise<BF16>(row_load16(src, b + 16 * lane), scale, inv, mx != 0);
-    for (int j = 0; j < copies; ++j)
-      row_store8(buffer_over(expanded_x + (long long)dest_row(j) * hidden, hidden), (b >> 1) + 8 * lane, q);
   }
 }
 
-// Routing in ONE launch for up to kFusedMaxEntries entries: every workgroup owns kFusedRows consecutive entries (its
+// Routing in ONE launch for up to kFusedMaxEntries entries: every workgroup owns the entries of some consecutive tokens (its
 // slice), finds their output rows by itself and copies their rows.  For that it counts, over ALL entries, how many carry
-// each expert id (total) and how many of those lie before its slice (before): the output row of entry i with id e is
+// each expert id and how many of those lie before its slice: the output row of entry i with id e is
 //     (entries with a smaller id) + (entries with id e before the slice) + (entries with id e inside the slice before i),
 // which is the position a stable sort gives it.  The counting is redundant across workgroups (a few thousand LDS
-// atomics each, on `rep` interleaved copies of the tables so that the lanes of a wavefront rarely meet on one address),
-// but nothing waits for another workgroup, so the sort, the index outputs and the row copy need no second launch.
-#ifndef MSCO_FUSED_ROWS
-#define MSCO_FUSED_ROWS 32
-#endif
-constexpr int kFusedRows = MSCO_FUSED_ROWS;   // 16, 32 or 64: one to four rows per wavefront
+// atomics each, both counts in the halves of one word, on `rep` interleaved copies of the table so that the lanes of a wavefront
+// rarely meet on one address), but nothing waits for another workgroup, so the sort, the index outputs and the row copy need no
+// second launch.
+//
+// A launch is a chain -- ids, counts, ranks; rows, maximum, scale, quantised rows -- of a few microseconds around a copy, so the
+// rows are requested in front of the chain and spread over all CUs: a workgroup for each of them (256), and a workgroup's sixteen wavefronts share the rows (1 << shift per row) where it has fewer tokens than wavefronts.
+// What is left of it, in cycles of one of 1728 workgroup slices of a 7168-element row: 4500 to the first row request's end, 2600 counting and
+// ranking, 3700 for the maximum (the row's arrival), the rest quantising and storing.  us, 32 entries per workgroup and a wavefront per row ->
+// this, bf16 rows quantised, buffers rotated: 1728 tokens x 1, 7168 wide 35.4 -> 16.1; 255 x 8, 7168 20.7 -> 8.8; 2048 x 8, 2048 wide 26.1 -> 13.8; 4096 x
+// 2, 4096 wide 20.4 -> 18.2; 4096 x 4, 5120 wide 40.7 -> 30.4; 509 x 8, 2048 wide 11.3 -> 8.0.
 constexpr int kFusedThreads = 1024;   // sixteen wavefronts: the counting is a chain of dependent LDS atomics per wavefront, four per SIMD overlap them
 constexpr int kFusedIdsPerThread = 16;
-constexpr long long kFusedMaxEntries = (long long)kFusedThreads * kFusedIdsPerThread;   // 16384
+constexpr long long kFusedMaxEntries = (long long)kFusedThreads * kFusedIdsPerThread;   // 16384: the two counts fit the halves of a word
+constexpr int kFusedMaxTopK = 1024;    // (a slice holds fewer than 64 + k entries)
 // QUANT: 0 copies rows of row_bytes bytes; 1 / 2 quantise float16 / bfloat16 rows to int8 and write their scales.
-template <int QUANT>
+// EARLY: the rows are requested in front of the counting; not where a wavefront has more of a row than its KV vectors.
+template <int QUANT, bool EARLY>
 __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsigned char *x, const int *expert_idx,
                                                                     unsigned char *expanded_x, float *expanded_scale,
                                                                     int *expanded_row_idx, int *count_or_cumsum,
-                                                                    int *before_capacity, long long n, int expert_num, int flag,
-                                                                    long long row_bytes, int k, int rep) {
-  extern __shared__ int lds[];   // total[rep][expert_num], before[rep][expert_num], base[expert_num], wave_sum[16], dest[kFusedRows]
-  int *total = lds;
-  int *before = total + rep * expert_num;
-  int *base = before + rep * expert_num;
-  int *wave_sum = base + expert_num;
-  int *dest = wave_sum + 16;
+                                                                    int *before_capacity, int n, int expert_num, int flag,
+                                                                    long long row_bytes, int k, int rep, int slice_tokens, int shift) {
+  extern __shared__ int lds[];   // counts[rep][expert_num], first[expert_num], wave_sum[16], row_max[16], dest[slice_tokens k]
+  int *counts = lds;
+  int *first = counts + rep * expert_num;
+  int *wave_sum = first + expert_num;
+  unsigned *row_max = reinterpret_cast<unsigned *>(wave_sum + 16);
+  int *dest = wave_sum + 32;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const long long start = (long long)blockIdx.x * kFusedRows;
-  constexpr int RPW = kFusedRows / 16;   // consecutive entries per wavefront
+  const int tokens = n / k, token0 = (int)blockIdx.x * slice_tokens, token_end = min(token0 + slice_tokens, tokens);
+  const int start = token0 * k, end = token_end * k;
   constexpr int KV = 8;                  // vectors of a row per lane and pass
-  const long long entry0 = start + RPW * wave;
-  for (int i = tid; i < 2 * rep * expert_num; i += kFusedThreads) lds[i] = 0;
+  const int slots = 16 >> shift, slot = wave >> shift;
+  WaveShare share;
+  share.sub = wave & ((1 << shift) - 1);
+  share.shift = shift;
+  for (int i = tid; i < rep * expert_num; i += kFusedThreads) counts[i] = 0;
   // all of a thread's ids are requested before the first is used: entries 4 (tid + 1024 j) .. + 3 (ids past n read as 0,
   // by the range check of the buffer load, and are skipped by their index; only the vector offset is range-checked)
-  const __amdgpu_buffer_rsrc_t rs_ids = buffer_over(expert_idx, n * 4);
+  const __amdgpu_buffer_rsrc_t rs_ids = buffer_over(expert_idx, 4ll * n);
   v4i ids[kFusedIdsPerThread / 4];
   static_for<kFusedIdsPerThread / 4>([&](auto j_c) {
     constexpr int J = decltype(j_c)::value;
     ids[J] = __builtin_amdgcn_raw_buffer_load_b128(rs_ids, (unsigned)(16 * (tid + kFusedThreads * J)), 0, 0);
   });
-  // the slice's own ids for the ranking by wavefront 0, requested now: a load issued where they are needed would put a
+  // the slice's first ids for the ranking by wavefront 0, requested now: a load issued where they are needed would put a
   // memory round trip between two barriers (other lanes ask beyond the list and get zeros)
-  const int slice_id = __builtin_amdgcn_raw_buffer_load_b32(
-      rs_ids, wave == 0 && lane < kFusedRows && start + lane < n ? (unsigned)(4 * (start + lane)) : 0xFFFFFFFCu, 0, 0);
-  // The plain copy requests the row of the wavefront's first entry right behind the ids (loads return in order: the
-  // counting must not wait for it): where it comes from is known from the entry's index alone (token = entry / k), only
-  // where it goes has to wait for the counting below.  (Measured: 0.4 us less for the copy at 8192 entries of 4 KiB; the
-  // quantising variant is 0.7 us slower with it.)
-  constexpr bool kPreload = QUANT == 0;
-  uint4 row0[KV];
-  if constexpr (kPreload) {
-    wave_load_row(row0, buffer_over(x + (long long)(entry0 < n ? (unsigned)entry0 / (unsigned)k : 0u) * row_bytes, entry0 < n ? row_bytes : 0),
-                  lane);
-  }
+  const int slice_id = __builtin_amdgcn_raw_buffer_load_b32(rs_ids, wave == 0 && start + lane < end ? (unsigned)(4 * (start + lane)) : 0xFFFFFFFCu, 0, 0);
+  // The wavefront's first row is requested behind every wavefront's ids (loads return in order: the counting must not wait for
+  // rows): where it comes from is known, only where it goes has to wait for the counting below.
   __syncthreads();
+  uint4 row[KV];
+  auto load = [&](int token) {
+    const __amdgpu_buffer_rsrc_t src = buffer_over(x + (long long)token * row_bytes, token < token_end ? row_bytes : 0);
+    wave_load_row(row, src, lane, share);
+    return src;
+  };
+  __amdgpu_buffer_rsrc_t src;
+  if constexpr (EARLY) src = load(token0 + slot);
   const int copy = (lane & (rep - 1)) * expert_num;   // rep is a power of two
   static_for<kFusedIdsPerThread / 4>([&](auto j_c) {
     constexpr int J = decltype(j_c)::value;
-    const long long i0 = 4ll * (tid + kFusedThreads * J);
-    static_for<4>([&](auto u_c) {
-      constexpr int U = decltype(u_c)::value;
-      if (i0 + U < n) {
-        const int e = clamp_expert(ids[J][U], expert_num);
-        atomicAdd(&total[copy + e], 1);
-        if (i0 + U < start) atomicAdd(&before[copy + e], 1);
-      }
-    });
+    if (4 * kFusedThreads * J < n) {
+      const int i0 = 4 * (tid + kFusedThreads * J);
+      static_for<4>([&](auto u_c) {
+        constexpr int U = decltype(u_c)::value;
+        if (i0 + U < n) atomicAdd(&counts[copy + clamp_expert(ids[J][U], expert_num)], i0 + U < start ? 0x10001 : 1);
+      });
+    }
   });
   __syncthreads();
-  // fold the copies; exclusive scan of the totals over the experts (one expert per thread)
-  int tsum = 0, bsum = 0;
-  if (tid < expert_num) {
-    for (int r = 0; r < rep; ++r) {
-      tsum += total[r * expert_num + tid];
-      bsum += before[r * expert_num + tid];
-    }
-    before[tid] = bsum;   // copy 0 now holds the folded value (a thread touches only its own expert)
+  // fold the copies; exclusive scan of the totals over the experts (one expert per thread): the first row of the slice's entries
+  int sum = 0;
+  if (tid < expert_num)
+    for (int r = 0; r < rep; ++r) sum += counts[r * expert_num + tid];
+  const int total = sum & 0xFFFF;
+  const int incl = wave_scan_add(total);
+  int offset = incl - total;
+  if (expert_num > 64) {
+    if (lane == 63) wave_sum[wave] = incl;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) offset += wave_sum[w];
   }
-  const int incl = wave_scan_add(tsum);
-  if (lane == 63) wave_sum[wave] = incl;
-  __syncthreads();
-  int offset = incl - tsum;
-  for (int w = 0; w < wave; ++w) offset += wave_sum[w];
   if (tid < expert_num) {
-    base[tid] = offset;
+    first[tid] = offset + (int)((unsigned)sum >> 16);
     if (blockIdx.x == 0) {
-      if (count_or_cumsum != nullptr && flag == 1) count_or_cumsum[tid] = offset + tsum;
-      if (count_or_cumsum != nullptr && flag == 2) count_or_cumsum[tid] = tsum;
+      if (count_or_cumsum != nullptr && flag == 1) count_or_cumsum[tid] = offset + total;
+      if (count_or_cumsum != nullptr && flag == 2) count_or_cumsum[tid] = total;
       if (before_capacity != nullptr) before_capacity[tid] = 0;
     }
   }
-  __syncthreads();
-  // the slice's entries, one per lane of wavefront 0: rank among equal ids inside the slice by ballots
+  if (expert_num > 64) __syncthreads();   // (up to 64 experts wavefront 0 reads what it wrote itself)
+  // the slice's entries, one per lane of wavefront 0, 64 at a time: rank among equal ids by ballots
   if (wave == 0) {
-    const long long i = start + lane;
-    const bool live = lane < kFusedRows && i < n;
-    const int e = live ? clamp_expert(slice_id, expert_num) : -1;
-    const int rank = __popcll(wave_match(e, live, id_bits(expert_num)) & ((1ull << lane) - 1ull));
-    if (live) {
-      const int d = base[e] + before[e] + rank;
-      dest[lane] = d;
-      expanded_row_idx[i] = d;
+    int id = slice_id;
+    for (int i0 = start; i0 < end; i0 += 64) {
+      const int i = i0 + lane;
+      const bool live = i < end;
+      if (i0 > start) id = live ? expert_idx[i] : 0;
+      const int e = live ? clamp_expert(id, expert_num) : -1;
+      const unsigned long long same = wave_match(e, live, id_bits(expert_num));
+      const int rank = __popcll(same & ((1ull << lane) - 1ull));
+      if (live) {
+        const int d = first[e] + rank;
+        dest[i - start] = d;
+        expanded_row_idx[i] = d;
+        if (end - i0 > 64 && rank + 1 == __popcll(same)) first[e] = d + 1;   // (the last of its id in these 64; every lane has read it)
+      }
     }
   }
   __syncthreads();
-  // move the rows: wavefront w takes the slice's entries RPW w .. RPW w + RPW - 1; neighbours of one token share a pass
-  int r = 0;
-  while (r < RPW) {
-    const long long i = entry0 + r;
-    if (i >= n) break;
-    const unsigned token = (unsigned)i / (unsigned)k;   // (entries fit 31 bits: 32-bit divisions)
-    int copies = 1;
-    while (r + copies < RPW && i + copies < n && (unsigned)(i + copies) / (unsigned)k == token) ++copies;
-    const int first = RPW * wave + r;
-    auto dest_row = [&](int j) { return __builtin_amdgcn_readfirstlane(dest[first + j]); };
-    const __amdgpu_buffer_rsrc_t src = buffer_over(x + (long long)token * row_bytes, row_bytes);
-    if (r != 0 || !kPreload) wave_load_row(row0, src, lane);
+  // move the rows: slot s of the workgroup takes its tokens s, s + slots, ..
+  for (int t = slot, pass = 0; pass * slots < slice_tokens; t += slots, ++pass) {
+    if (pass > 0 || !EARLY) src = load(token0 + t);
+    const bool live = token0 + t < token_end;
+    // (a token's rows in one register, entry j in lane j: an LDS read per copy and piece of the row is a wait of its own)
+    const int dest_lane = live ? dest[t * k + min(lane, k - 1)] : 0;
+    auto dest_row = [&](int j) { return j < 64 ? __builtin_amdgcn_readlane(dest_lane, j) : __builtin_amdgcn_readfirstlane(dest[t * k + j]); };
     if constexpr (QUANT == 0) {
-      wave_copy_row(row0, src, lane, copies, dest_row, expanded_x, row_bytes);
+      if (live) wave_copy_row(row, src, lane, share, k, dest_row, expanded_x, row_bytes);
     } else {
-      wave_quantise_row<QUANT == 2>(row0, src, lane, copies, dest_row, reinterpret_cast<signed char *>(expanded_x),
-                                    expanded_scale, row_bytes / 2);
+      unsigned mx = live ? wave_row_max(row, src, lane, share, row_bytes) : 0;
+      if (shift > 0) {
+        if (lane == 0) row_max[wave] = mx;   // (rows are shared only where one pass does: slots >= slice_tokens)
+        __syncthreads();
+        for (int w = 0; w < 1 << shift; ++w) mx = max(mx, row_max[(slot << shift) + w]);
+        mx = (unsigned)__builtin_amdgcn_readfirstlane((int)mx);
+      }
+      if (live)
+        wave_quantise_row<QUANT == 2>(row, mx, src, lane, share, k, dest_row, reinterpret_cast<signed char *>(expanded_x), expanded_scale, row_bytes / 2);
     }
-    r += copies;
   }
+}
+
+// tokens per workgroup and (as a power of two) wavefronts per row of that launch
+struct FusedShape { int slice_tokens, shift; };
+inline FusedShape fused_shape(long long tokens, long long row_bytes) {
+  FusedShape f;
+  f.slice_tokens = (int)((tokens + 255) / 256);
+  f.shift = 0;
+  while (f.shift < 4 && (2 << f.shift) * f.slice_tokens <= 16 && (2048ll << f.shift) < row_bytes) ++f.shift;
+  return f;
 }
 
 // The row movement behind the sort for problems beyond the single launch: one wavefront per token reads its row once and
@@ -463,8 +523,9 @@ __global__ void __launch_bounds__(256) route_scatter_kernel(const unsigned char 
   const int *dests = expanded_row_idx + token * k;
   const __amdgpu_buffer_rsrc_t src = buffer_over(x + token * row_bytes, row_bytes);
   uint4 first[8];
-  wave_load_row(first, src, lane);
-  wave_copy_row(first, src, lane, k, [&](int j) { return __builtin_amdgcn_readfirstlane(dests[j]); }, expanded_x, row_bytes);
+  const WaveShare share;
+  wave_load_row(first, src, lane, share);
+  wave_copy_row(first, src, lane, share, k, [&](int j) { return __builtin_amdgcn_readfirstlane(dests[j]); }, expanded_x, row_bytes);
 }
 
 // Per-row dynamic int8 quantisation on the way to the sorted rows, for problems beyond the single launch: one wavefront
@@ -479,8 +540,10 @@ __global__ void __launch_bounds__(256) route_scatter_quant_kernel(const unsigned
   const int *dests = expanded_row_idx + token * k;
   const __amdgpu_buffer_rsrc_t src = buffer_over(x + token * hidden, 2 * hidden);
   uint4 kept[16];
-  wave_load_row(kept, src, lane);
-  wave_quantise_row<BF16>(kept, src, lane, k, [&](int j) { return __builtin_amdgcn_readfirstlane(dests[j]); }, expanded_x,
+  const WaveShare share;
+  wave_load_row(kept, src, lane, share);
+  const unsigned mx = wave_row_max(kept, src, lane, share, 2 * hidden);
+  wave_quantise_row<BF16>(kept, mx, src, lane, share, k, [&](int j) { return __builtin_amdgcn_readfirstlane(dests[j]); }, expanded_x,
                           expanded_scale, hidden);
 }
 
@@ -499,7 +562,9 @@ typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 // K: top_k as a compile-time constant (the row indices, the probabilities and the K row pieces of a pass are then all
 // requested before the first one is used; with a run-time loop every step waits for two dependent loads), 0: any top_k
 // kUnpermuteU: 2048-element pieces of the row a workgroup takes together (all their row vectors are requested before
-// the first is used: with many tokens, four pieces measured 91 us where one piece takes 97 us at 4096 x top-8 x 7168)
+// the first is used: with many tokens, four pieces measured 91 us where one piece takes 97 us at 4096 x top-8 x 7168).
+// bfloat16, loads that wait for each other's branches and roundings by hand -> this, us: 4096 x 8 x 7168 127 -> 93, 512 x 8 x 7168 18.2 -> 13.1,
+// 1000 x 4 x 5120 13.3 -> 10.3, 64 x 8 x 7168 6.5 -> 4.2.
 template <bool BF16, int K, int kUnpermuteU>
 __global__ void __launch_bounds__(256) unpermute_kernel(const unsigned short *permuted, const int *sorted_indices,
                                                         const unsigned short *probs, unsigned short *out, int top_k_arg,
@@ -517,7 +582,13 @@ __global__ void __launch_bounds__(256) unpermute_kernel(const unsigned short *pe
     }
   }
   // blockIdx.y walks the row in pieces of kUnpermuteU x 2048 elements: one pass per workgroup, so nothing waits for a
-  // previous pass; a thread requests its kUnpermuteU x K vectors before it uses the first
+  // previous pass; a thread requests its kUnpermuteU x K vectors before it uses the first (through descriptors over exactly one
+  // row: what lies past its end reads as zeros, and no lane branches around a load and waits for it there)
+  __amdgpu_buffer_rsrc_t src[KK];
+  if constexpr (K > 0) {
+#pragma unroll
+    for (int kk = 0; kk < K; ++kk) src[kk] = buffer_over(permuted + rows[kk] * hidden, 2 * hidden);
+  }
   for (long long v0 = (long long)blockIdx.y * kUnpermuteU * 256 + threadIdx.x; v0 * 8 < hidden; v0 += (long long)gridDim.y * kUnpermuteU * 256) {
     uint4 all_pieces[kUnpermuteU][KK];
     if constexpr (K > 0) {
@@ -525,8 +596,9 @@ __global__ void __launch_bounds__(256) unpermute_kernel(const unsigned short *pe
       for (int u = 0; u < kUnpermuteU; ++u)
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
-          const long long hu = (v0 + u * 256) * 8;
-          all_pieces[u][kk] = hu < hidden ? MSCO_ROW_LOAD(reinterpret_cast<const uint4 *>(permuted + rows[kk] * hidden + hu)) : make_uint4(0, 0, 0, 0);
+          const long long byte = (v0 + u * 256) * 16;
+          const rq_v4u v = __builtin_bit_cast(rq_v4u, __builtin_amdgcn_raw_buffer_load_b128(src[kk], byte > 0x7FFFFFFFll ? 0x7FFFFFFFu : (unsigned)byte, 0, kStreamAux));
+          all_pieces[u][kk] = make_uint4(v.x, v.y, v.z, v.w);
         }
     }
 #pragma unroll
@@ -567,15 +639,15 @@ __global__ void __launch_bounds__(256) unpermute_kernel(const unsigned short *pe
           }
         }
       } else {
+        // bfloat16: two values per conversion (v_cvt_pk_bf16_f32 rounds like the golden; by hand it is six instructions per value, and the
+        // arithmetic is then what a workgroup spends its time on)
         const float p = bf16_bits_to_f32(pbits);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const unsigned short v = (unsigned short)(w[j >> 1] >> (16 * (j & 1)));
-          float prod = p * bf16_bits_to_f32(v);
-          asm volatile("" : "+v"(prod));
-          float sum = acc[j] + bf16_bits_to_f32(f32_to_bf16_rne(prod));
-          asm volatile("" : "+v"(sum));
-          acc[j] = bf16_bits_to_f32(f32_to_bf16_rne(sum));
+        for (int d = 0; d < 4; ++d) {
+          const unsigned prod = pack_bf16x2(p * __uint_as_float(w[d] << 16), p * __uint_as_float(w[d] & 0xFFFF0000u));
+          const unsigned sum = pack_bf16x2(acc[2 * d] + __uint_as_float(prod << 16), acc[2 * d + 1] + __uint_as_float(prod & 0xFFFF0000u));
+          acc[2 * d] = __uint_as_float(sum << 16);
+          acc[2 * d + 1] = __uint_as_float(sum & 0xFFFF0000u);
         }
       }
         };
@@ -587,7 +659,7 @@ __global__ void __launch_bounds__(256) unpermute_kernel(const unsigned short *pe
     }
     unsigned short ob[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ob[j] = to_elem<BF16>(acc[j]);   // exact: acc already holds an element-type value
+    for (int j = 0; j < 8; ++j) ob[j] = BF16 ? (unsigned short)(__float_as_uint(acc[j]) >> 16) : to_elem<false>(acc[j]);   // exact: acc already holds an element-type value
     uint4 o;
     o.x = ob[0] | ((unsigned)ob[1] << 16); o.y = ob[2] | ((unsigned)ob[3] << 16);
     o.z = ob[4] | ((unsigned)ob[5] << 16); o.w = ob[6] | ((unsigned)ob[7] << 16);
@@ -636,20 +708,24 @@ static int route_and_gather(const void *x, const int32_t *expert_idx, void *expa
   if (count_or_cumsum_flag != 0 && expert_tokens_count_or_cumsum == nullptr) return MSCO_ERR_INVALID_ARG;
   if (workspace == nullptr || workspace_bytes < msco_moe_init_routing_v2_workspace_bytes(num_rows, k, expert_num))
     return MSCO_ERR_WORKSPACE;
-  if (n <= kFusedMaxEntries) {
+  if (n <= kFusedMaxEntries && k <= kFusedMaxTopK) {
     // small problems: the sort and the row movement in one launch, no workspace traffic
+    const long long row_bytes = (long long)hidden * (quant_dtype == MSCO_DT_NONE ? elem_bytes : 2);
+    const FusedShape f = fused_shape(num_rows, row_bytes);
     int rep = 8;
     while (rep > 1 && rep * expert_num > 512) rep /= 2;
-    const size_t lds_bytes = (size_t)(2 * rep * expert_num + expert_num + 16 + kFusedRows) * sizeof(int);
-    const dim3 grid((unsigned)((n + kFusedRows - 1) / kFusedRows)), block(kFusedThreads);
+    const size_t lds_bytes = (size_t)((rep + 1) * expert_num + 32 + f.slice_tokens * k) * sizeof(int);
+    const dim3 grid((unsigned)((num_rows + f.slice_tokens - 1) / f.slice_tokens)), block(kFusedThreads);
+    const bool late = quant_dtype != MSCO_DT_NONE && row_bytes > 8192ll << f.shift;
 #define MSCO_ROUTE_FUSED(Q)                                                                                                  \
-    hipLaunchKernelGGL(route_fused_kernel<Q>, grid, block, lds_bytes, s, static_cast<const unsigned char *>(x), expert_idx,   \
+    auto kern = late ? route_fused_kernel<Q, Q == 0> : route_fused_kernel<Q, true>;                                           \
+    hipLaunchKernelGGL(kern, grid, block, lds_bytes, s, static_cast<const unsigned char *>(x), expert_idx,   \
                        static_cast<unsigned char *>(expanded_x), expanded_scale, expanded_row_idx,                            \
-                       expert_tokens_count_or_cumsum, expert_tokens_before_capacity, n, (int)expert_num,                      \
-                       (int)count_or_cumsum_flag, (long long)hidden * (quant_dtype == MSCO_DT_NONE ? elem_bytes : 2), (int)k, rep)
-    if (quant_dtype == MSCO_DT_NONE) MSCO_ROUTE_FUSED(0);
-    else if (quant_dtype == MSCO_DT_F16) MSCO_ROUTE_FUSED(1);
-    else MSCO_ROUTE_FUSED(2);
+                       expert_tokens_count_or_cumsum, expert_tokens_before_capacity, (int)n, (int)expert_num,                 \
+                       (int)count_or_cumsum_flag, row_bytes, (int)k, rep, f.slice_tokens, f.shift)
+    if (quant_dtype == MSCO_DT_NONE) { MSCO_ROUTE_FUSED(0); }
+    else if (quant_dtype == MSCO_DT_F16) { MSCO_ROUTE_FUSED(1); }
+    else { MSCO_ROUTE_FUSED(2); }
 #undef MSCO_ROUTE_FUSED
     return hipGetLastError() == hipSuccess ? MSCO_OK : MSCO_ERR_DEVICE;
   }
@@ -712,8 +788,9 @@ int msco_moe_token_unpermute(const void *permuted_tokens, const int32_t *sorted_
   const auto *pt = static_cast<const unsigned short *>(permuted_tokens);
   const auto *pr = static_cast<const unsigned short *>(probs);
   auto *o = static_cast<unsigned short *>(out);
-  // enough tokens to fill the chip with one workgroup per four pieces: fewer, larger workgroups; else one per piece
-  const int u = (num_tokens >= 1024 && top_k <= 8) ? 4 : 1;
+  // enough tokens to fill the chip with one workgroup per four pieces: fewer, larger workgroups; else one per piece (and where a
+  // row is one piece: 4096 x top-2 x 2048 10.2 against 11.2 us)
+  const int u = (num_tokens >= 1024 && top_k <= 8 && hidden > 2048) ? 4 : 1;
   const long long piece = 2048ll * u;
   const dim3 grid((unsigned)num_tokens, (unsigned)((hidden + piece - 1) / piece > 16 ? 16 : (hidden + piece - 1) / piece)), block(256);
   const bool bf = dtype == MSCO_DT_BF16;
@@ -727,7 +804,7 @@ int msco_moe_token_unpermute(const void *permuted_tokens, const int32_t *sorted_
       else hipLaunchKernelGGL((unpermute_kernel<false, K, 1>), grid, block, 0, s, pt, sorted_indices, pr, o, (int)top_k, (long long)hidden);    \
     }                                                                                                                   \
   } while (0)
-  switch (top_k) {
+  switch (2 * hidden <= 0x7FFFFFFF ? top_k : 0) {   // (a row has to fit a buffer descriptor)
     case 1: MSCO_UNPERMUTE(1); break;
     case 2: MSCO_UNPERMUTE(2); break;
     case 4: MSCO_UNPERMUTE(4); break;

@@ -335,6 +335,44 @@ def test_routing_with_dynamic_quantisation_is_bit_exact(n_rows, h, k, e, bf16):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_rows,h,k,e", [(1, 24, 1, 1), (1, 16384, 2, 8), (2, 40968, 70, 100), (3, 2056, 200, 64), (5, 1016, 64, 65),
+                                          (255, 7168, 8, 64), (257, 5120, 4, 16), (700, 2048, 8, 128), (1281, 3080, 4, 63), (4097, 1024, 1, 1024),
+                                          (2048, 4096, 8, 256)])
+def test_one_launch_routing_with_rows_shared_by_wavefronts(n_rows, h, k, e):
+    """Tokens per workgroup 1 to 17, wavefronts per row 1 to 16, rows beyond what the wavefronts keep, slices of more than 64
+    entries, expert tables of one wavefront and of several: quantised rows, copied rows, indices and boundaries, bit for bit."""
+    rng = np.random.default_rng(n_rows * 7 + h)
+    x = rng.uniform(-3, 3, (n_rows, h)).astype(np.float16)
+    x[-1, -1] = 11.0                                                               # the last vector holds the maximum
+    idx = np.minimum(rng.integers(0, e, (n_rows, k)), rng.integers(0, e, (n_rows, k))).astype(np.int32)
+    ref_rows, ref_idx, ref_tok = M.moe_init_routing_v2(x, idx, e, 1)
+    ref_q, ref_s = M.dyn_quant(ref_rows)
+    ex, sc, ridx, tok = _route_quant_gpu(np.ascontiguousarray(x.view(np.uint16)), False, idx, e, 1)
+    assert np.array_equal(ridx, ref_idx) and np.array_equal(tok, ref_tok)
+    assert np.array_equal(sc.view(np.uint32), ref_s.view(np.uint32)) and np.array_equal(ex, ref_q)
+    got = _route_gpu(x, idx, e, 1)
+    assert np.array_equal(got[0].view(np.uint16), ref_rows.view(np.uint16)) and np.array_equal(got[1], ref_idx) and np.array_equal(got[2], ref_tok)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("top_k", [1, 2, 4, 8])
+@pytest.mark.parametrize("tokens,hidden", [(5, 2040), (1025, 6152)])
+def test_token_unpermute_bf16_rounds_like_the_golden(tokens, hidden, top_k):
+    """bfloat16 products and sums rounded two at a time by the hardware: ties, subnormals, infinities and the largest values as
+    by hand; rows that end inside a workgroup's pieces."""
+    rng = np.random.default_rng(tokens + top_k)
+    pt = rng.integers(0, 1 << 16, (tokens * top_k, hidden)).astype(np.uint16)
+    pt = np.where((pt & 0x7F80) == 0x7F80, pt & 0xFF80, pt)                        # infinities, no NaN
+    pr = (rng.standard_normal((tokens, top_k)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    si = rng.permutation(tokens * top_k).astype(np.int32)
+    with np.errstate(all="ignore"):
+        want = M.moe_token_unpermute_bf16(pt, si, pr)
+    got = _unpermute_gpu(pt, si, pr, cabi.DT_BF16)
+    nan = lambda b: (b & 0x7FFF) > 0x7F80                                          # (inf - inf: a NaN either way)
+    assert np.array_equal(nan(got), nan(want)) and np.array_equal(got[~nan(want)], want[~nan(want)])
+
+
+@pytest.mark.gpu
 def test_routing_with_dynamic_quantisation_rejects_what_it_cannot_take():
     with pytest.raises(RuntimeError):                                               # float32 activations
         cabi.moe_init_routing_v2_quant(1, 1, 1, 1, 1, None, None, 1, 0, 4, 64, 2, 8, cabi.DT_F32, 1)
