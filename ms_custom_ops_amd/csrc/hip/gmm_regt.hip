@@ -42,7 +42,6 @@ namespace {
 typedef long long i64;
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef int v2i __attribute__((ext_vector_type(2)));
-typedef unsigned short v8us __attribute__((ext_vector_type(8), aligned(2)));   // antiquant rows may start at any element
 
 template <int XT, int WB, int R, int CPL, int WN>
 struct RtShape {
@@ -53,7 +52,9 @@ struct RtShape {
   static constexpr int kDw = CPL * WB / 32;             // dwords per lane and K row
   static constexpr int kCols = 16 * CPL * WN;
   static constexpr int kRed = WN * kWk * 8 * 1024;      // 16 rows x 8 word positions of every wave's accumulators
-  static constexpr size_t kLds = (size_t)kRed + WN * kWk * R * 64 + 16;   // + row sums of x per wave, ticket
+  static constexpr int kEp = kRed + WN * kWk * R * 64 + 16;   // + row sums of x per wave, ticket
+  static_assert(kThreads == kCols, "a thread brings the epilogue operands of one column");
+  static constexpr size_t kLds = (size_t)kEp + 8 * kCols + 64 * R;   // + the columns' scales and offsets (biases), the rows' scales
   static constexpr size_t kSliceWords = (size_t)R * (16 * kCols / 2 + 8);   // 64-bit words of a K slice's partial tile (+ row sums)
 };
 
@@ -212,6 +213,29 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
       for (int t = 0; t < L; ++t) rt_mfma<XT>(rs[t], xbuf[B][t], ones_frag);
     }
   };
+  // Epilogue operands, one column (and one row) per thread: requested here and handed over through LDS behind the loop.  Asked for where
+  // they are used, they cost a memory round trip of 1 to 2 us behind the last weight (6 rows over 16 experts, 1568 x 2048, two slices:
+  // 4700 of 24000 cycles from the last slice's arrival to the end); int8 x looked its scales and biases up one by one.  us, before -> now: 25 rows
+  // over 32 experts, 4064 x 1296, int8 x on 4 bits 28.8 -> 25.4; 120 decode shapes: int8 x on 4 bits 0.88 of the time, 16-bit x 0.975.  Nothing is
+  // converted here: that would wait.
+  unsigned ep_scale = 0x3F800000u, ep_other = 0u;   // scale: 16 or 32 bits as they are; offset or bias
+  float ep_pt = 1.0f;
+  {
+    const bool in = n0 + tid < p.n;
+    if constexpr (FP) {
+      const unsigned at = in ? (unsigned)(n0 + tid) * 2u : kBufferOob;
+      const long long row = (long long)grp * p.n * 2;
+      ep_scale = (unsigned)__builtin_amdgcn_raw_buffer_load_b16(buffer_over(static_cast<const char *>(p.aq_scale) + row, 2ll * p.n), at, 0, 0);
+      ep_other = (unsigned)__builtin_amdgcn_raw_buffer_load_b16(buffer_over(static_cast<const char *>(p.aq_offset) + (p.aq_offset ? row : 0), p.aq_offset ? 2ll * p.n : 0), at, 0, 0);
+    } else if (in) {
+      const long long idx = (p.scale_per_group ? (long long)grp * p.n : 0) + n0 + tid, at = p.scale_is_scalar ? 0 : idx;
+      if (p.scale_dtype == DT_F32) ep_scale = reinterpret_cast<const unsigned *>(p.scale)[at];
+      else if (p.scale_dtype == DT_BF16) ep_scale = reinterpret_cast<const unsigned short *>(p.scale)[at];
+      else if (p.scale_dtype != DT_NONE) ep_scale = reinterpret_cast<const unsigned *>(p.scale)[2 * at];
+      if (p.bias) ep_other = (unsigned)p.bias[idx];
+    }
+    if (!FP && p.per_token && tid < chunk_rows) ep_pt = p.per_token[m0 + tid];
+  }
   static_for<NB - 1>([&](auto b_c) { issue(b_c, s_begin + wk + WK * decltype(b_c)::value); });
   for (int s = s_begin + wk; s < s_end; s += NB * WK) {
     static_for<NB>([&](auto b_c) {
@@ -235,6 +259,16 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
       for (int t = 0; t < L; ++t) *reinterpret_cast<v4f *>(red_rs + wave * 16 * R + 16 * t + 4 * h) = rs[t];
     }
   }
+  float *s_scale = reinterpret_cast<float *>(smem + S::kEp), *s_pt = s_scale + 2 * S::kCols;
+  int *s_other = reinterpret_cast<int *>(s_scale + S::kCols);   // offsets as float32, biases as they are
+  if constexpr (FP) {
+    s_scale[tid] = BF16 ? __uint_as_float(ep_scale << 16) : f16_bits_to_f32((unsigned short)ep_scale);
+    s_other[tid] = __float_as_int(BF16 ? __uint_as_float(ep_other << 16) : f16_bits_to_f32((unsigned short)ep_other));
+  } else {
+    s_scale[tid] = __uint_as_float(p.scale_dtype == DT_BF16 ? ep_scale << 16 : ep_scale);
+    s_other[tid] = (int)ep_other;
+    if (tid < 16 * R) s_pt[tid] = ep_pt;
+  }
   // item u of this thread: lane position `lane` of wave column iwn, row ir of the lane's four
   auto item_wn = [&](int u) { return (tid + NT * u) >> 8; };
   auto item_row = [&](int u) { return 4 * h + (((tid + NT * u) >> 6) & 3); };
@@ -243,28 +277,21 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
     if (n >= p.n) return;
     constexpr int shift = WB == 4 ? 4 : 0;   // the operands were 16 times the nibbles: exact
     float f[8];
+    const float *sc = s_scale + (n - n0);
+    const int *other = s_other + (n - n0);
     if constexpr (FP) {
-      const long long at = ((long long)grp * p.n + n) * 2;
-      const v8us s8 = *reinterpret_cast<const v8us *>(static_cast<const char *>(p.aq_scale) + at);
-      v8us o8 = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (p.aq_offset) o8 = *reinterpret_cast<const v8us *>(static_cast<const char *>(p.aq_offset) + at);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const unsigned short sb = s8[j], ob = o8[j];
-        const float sc = BF16 ? bf16_bits_to_f32(sb) : f16_bits_to_f32(sb);
-        const float of = BF16 ? bf16_bits_to_f32(ob) : f16_bits_to_f32(ob);
-        f[j] = fmaf(of, xs, v[j] * (1.0f / (1 << shift))) * sc;
-      }
+      for (int j = 0; j < 8; ++j) f[j] = fmaf(__int_as_float(other[j]), xs, v[j] * (1.0f / (1 << shift))) * sc[j];
     } else {
       if (p.out_dtype == DT_I32) {
         int *dst = reinterpret_cast<int *>(p.out) + (long long)(m0 + row) * p.n + n;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dst[j] = (v[j] >> shift) + load_bias(p, grp, n + j);
+        for (int j = 0; j < 8; ++j) dst[j] = (v[j] >> shift) + other[j];
         return;
       }
-      const float pt = p.per_token ? p.per_token[m0 + row] : 1.0f;
+      const float pt = s_pt[row];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = dequant((v[j] >> shift) + load_bias(p, grp, n + j), load_scale(p, grp, n + j), pt);
+      for (int j = 0; j < 8; ++j) f[j] = dequant((v[j] >> shift) + other[j], sc[j], pt);
     }
     unsigned q[4];
     activate_n(f, p.act_type);
@@ -325,37 +352,45 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
   if (*s_ticket != (unsigned)(p.split_k - 1)) return;
   if (tid == 0) __hip_atomic_store(&p.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll 1
-  for (int item = 0; item < L * NJ * ITEMS; ++item) {
-    const int t = item / (NJ * ITEMS), j8 = item / ITEMS % NJ, u = item % ITEMS;
+  for (int tu = 0; tu < L * ITEMS; ++tu) {
+    const int t = tu / ITEMS, u = tu % ITEMS;
     const int iwn = item_wn(u), row = 16 * t + item_row(u);
     if (row >= chunk_rows) continue;
-    Elem v[8];
+    Elem v[NJ][8];   // (both pieces of a row are requested together)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = 0;
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[j][e] = 0;
     float xs = 0.f;
     for (int s0 = 0; s0 < p.split_k; s0 += 4) {
-      i64 part[4][4];
+      i64 part[4][NJ][4];
       float ps[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const i64 *src = base + (long long)min(s0 + q, p.split_k - 1) * S::kSliceWords;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) part[q][e] = __hip_atomic_load(src + (item * 4 + e) * NT + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            part[q][j][e] = __hip_atomic_load(src + (((t * NJ + j) * ITEMS + u) * 4 + e) * NT + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         ps[q] = FP ? __hip_atomic_load(reinterpret_cast<const float *>(src + kSums) + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         if (s0 + q < p.split_k) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[2 * e] += __builtin_bit_cast(Elem, (unsigned)(unsigned long long)part[q][e]);
-            v[2 * e + 1] += __builtin_bit_cast(Elem, (unsigned)((unsigned long long)part[q][e] >> 32));
-          }
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[j][2 * e] += __builtin_bit_cast(Elem, (unsigned)(unsigned long long)part[q][j][e]);
+              v[j][2 * e + 1] += __builtin_bit_cast(Elem, (unsigned)((unsigned long long)part[q][j][e] >> 32));
+            }
           xs += ps[q];
         }
       }
     }
-    finish(row, n0 + 16 * CPL * iwn + CPL * c16 + 8 * j8, v, xs);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) finish(row, n0 + 16 * CPL * iwn + CPL * c16 + 8 * j, v[j], xs);
   }
 }
 
