@@ -429,6 +429,32 @@ void plan_few_rows(msco_gmm_op *op, int &family) {
   op->tile_cfg = tiles * 8 <= cus * 9 ? TILE_32x128 : nk || k < 1024 ? TILE_64x128 : TILE_32x256;
 }
 
+// Tiles just too many for one round of the chip.  128 x 128 and 64 x 128 tiles that are one to a CU walk K in 128-byte slabs with nothing
+// masked; with more of them than CUs the plan gives them 64-byte slabs and two or three workgroups share a CU's loads, which takes about
+// twice as long.  The next shape in one round (or in fewer, larger workgroups) is then the better one.  us, the tile picked above -> this,
+// 1200 random shapes, all forms measured on each (one group of 33 to 4096 rows; 8 to 128 groups, even and uneven routings):
+//   [E,K,N], 128 x 128 -> 128 x 256 from K = 1024: 45 shapes at 0.84 (0.63 .. 1.00); 8 experts, 165 rows, 7168 x 3696 122 -> 79; one group, 947 rows,
+//   4224 x 4704 43 -> 34; not where N leaves a quarter of the wider tiles empty (8 experts, 718 rows, 1792 x 560 14.7 -> 19.6) or K is short
+//   (10812 rows, 768 x 640 12.1 -> 15.7).
+//   [E,K,N] and [E,N,K], 64 x 128 -> 128 x 128 from K = 2048 where those are one round: 12 shapes at 0.72 (0.59 .. 0.84); 8 experts, 97 rows, 5312 x
+//   2368 55 -> 34; one group, 156 rows, 5184 x 13856 51 -> 39; shorter K 0.97 .. 1.11.  [E,N,K] tiles of 128 x 256 gain less (one group 0.94,
+//   several 0.99, from 0.77 to 1.58) and are not taken.
+//   Packed weights stay (128 x 256 tiles for several groups 0.95, from 0.81 to 1.31; 64 x 128 for one group 0.94, from 0.77 to 1.04).
+// 600 other shapes: 21 changed, 0.83 of the time, the worst 1.01.
+void plan_one_round(msco_gmm_op *op) {
+  const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
+  const bool packed = is_packed(op->desc), kn = !packed && !op->desc.transpose_b;
+  auto tiles = [&](int64_t bm, int64_t bn) {   // an average group's and a tenth more rows (real routings are uneven)
+    const int64_t groups = std::max<int64_t>(1, std::min(e, m)), rows = e == 1 ? m : (11 * m + 10 * e - 1) / (10 * e);
+    return groups * ((rows + bm - 1) / bm) * ((n + bn - 1) / bn);
+  };
+  if (op->tile_cfg == TILE_128x128 && tiles(128, 128) > cus) {
+    if (kn && k >= 1024 && n * 4 >= (n + 255) / 256 * 256 * 3) op->tile_cfg = TILE_128x256;
+  } else if (op->tile_cfg == TILE_64x128 && !packed && k >= 2048 && tiles(64, 128) > cus && tiles(128, 128) <= cus) {
+    op->tile_cfg = TILE_128x128;
+  }
+}
+
 void choose_plan(msco_gmm_op *op) {
   const msco_gmm_desc &d = op->desc;
   const int num_cus = op->num_cus;
@@ -568,7 +594,10 @@ void choose_plan(msco_gmm_op *op) {
       op->tile_cfg = TILE_64x128;
     }
   }
-  if (d.kernel_override == OV_AUTO && aligned && is_w8a8(d) && !is_w4(d)) plan_few_rows(op, family);
+  if (d.kernel_override == OV_AUTO && aligned && is_w8a8(d) && !is_w4(d)) {
+    if (family == FAM_TILE) plan_one_round(op);
+    plan_few_rows(op, family);
+  }
   switch (d.kernel_override) {
     case OV_TILE_256: family = FAM_TILE; op->tile_cfg = TILE_256x256; break;
     case OV_TILE_256_W4: family = FAM_TILE; op->tile_cfg = TILE_256x256_W4; break;
