@@ -439,6 +439,9 @@ void plan_few_rows(msco_gmm_op *op, int &family) {
 //   [E,K,N] and [E,N,K], 64 x 128 -> 128 x 128 from K = 2048 where those are one round: 12 shapes at 0.72 (0.59 .. 0.84); 8 experts, 97 rows, 5312 x
 //   2368 55 -> 34; one group, 156 rows, 5184 x 13856 51 -> 39; shorter K 0.97 .. 1.11.  [E,N,K] tiles of 128 x 256 gain less (one group 0.94,
 //   several 0.99, from 0.77 to 1.58) and are not taken.
+//   [E,N,K], several groups, more than two 128 x 128 tiles per CU -> the persistent kernel where its tiles are one round on more than half of the
+//   CUs, from K = 2048: 25 shapes at 0.78 (0.54 .. 1.04); 16 experts, 627 rows, 5472 x 1168 146 -> 79; 32 experts, 296 rows, 3520 x 864 71 -> 56.
+//   ([E,K,N] from 128 x 256 tiles: 0.83, but up to 1.25.)
 //   Packed weights stay (128 x 256 tiles for several groups 0.95, from 0.81 to 1.31; 64 x 128 for one group 0.94, from 0.77 to 1.04).
 // 600 other shapes: 21 changed, 0.83 of the time, the worst 1.01.
 void plan_one_round(msco_gmm_op *op) {
@@ -450,6 +453,7 @@ void plan_one_round(msco_gmm_op *op) {
   };
   if (op->tile_cfg == TILE_128x128 && tiles(128, 128) > cus) {
     if (kn && k >= 1024 && n * 4 >= (n + 255) / 256 * 256 * 3) op->tile_cfg = TILE_128x256;
+    else if (!packed && !kn && e > 1 && e <= 1024 && k >= 2048 && tiles(128, 128) > 2 * cus && tiles(256, 256) * 2 > cus && tiles(256, 256) <= cus) op->tile_cfg = TILE_256x256_W4;
   } else if (op->tile_cfg == TILE_64x128 && !packed && k >= 2048 && tiles(64, 128) > cus && tiles(128, 128) <= cus) {
     op->tile_cfg = TILE_128x128;
   }

@@ -11,7 +11,8 @@ PICKS = [(720, 1024, 5632, 1, False, False, "tile_128x256"), (720, 1008, 5632, 1
          (720, 4096, 5632, 1, False, True, "tile_128x128"),
          (1320, 7168, 3696, 8, False, False, "tile_128x256"), (5744, 1792, 560, 8, False, False, "tile_128x128"),
          (776, 2048, 2368, 8, False, False, "tile_128x128"), (776, 2032, 2368, 8, False, False, "tile_64x128"),
-         (776, 2048, 2368, 8, True, False, "tile_128x128")]
+         (776, 2048, 2368, 8, True, False, "tile_128x128"), (4736, 2048, 1248, 32, True, False, "tile_256x256x128_w4"),
+         (4736, 2032, 1248, 32, True, False, "tile_128x128"), (4736, 2048, 1248, 32, False, False, "tile_128x256")]
 
 
 def _op(m, k, n, e, nk, packed):
