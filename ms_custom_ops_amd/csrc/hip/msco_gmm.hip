@@ -648,13 +648,19 @@ void choose_plan(msco_gmm_op *op) {
       // s = 1 / 2 / 3: 20.9 / 18.0 / 24.3 us, the third slice starting a second round).  Of the 32 x 128 tiles two share a CU, in a
       // fifth more time than one alone, and the exchange is half as large: 128 experts, 24 rows, 3264 x 976, s = 1 / 2: 21.7 / 16.9; 16 experts,
       // 18 rows, 3392 x 1168: 16.0 / 14.3; 8 experts, 16 rows, 6400 x 2304: 32.6 / 30.3; 16 experts, 12 rows, 608 x 2096: 7.8 / 9.7.
+      // One group (206 random shapes of 1 to 400 rows, every split measured): a slice adds less than that -- 4 and 6 in place of 6 and 8, and 2
+      // once -- but a launch that fills more than 15/16 of the CUs with 32 x 128 tiles already takes what two on a CU take, 1.6 times one
+      // alone (4 rows, 2272 x 10448, s = 2 / 3: 11.5 / 14.0).  32 x 128 0.971 of the time, none slower (7 rows, 6176 x 10464 26.2 -> 21.5; 3 rows,
+      // 7552 x 4256 15.4 -> 14.0), 64 x 128 0.991 (41 rows, 2720 x 1200 10.9 -> 9.6).
       const int cus = or_default(tuning().tile_target_wgs, num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       const int cap = (int)std::max<int64_t>(1, ((k + 63) / 64) / kTileMinSlabs);
       auto split_cost = [&](int sl) {
         const int64_t slabs = ((k + 63) / 64 + sl - 1) / sl;
-        const int64_t rounds = (t * sl + cus - 1) / cus;
-        const int64_t fifths = few && rounds > 1 ? (rounds + 1) / 2 * 6 : rounds * 5;
-        const int64_t exchange = sl > 1 ? (int64_t)(4 + bm * bn / 2048) * sl - 2 : 0;
+        const bool one_small = e == 1 && (few || op->tile_cfg == TILE_64x128);
+        const int64_t slots = few && e == 1 && sl > 1 ? cus * 15 / 16 : cus;
+        const int64_t rounds = (t * sl + slots - 1) / slots;
+        const int64_t fifths = few && rounds > 1 ? (rounds + 1) / 2 * (e == 1 ? 8 : 6) : rounds * 5;
+        const int64_t exchange = sl <= 1 ? 0 : one_small ? (int64_t)(2 + bm * bn / 2048) * sl + 2 : (int64_t)(4 + bm * bn / 2048) * sl - 2;
         return fifths * (slabs + 10 + exchange);
       };
       int want = 1;
@@ -803,7 +809,7 @@ void choose_plan(msco_gmm_op *op) {
       want = std::max(1, std::min(std::min(want, kMaxSplitK), cap));
     } else if (is_packed(d)) {
       // Packed weights: strips as wide as still give every CU a workgroup without splitting K (a slice holds at
-      // most 128 blocks of 64 bytes), then a K split up to about two workgroups per CU.
+      // most 128 blocks of 64 bytes).
       const int64_t col_groups = (n + 15) / 16, k_blocks = (k + 63) / 64;
       const int slice_blocks = is_w8a8(d) ? 128 : 64;
       const int floor_split = (int)((k_blocks + slice_blocks - 1) / slice_blocks);
@@ -815,10 +821,13 @@ void choose_plan(msco_gmm_op *op) {
       op->strip_groups = groups;
       op->n_strips = (int)((col_groups + groups - 1) / groups);
       op->skinny_cols = groups * 16;
-      const int64_t base = (int64_t)op->n_strips * active;
-      want = (int)(kTargetWorkgroups / std::max<int64_t>(base, 1));
-      cap = std::max<int>(1, (int)(k_blocks / 16));      // a slice keeps at least 16 blocks
-      want = std::max(floor_split, std::min(std::min(want, kMaxSplitK), cap));
+      // No split beyond that: a strip of one column group is a walk of K / 256 requests per wave, and the exchange costs more than any
+      // of it saves (us, two workgroups per CU through a split -> none: one row, 2688 x 2800 8.1 -> 5.1; 13 rows, 8128 x 1568 13.0 -> 7.9; 5 rows
+      // over 32 experts, 5536 x 576 8.9 -> 6.7; 16-bit x, one row, 3520 x 3920 9.9 -> 6.9).
+      // Two slices are left where at most two thirds of the CUs have a strip and there are no more than 1024 columns and K is 4096 or more: about what
+      // none takes (two rows, 8096 x 1120: 7.1 / 7.8 with one / two slices, 10.0 with the seven planned before).
+      want = floor_split;
+      if (col_groups <= 64 && (int64_t)op->n_strips * active * 3 <= 2 * (int64_t)num_cus && k_blocks >= 64) want = std::max(want, 2);
       cap = kMaxSplitK * 64;
     } else if (wide16) {
       // at most one 16-wave workgroup per CU, every wave keeps at least one block
