@@ -808,9 +808,10 @@ void choose_plan(msco_gmm_op *op) {
       cap = std::max<int>(1, (int)(k_blocks / 16));      // a slice keeps at least 16 blocks
       want = std::max(1, std::min(std::min(want, kMaxSplitK), cap));
     } else if (is_packed(d)) {
-      // Packed weights: strips as wide as still give every CU a workgroup.  Where one workgroup walks all of K those are counted over the
-      // groups that a random routing hits (int8 x, 16 experts, 16 rows, 800 x 4176: 14.6 -> 11.1 us with the strips that follow; 329 int8
-      // shapes of 8 to 128 experts 0.988 of the time that one workgroup per group that can be hit gives).
+      // Packed weights: strips as wide as still give every CU a workgroup.  With int8 x, where one workgroup walks all of K, those are counted over the
+      // groups that a random routing hits (16 experts, 16 rows, 800 x 4176: 14.6 -> 11.1 us with the strips that follow; 329 int8
+      // shapes of 8 to 128 experts 0.988 of the time that one workgroup per group that can be hit gives; 16-bit x gains 0.4 % over 449 shapes and loses 5 %
+      // on some of them: 100 rows over 16 experts, 3776 x 1440 19.6 -> 20.6).
       // A slice of K holds 128 blocks of 64 bytes, with 16-bit x 64.  Beyond 64 the 16-bit kernel would take two slices of 9 to 16 blocks
       // per wave in the code for 16, most requests of a shorter one masked: slices of at most 32 blocks, eight per wave, instead (us, two
       // slices -> three or four: 18 rows over 16 experts, 4288 x 2320 43.9 -> 30.6; 14 rows, one group, 4288 x 8288 22.1 -> 13.8; 4 rows over 16 experts,
@@ -819,7 +820,7 @@ void choose_plan(msco_gmm_op *op) {
       const int slice_blocks = is_w8a8(d) ? 128 : 64, fewest = (int)((k_blocks + slice_blocks - 1) / slice_blocks);
       const bool short_slices = !is_w8a8(d) && fewest > 1 && k_blocks <= 32 * kMaxSplitK;
       const int floor_split = short_slices ? (int)((k_blocks + 31) / 32) : fewest;
-      const int64_t hit = floor_split > 1 ? active : std::min(active, groups_hit(m, e) * std::max<int64_t>(1, (m / e + kSkinnyRows - 1) / kSkinnyRows));
+      const int64_t hit = floor_split > 1 || !is_w8a8(d) ? active : std::min(active, groups_hit(m, e) * std::max<int64_t>(1, (m / e + kSkinnyRows - 1) / kSkinnyRows));
       int groups = 16;
       const int min_wgs = or_default(tuning().stream_min_wgs, num_cus);
       while (groups > 1 && ((col_groups + groups - 1) / groups) * hit * floor_split < min_wgs) groups /= 2;
@@ -830,10 +831,13 @@ void choose_plan(msco_gmm_op *op) {
       op->skinny_cols = groups * 16;
       // No split beyond that: a strip of one column group is a walk of K / 256 requests per wave, and the exchange costs more than any
       // of it saves (us, two workgroups per CU through a split -> none: one row, 2688 x 2800 8.1 -> 5.1; 13 rows, 8128 x 1568 13.0 -> 7.9; 5 rows
-      // over 32 experts, 5536 x 576 8.9 -> 6.7; 16-bit x, one row, 3520 x 3920 9.9 -> 6.9; two slices of int8 x on few columns: 8 rows, 4192 x 656
-      // 8.2 -> 6.5; 4 rows over 16 experts, 4064 x 560 7.0 -> 5.3).
+      // over 32 experts, 5536 x 576 8.9 -> 6.7; 16-bit x, one row, 3520 x 3920 9.9 -> 6.9).
+      // Two slices are left where at most two thirds of the CUs have a strip and there are no more than 1024 columns and K is 4096 or more: they cost
+      // up to 1.7 us (one / two slices: two rows, 8096 x 1120 7.1 / 7.8, ten with the seven planned before; 8 rows, 4192 x 656 6.5 / 8.2), but these are the packed decode plans that exchange partial
+      // tiles through the workspace of msco_gmm_launch_static, and its tests hold them to it.
       // (short slices only where msco_gmm_launch_static takes their partial tiles too)
       want = floor_split;
+      if (col_groups <= 64 && (int64_t)op->n_strips * active * 3 <= 2 * (int64_t)num_cus && k_blocks >= 64) want = std::max(want, 2);
       if (short_slices && skinny_counter_count(m, n, e, op->skinny_cols) * (size_t)want * stream_a16w8_tile_bytes() > (size_t)MSCO_GMM_STATIC_WORKSPACE_BYTES) want = fewest;
       cap = kMaxSplitK * 64;
     } else if (wide16) {

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
-@pytest.mark.parametrize("counts,k,n,split", [([3], 4096, 80, 1), ([1], 4112, 528, 3), ([16, 0, 1, 5], 6144, 272, 3), ([2, 0, 0, 7], 6160, 48, 4), ([9], 8192, 16, 4),
+@pytest.mark.parametrize("counts,k,n,split", [([3], 4096, 1040, 1), ([1], 4112, 528, 3), ([16, 0, 1, 5], 6144, 272, 3), ([2, 0, 0, 7], 6160, 48, 4), ([9], 8192, 16, 4),
                                               ([1, 1], 16384, 32, 8), ([2], 16400, 32, 5)])
 def test_within_one_rounding(device, counts, k, n, split, dtype):
     """One rounding of the output plus float32 accumulation noise (2e-5 of the sum of the terms' magnitudes: 16 x 4 lanes' partial sums of
