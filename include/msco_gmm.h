@@ -156,13 +156,17 @@ MSCO_API int msco_gmm_create(const msco_gmm_desc *desc, msco_gmm_handle *out_han
 /* Fix the shapes (shape-dependent work of Resize: kernel choice, grid, workspace size).
  * m = rows of x, k = reduction length, n = output columns, e = number of groups.
  * Replaces UpdateShape + Tiling + GetWorkspaceSize.  May be called again with new shapes, but only while no launch
- * of this handle is in flight on any stream: planning re-zeroes (with a synchronous hipMemset) the arrival counters
+ * of this handle is in flight on any stream: planning re-zeroes (and waits for it) the arrival counters
  * that a split-K launch of the handle reduces through, and may free and re-allocate them.  Callers that re-plan per
- * shape keep one handle per (shape, stream), as the operator layer's plan cache does. */
+ * shape keep one handle per (shape, stream), as the operator layer's plan cache does.  Planning and destroying are also
+ * allowed while a stream of the calling thread is captured into a graph. */
 MSCO_API int msco_gmm_plan(msco_gmm_handle h, int64_t m, int64_t k, int64_t n, int64_t e, size_t *workspace_bytes);
 
 /* Enqueue the computation.  inputs[MSCO_IN_COUNT] are device pointers (NULL = absent);
- * out is [M,N] in out_dtype; stream is a hipStream_t (NULL = default stream). */
+ * out is [M,N] in out_dtype; stream is a hipStream_t (NULL = default stream).  Launches on a stream that is captured
+ * may be replayed after the handle is re-planned or destroyed, and beside its other launches: the launches that one capture
+ * records reduce through arrival counters of their own (16 MiB per GPU for all of them; beyond, through the handle's,
+ * which are then kept until the process ends and share the handle's one-stream rule). */
 MSCO_API int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, void *workspace,
                     size_t workspace_bytes, void *stream);
 

@@ -104,7 +104,11 @@ struct msco_gmm_op {
   int64_t widen_bytes = 0;   // 4-bit weights without a kernel of their own for the shape: int8 copy of them at the front of the workspace
   size_t workspace_bytes = 0;
   unsigned *counters = nullptr;
-  size_t counters_cap = 0;
+  size_t counters_cap = 0, counters_used = 0;   // allocated; of the present plan
+  bool counters_recorded = false;               // a recorded graph counts with `counters`: they are never freed
+  unsigned *recorded = nullptr;                 // counters of the launches that capture `recorded_id` records
+  size_t recorded_cap = 0;
+  unsigned long long recorded_id = 0;
   int num_cus = kDefaultCUs;   // compute units of the device that was current at create time
   std::string info;
   std::mutex mu;
@@ -936,6 +940,96 @@ int msco_gmm_create(const msco_gmm_desc *desc, msco_gmm_handle *out_handle) {
   return MSCO_OK;
 }
 
+// Planning allocates, clears and frees counters, also while a stream of this thread is being captured (the first call of a shape under
+// capture plans there): the runtime refuses these calls in the default capture mode and spoils the capture.  Relaxed, it takes
+// them, as none of them belongs to the captured stream -- but nothing on the null stream, so clearing has a stream of its own.
+namespace {
+constexpr int kMaxDevices = 64;
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  RelaxedCapture(const RelaxedCapture &) = delete;
+};
+
+std::mutex g_clear_mu;
+hipStream_t g_clear_stream[kMaxDevices] = {};
+
+bool clear_counters(unsigned *counters, size_t count) {   // and wait for it
+  int dev = -1;
+  hipStream_t stream = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_clear_mu);
+    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices &&
+        (g_clear_stream[dev] != nullptr || hipStreamCreateWithFlags(&g_clear_stream[dev], hipStreamNonBlocking) == hipSuccess))
+      stream = g_clear_stream[dev];
+  }
+  if (stream != nullptr && hipMemsetAsync(counters, 0, count * sizeof(unsigned), stream) == hipSuccess && hipStreamSynchronize(stream) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+void free_counters(msco_gmm_op *h) {
+  if (h->counters != nullptr && !h->counters_recorded) (void)hipFree(h->counters);
+  h->counters = nullptr;
+  h->counters_cap = 0;
+  h->counters_recorded = false;
+}
+
+// A recorded launch is replayed whenever its graph is: after the handle is gone or re-planned, and beside eager launches and other graphs.
+// So the launches that one capture records through one handle (they are ordered) count in a range of this array that is handed
+// out once.  It is zero when the library is loaded, counters reset themselves at the end of a launch, nothing is
+// allocated under capture.  Once it is used up, a recorded launch counts with its handle's own counters, which then stay allocated.
+constexpr size_t kRecordedCounters = (size_t)4 << 20;
+static __device__ unsigned recorded_counters[kRecordedCounters];
+std::mutex g_recorded_mu;
+unsigned *g_recorded_ptr[kMaxDevices] = {};
+size_t g_recorded_used[kMaxDevices] = {};
+
+unsigned *take_recorded_counters(size_t count) {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  std::lock_guard<std::mutex> lock(g_recorded_mu);
+  if (g_recorded_ptr[dev] == nullptr) {
+    void *ptr = nullptr;
+    if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(recorded_counters)) != hipSuccess || ptr == nullptr) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    g_recorded_ptr[dev] = static_cast<unsigned *>(ptr);
+  }
+  count = (count + 15) / 16 * 16;   // (ranges of different captures share no 64-byte piece)
+  if (count > kRecordedCounters - g_recorded_used[dev]) return nullptr;
+  unsigned *at = g_recorded_ptr[dev] + g_recorded_used[dev];
+  g_recorded_used[dev] += count;
+  return at;
+}
+
+// the arrival counters of a launch on `stream`
+unsigned *launch_counters(msco_gmm_op *h, hipStream_t stream) {
+  if (h->split_k <= 1 || h->counters == nullptr || stream == nullptr) return h->counters;   // (the null stream is not captured)
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return h->counters;
+  }
+  if (status != hipStreamCaptureStatusActive) return h->counters;
+  std::lock_guard<std::mutex> lock(h->mu);
+  if (h->recorded == nullptr || h->recorded_id != id || h->recorded_cap < h->counters_used) {
+    h->recorded = take_recorded_counters(h->counters_used);
+    h->recorded_cap = h->recorded != nullptr ? h->counters_used : 0;
+    h->recorded_id = id;
+  }
+  if (h->recorded != nullptr) return h->recorded;
+  h->counters_recorded = true;
+  return h->counters;
+}
+}  // namespace
+
 int msco_gmm_plan(msco_gmm_handle h, int64_t m, int64_t k, int64_t n, int64_t e, size_t *workspace_bytes) {
   if (h == nullptr) return MSCO_ERR_INVALID_ARG;
   if (m < 0 || k <= 0 || n <= 0 || e <= 0) return MSCO_ERR_SHAPE;
@@ -953,26 +1047,20 @@ int msco_gmm_plan(msco_gmm_handle h, int64_t m, int64_t k, int64_t n, int64_t e,
                         : h->family == FAM_REGT ? (size_t)chunk_slots(p, 16 * h->row_blocks) * h->n_strips
                         : h->family == FAM_TILE ? tile_count_bound(h->tile_cfg, m, n, e)
                                               : skinny_counter_count(m, n, e, h->skinny_cols);
+    const RelaxedCapture relaxed;
+    h->counters_used = need;
     if (need > h->counters_cap) {
-      if (h->counters) (void)hipFree(h->counters);
-      h->counters = nullptr;
-      h->counters_cap = 0;
+      free_counters(h);
       if (hipMalloc(reinterpret_cast<void **>(&h->counters), need * sizeof(unsigned)) != hipSuccess) {
         (void)hipGetLastError();
         return MSCO_ERR_DEVICE;
       }
-      if (hipMemset(h->counters, 0, need * sizeof(unsigned)) != hipSuccess) {
-        (void)hipGetLastError();
-        return MSCO_ERR_DEVICE;
-      }
+      if (!clear_counters(h->counters, need)) return MSCO_ERR_DEVICE;
       h->counters_cap = need;
     } else if (h->counters != nullptr) {
       // the counters reset themselves at the end of a launch; one that was abandoned half-way (a failed launch, a
       // destroyed stream) may have left tickets behind, so a new plan starts from zero again
-      if (hipMemset(h->counters, 0, h->counters_cap * sizeof(unsigned)) != hipSuccess) {
-        (void)hipGetLastError();
-        return MSCO_ERR_DEVICE;
-      }
+      if (!clear_counters(h->counters, h->counters_cap)) return MSCO_ERR_DEVICE;
     }
   }
   h->planned = true;
@@ -1026,7 +1114,7 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
     p.w = static_cast<const int8_t *>(workspace);
     p.partial = reinterpret_cast<int32_t *>(static_cast<char *>(workspace) + h->widen_bytes);
   }
-  p.counters = h->counters;
+  p.counters = launch_counters(h, static_cast<hipStream_t>(stream));
   p.m = (int)h->m; p.k = (int)h->k; p.n = (int)h->n; p.e = (int)h->e;
   p.gl_dtype = d.group_list_dtype;
   p.gl_type = d.group_list_type;
@@ -1085,7 +1173,6 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
 // is looked up once with hipGetSymbolAddress, with that device current, and kept.
 namespace {
 static __device__ __align__(256) unsigned char scratch[MSCO_GMM_STATIC_WORKSPACE_BYTES];
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void *g_scratch_ptr[kMaxDevices] = {};
 
@@ -1154,7 +1241,10 @@ int msco_pack_weight(const void *src, void *dst, int64_t e, int64_t k, int64_t n
 
 int msco_gmm_destroy(msco_gmm_handle h) {
   if (h == nullptr) return MSCO_ERR_INVALID_ARG;
-  if (h->counters) (void)hipFree(h->counters);
+  {
+    const RelaxedCapture relaxed;
+    free_counters(h);
+  }
   delete h;
   return MSCO_OK;
 }

@@ -112,3 +112,101 @@ def test_moe_chain_is_graph_capturable(device):
         torch.cuda.synchronize()
         assert torch.equal(out, eager), replay
     op.close()
+
+
+def _weight_only(m, k, n, e, seed):
+    """A weight-only grouped call through the Python operator; plans with 16 to 128 rows per group and a long K split it."""
+    import ms_custom_ops_amd as ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    x = torch.randn((m, k), dtype=torch.bfloat16, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (e, k, n), dtype=torch.int8, device="cuda", generator=g)
+    s = (torch.rand(e, n, device="cuda", generator=g) * 1e-3).to(torch.bfloat16)
+    gl = torch.tensor([(m * (i + 1)) // e for i in range(e)], dtype=torch.int64, device="cuda")
+    return lambda: ops.grouped_matmul_v4_cops([x], [w], antiquant_scale=[s], group_list=gl, split_item=3, group_type=0)[0]
+
+
+def _dense(m, k, n, seed):
+    import ms_custom_ops_amd as ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    x = torch.randint(-127, 128, (m, k), dtype=torch.int8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (k, n), dtype=torch.int8, device="cuda", generator=g)
+    s = torch.rand(n, device="cuda", generator=g) * 1e-3
+    return lambda: ops.quant_batch_matmul(x, w, s)
+
+
+# (calls whose plan splits K, and one that does not)
+_CALLS = [(_weight_only, (816, 6336, 544, 16)), (_dense, (13, 7952, 5392)), (_dense, (40, 4096, 512)), (_dense, (2048, 1024, 1024))]
+
+
+@pytest.mark.parametrize("call", _CALLS, ids=["weight_only_split_k", "few_rows_split_k", "small_tile_split_k", "tile"])
+def test_first_call_of_a_shape_under_capture_and_replays_after_its_plan_is_gone(device, call):
+    """Planning allocates and clears arrival counters; inside a capture it has to go through.  70 other shapes then push the plan out of the
+    operators' cache (64 plans per process): the recorded launches keep counters of their own, so replays stay right."""
+    make, args = call
+    f = make(*args, seed=5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = f()
+    eager = f().clone()
+    torch.cuda.synchronize()
+    assert eager.ne(0).any()
+
+    def replays():
+        for _ in range(3):
+            out.fill_(7)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager)
+            assert torch.equal(f(), eager)
+
+    replays()
+    for i in range(70):
+        _dense(1 + i % 16, 1024 + 16 * i, 256, seed=i)()
+    replays()
+
+
+def test_graphs_of_one_shape_replayed_side_by_side(device):
+    """Two graphs recorded on the same stream from one shape, and eager calls, at the same time on three streams."""
+    fs = [_weight_only(816, 6336, 544, 16, seed=s) for s in (1, 2, 3)]
+    want = [f().clone() for f in fs]
+    torch.cuda.synchronize()
+    graphs, outs = [], []
+    for f in fs[:2]:
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            outs.append(f())
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for o in outs:
+            o.fill_(7)
+        torch.cuda.synchronize()
+        for g, st in zip(graphs, streams):
+            with torch.cuda.stream(st):
+                g.replay()
+        eager = fs[2]()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], want[0]) and torch.equal(outs[1], want[1]) and torch.equal(eager, want[2])
+
+
+def test_a_plan_leaves_the_cache_while_a_stream_is_captured(device):
+    """Planning 70 shapes inside one capture evicts plans that other calls allocated counters for."""
+    f = _dense(13, 7952, 5392, seed=1)
+    want = f().clone()
+    small = [_dense(1 + i % 16, 1040 + 16 * i, 272, seed=i) for i in range(70)]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = [g() for g in small]
+    for _ in range(2):
+        for o in outs:
+            o.fill_(7)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, g()) for o, g in zip(outs, small))
+    assert torch.equal(f(), want)
