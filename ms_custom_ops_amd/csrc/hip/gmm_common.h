@@ -47,7 +47,6 @@ struct GmmParams {
   int x_dtype;              // DT_I8 / DT_BF16 / DT_F16
   int split_k;              // number of K splits across workgroups (skinny kernels)
   int n_strips;             // ceil(N / kSkinnyCols)
-  int max_chunks;           // ceil(M / kSkinnyRows): 16-row chunks a group can have (skinny W8A8 kernel)
   int strip_groups;         // packed-layout kernels: 16-column groups per strip (1..16); n_strips counts these strips
   int act_type;             // ACT_*: activation on the float32 result before the output cast (never with int32 output)
   int x_via_lds;            // packed-layout W8A8 decode kernel: stage the chunk's x rows through LDS (pays from about 8 rows per chunk)

@@ -54,11 +54,10 @@ inline long long xcd_slots(const GmmParams &p, int rows_per_chunk) {
 // range; waves split K and reduce through LDS, workgroups split K and reduce through the workspace.
 // wide16: the 16-wave / 128-column-strip variant for small weight sets, else 4 waves / 256-column strips
 hipError_t launch_skinny_w8a8(const GmmParams &p, bool nk, bool wide16, hipStream_t stream);
-size_t skinny_workspace_bytes(int64_t m, int64_t n, int64_t e, int split_k, int cols);
-size_t skinny_counter_count(int64_t m, int64_t n, int64_t e, int cols);
+size_t decode_tiles(int64_t m, int64_t n, int64_t e, int rows_per_chunk, int cols);   // partial tiles (per K slice) and counters of the decode kernels
 
 // Decode kernels for weights in the packed layout (gmm_stream.hip): 4 waves, strips of up to 256 columns, K slices of
-// at most 128 blocks of 64 bytes (split_k chosen accordingly); workspace and counters as for the 4-wave skinny kernel.
+// at most 128 blocks of 64 bytes (split_k chosen accordingly).
 hipError_t launch_stream_w8a8(const GmmParams &p, hipStream_t stream);
 hipError_t launch_stream_a16w8(const GmmParams &p, hipStream_t stream);   // K slices of at most 64 blocks
 // more than 16 rows per group on packed weights: chunks of 16 tch rows (tch = 2, 4, 8), strips of 64 columns

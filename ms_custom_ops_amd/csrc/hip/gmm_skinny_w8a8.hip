@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(SK_THREADS, NK ? 3 : 4) gmm_w8a8_skinny_kernel
     // bypass the per-XCD L2 for this data only, so no cache-wide write-back / invalidate fence is
     // needed.  Every wavefront waits for its own stores (vmcnt == 0) before the barrier that precedes the counter bump.  A tile is kept in
     // the threads' own fragment order: slice s, 64-bit word e of thread t at ((s * 8 + e) * 256 + t).
-    const long long tile = ((long long)grp * p.max_chunks + mc) * p.n_strips + strip;
+    const long long tile = (long long)blockIdx.y * p.n_strips + strip;
     i64 *base = reinterpret_cast<i64 *>(p.partial) + tile * p.split_k * (SK_TILE_INTS / 2);
     if (rows_ok) {
       i64 *mine = base + (long long)ks * (SK_TILE_INTS / 2) + tid;
@@ -360,7 +360,7 @@ __global__ void __launch_bounds__(W16_THREADS) gmm_w8a8_skinny16_kernel(const Gm
 
   if (p.split_k > 1) {
     // cross-workgroup reduction, as in the 4-wave kernel; slice s, word e of reducer t at ((s * 2 + e) * 512 + t)
-    const long long tile = ((long long)grp * p.max_chunks + mc) * gridDim.x + strip;
+    const long long tile = (long long)blockIdx.y * gridDim.x + strip;
     i64 *base = reinterpret_cast<i64 *>(p.partial) + tile * p.split_k * W16_TILE_WORDS;
     if (rows_ok) {
       i64 *mine = base + (long long)ks * W16_TILE_WORDS + tid;
@@ -432,17 +432,14 @@ __global__ void __launch_bounds__(W16_THREADS) gmm_w8a8_skinny16_kernel(const Gm
   }
 }
 
-// one arrival counter per (group, 16-row chunk, strip of `cols` columns)
-size_t skinny_counter_count(int64_t m, int64_t n, int64_t e, int cols) {
-  const int64_t strips = (n + cols - 1) / cols;
-  const int64_t max_chunks = (m + kSkinnyRows - 1) / kSkinnyRows;
-  return (size_t)(e * (max_chunks > 0 ? max_chunks : 1) * strips);
-}
-
-size_t skinny_workspace_bytes(int64_t m, int64_t n, int64_t e, int split_k, int cols) {
-  if (split_k <= 1) return 0;
-  // one 16 x cols tile of 4-byte partial sums per (tile, K slice)
-  return skinny_counter_count(m, n, e, cols) * (size_t)split_k * kSkinnyRows * cols * 4;
+// Partial tiles and arrival counters of the decode kernels: one per (chunk slot, strip of `cols` columns).  A workgroup's slot is its grid.y, and
+// a launch has chunk_slots of them.  (Numbered by group and chunk of the group, as if every group could hold all rows, they were 10 to 30 times
+// as many: 294 rows over 64 experts, 5120 x 13200, two slices 2.2 GB, 163 MB now.)
+size_t decode_tiles(int64_t m, int64_t n, int64_t e, int rows_per_chunk, int cols) {
+  GmmParams p{};
+  p.m = (int)m;
+  p.e = (int)e;
+  return (size_t)chunk_slots(p, rows_per_chunk) * (size_t)((n + cols - 1) / cols);
 }
 
 hipError_t launch_skinny_w8a8(const GmmParams &p, bool nk, bool wide16, hipStream_t stream) {

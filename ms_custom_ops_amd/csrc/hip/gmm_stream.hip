@@ -226,7 +226,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_w8a8_stream_kernel(const Gm
   if (p.split_k > 1) {
     // cross-workgroup reduction through the workspace with agent-scope relaxed atomics (no cache-wide
     // fences); slice s, 64-bit word e of thread t at ((s * 8 + e) * 256 + t); the last arriver adds up
-    const long long tile = ((long long)grp * p.max_chunks + mc) * p.n_strips + strip;
+    const long long tile = (long long)blockIdx.y * p.n_strips + strip;
     i64 *base = reinterpret_cast<i64 *>(p.partial) + tile * p.split_k * (ST_TILE_INTS / 2);
     if (rows_ok) {
       i64 *mine = base + (long long)ks * (ST_TILE_INTS / 2) + tid;
@@ -458,7 +458,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_w8a8_streamm_kernel(const G
 
   if (p.split_k > 1) {
     // slice s, fragment word (j, half) of thread t at ((s * OWN + j) * 2 + half) * 256 + t, 64-bit words
-    const long long tile_id = ((long long)grp * p.max_chunks + mc) * p.n_strips + strip;
+    const long long tile_id = (long long)blockIdx.y * p.n_strips + strip;
     i64 *base = reinterpret_cast<i64 *>(p.partial) + tile_id * p.split_k * (S::kTileInts / 2);
     i64 *mine = base + (long long)ks * (S::kTileInts / 2) + tid;
 #pragma unroll
@@ -543,7 +543,7 @@ static hipError_t streamm_launch(const GmmParams &p, const dim3 &grid, hipStream
   return hipGetLastError();
 }
 
-// tch = 16-row fragments per chunk (2, 4 or 8); p.max_chunks counts chunks of 16 tch rows, p.n_strips strips of 64 columns
+// tch = 16-row fragments per chunk (2, 4 or 8); p.n_strips strips of 64 columns
 hipError_t launch_streamm_w8a8(const GmmParams &p, int tch, hipStream_t stream) {
   if (p.m == 0) return hipSuccess;
   const dim3 grid((unsigned)p.n_strips, chunk_slots(p, 16 * tch), (unsigned)p.split_k);
@@ -722,7 +722,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_a16w8_stream_kernel(const G
   if (p.split_k > 1) {
     // float32 partials through the workspace, added in slice order by the last arriver.  Slice s: word e (0..7) of
     // thread t at (s * SA_TILE_WORDS + e * 256 + t); row sums of wave 0's lanes at (... + 2048 + 2 lane + {0, 1})
-    const long long tile = ((long long)grp * p.max_chunks + mc) * p.n_strips + strip;
+    const long long tile = (long long)blockIdx.y * p.n_strips + strip;
     i64 *base = reinterpret_cast<i64 *>(p.partial) + tile * p.split_k * SA_TILE_WORDS;
     auto pack = [](float lo, float hi) {
       return (i64)(((unsigned long long)__float_as_uint(hi) << 32) | __float_as_uint(lo));
@@ -1355,7 +1355,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_a16w8_rows32_kernel(const G
     typedef long long i64;
     constexpr int WORDS = GP * TR * 8;
     unsigned *s_ticket = reinterpret_cast<unsigned *>(st_smem + S::kTile + S::kRows * 4);
-    const long long tile = ((long long)grp * p.max_chunks + mc) * p.n_strips + strip;
+    const long long tile = (long long)blockIdx.y * p.n_strips + strip;
     i64 *base = reinterpret_cast<i64 *>(p.partial) + tile * p.split_k * (long long)S::kSliceWords;
     i64 *mine = base + (long long)ks * (long long)S::kSliceWords;
     auto pack = [](float lo, float hi) { return (i64)(((unsigned long long)__float_as_uint(hi) << 32) | __float_as_uint(lo)); };
@@ -1492,7 +1492,7 @@ static hipError_t rows32_launch_a16w8(const GmmParams &p, const dim3 &grid, hipS
 // workspace bytes of one (chunk, strip, K slice) partial tile of the 128-row kernel: accumulators and row sums
 size_t rows32_a16w8_slice_bytes(int strip_groups) { return ((size_t)128 * 16 * strip_groups + 128) * 4; }
 
-// tch = 16-row fragments per chunk (2, 4 or 8); p.max_chunks counts chunks of 16 tch rows; p.strip_groups = column groups
+// tch = 16-row fragments per chunk (2, 4 or 8); p.strip_groups = column groups
 // per strip (8 or 16: strips of 128 or 256 columns), p.n_strips strips
 hipError_t launch_streamm_a16w8(const GmmParams &p, int tch, bool packed, hipStream_t stream) {
   if (p.m == 0) return hipSuccess;

@@ -88,7 +88,6 @@ struct msco_gmm_op {
   int family = FAM_NONE;
   int tile_cfg = 0;
   int split_k = 1;
-  int max_chunks = 1;
   int skinny_wide16 = 0;
   int skinny_cols = kSkinnyCols;
   int n_strips = 0;
@@ -469,7 +468,6 @@ void choose_plan(msco_gmm_op *op) {
   const int64_t m = op->m, k = op->k, n = op->n, e = op->e;
   const bool aligned = (k % 16 == 0) && (n % 16 == 0) && k >= 16 && n >= 16;
   op->split_k = 1;
-  op->max_chunks = 1;
   op->skinny_wide16 = 0;
   op->skinny_cols = kSkinnyCols;
   op->n_strips = (int)((n + kSkinnyCols - 1) / kSkinnyCols);
@@ -764,12 +762,12 @@ void choose_plan(msco_gmm_op *op) {
     if (tuning().stream_tch == 1 || tuning().stream_tch == 2 || tuning().stream_tch == 4 || tuning().stream_tch == 8)
       op->stream_tch = tuning().stream_tch;
   }
+  int64_t max_chunks = 1;   // chunks of 16 * stream_tch rows that a group can have
   if (family == FAM_SKINNY) {
-    // grid.y enumerates (group, chunk of 16 * stream_tch rows)
+    // grid.y enumerates (group, chunk) pairs
     const int64_t chunk_rows = (int64_t)kSkinnyRows * op->stream_tch;
-    op->max_chunks = (int)((m + chunk_rows - 1) / chunk_rows);
-    if (op->max_chunks < 1) op->max_chunks = 1;
-    if (e * op->max_chunks > 65535) {
+    max_chunks = std::max<int64_t>(1, (m + chunk_rows - 1) / chunk_rows);
+    if (e * max_chunks > 65535) {
       family = FAM_GENERIC;
       rows16_fits = is_a16w8(d);
     }
@@ -777,7 +775,7 @@ void choose_plan(msco_gmm_op *op) {
   if (family == FAM_SKINNY) {
     // Only shapes enter: the number of (group, chunk) pairs that can hold rows is estimated from M and E.
     const int64_t active = std::max<int64_t>(
-      1, std::min<int64_t>(e * op->max_chunks, std::min<int64_t>(m, e) + m / (kSkinnyRows * op->stream_tch)));
+      1, std::min<int64_t>(e * max_chunks, std::min<int64_t>(m, e) + m / (kSkinnyRows * op->stream_tch)));
     const int64_t tiles128 = ((n + 127) / 128) * active;
     int wide16 = is_w8a8(d) && tiles128 <= num_cus && !is_packed(d);
     const int forced_variant = tuning().skinny_wide16;
@@ -797,8 +795,8 @@ void choose_plan(msco_gmm_op *op) {
       const int64_t base = (int64_t)op->n_strips * active, k_blocks = (k + 63) / 64;
       if (e == 1 && base < num_cus && tuning().stream_tch == 0) {
         op->stream_tch = 8;
-        op->max_chunks = (int)((m + 127) / 128);
-        want = (int)std::min<int64_t>(kTargetWorkgroups / std::max<int64_t>((int64_t)op->n_strips * op->max_chunks, 1), kMaxSplitK);
+        max_chunks = (m + 127) / 128;
+        want = (int)std::min<int64_t>(kTargetWorkgroups / std::max<int64_t>((int64_t)op->n_strips * max_chunks, 1), kMaxSplitK);
         cap = std::max<int>(1, (int)(k_blocks / 8));
       }
     } else if (is_packed(d) && op->stream_tch > 1) {
@@ -842,7 +840,7 @@ void choose_plan(msco_gmm_op *op) {
       // (short slices only where msco_gmm_launch_static takes their partial tiles too)
       want = floor_split;
       if (col_groups <= 64 && (int64_t)op->n_strips * active * 3 <= 2 * (int64_t)num_cus && k_blocks >= 64) want = std::max(want, 2);
-      if (short_slices && skinny_counter_count(m, n, e, op->skinny_cols) * (size_t)want * stream_a16w8_tile_bytes() > (size_t)MSCO_GMM_STATIC_WORKSPACE_BYTES) want = fewest;
+      if (short_slices && decode_tiles(m, n, e, kSkinnyRows, op->skinny_cols) * (size_t)want * stream_a16w8_tile_bytes() > (size_t)MSCO_GMM_STATIC_WORKSPACE_BYTES) want = fewest;
       cap = kMaxSplitK * 64;
     } else if (wide16) {
       // at most one 16-wave workgroup per CU, every wave keeps at least one block
@@ -867,19 +865,12 @@ void choose_plan(msco_gmm_op *op) {
     if (op->stream_tch > 1 && !is_w8a8(d) && !(e == 1 && op->stream_tch == 8)) want = 1;   // the multi-row weight-only kernels walk all of K, but for one group in 128-row chunks
     op->split_k = want;
     if (!is_packed(d) && !(op->stream_tch > 1 && !is_w8a8(d))) op->skinny_cols = wide16 ? 128 : kSkinnyCols;
-    if (op->stream_tch > 1 && !is_w8a8(d)) {
-      op->workspace_bytes = op->split_k > 1 ? (size_t)e * op->max_chunks * op->n_strips * op->split_k * rows32_a16w8_slice_bytes(op->strip_groups) : 0;
-    } else if (is_packed(d)) {
-      // the packed-layout kernels keep a full 16 x 256 partial tile per (strip, K slice) whatever the strip's width
-      const size_t tile_bytes = !is_w8a8(d)           ? stream_a16w8_tile_bytes()
-                                : op->stream_tch > 1 ? streamm_tile_bytes(op->stream_tch)
-                                                     : (size_t)kSkinnyRows * kSkinnyCols * 4;
-      const size_t tiles = op->stream_tch > 1 ? (size_t)e * op->max_chunks * op->n_strips
-                                              : skinny_counter_count(m, n, e, op->skinny_cols);
-      op->workspace_bytes = op->split_k > 1 ? tiles * (size_t)op->split_k * tile_bytes : 0;
-    } else {
-      op->workspace_bytes = is_w8a8(d) ? skinny_workspace_bytes(m, n, e, op->split_k, op->skinny_cols) : 0;   // (weight-only: plan_regt's)
-    }
+    size_t slice_bytes = (size_t)kSkinnyRows * op->skinny_cols * 4;
+    if (op->stream_tch > 1 && !is_w8a8(d)) slice_bytes = rows32_a16w8_slice_bytes(op->strip_groups);
+    else if (is_packed(d))   // (the packed-layout kernels keep a full 16 x 256 partial tile per (strip, K slice) whatever the strip's width)
+      slice_bytes = !is_w8a8(d) ? stream_a16w8_tile_bytes() : op->stream_tch > 1 ? streamm_tile_bytes(op->stream_tch) : (size_t)kSkinnyRows * kSkinnyCols * 4;
+    else if (!is_w8a8(d)) slice_bytes = 0;   // (plan_regt's)
+    op->workspace_bytes = op->split_k > 1 ? decode_tiles(m, n, e, kSkinnyRows * op->stream_tch, op->skinny_cols) * (size_t)op->split_k * slice_bytes : 0;
   }
   op->family = family;
   op->widen_bytes = 0;
@@ -1046,7 +1037,7 @@ int msco_gmm_plan(msco_gmm_handle h, int64_t m, int64_t k, int64_t n, int64_t e,
     const size_t need = h->family == FAM_ROWS16 ? (size_t)chunk_slots(p, 128) * h->n_strips
                         : h->family == FAM_REGT ? (size_t)chunk_slots(p, 16 * h->row_blocks) * h->n_strips
                         : h->family == FAM_TILE ? tile_count_bound(h->tile_cfg, m, n, e)
-                                              : skinny_counter_count(m, n, e, h->skinny_cols);
+                                              : decode_tiles(m, n, e, kSkinnyRows * h->stream_tch, h->skinny_cols);
     const RelaxedCapture relaxed;
     h->counters_used = need;
     if (need > h->counters_cap) {
@@ -1125,7 +1116,6 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   p.x_dtype = d.x_dtype;
   p.split_k = h->split_k;
   p.n_strips = h->n_strips;
-  p.max_chunks = h->max_chunks;
   p.strip_groups = h->strip_groups;
   p.act_type = d.act_type;
   // rows a 16-row chunk is expected to hold (shapes only): measured on the dense 45 MB decode, 16 rows 13.1 -> 12.35 us with
