@@ -651,16 +651,18 @@ void choose_plan(msco_gmm_op *op) {
       // fifth more time than one alone, and the exchange is half as large: 128 experts, 24 rows, 3264 x 976, s = 1 / 2: 21.7 / 16.9; 16 experts,
       // 18 rows, 3392 x 1168: 16.0 / 14.3; 8 experts, 16 rows, 6400 x 2304: 32.6 / 30.3; 16 experts, 12 rows, 608 x 2096: 7.8 / 9.7.
       // One group (206 random shapes of 1 to 400 rows, every split measured): a slice adds less than that -- 4 and 6 in place of 6 and 8, and 2
-      // once -- but a launch that fills more than 15/16 of the CUs with 32 x 128 tiles already takes what two on a CU take, 1.6 times one
-      // alone (4 rows, 2272 x 10448, s = 2 / 3: 11.5 / 14.0).  32 x 128 0.971 of the time, none slower (7 rows, 6176 x 10464 26.2 -> 21.5; 3 rows,
-      // 7552 x 4256 15.4 -> 14.0), 64 x 128 0.991 (41 rows, 2720 x 1200 10.9 -> 9.6).
+      // once -- and two 32 x 128 tiles on a CU take 1.6 times one alone.  32 x 128 0.971 of the time, none slower (7 rows, 6176 x 10464 26.2 ->
+      // 21.5; 3 rows, 7552 x 4256 15.4 -> 14.0), 64 x 128 0.991 (41 rows, 2720 x 1200 10.9 -> 9.6).  Its rounds are those of an XCD, which takes an
+      // eighth of the tiles, rounded up, with all their slices: three slices of 81 to 85 tiles are 33 workgroups for 32 CUs.  Counted over the
+      // chip that was one round.  7778 random shapes that this changes, 0.83 of the time, one slower by more than 0.05: 64 x 128, three
+      // slices -> two 0.77 (72 rows, 2688 x 5280 15.4 -> 12.7), 32 x 128, 62 to 64 tiles, three -> four 0.95.
       const int cus = or_default(tuning().tile_target_wgs, num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       const int cap = (int)std::max<int64_t>(1, ((k + 63) / 64) / kTileMinSlabs);
       auto split_cost = [&](int sl) {
         const int64_t slabs = ((k + 63) / 64 + sl - 1) / sl;
         const bool one_small = e == 1 && (few || op->tile_cfg == TILE_64x128);
-        const int64_t slots = few && e == 1 && sl > 1 ? cus * 15 / 16 : cus;
-        const int64_t rounds = (t * sl + slots - 1) / slots;
+        const int64_t xcd_cus = std::max(1, cus / kNumXcd);
+        const int64_t rounds = e == 1 ? ((t + kNumXcd - 1) / kNumXcd * sl + xcd_cus - 1) / xcd_cus : (t * sl + cus - 1) / cus;
         const int64_t fifths = few && rounds > 1 ? (rounds + 1) / 2 * (e == 1 ? 8 : 6) : rounds * 5;
         const int64_t exchange = sl <= 1 ? 0 : one_small ? (int64_t)(2 + bm * bn / 2048) * sl + 2 : (int64_t)(4 + bm * bn / 2048) * sl - 2;
         return fifths * (slabs + 10 + exchange);

@@ -1,0 +1,29 @@
+"""K slices of the small tiles: which split the plan takes where the tiles of an XCD (an eighth of all, rounded up) with their slices just fit its 32
+CUs and where they just do not.  256 CUs."""
+import re
+
+import pytest
+
+from ms_custom_ops_amd import cabi
+
+
+def _plan(m, k, n, e=1, nk=False, packed=False):
+    op = cabi.GmmOp(x_dtype=cabi.DT_I8, weight_dtype=cabi.DT_I8, out_dtype=cabi.DT_BF16, scale_dtype=cabi.DT_F32, scale_per_group=1, transpose_b=int(nk),
+                    weight_layout=cabi.WL_PACKED if packed else cabi.WL_ROW_MAJOR, **({} if e == 1 else dict(group_list_dtype=cabi.DT_I64)))
+    try:
+        op.plan(m, k, n, e)
+    except cabi.BackendError:
+        pass   # (a split plan allocates counters on the device; the plan itself stands)
+    info = op.plan_info()
+    op.close()
+    return info.split("kernel=")[1].split()[0], int(re.search(r"split_k=(\d+)", info)[1])
+
+
+@pytest.mark.parametrize("m,k,n,nk,packed,kernel,split", [
+    (72, 2688, 5120, True, False, "w8a8_tile_64x128", 3), (72, 2688, 5280, True, False, "w8a8_tile_64x128", 2),      # 80 and 84 tiles
+    (72, 2688, 5280, False, True, "w8a8_tile_64x128", 2), (244, 2912, 2688, True, False, "w8a8_tile_64x128", 2),
+    (40, 16384, 6144, False, True, "w8a8_tile_64x128", 5), (40, 16384, 6272, False, True, "w8a8_tile_64x128", 4),      # 48 and 49
+    (19, 3296, 8192, False, False, "w8a8_skinny_tile_32x128", 4), (19, 3296, 8320, False, False, "w8a8_skinny_tile_32x128", 3),   # 64 and 65
+    (4, 2272, 10240, False, False, "w8a8_skinny_tile_32x128", 3), (4, 2272, 10448, False, False, "w8a8_skinny_tile_32x128", 2)])
+def test_one_group(m, k, n, nk, packed, kernel, split):
+    assert _plan(m, k, n, nk=nk, packed=packed) == (kernel, split)
