@@ -658,12 +658,16 @@ void choose_plan(msco_gmm_op *op) {
       // slices -> two 0.77 (72 rows, 2688 x 5280 15.4 -> 12.7), 32 x 128, 62 to 64 tiles, three -> four 0.95.
       const int cus = or_default(tuning().tile_target_wgs, num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       const int cap = (int)std::max<int64_t>(1, ((k + 63) / 64) / kTileMinSlabs);
+      // (several groups, 11 to 16 rows each on average: all of them hold rows, some of them more than a tile, and a second tile per CU costs what it
+      // costs with one group.  2411 such shapes 0.85 of the time of the splits before, none
+      // with an even routing slower than 64 x 128 tiles; up to 10 rows a group the 1.2 times stand, as a random routing leaves groups empty)
+      const bool full_groups = (m + e - 1) / e * 3 / 2 > kSkinnyRows;
       auto split_cost = [&](int sl) {
         const int64_t slabs = ((k + 63) / 64 + sl - 1) / sl;
         const bool one_small = e == 1 && (few || op->tile_cfg == TILE_64x128);
         const int64_t xcd_cus = std::max(1, cus / kNumXcd);
         const int64_t rounds = e == 1 ? ((t + kNumXcd - 1) / kNumXcd * sl + xcd_cus - 1) / xcd_cus : (t * sl + cus - 1) / cus;
-        const int64_t fifths = few && rounds > 1 ? (rounds + 1) / 2 * (e == 1 ? 8 : 6) : rounds * 5;
+        const int64_t fifths = few && rounds > 1 ? (rounds + 1) / 2 * (e == 1 || full_groups ? 8 : 6) : rounds * 5;
         const int64_t exchange = sl <= 1 ? 0 : one_small ? (int64_t)(2 + bm * bn / 2048) * sl + 2 : (int64_t)(4 + bm * bn / 2048) * sl - 2;
         return fifths * (slabs + 10 + exchange);
       };
