@@ -658,9 +658,9 @@ void choose_plan(msco_gmm_op *op) {
       // slices -> two 0.77 (72 rows, 2688 x 5280 15.4 -> 12.7), 32 x 128, 62 to 64 tiles, three -> four 0.95.
       const int cus = or_default(tuning().tile_target_wgs, num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       const int cap = (int)std::max<int64_t>(1, ((k + 63) / 64) / kTileMinSlabs);
-      // (several groups, 11 to 16 rows each on average: all of them hold rows, some of them more than a tile, and a second tile per CU costs what it
+      // (several groups, more than 11 and up to 16 rows each on average: all of them hold rows, some of them more than a tile, and a second tile per CU costs what it
       // costs with one group.  2411 such shapes 0.85 of the time of the splits before, none
-      // with an even routing slower than 64 x 128 tiles; up to 10 rows a group the 1.2 times stand, as a random routing leaves groups empty)
+      // with an even routing slower than 64 x 128 tiles; up to 11 rows a group the 1.2 times stand, as a random routing leaves groups empty)
       const bool full_groups = (m + e - 1) / e * 3 / 2 > kSkinnyRows;
       auto split_cost = [&](int sl) {
         const int64_t slabs = ((k + 63) / 64 + sl - 1) / sl;

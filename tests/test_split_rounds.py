@@ -30,7 +30,7 @@ def test_one_group(m, k, n, nk, packed, kernel, split):
 
 
 @pytest.mark.parametrize("m,k,n,e,split", [
-    (352, 3616, 832, 32, 1), (320, 3616, 832, 32, 2),      # 11 and 10 rows a group, 224 tiles: two to a CU cost 1.6 and 1.2 times one
-    (352, 3616, 512, 32, 2), (112, 3680, 3680, 8, 1), (112, 3680, 1920, 8, 2)])
+    (353, 3616, 832, 32, 1), (352, 3616, 832, 32, 2),      # more than 11 rows a group and 11, 224 tiles: two to a CU cost 1.6 and 1.2 times one
+    (384, 3616, 512, 32, 2), (112, 3680, 3680, 8, 1), (112, 3680, 1920, 8, 2)])
 def test_several_groups_on_32_row_tiles(m, k, n, e, split):
     assert _plan(m, k, n, e) == ("w8a8_skinny_tile_32x128", split)
