@@ -447,19 +447,39 @@ void plan_few_rows(msco_gmm_op *op, int &family) {
 //   ([E,K,N] from 128 x 256 tiles: 0.83, but up to 1.25.)
 //   Packed weights stay (128 x 256 tiles for several groups 0.95, from 0.81 to 1.31; 64 x 128 for one group 0.94, from 0.77 to 1.04).
 // 600 other shapes: 21 changed, 0.83 of the time, the worst 1.01.
-void plan_one_round(msco_gmm_op *op) {
+// Which side of a round a launch of several groups falls is counted with the mean over the routings of its row tiles: "a tenth more rows" jumps by a
+// tile per group just below a multiple of the tile (8 experts, 121 rows each: three 64-row tiles, 2.4 on average).
+// A random routing scatters a group's rows around their average by about its root.  Shapes between the two counts, us, the wider tile / the other:
+// 128 x 256 where 128 x 128 are expected to be 180 .. 250 tiles 1.36 times as long (8 experts, 1988 rows, 4032 x 1776 45.6 / 34.4), 260 and more
+// 0.91; 128 x 128 where 64 x 128 are 180 .. 236 1.08 (skewed routings 1.07), 248 .. 256 0.99; a K split of 128 x 128 tiles that fill
+// more than half of a round 1.25 (16 experts, 2872 rows, 3168 x 592, [E,N,K] two slices 33.5, 64 x 128 22.8).
+double expected_row_tiles(double avg, double bm) {
+  const double sd = std::sqrt(std::max(avg, 1e-9));
+  const double sure = std::max(0.0, std::floor((avg - 5.0 * sd) / bm));
+  double tiles = sure;
+  for (double rows = sure * bm + 0.5; rows < avg + 5.0 * sd; rows += bm) tiles += 0.5 * std::erfc((rows - avg) / (sd * std::sqrt(2.0)));
+  return std::max(tiles, 1e-3);
+}
+
+bool plan_one_round(msco_gmm_op *op) {   // true: K is not to be split
   const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
   const bool packed = is_packed(op->desc), kn = !packed && !op->desc.transpose_b;
   auto tiles = [&](int64_t bm, int64_t bn) {   // an average group's and a tenth more rows (real routings are uneven)
     const int64_t groups = std::max<int64_t>(1, std::min(e, m)), rows = e == 1 ? m : (11 * m + 10 * e - 1) / (10 * e);
     return groups * ((rows + bm - 1) / bm) * ((n + bn - 1) / bn);
   };
+  auto expected = [&](int64_t bm, int64_t bn) {
+    return (e == 1 ? (double)((m + bm - 1) / bm) : (double)std::min(e, m) * expected_row_tiles((double)m / (double)std::min(e, m), (double)bm)) * (double)((n + bn - 1) / bn);
+  };
   if (op->tile_cfg == TILE_128x128 && tiles(128, 128) > cus) {
-    if (kn && k >= 1024 && n * 4 >= (n + 255) / 256 * 256 * 3) op->tile_cfg = TILE_128x256;
+    if (kn && k >= 1024 && n * 4 >= (n + 255) / 256 * 256 * 3 && (e == 1 || expected(128, 128) > (double)cus)) op->tile_cfg = TILE_128x256;
     else if (!packed && !kn && e > 1 && e <= 1024 && k >= 2048 && tiles(128, 128) > 2 * cus && tiles(256, 256) * 2 > cus && tiles(256, 256) <= cus) op->tile_cfg = TILE_256x256_W4;
-  } else if (op->tile_cfg == TILE_64x128 && !packed && k >= 2048 && tiles(64, 128) > cus && tiles(128, 128) <= cus) {
+  } else if (op->tile_cfg == TILE_64x128 && !packed && k >= 2048 && tiles(64, 128) > cus && expected(64, 128) * 16 > (double)(cus * 15) && tiles(128, 128) <= cus) {
     op->tile_cfg = TILE_128x128;
+    // (a K split of more than half a round would make two rounds of one)
+    return expected(128, 128) * 2 > (double)cus;
   }
+  return false;
 }
 
 void choose_plan(msco_gmm_op *op) {
@@ -600,8 +620,9 @@ void choose_plan(msco_gmm_op *op) {
       op->tile_cfg = TILE_64x128;
     }
   }
+  bool one_round = false;
   if (d.kernel_override == OV_AUTO && aligned && is_w8a8(d) && !is_w4(d)) {
-    if (family == FAM_TILE) plan_one_round(op);
+    one_round = family == FAM_TILE && plan_one_round(op);
     plan_few_rows(op, family);
   }
   switch (d.kernel_override) {
@@ -672,7 +693,7 @@ void choose_plan(msco_gmm_op *op) {
         return fifths * (slabs + 10 + exchange);
       };
       int want = 1;
-      if (t <= (few ? 2 * kTileSplitMaxTiles : kTileSplitMaxTiles)) {
+      if (!one_round && t <= (few ? 2 * kTileSplitMaxTiles : kTileSplitMaxTiles)) {
         for (int sl = 2; sl <= std::min(kMaxSplitK, cap); ++sl)
           if (split_cost(sl) < split_cost(want)) want = sl;
       }

@@ -56,3 +56,20 @@ def test_exact(device, m, k, n, e, nk, packed, must):
     want = O.grouped_matmul_w8a8(x, w, ends, None, s, None)
     rows = int(ends[-1])
     assert np.array_equal(out.cpu().numpy().view(np.uint16)[:rows], np.asarray(want).view(np.uint16)[:rows])
+
+
+# several groups, counted with the mean of their row tiles over random routings: both sides of the lines, and a K split that would make two rounds
+@pytest.mark.parametrize("m,k,n,e,nk,must,split", [
+    (1960, 4032, 1776, 8, False, "tile_128x128", 1), (2120, 4032, 1776, 8, False, "tile_128x256", 1),            # 250 and 302 tiles of 128 x 128 expected
+    (920, 6400, 1712, 8, True, "tile_64x128", 1), (1016, 6400, 1712, 8, True, "tile_128x128", 1),                # 236 and 274 of 64 x 128
+    (2872, 3168, 592, 16, True, "tile_128x128", 1), (2900, 6688, 544, 8, True, "tile_128x128", 2)])              # 160 and 125 of 128 x 128 instead
+def test_the_rule_counts_a_mean_routing(m, k, n, e, nk, must, split):
+    op = cabi.GmmOp(x_dtype=cabi.DT_I8, weight_dtype=cabi.DT_I8, out_dtype=cabi.DT_BF16, scale_dtype=cabi.DT_F32, scale_per_group=1, transpose_b=int(nk),
+                    group_list_dtype=cabi.DT_I64, group_list_type=1)
+    try:
+        op.plan(m, k, n, e)
+    except cabi.BackendError:
+        pass   # (a split plan allocates counters on the device; the plan itself stands)
+    info = op.plan_info()
+    op.close()
+    assert must in info and f"split_k={split} " in info, info
