@@ -416,8 +416,10 @@ int64_t few_row_tiles(int64_t m, int64_t n, int64_t e) { return groups_hit(m, e)
 //   more: 32 x 256 (8 experts, 32 rows, 5632 x 5120 60.4 -> 48.7, 32 x 128: 62.4), or, where K below 1024 leaves its three-slab ring too
 //   little to walk, 64 x 128 with 64-byte slabs and three workgroups per CU (16 experts, 162 rows, 864 x 4112 22.7 -> 15.3, 32 x 256: 18.8).
 // The decode kernels keep what leaves most CUs idle whatever the tile, because their 16 waves split K inside a workgroup: a handful of
-// rows over dozens of experts (64 experts, 1 row, 2272 x 800: 8.3 against 9.9; 5 rows, 800 x 1824: 8.0 against 8.8) and one group of ten
-// tiles and a long K (1 row, 3744 x 1120: 9.5 against 10.4).  They also keep K below 512 (not measured).  On [E,N,K] weights several groups take 64 x 128
+// rows over dozens of experts (64 experts, 1 row, 2272 x 800: 8.3 against 9.9; 5 rows, 800 x 1824: 8.0 against 8.8), one group of ten
+// tiles and a long K (1 row, 3744 x 1120: 9.5 against 10.4), and several groups where that is K / 192 tiles, at least ten (2 rows over 16 experts,
+// 7712 x 656: 13.6 against 16.9; 3082 such [E,K,N] shapes 0.93 of the time of 32 x 128 tiles, 0.85 to 0.97 from few tiles to the line; 1288 of
+// them had become slower by more than 5 % with those, 14 are left).  They also keep K below 512 (not measured).  On [E,N,K] weights several groups take 64 x 128
 // tiles already, which are as fast (60 shapes: 0.98), but for more than 32 experts and up to 64 rows (41 rows over 64 experts, 4352 x 688: 27.9 ->
 // 20.3; 52 rows, 544 x 10576: 17.2 -> 15.3 with 64 x 128 tiles), where the decode kernels' plan dates from launches with workgroups for experts
 // without rows.
@@ -427,7 +429,7 @@ void plan_few_rows(msco_gmm_op *op, int &family) {
   if (is_packed(op->desc) || k < 512 || (e == 1 ? m > 32 : m > 16 * e)) return;
   const int64_t tiles = few_row_tiles(m, n, e);
   if (e == 1 && !nk && m <= kSkinnyRows && tiles <= 10 && k >= 2048) return;
-  if (e > 1 && ((nk && family != FAM_SKINNY) || tiles <= 10 || (e >= 32 && m <= 5))) return;
+  if (e > 1 && ((nk && family != FAM_SKINNY) || tiles <= 10 || (!nk && family == FAM_SKINNY && tiles * 192 <= k) || (e >= 32 && m <= 5))) return;
   family = FAM_TILE;
   op->tile_cfg = tiles * 8 <= cus * 9 ? TILE_32x128 : nk || k < 1024 ? TILE_64x128 : TILE_32x256;
 }

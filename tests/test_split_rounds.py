@@ -34,3 +34,10 @@ def test_one_group(m, k, n, nk, packed, kernel, split):
     (384, 3616, 512, 32, 2), (112, 3680, 3680, 8, 1), (112, 3680, 1920, 8, 2)])
 def test_several_groups_on_32_row_tiles(m, k, n, e, split):
     assert _plan(m, k, n, e) == ("w8a8_skinny_tile_32x128", split)
+
+
+@pytest.mark.parametrize("m,k,n,e,kernel", [
+    (6, 5760, 560, 128, "w8a8_skinny_16w"), (6, 5744, 560, 128, "w8a8_skinny_tile_32x128"),      # 30 tiles, 30 times 192 and less
+    (2, 7712, 656, 16, "w8a8_skinny_16w"), (2, 4576, 1136, 16, "w8a8_skinny_16w"), (2, 3072, 1136, 16, "w8a8_skinny_tile_32x128")])
+def test_few_tiles_and_a_long_k_stay_with_the_decode_kernels(m, k, n, e, kernel):
+    assert _plan(m, k, n, e)[0] == kernel
