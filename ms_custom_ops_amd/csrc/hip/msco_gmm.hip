@@ -296,6 +296,15 @@ void plan_regt(msco_gmm_op *op) {
   }
 }
 
+// Mean number of bm-row tiles of a group that holds `avg` rows on average: a random routing scatters them by about the root of that.
+double expected_row_tiles(double avg, double bm) {
+  const double sd = std::sqrt(std::max(avg, 1e-9));
+  const double sure = std::max(0.0, std::floor((avg - 5.0 * sd) / bm));
+  double tiles = sure;
+  for (double rows = sure * bm + 0.5; rows < avg + 5.0 * sd; rows += bm) tiles += 0.5 * std::erfc((rows - avg) / (sd * std::sqrt(2.0)));
+  return std::max(tiles, 1e-3);
+}
+
 // Weight-only on packed or [E,K,N] weights beyond one 16-row chunk per group: the forms of the 128-row kernel
 // (gmm_rows_a16w8_kernel.h) -- strips of 512 columns, strips of 256 with two workgroups per CU, strips of 256 whose K blocks two
 // sets of waves share, the last two with a K split -- against the 32- and 64-row kernels, by a model of the time in us.  All
@@ -331,7 +340,11 @@ double rows16_us(int64_t m, int64_t k, int64_t n, int64_t e, int64_t cus, bool p
   const double wgs = (double)((n + f.cols - 1) / f.cols) * (double)(groups * chunks * f.split);
   const bool pairs = f.cols == 256 && f.sets == 1 && wgs > (double)cus;
   const Rows16Cost &c = kRows16[packed][f.cols == 512 ? 0 : f.sets == 2 ? 3 : pairs ? 2 : 1];
-  const double r = chip_rounds(wgs, pairs ? 2.0 * (double)cus : (double)cus);
+  // (packed weights, two sets: a second round is a whole one.  257 .. 351 workgroups at w / CUs + 0.5 rounds were picked over the 32- and 64-row
+  // kernels and took 1.1 times as long: 8 experts, 210 rows, 5472 x 8816 88 against 108 us)
+  const bool two_rounds = packed && f.sets == 2 && wgs <= 2.0 * (double)cus &&
+                          (double)((n + f.cols - 1) / f.cols) * (double)(groups * f.split) * (e == 1 ? (double)chunks : expected_row_tiles((double)m / (double)groups, 128.0)) > (double)cus;
+  const double r = two_rounds ? 2.0 : chip_rounds(wgs, pairs ? 2.0 * (double)cus : (double)cus);
   const double us = c.fixed + r * (c.round + blocks * (c.block + c.rows * rb)) + c.stream * rows_stream_us(m, k, n, e, bits) + (f.split > 1 ? c.split + c.slice * rb * r * (f.split - 1) : 0.0);
   return pairs && r > 3 && rb >= 6 ? 1.07 * us : us;   // (what the fit is off by there: x comes in twice per CU)
 }
@@ -451,18 +464,10 @@ void plan_few_rows(msco_gmm_op *op, int &family) {
 // 600 other shapes: 21 changed, 0.83 of the time, the worst 1.01.
 // Which side of a round a launch of several groups falls is counted with the mean over the routings of its row tiles: "a tenth more rows" jumps by a
 // tile per group just below a multiple of the tile (8 experts, 121 rows each: three 64-row tiles, 2.4 on average).
-// A random routing scatters a group's rows around their average by about its root.  Shapes between the two counts, us, the wider tile / the other:
+// Shapes between the two counts, us, the wider tile / the other:
 // 128 x 256 where 128 x 128 are expected to be 180 .. 250 tiles 1.36 times as long (8 experts, 1988 rows, 4032 x 1776 45.6 / 34.4), 260 and more
 // 0.91; 128 x 128 where 64 x 128 are 180 .. 236 1.08 (skewed routings 1.07), 248 .. 256 0.99; a K split of 128 x 128 tiles that fill
 // more than half of a round 1.25 (16 experts, 2872 rows, 3168 x 592, [E,N,K] two slices 33.5, 64 x 128 22.8).
-double expected_row_tiles(double avg, double bm) {
-  const double sd = std::sqrt(std::max(avg, 1e-9));
-  const double sure = std::max(0.0, std::floor((avg - 5.0 * sd) / bm));
-  double tiles = sure;
-  for (double rows = sure * bm + 0.5; rows < avg + 5.0 * sd; rows += bm) tiles += 0.5 * std::erfc((rows - avg) / (sd * std::sqrt(2.0)));
-  return std::max(tiles, 1e-3);
-}
-
 bool plan_one_round(msco_gmm_op *op) {   // true: K is not to be split
   const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
   const bool packed = is_packed(op->desc), kn = !packed && !op->desc.transpose_b;
