@@ -24,6 +24,8 @@ def _plan(m, k, n, e, layout="kn", bits=8, override=0):
     (800, 512, 2048, 8, "kn", 8, "a16w8_rows128x256", 1), (800, 496, 2048, 8, "kn", 8, "a16w8_skinny_rows", 1),
     # 4-bit weights: beyond 30 rows a group the 128-row kernel reads the nibbles
     (240, 2048, 4096, 8, "kn", 4, "a16w4_skinny_regt", 2), (600, 2048, 4096, 8, "kn", 4, "a16w4_rows128x256_2", 1),
+    # ... but up to 43 rows the register-transpose kernels stay where its workgroups fill no more than half of the chip (128 and 136 of them)
+    (330, 4416, 4096, 8, "kn", 4, "a16w4_skinny_regt", 1), (330, 4416, 4352, 8, "kn", 4, "a16w4_rows128x256_2", 1), (352, 4416, 4096, 8, "kn", 4, "a16w4_rows128x256_2", 1),
     # strips of 512 columns where they fill the chip, of 256 where they do not, two sets of waves with a K split where those do not either
     (4096, 4096, 14336, 8, "packed", 8, "a16w8_rows128", 1), (131072, 1024, 1024, 128, "packed", 8, "a16w8_rows128x256", 1),
     (816, 6336, 544, 16, "kn", 8, "a16w8_rows128x256_2", 3),
