@@ -872,13 +872,10 @@ void choose_plan(msco_gmm_op *op) {
       op->skinny_cols = groups * 16;
       // No split beyond that: a strip of one column group is a walk of K / 256 requests per wave, and the exchange costs more than any
       // of it saves (us, two workgroups per CU through a split -> none: one row, 2688 x 2800 8.1 -> 5.1; 13 rows, 8128 x 1568 13.0 -> 7.9; 5 rows
-      // over 32 experts, 5536 x 576 8.9 -> 6.7; 16-bit x, one row, 3520 x 3920 9.9 -> 6.9).
-      // Two slices are left where at most two thirds of the CUs have a strip and there are no more than 1024 columns and K is 4096 or more: they cost
-      // up to 1.7 us (one / two slices: two rows, 8096 x 1120 7.1 / 7.8, ten with the seven planned before; 8 rows, 4192 x 656 6.5 / 8.2), but these are the packed decode plans that exchange partial
-      // tiles through the workspace of msco_gmm_launch_static, and its tests hold them to it.
+      // over 32 experts, 5536 x 576 8.9 -> 6.7; 16-bit x, one row, 3520 x 3920 9.9 -> 6.9; up to 1024 columns and K from 4096, where two slices stayed
+      // longest: 8336 shapes, two slices 1.14 of the time of one, K = 4096 1.15 to 1.19, K = 8192 1.07 to 1.17).
       // (short slices only where msco_gmm_launch_static takes their partial tiles too)
       want = floor_split;
-      if (col_groups <= 64 && (int64_t)op->n_strips * active * 3 <= 2 * (int64_t)num_cus && k_blocks >= 64) want = std::max(want, 2);
       if (short_slices && decode_tiles(m, n, e, kSkinnyRows, op->skinny_cols) * (size_t)want * stream_a16w8_tile_bytes() > (size_t)MSCO_GMM_STATIC_WORKSPACE_BYTES) want = fewest;
       cap = kMaxSplitK * 64;
     } else if (wide16) {

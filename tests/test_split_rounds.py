@@ -41,3 +41,8 @@ def test_several_groups_on_32_row_tiles(m, k, n, e, split):
     (2, 7712, 656, 16, "w8a8_skinny_16w"), (2, 4576, 1136, 16, "w8a8_skinny_16w"), (2, 3072, 1136, 16, "w8a8_skinny_tile_32x128")])
 def test_few_tiles_and_a_long_k_stay_with_the_decode_kernels(m, k, n, e, kernel):
     assert _plan(m, k, n, e)[0] == kernel
+
+
+@pytest.mark.parametrize("m,k,n,e", [(16, 8192, 1024, 1), (24, 4096, 512, 4), (8, 4192, 656, 1), (2, 8096, 1024, 1)])
+def test_packed_decode_walks_k_in_one_slice(m, k, n, e):
+    assert _plan(m, k, n, e, packed=True) == ("w8a8_stream", 1)

@@ -24,7 +24,7 @@ def _problem(seed, m, k, n, e, group_list, packed):
     tg = to_dev(np.asarray(group_list, dtype=np.int64))
     op = cabi.GmmOp(x_dtype=cabi.DT_I8, out_dtype=cabi.DT_BF16, group_list_dtype=cabi.DT_I64, bias_dtype=cabi.DT_I32,
                     scale_dtype=cabi.DT_F32, per_token_dtype=cabi.DT_F32,
-                    weight_layout=cabi.WL_PACKED if packed else cabi.WL_ROW_MAJOR)
+                    weight_layout=cabi.WL_PACKED if packed else cabi.WL_ROW_MAJOR, force_split_k=2 if packed else 0)
     ws = op.plan(m, k, n, e)
     ins = [t.data_ptr() for t in (tx, tw, tb, ts, tg, tp)] + [None, None]
     keep = (tx, tw, ts, tp, tb, tg)
@@ -45,8 +45,8 @@ def _both(op, ws, ins, shape):
 
 @pytest.mark.parametrize("packed", [True, False])
 def test_static_workspace_launch_matches_the_workspace_launch_twice_in_a_row(packed):
-    # a dense decode with a long K and then a smaller grouped decode: both plans split K across workgroups, so both
-    # exchange partial tiles through the workspace
+    # a dense decode with a long K and then a smaller grouped decode, K split across workgroups (on packed weights because the
+    # descriptor says so: the plan of its own accord does not), so that both exchange partial tiles through the workspace
     first = _problem(1, 16, 8192, 1024, 1, [16], packed)
     second = _problem(2, 24, 4096, 512, 4, [5, 5, 17, 24], packed)
     for op, ws, ins, keep, shape in (first, second):
