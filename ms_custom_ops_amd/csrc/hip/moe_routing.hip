@@ -267,7 +267,8 @@ __device__ __forceinline__ void wave_load_row(uint4 (&kept)[KV], __amdgpu_buffer
   });
 }
 
-// `first`: what wave_load_row brought of this row; dest_row(j): the j-th destination row
+// `first`: what wave_load_row brought of this row; dest_row(j): the j-th destination row.  (A store of vectors that all lie past the row's end writes
+// nothing but takes as long as one that does, once per copy: 2080 2-byte elements, 803 tokens x 8 14.8 against 9.5 us without it.)
 template <int KV, typename DestFn>
 __device__ __forceinline__ void wave_copy_row(const uint4 (&first)[KV], __amdgpu_buffer_rsrc_t src, int lane, const WaveShare &share, int copies,
                                               DestFn dest_row, unsigned char *expanded_x, long long row_bytes) {
@@ -275,7 +276,7 @@ __device__ __forceinline__ void wave_copy_row(const uint4 (&first)[KV], __amdgpu
     const __amdgpu_buffer_rsrc_t dst = buffer_over(expanded_x + (long long)dest_row(j) * row_bytes, row_bytes);
     static_for<KV>([&](auto u_c) {
       constexpr int U = decltype(u_c)::value;
-      row_store16(dst, share.at(U) + 16 * lane, first[U]);   // kept cacheable: the matmul reads it next
+      if (share.at(U) < row_bytes) row_store16(dst, share.at(U) + 16 * lane, first[U]);   // kept cacheable: the matmul reads it next
     });
   }
   for (long long b0 = share.pass_bytes(KV); b0 < row_bytes; b0 += share.pass_bytes(KV)) {
@@ -285,7 +286,7 @@ __device__ __forceinline__ void wave_copy_row(const uint4 (&first)[KV], __amdgpu
       const __amdgpu_buffer_rsrc_t dst = buffer_over(expanded_x + (long long)dest_row(j) * row_bytes, row_bytes);
       static_for<KV>([&](auto u_c) {
         constexpr int U = decltype(u_c)::value;
-        row_store16(dst, b0 + share.at(U) + 16 * lane, buf[U]);
+        if (b0 + share.at(U) < row_bytes) row_store16(dst, b0 + share.at(U) + 16 * lane, buf[U]);
       });
     }
   }
@@ -382,6 +383,19 @@ constexpr int kFusedThreads = 1024;   // sixteen wavefronts: the counting is a c
 constexpr int kFusedIdsPerThread = 16;
 constexpr long long kFusedMaxEntries = (long long)kFusedThreads * kFusedIdsPerThread;   // 16384: the two counts fit the halves of a word
 constexpr int kFusedMaxTopK = 1024;    // (a slice holds fewer than 64 + k entries)
+// A wavefront writes a token's rows one after the other; with dozens of experts per token that is what a launch takes, so beyond 8 of them spare slots
+// (and from 8 on spare CUs: one workgroup fits a CU) take four rows each.  us, plain copy, 2 x 64 rows of 4136 2-byte elements 32 -> 7.5, 4 x 200 of
+// 7944 94 -> 12, 1 x 8 of 4192 8.3 -> 6.6.
+struct FusedShares { int teams, parts, rows; };   // rows: of a token that one team of one workgroup writes
+inline FusedShares fused_shares(long long slices, int slots, int slice_tokens, long long k) {
+  auto take = [&](long long spare, long long want) { return (int)std::max<long long>(1, std::min(spare, want)); };
+  FusedShares f{1, 1, (int)k};
+  if (k > 8) f.teams = take(slots / slice_tokens, (k + 3) / 4);
+  if (k >= 8) f.parts = take(256 / slices, (k + 4 * f.teams - 1) / (4 * f.teams));
+  f.rows = (int)((k + f.teams * f.parts - 1) / (f.teams * f.parts));
+  return f;
+}
+
 // QUANT: 0 copies rows of row_bytes bytes; 1 / 2 quantise float16 / bfloat16 rows to int8 and write their scales.
 // EARLY: the rows are requested in front of the counting; not where a wavefront has more of a row than its KV vectors.
 template <int QUANT, bool EARLY>
@@ -389,7 +403,8 @@ __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsign
                                                                     unsigned char *expanded_x, float *expanded_scale,
                                                                     int *expanded_row_idx, int *count_or_cumsum,
                                                                     int *before_capacity, int n, int expert_num, int flag,
-                                                                    long long row_bytes, int k, int rep, int slice_tokens, int shift) {
+                                                                    long long row_bytes, int k, int rep, int slice_tokens, int shift, int teams,
+                                                                    int share_rows) {
   extern __shared__ int lds[];   // counts[rep][expert_num], first[expert_num], wave_sum[16], row_max[16], dest[slice_tokens k]
   int *counts = lds;
   int *first = counts + rep * expert_num;
@@ -401,6 +416,16 @@ __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsign
   const int start = token0 * k, end = token_end * k;
   constexpr int KV = 8;                  // vectors of a row per lane and pass
   const int slots = 16 >> shift, slot = wave >> shift;
+  // Who writes which of a token's k rows: parts of them go to the workgroups along grid.y (each ranks all of them), and in a workgroup to teams of slots
+  // where it has slots to spare.  A slot past the teams has no token.
+  const int part = (int)blockIdx.y;
+  int team = 0, slot_token = slot, copy0 = 0, copies = k;
+  if (share_rows < k) {   // (no division where nothing is shared: a hundred instructions on a cold instruction cache)
+    team = teams > 1 ? slot / slice_tokens : 0;
+    slot_token = team < teams ? slot - team * slice_tokens : slice_tokens;
+    copy0 = min((part * teams + min(team, teams - 1)) * share_rows, k);
+    copies = min(share_rows, k - copy0);
+  }
   WaveShare share;
   share.sub = wave & ((1 << shift) - 1);
   share.shift = shift;
@@ -426,7 +451,7 @@ __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsign
     return src;
   };
   __amdgpu_buffer_rsrc_t src;
-  if constexpr (EARLY) src = load(token0 + slot);
+  if constexpr (EARLY) src = load(token0 + slot_token);
   const int copy = (lane & (rep - 1)) * expert_num;   // rep is a power of two
   static_for<kFusedIdsPerThread / 4>([&](auto j_c) {
     constexpr int J = decltype(j_c)::value;
@@ -453,7 +478,7 @@ __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsign
   }
   if (tid < expert_num) {
     first[tid] = offset + (int)((unsigned)sum >> 16);
-    if (blockIdx.x == 0) {
+    if (blockIdx.x == 0 && part == 0) {
       if (count_or_cumsum != nullptr && flag == 1) count_or_cumsum[tid] = offset + total;
       if (count_or_cumsum != nullptr && flag == 2) count_or_cumsum[tid] = total;
       if (before_capacity != nullptr) before_capacity[tid] = 0;
@@ -473,21 +498,21 @@ __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsign
       if (live) {
         const int d = first[e] + rank;
         dest[i - start] = d;
-        expanded_row_idx[i] = d;
+        if (part == 0) expanded_row_idx[i] = d;
         if (end - i0 > 64 && rank + 1 == __popcll(same)) first[e] = d + 1;   // (the last of its id in these 64; every lane has read it)
       }
     }
   }
   __syncthreads();
-  // move the rows: slot s of the workgroup takes its tokens s, s + slots, ..
-  for (int t = slot, pass = 0; pass * slots < slice_tokens; t += slots, ++pass) {
+  // move the rows: slot s of the workgroup takes its tokens s, s + slots, .. (teams: one token)
+  for (int t = slot_token, pass = 0; pass * slots < slice_tokens; t += slots, ++pass) {
     if (pass > 0 || !EARLY) src = load(token0 + t);
     const bool live = token0 + t < token_end;
     // (a token's rows in one register, entry j in lane j: an LDS read per copy and piece of the row is a wait of its own)
-    const int dest_lane = live ? dest[t * k + min(lane, k - 1)] : 0;
-    auto dest_row = [&](int j) { return j < 64 ? __builtin_amdgcn_readlane(dest_lane, j) : __builtin_amdgcn_readfirstlane(dest[t * k + j]); };
+    const int dest_lane = live ? dest[t * k + min(copy0 + lane, k - 1)] : 0;
+    auto dest_row = [&](int j) { return j < 64 ? __builtin_amdgcn_readlane(dest_lane, j) : __builtin_amdgcn_readfirstlane(dest[t * k + copy0 + j]); };
     if constexpr (QUANT == 0) {
-      if (live) wave_copy_row(row, src, lane, share, k, dest_row, expanded_x, row_bytes);
+      if (live) wave_copy_row(row, src, lane, share, copies, dest_row, expanded_x, row_bytes);
     } else {
       unsigned mx = live ? wave_row_max(row, src, lane, share, row_bytes) : 0;
       if (shift > 0) {
@@ -497,7 +522,7 @@ __global__ void __launch_bounds__(kFusedThreads) route_fused_kernel(const unsign
         mx = (unsigned)__builtin_amdgcn_readfirstlane((int)mx);
       }
       if (live)
-        wave_quantise_row<QUANT == 2>(row, mx, src, lane, share, k, dest_row, reinterpret_cast<signed char *>(expanded_x), expanded_scale, row_bytes / 2);
+        wave_quantise_row<QUANT == 2>(row, mx, src, lane, share, copies, dest_row, reinterpret_cast<signed char *>(expanded_x), expanded_scale, row_bytes / 2);
     }
   }
 }
@@ -715,14 +740,16 @@ static int route_and_gather(const void *x, const int32_t *expert_idx, void *expa
     int rep = 8;
     while (rep > 1 && rep * expert_num > 512) rep /= 2;
     const size_t lds_bytes = (size_t)((rep + 1) * expert_num + 32 + f.slice_tokens * k) * sizeof(int);
-    const dim3 grid((unsigned)((num_rows + f.slice_tokens - 1) / f.slice_tokens)), block(kFusedThreads);
+    const long long slices = (num_rows + f.slice_tokens - 1) / f.slice_tokens;
+    const FusedShares shares = fused_shares(slices, 16 >> f.shift, f.slice_tokens, k);
+    const dim3 grid((unsigned)slices, (unsigned)shares.parts), block(kFusedThreads);
     const bool late = quant_dtype != MSCO_DT_NONE && row_bytes > 8192ll << f.shift;
 #define MSCO_ROUTE_FUSED(Q)                                                                                                  \
     auto kern = late ? route_fused_kernel<Q, Q == 0> : route_fused_kernel<Q, true>;                                           \
     hipLaunchKernelGGL(kern, grid, block, lds_bytes, s, static_cast<const unsigned char *>(x), expert_idx,   \
                        static_cast<unsigned char *>(expanded_x), expanded_scale, expanded_row_idx,                            \
                        expert_tokens_count_or_cumsum, expert_tokens_before_capacity, (int)n, (int)expert_num,                 \
-                       (int)count_or_cumsum_flag, row_bytes, (int)k, rep, f.slice_tokens, f.shift)
+                       (int)count_or_cumsum_flag, row_bytes, (int)k, rep, f.slice_tokens, f.shift, shares.teams, shares.rows)
     if (quant_dtype == MSCO_DT_NONE) { MSCO_ROUTE_FUSED(0); }
     else if (quant_dtype == MSCO_DT_F16) { MSCO_ROUTE_FUSED(1); }
     else { MSCO_ROUTE_FUSED(2); }

@@ -339,8 +339,8 @@ def test_routing_with_dynamic_quantisation_is_bit_exact(n_rows, h, k, e, bf16):
                                           (255, 7168, 8, 64), (257, 5120, 4, 16), (700, 2048, 8, 128), (1281, 3080, 4, 63), (4097, 1024, 1, 1024),
                                           (2048, 4096, 8, 256)])
 def test_one_launch_routing_with_rows_shared_by_wavefronts(n_rows, h, k, e):
-    """Tokens per workgroup 1 to 17, wavefronts per row 1 to 16, rows beyond what the wavefronts keep, slices of more than 64
-    entries, expert tables of one wavefront and of several: quantised rows, copied rows, indices and boundaries, bit for bit."""
+    """Tokens per workgroup 1 to 17, wavefronts per row 1 to 16, slices of more than 64 entries, expert tables of one wavefront and of
+    several: quantised rows, copied rows, indices and boundaries, bit for bit."""
     rng = np.random.default_rng(n_rows * 7 + h)
     x = rng.uniform(-3, 3, (n_rows, h)).astype(np.float16)
     x[-1, -1] = 11.0                                                               # the last vector holds the maximum
@@ -352,6 +352,36 @@ def test_one_launch_routing_with_rows_shared_by_wavefronts(n_rows, h, k, e):
     assert np.array_equal(sc.view(np.uint32), ref_s.view(np.uint32)) and np.array_equal(ex, ref_q)
     got = _route_gpu(x, idx, e, 1)
     assert np.array_equal(got[0].view(np.uint16), ref_rows.view(np.uint16)) and np.array_equal(got[1], ref_idx) and np.array_equal(got[2], ref_tok)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("n_rows,h,k,e", [
+    (2100, 5120, 4, 64), (3000, 8200, 2, 8), (4099, 4104, 1, 16), (2049, 16392, 1, 1),     # rows longer than the 8 KiB that a wavefront keeps, none shared
+    (1, 4192, 8, 256), (130, 2080, 8, 300), (39, 584, 200, 256), (97, 1880, 64, 1024),     # a token's rows over workgroups, over teams of a workgroup, over both
+    (1, 8, 9, 9), (7, 72, 1024, 3), (255, 264, 17, 2), (2, 7944, 33, 40)])
+def test_one_launch_routing_of_long_rows_and_of_many_rows_per_token(n_rows, h, k, e, bf16):
+    """The launch's loops over what a wavefront does not keep in registers, and every way a token's rows are shared out: quantised rows, copied
+    rows, indices and boundaries, bit for bit."""
+    assert n_rows * k <= 16384   # (more entries take the separate launches)
+    rng = np.random.default_rng(n_rows * 11 + h + k)
+    x32 = rng.uniform(-3, 3, (n_rows, h)).astype(np.float32)
+    x32[-1, -1] = 11.0                                                             # the last vector holds the maximum
+    if bf16:
+        bits = (x32.view(np.uint32) >> 16).astype(np.uint16)
+        vals = M.bf16_bits_to_f32(bits)
+    else:
+        vals = x32.astype(np.float16)
+        bits = vals.view(np.uint16)
+    idx = np.minimum(rng.integers(0, e, (n_rows, k)), rng.integers(0, e, (n_rows, k))).astype(np.int32)
+    ref_rows, ref_idx, ref_tok = M.moe_init_routing_v2(vals, idx, e, 1)
+    ref_q, ref_s = M.dyn_quant(ref_rows)
+    ex, sc, ridx, tok = _route_quant_gpu(np.ascontiguousarray(bits), bf16, idx, e, 1)
+    assert np.array_equal(ridx, ref_idx) and np.array_equal(tok, ref_tok)
+    assert np.array_equal(sc.view(np.uint32), ref_s.view(np.uint32)) and np.array_equal(ex, ref_q)
+    got = _route_gpu(bits.view(np.float16), idx, e, 1)                             # (a copy of two-byte elements)
+    want = M.moe_init_routing_v2(bits.view(np.float16), idx, e, 1)
+    assert np.array_equal(got[0].view(np.uint16), want[0].view(np.uint16)) and np.array_equal(got[1], ref_idx) and np.array_equal(got[2], ref_tok)
 
 
 @pytest.mark.gpu
