@@ -403,6 +403,18 @@ def test_token_unpermute_bf16_rounds_like_the_golden(tokens, hidden, top_k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("top_k", [1, 2, 3, 4, 8])
+@pytest.mark.parametrize("tokens,hidden", [(1025, 2056), (3, 2040)])
+def test_token_unpermute_f16_at_the_edges_of_a_piece(tokens, hidden, top_k):
+    """float16 rows that end just inside and just past a workgroup's 2048 elements, its loads under a condition."""
+    rng = np.random.default_rng(tokens + top_k + hidden)
+    pt, pr = rng.standard_normal((tokens * top_k, hidden)).astype(np.float16), rng.random((tokens, top_k)).astype(np.float16)
+    si = rng.permutation(tokens * top_k).astype(np.int32)
+    got = _unpermute_gpu(pt.view(np.uint16), si, pr.view(np.uint16), cabi.DT_F16)
+    assert np.array_equal(got, M.moe_token_unpermute(pt, si, pr).view(np.uint16))
+
+
+@pytest.mark.gpu
 def test_routing_with_dynamic_quantisation_rejects_what_it_cannot_take():
     with pytest.raises(RuntimeError):                                               # float32 activations
         cabi.moe_init_routing_v2_quant(1, 1, 1, 1, 1, None, None, 1, 0, 4, 64, 2, 8, cabi.DT_F32, 1)
