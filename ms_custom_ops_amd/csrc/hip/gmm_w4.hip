@@ -12,8 +12,8 @@
 //     with the low and the high nibbles of a weight word;
 //   * a wavefront takes blocks of C neighbouring columns per lane segment, lane L holding the 16-byte pieces L, L + 64, ... of a
 //     column (32 consecutive k, always inside one K group), and requests the next block while it multiplies this one: the
-//     group look-up, the x rows and the first round trip are paid once per workgroup, of which the launch has about four
-//     per CU.  nibbles are multiplied as u ^ 8 in [0, 15] with v_dot4_i32_i8 and 8 * sum(x) of the piece is subtracted
+//     group look-up, the x rows and the first round trip are paid once per workgroup, of which the launch has four
+//     per CU and more (launch_a8w4).  nibbles are multiplied as u ^ 8 in [0, 15] with v_dot4_i32_i8 and 8 * sum(x) of the piece is subtracted
 //     (u ^ 8 = s + 8 for the signed nibble s); the int32 sum of a piece is exact, is scaled by its K group's float32
 //     scale and added up in float32; the lanes' sums of C columns are added in a tree that halves the columns a lane
 //     holds with every step.
@@ -27,7 +27,7 @@ namespace {
 constexpr int W4_MAX_K = 8192;
 constexpr int W4_LDS_BYTES = 32 * 1024;              // x rows in LDS at a time: 32 KiB / K, at most W4_MAX_ROWS
 constexpr int W4_MAX_ROWS = 16;
-constexpr int W4_TARGET_WGS = 1024;                  // four workgroups per CU
+constexpr int W4_TARGET_WGS = 1024;                  // four workgroups per CU (one group; see launch_a8w4)
 constexpr int w4_cols(int p) { return p == 1 ? 8 : 4; }   // columns of a block per lane segment: 32 weight registers (64 with the longest K)
 inline int w4_rows(int64_t k, int64_t m) {
   int64_t r = W4_LDS_BYTES / k;
@@ -202,6 +202,25 @@ __global__ void __launch_bounds__(256, VEC ? 3 : 2) gmm_a8w4_kernel(const int8_t
 
   Block even, odd;   // (the longest K has one block in flight: with half as many columns each, or both blocks, slower, 14.5 against 12.4 us)
   const int stride = (int)gridDim.x;
+  if constexpr (P == 4) {
+    // A block's weights stay in registers for all rows of the group: a group with more rows than LDS holds (four to seven with this K) brings its rows
+    // once per block, not its weights once per batch of rows (one group of 16 and more rows 0.80 -> 0.68 of the time of a launch with one block per workgroup)
+    int staged = -1;   // the batch of rows in LDS
+    for (int block = (int)blockIdx.x; block < blocks; block += stride) {
+      request(even, block);
+      for (int r0 = g_start; r0 < g_end; r0 += lds_rows) {
+        const int rows = min(lds_rows, g_end - r0);
+        if (staged != r0) {
+          if (staged >= 0) __syncthreads();   // the rows before are no longer read
+          stage_rows(r0, rows);
+          __syncthreads();
+          staged = r0;
+        }
+        multiply(even, block, r0, rows);
+      }
+    }
+    return;
+  }
   for (int r0 = g_start; r0 < g_end; r0 += lds_rows) {
     const int rows = min(lds_rows, g_end - r0);
     int block = (int)blockIdx.x;
@@ -209,13 +228,6 @@ __global__ void __launch_bounds__(256, VEC ? 3 : 2) gmm_a8w4_kernel(const int8_t
     if (r0 != g_start) __syncthreads();   // the rows before are no longer read
     stage_rows(r0, rows);
     __syncthreads();
-    if constexpr (P == 4) {
-      for (; block < blocks; block += stride) {
-        multiply(even, block, r0, rows);
-        request(even, block + stride);
-      }
-      continue;
-    }
     for (; block < blocks; block += 2 * stride) {
       request(odd, block + stride);
       multiply(even, block, r0, rows);
@@ -235,7 +247,10 @@ hipError_t launch_a8w4(const int8_t *x, const unsigned char *w, const int *group
   const int block_cols = 4 * C * (64 / lanes_per_col), blocks = (n + block_cols - 1) / block_cols;
   const int slots = e < m ? e : m;
   // (slots past the last group that holds rows leave at once: counting them all makes the shares of the columns larger, not smaller)
-  int shares = (W4_TARGET_WGS + slots - 1) / slots;
+  // With several groups the launch ends with the largest one, which does rows x columns of work in its shares: more of them, by twice the average rows of a
+  // group, let the others' CUs take part (172 rows over 64 experts, 8064 x 6128 701 -> 372 us; 106 rows, 5312 x 6064 431 -> 246; 12342 random
+  // shapes 0.95 of the time; one group is even whatever the shares)
+  int shares = (W4_TARGET_WGS + slots - 1) / slots * (slots > 1 ? (2 * m + slots - 1) / slots : 1);
   shares = shares < blocks ? shares : blocks;
   const int steps = (blocks + shares - 1) / shares;
   const dim3 grid((unsigned)((blocks + steps - 1) / steps), (unsigned)slots);

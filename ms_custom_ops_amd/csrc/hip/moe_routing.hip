@@ -268,7 +268,7 @@ __device__ __forceinline__ void wave_load_row(uint4 (&kept)[KV], __amdgpu_buffer
 }
 
 // `first`: what wave_load_row brought of this row; dest_row(j): the j-th destination row.  (A store of vectors that all lie past the row's end writes
-// nothing but takes as long as one that does, once per copy: 2080 2-byte elements, 803 tokens x 8 14.8 against 9.5 us without it.)
+// nothing but takes as long as one that does, once per copy: 2080 2-byte elements, 803 tokens x 8 14.7 against 9.9 us without it.)
 template <int KV, typename DestFn>
 __device__ __forceinline__ void wave_copy_row(const uint4 (&first)[KV], __amdgpu_buffer_rsrc_t src, int lane, const WaveShare &share, int copies,
                                               DestFn dest_row, unsigned char *expanded_x, long long row_bytes) {
@@ -384,8 +384,8 @@ constexpr int kFusedIdsPerThread = 16;
 constexpr long long kFusedMaxEntries = (long long)kFusedThreads * kFusedIdsPerThread;   // 16384: the two counts fit the halves of a word
 constexpr int kFusedMaxTopK = 1024;    // (a slice holds fewer than 64 + k entries)
 // A wavefront writes a token's rows one after the other; with dozens of experts per token that is what a launch takes, so beyond 8 of them spare slots
-// (and from 8 on spare CUs: one workgroup fits a CU) take four rows each.  us, plain copy, 2 x 64 rows of 4136 2-byte elements 32 -> 7.5, 4 x 200 of
-// 7944 94 -> 12, 1 x 8 of 4192 8.3 -> 6.6.
+// (and from 8 on spare CUs: one workgroup fits a CU) take four rows each.  us, plain copy, 2 x 64 rows of 4136 2-byte elements 32 -> 5.9, 4 x 200 of
+// 7944 94 -> 10, 1 x 8 of 4192 8.3 -> 5.8.
 struct FusedShares { int teams, parts, rows; };   // rows: of a token that one team of one workgroup writes
 inline FusedShares fused_shares(long long slices, int slots, int slice_tokens, long long k) {
   auto take = [&](long long spare, long long want) { return (int)std::max<long long>(1, std::min(spare, want)); };

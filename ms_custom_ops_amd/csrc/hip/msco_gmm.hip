@@ -470,7 +470,7 @@ void plan_few_rows(msco_gmm_op *op, int &family) {
 // Which side of a round a launch of several groups falls is counted with the mean over the routings of its row tiles: "a tenth more rows" jumps by a
 // tile per group just below a multiple of the tile (8 experts, 121 rows each: three 64-row tiles, 2.4 on average).
 // Shapes between the two counts, us, the wider tile / the other:
-// 128 x 256 where 128 x 128 are expected to be 180 .. 250 tiles 1.36 times as long (8 experts, 1988 rows, 4032 x 1776 45.6 / 34.4), 260 and more
+// 128 x 256 where 128 x 128 are expected to be 180 .. 250 tiles 1.36 times as long (8 experts, 490 tokens x 4, 4032 x 1776 45.5 / 32.1), 260 and more
 // 0.91; 128 x 128 where 64 x 128 are 180 .. 236 1.08 (skewed routings 1.07), 248 .. 256 0.99; a K split of 128 x 128 tiles that fill
 // more than half of a round 1.25 (16 experts, 2872 rows, 3168 x 592, [E,N,K] two slices 33.5, 64 x 128 22.8).
 bool plan_one_round(msco_gmm_op *op) {   // true: K is not to be split
@@ -688,12 +688,12 @@ void choose_plan(msco_gmm_op *op) {
       // 21.5; 3 rows, 7552 x 4256 15.4 -> 14.0), 64 x 128 0.991 (41 rows, 2720 x 1200 10.9 -> 9.6).  Its rounds are those of an XCD, which takes an
       // eighth of the tiles, rounded up, with all their slices: three slices of 81 to 85 tiles are 33 workgroups for 32 CUs.  Counted over the
       // chip that was one round.  7778 random shapes that this changes, 0.83 of the time, one slower by more than 0.05: 64 x 128, three
-      // slices -> two 0.77 (72 rows, 2688 x 5280 15.4 -> 12.7), 32 x 128, 62 to 64 tiles, three -> four 0.95.
+      // slices -> two 0.77 (72 rows, 2688 x 5280, [E,N,K] 15.6 -> 11.3), 32 x 128, 62 to 64 tiles, three -> four 0.95.
       const int cus = or_default(tuning().tile_target_wgs, num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       const int cap = (int)std::max<int64_t>(1, ((k + 63) / 64) / kTileMinSlabs);
       // (several groups, more than 11 and up to 16 rows each on average: all of them hold rows, some of them more than a tile, and a second tile per CU costs what it
       // costs with one group.  2411 such shapes 0.85 of the time of the splits before, none
-      // with an even routing slower than 64 x 128 tiles; up to 11 rows a group the 1.2 times stand, as a random routing leaves groups empty)
+      // with an even routing slower than 64 x 128 tiles (32 experts, 364 rows, 3616 x 832 28.3 -> 22.1); up to 11 rows a group the 1.2 times stand, as a random routing leaves groups empty)
       const bool full_groups = (m + e - 1) / e * 3 / 2 > kSkinnyRows;
       auto split_cost = [&](int sl) {
         const int64_t slabs = ((k + 63) / 64 + sl - 1) / sl;
