@@ -14,9 +14,13 @@
 //     [E,K,N]: a lane requests four neighbouring columns of its 16 K rows; column j of two rows is converted and packed by
 //     the same instructions (byte select), so the turn costs nothing.  The output column of MFMA column c of word position j
 //     then is 4 c + j.
-//     4-bit [E,K,N]: two bytes hold the lane's four columns of a row; four instructions make signed bytes of two rows, at 16 times
-//     their value (exact in either type, taken out of the sums again), and the rest is the same: bit for bit what the int8 copy of
-//     the weights gives, without the launch that writes it (1.5 bytes per weight) and the second byte of every later read.
+//     4-bit [E,K,N]: two bytes hold the lane's four columns of a row; a word holds two rows.  bfloat16 x: one conversion of a
+//     signed 4-bit number each, at a sixteenth of its value (products and sums stay exact where they are subnormal, and none is
+//     infinite that the numbers themselves keep finite; bytes at 16 times the value lost the sums above 2^124 and took 1.01 of
+//     the time, nibbles taken out one by one at their value 1.06).  float16 x: four instructions make signed bytes of two rows,
+//     at 16 times their value (exact, and float16 products are far from the end of float32).  The epilogue takes the factor out.
+//     Bit for bit what the int8 copy of the weights gives, without the launch that writes it (1.5 bytes per weight) and the
+//     second byte of every later read.
 //   * the weights are the MFMA's first operand: a lane ends up with neighbouring columns of one row ([E,K,N]: 16; packed: 8,
 //     once two lane rows have changed places), stored straight from the accumulators.
 //   * x goes straight into a ring of LDS stages of 64 K positions (128 bytes) per row; 16-byte piece q of row r sits at piece
@@ -74,6 +78,13 @@ __device__ __forceinline__ int xa_pair(unsigned w0, unsigned w1) {
     const unsigned bytes = perm(w1, w0, 0x0C000C00u | ((4u + B1) << 16) | B0) ^ 0x64806480u;
     return __builtin_bit_cast(int, __builtin_bit_cast(v2h, bytes) + v2h{(_Float16)-1152.0f, (_Float16)-1152.0f});
   }
+}
+
+// Signed 4-bit numbers in the low halves of bytes B0 and B1 -> two bfloat16 values, a sixteenth of the numbers, exact.
+template <int B0, int B1>
+__device__ __forceinline__ int xa_nibble_pair(unsigned w) {
+  const float f0 = __builtin_amdgcn_cvt_off_f32_i4((int)(w >> (8 * B0) & 0xFFu)), f1 = __builtin_amdgcn_cvt_off_f32_i4((int)(w >> (8 * B1) & 0xFFu));
+  return (int)perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
 }
 
 // acc += a x b in the registers of acc (left to the compiler, accumulator blocks move between the unrolled K blocks, and the
@@ -173,14 +184,22 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
     if constexpr (KN) {
       constexpr int R = 8 * HALF + 2 * D;
       if constexpr (W4) {
-        // four columns of two rows: 16 times their values as signed bytes, the even columns in one word and the odd ones in the other
+        // four columns of two rows in one word: the even columns in the low halves of its bytes, the odd ones in the high halves
         int &even = raw[SET][R / 4][R % 4], &odd = raw[SET][(R + 1) / 4][(R + 1) % 4];
         if constexpr (J == 0) {
           const unsigned both = (unsigned)even | (unsigned)odd << 16;
-          even = (int)((both << 4) & 0xF0F0F0F0u);
-          odd = (int)(both & 0xF0F0F0F0u);
+          if constexpr (BF16) {          // (the conversion looks at the low half of a byte alone)
+            even = (int)both;
+            odd = (int)(both >> 4);
+            asm("" : "+v"(odd));         // (or the shift joins the byte select: one more instruction for each weight)
+          } else {                       // 16 times their values as signed bytes
+            even = (int)((both << 4) & 0xF0F0F0F0u);
+            odd = (int)(both & 0xF0F0F0F0u);
+          }
         }
-        f[J][D] = xa_pair<BF16, J / 2, 2 + J / 2>((unsigned)(J % 2 == 0 ? even : odd), (unsigned)(J % 2 == 0 ? even : odd));
+        const unsigned w = (unsigned)(J % 2 == 0 ? even : odd);
+        if constexpr (BF16) f[J][D] = xa_nibble_pair<J / 2, 2 + J / 2>(w);
+        else f[J][D] = xa_pair<false, J / 2, 2 + J / 2>(w, w);
       } else f[J][D] = xa_pair<BF16, J, J>((unsigned)raw[SET][R / 4][R % 4], (unsigned)raw[SET][(R + 1) / 4][(R + 1) % 4]);
     } else {
       constexpr int W = 2 * HALF + D / 2;
@@ -419,7 +438,7 @@ __device__ __forceinline__ void rows_a16w8_run(const GmmParams &p, unsigned char
       if (live && row < chunk_rows) {
         unsigned q[NV / 2];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) a[v] = fmaf(of[v], xs_row, W4 ? a[v] * 0.0625f : a[v]) * sc[v];
+        for (int v = 0; v < NV; ++v) a[v] = fmaf(of[v], xs_row, W4 ? a[v] * (BF16 ? 16.0f : 0.0625f) : a[v]) * sc[v];
         if constexpr (decltype(act_c)::value) activate_n(a, p.act_type);
         pack_half_n(a, BF16 ? DT_BF16 : DT_F16, q);
         uint4 *dst = reinterpret_cast<uint4 *>(reinterpret_cast<unsigned short *>(p.out) + (long long)(m0 + row) * p.n + n);
