@@ -3,6 +3,7 @@ import numpy as np
 import torch
 
 from ms_custom_ops_amd import cabi
+from oracle import gmm_oracle as O
 
 _NP2DT = {np.dtype(np.int32): cabi.DT_I32, np.dtype(np.int64): cabi.DT_I64}
 
@@ -66,15 +67,15 @@ def run_w8a8(x, w, group_list, bias=None, scale=None, per_token=None, *, out="bf
 
 
 def run_a16w8(x_bits, w, scale_bits, offset_bits, group_list, *, dtype="bf16", override=0, group_list_type=0, packed=False,
-              act_type=0):
+              act_type=0, bits=8, force_split_k=0):
     m, k = x_bits.shape
     e, _, n = w.shape
     dt = cabi.DT_BF16 if dtype == "bf16" else cabi.DT_F16
-    tx, tw, ts, to = to_dev(x_bits), to_dev(w), to_dev(scale_bits), to_dev(offset_bits)
+    tx, tw, ts, to = to_dev(x_bits), to_dev(O.pack_int4(w) if bits == 4 else w), to_dev(scale_bits), to_dev(offset_bits)
     tg = to_dev(np.asarray(group_list).astype(np.int64))
     if packed:
         tw = pack_on_device(tw, e, k, n)
-    op = cabi.GmmOp(x_dtype=dt, out_dtype=dt, group_list_dtype=cabi.DT_I64, group_list_type=group_list_type,
+    op = cabi.GmmOp(x_dtype=dt, out_dtype=dt, weight_dtype=cabi.DT_I4 if bits == 4 else cabi.DT_I8, force_split_k=force_split_k, group_list_dtype=cabi.DT_I64, group_list_type=group_list_type,
                     antiquant_dtype=dt, has_antiquant_offset=int(to is not None), kernel_override=override, act_type=act_type,
                     weight_layout=cabi.WL_PACKED if packed else cabi.WL_ROW_MAJOR)
     ws = op.plan(m, k, n, e)

@@ -199,3 +199,54 @@ def test_fused_activation_weight_only_128_row_chunks(act, packed):
     assert not np.array_equal(bits, plain)
     if act == O.ACT_RELU:
         assert np.array_equal(bits, np.where(O.bf16_bits_to_f32(plain) < 0, np.uint16(0), plain))
+
+
+@pytest.mark.parametrize("act", ACTS)
+@pytest.mark.parametrize("bits,packed", [(8, False), (8, True), (4, False)])
+@pytest.mark.parametrize("override,split,strips", [(cabi.OV_ROWS16, 0, "rows128 "), (cabi.OV_ROWS16_256, 1, "rows128x256 "), (cabi.OV_ROWS16_256, 3, "rows128x256 "),
+                                                   (cabi.OV_ROWS16_256X2, 1, "rows128x256_2 "), (cabi.OV_ROWS16_256X2, 2, "rows128x256_2 "),
+                                                   (cabi.OV_ROWS16_256X2, 4, "rows128x256_2 ")])
+def test_fused_activation_weight_only_128_row_forms(override, split, strips, bits, packed, act):
+    """Every form of the 128-row kernel: strips of 512 and 256 columns, two sets of waves, K slices, 4-bit weights."""
+    from gpu_utils import run_a16w8
+    rng = np.random.default_rng(6)
+    m, k, n, e, gl = 333, 1104, 528, 3, [129, 130, 333]
+    x_bits = O.f32_to_bf16_bits(rng.standard_normal((m, k)).astype(np.float32))
+    top = 127 if bits == 8 else 7
+    w = rng.integers(-top - 1, top + 1, (e, k, n), dtype=np.int8)
+    s_bits = O.f32_to_bf16_bits((rng.uniform(1e-3, 1e-2, (e, n)) * (1 if bits == 8 else 10)).astype(np.float32))
+    o_bits = O.f32_to_bf16_bits(rng.integers(-8, 9, (e, n)).astype(np.float32))
+    plain, info = run_a16w8(x_bits, w, s_bits, o_bits, gl, packed=packed, override=override, bits=bits, force_split_k=split)
+    got_bits, info = run_a16w8(x_bits, w, s_bits, o_bits, gl, packed=packed, override=override, bits=bits, force_split_k=split, act_type=act)
+    assert strips in info and "widened" not in info and ("a16w4" in info) == (bits == 4) and f"split_k={max(split, 1)} " in info, info
+    xv, sv, ov = (O.bf16_bits_to_f32(b) for b in (x_bits, s_bits, o_bits))
+    exact = O.a16w8_grouped_f64(xv, w, sv, ov, gl)
+    # (bars as above: one bfloat16 rounding and float32 sums, whose terms are at most |x| (|w| + |o|) s)
+    mag = np.abs(xv).astype(np.float64).sum(1, keepdims=True) * (top + 1 + 8) * float(np.abs(sv).max())
+    ref, got = O.activation(exact.astype(np.float32), act), O.bf16_bits_to_f32(got_bits).astype(np.float64)
+    assert (np.abs(got - ref) <= 2.0 ** -7 * np.abs(ref) + 1.13 * (2.0 ** -7 * np.abs(exact) + 1e-5 * mag) + 1e-30).all(), info
+    pre = O.bf16_bits_to_f32(plain)
+    assert not np.array_equal(got_bits, plain)
+    if act == O.ACT_RELU:
+        assert np.array_equal(got_bits, np.where(pre < 0, np.uint16(0), plain))
+
+
+@pytest.mark.parametrize("act", ACTS)
+@pytest.mark.parametrize("override,transpose_b,columns", [(cabi.OV_TILE_32x128, False, 128), (cabi.OV_TILE_32x128, True, 128), (cabi.OV_TILE_32x256, False, 256)])
+def test_fused_activation_32_row_tiles(override, transpose_b, columns, act):
+    """Tiles of 32 rows: groups that end inside a tile, a last strip that is not full."""
+    from gpu_utils import run_w8a8
+    m, k, n, e, gl = 333, 256 + 48, 384 + 16, 8, [5, 5, 40, 100, 100, 230, 300, 333]
+    rng = np.random.default_rng(18)
+    x, w = rng.integers(-127, 128, (m, k), dtype=np.int8), rng.integers(-127, 128, (e, k, n), dtype=np.int8)
+    scale, pt = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), rng.uniform(1e-2, 1e-1, m).astype(np.float32)
+    pre, ref64 = _reference(x, w, gl, None, scale, pt, act)
+    for out in ("bf16", "f16"):
+        bits, info = run_w8a8(x, w, gl, None, scale, pt, out=out, transpose_b=transpose_b, override=override, act_type=act, launches=2)
+        assert f"tile_32x{columns}" in info, info
+        got = O.bf16_bits_to_f32(bits) if out == "bf16" else bits.view(np.float16).astype(np.float32)
+        if act == O.ACT_RELU:
+            want = O.f32_to_bf16_bits(ref64.astype(np.float32)) if out == "bf16" else O.f32_to_f16(ref64.astype(np.float32)).view(np.uint16)
+            assert np.array_equal(bits, want), info
+        else:
+            _assert_close(got, ref64, out, info)
