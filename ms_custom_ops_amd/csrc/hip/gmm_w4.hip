@@ -250,9 +250,8 @@ hipError_t launch_a8w4(const int8_t *x, const unsigned char *w, const int *group
   // With several groups the launch ends with the largest one, which does rows x columns of work in its shares: more of them, by twice the average rows of a
   // group, let the others' CUs take part (172 rows over 64 experts, 8064 x 6128 701 -> 372 us; 106 rows, 5312 x 6064 431 -> 246; 12342 random
   // shapes 0.95 of the time; one group is even whatever the shares)
-  int shares = (W4_TARGET_WGS + slots - 1) / slots * (slots > 1 ? (2 * m + slots - 1) / slots : 1);
-  shares = shares < blocks ? shares : blocks;
-  const int steps = (blocks + shares - 1) / shares;
+  const long long wanted = (W4_TARGET_WGS + slots - 1ll) / slots * (slots > 1 ? (2ll * m + slots - 1) / slots : 1);
+  const int shares = wanted < blocks ? (int)wanted : blocks, steps = (blocks + shares - 1) / shares;
   const dim3 grid((unsigned)((blocks + steps - 1) / steps), (unsigned)slots);
   const int rows = w4_rows(k, m);
   const size_t lds = (size_t)rows * (size_t)k;
