@@ -37,7 +37,7 @@ inline int w4_rows(int64_t k, int64_t m) {
 
 __device__ __forceinline__ int dot4(int a, int b, int c) { return __builtin_amdgcn_sdot4(a, b, c, false); }
 
-// P = 16-byte pieces of a column per lane (K <= 2048 P); VEC: a lane's C scales of a K group are one request (N % C == 0)
+// P = 16-byte pieces of a column per lane (K <= 2048 P); VEC: four scales of a lane's columns are one request (N % 4 == 0)
 template <int P, bool VEC>
 __global__ void __launch_bounds__(256, VEC ? 3 : 2) gmm_a8w4_kernel(const int8_t *x, const unsigned char *w, const int *group_list,
                                                        const float *x_scale, const float *w_scale, unsigned short *out, int m,
@@ -116,17 +116,13 @@ __global__ void __launch_bounds__(256, VEC ? 3 : 2) gmm_a8w4_kernel(const int8_t
       for (int c = 0; c < C; ++c)
         b.w[i][c] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, live && col_lane + c < cols ? (unsigned)(col_lane + c) * (unsigned)(k / 2) + 16u * (unsigned)p : 0xFFFFFFF0u, 0, 0);
       const unsigned at = 4u * ((unsigned)(p / pieces_per_group) * (unsigned)n + (unsigned)col_lane);
-      if constexpr (VEC && C % 4 == 0) {
+      if constexpr (VEC) {
 #pragma unroll
         for (int c = 0; c < C; c += 4) {
           const v4i v = __builtin_amdgcn_raw_buffer_load_b128(rs_s, live && col_lane < cols ? at + 4u * c : 0xFFFFFFF0u, 0, 0);
 #pragma unroll
           for (int q = 0; q < 4; ++q) b.s[i][c + q] = __uint_as_float((unsigned)v[q]);
         }
-      } else if constexpr (VEC) {
-        const unsigned long long v = __builtin_bit_cast(unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(rs_s, live && col_lane < cols ? at : 0xFFFFFFF0u, 0, 0));
-        b.s[i][0] = __uint_as_float((unsigned)v);
-        b.s[i][1] = __uint_as_float((unsigned)(v >> 32));
       } else {
 #pragma unroll
         for (int c = 0; c < C; ++c)
@@ -255,7 +251,7 @@ hipError_t launch_a8w4(const int8_t *x, const unsigned char *w, const int *group
   const dim3 grid((unsigned)((blocks + steps - 1) / steps), (unsigned)slots);
   const int rows = w4_rows(k, m);
   const size_t lds = (size_t)rows * (size_t)k;
-  auto kern = n % (C < 4 ? C : 4) == 0 ? gmm_a8w4_kernel<P, true> : gmm_a8w4_kernel<P, false>;
+  auto kern = n % 4 == 0 ? gmm_a8w4_kernel<P, true> : gmm_a8w4_kernel<P, false>;
   hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, x, w, group_list, x_scale, w_scale, out, m, k, n, e, group_size, rows);
   return hipGetLastError();
 }
