@@ -11,9 +11,10 @@
 //             operands of 16 times their value ((c << 4) & 0xF0.., c & 0xF0..): 20 instructions per 32 weights, nothing to
 //             sign-extend, and the int32 sums are exactly 16 times the true ones (K x 2^14 < 2^31 is checked by the plan, for this form alone).
 //   16-bit x  v_mfma_f32_16x16x32, KR = 8.  A signed byte of two rows each goes through v_cvt_f32_i32 (byte select) and
-//             one pack: exact in bf16 and f16.  4-bit weights enter as 16 times their value (the same masks as above):
-//             every product and every rounding is 16 times the one 8-bit weights of the same value give, so with the
-//             same chunks the results are the same bits.  The antiquant offset is folded into the epilogue with the row sums of x (one MFMA
+//             one pack: exact in bf16 and f16.  4-bit weights enter as a sixteenth of their value (one conversion takes the low half
+//             of a byte): every product and every rounding is a sixteenth of the one 8-bit weights of the same value give, so with
+//             the same chunks the results are the same bits (16 times the value, which this was, loses sums from 2^124 on; a sixteenth
+//             loses nothing: products are multiples of 2^-137).  The antiquant offset is folded into the epilogue with the row sums of x (one MFMA
 //             against ones per x fragment):  out = s * (sum_k x w + o sum_k x).
 //
 // The output column of MFMA column c of word position j is CPL c + j: a permutation that only the epilogue sees.
@@ -77,6 +78,13 @@ __device__ __forceinline__ void load_words(int *w, __amdgpu_buffer_rsrc_t rs, un
 template <bool BF16, int B>
 __device__ __forceinline__ int byte_pair(unsigned lo, unsigned hi) {
   const float f0 = (float)(int)(signed char)(lo >> (8 * B)), f1 = (float)(int)(signed char)(hi >> (8 * B));
+  if constexpr (BF16) return (int)perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+  else return __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(f0, f1));
+}
+// the signed 4-bit numbers in the low halves of these bytes -> a sixteenth of each
+template <bool BF16, int B>
+__device__ __forceinline__ int nibble_pair(unsigned lo, unsigned hi) {
+  const float f0 = __builtin_amdgcn_cvt_off_f32_i4((int)(lo >> (8 * B) & 0xFFu)), f1 = __builtin_amdgcn_cvt_off_f32_i4((int)(hi >> (8 * B) & 0xFFu));
   if constexpr (BF16) return (int)perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
   else return __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(f0, f1));
 }
@@ -186,19 +194,19 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
           for (int t = 0; t < L; ++t) rt_mfma<XT>(acc[4 * D + Q][t], xbuf[B][t], f);
         });
       } else {
-        unsigned even[8], odd[8];   // 16 times columns 0, 2, 4, 6 and 1, 3, 5, 7 of the word as signed bytes
+        unsigned odd[8];   // columns 1, 3, 5, 7 of the word in the low halves of the bytes, where 0, 2, 4, 6 are in the word itself
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          even[i] = ((unsigned)wbuf[B][i][D] << 4) & 0xF0F0F0F0u;
-          odd[i] = (unsigned)wbuf[B][i][D] & 0xF0F0F0F0u;
+          odd[i] = (unsigned)wbuf[B][i][D] >> 4;
+          asm("" : "+v"(odd[i]));   // (or the shift joins the byte select: one more instruction for each weight)
         }
         static_for<4>([&](auto b4_c) {
           constexpr int Q = decltype(b4_c)::value;
           v4i fe, fo;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            fe[q] = byte_pair<BF16, Q>(even[2 * q], even[2 * q + 1]);
-            fo[q] = byte_pair<BF16, Q>(odd[2 * q], odd[2 * q + 1]);
+            fe[q] = nibble_pair<BF16, Q>((unsigned)wbuf[B][2 * q][D], (unsigned)wbuf[B][2 * q + 1][D]);
+            fo[q] = nibble_pair<BF16, Q>(odd[2 * q], odd[2 * q + 1]);
           }
 #pragma unroll
           for (int t = 0; t < L; ++t) {
@@ -275,13 +283,13 @@ __device__ __forceinline__ void regt_run(const GmmParams &p, unsigned char *smem
 
   auto finish = [&](int row, int n, const Elem (&v)[8], float xs) {
     if (n >= p.n) return;
-    constexpr int shift = WB == 4 ? 4 : 0;   // the operands were 16 times the nibbles: exact
+    constexpr int shift = WB == 4 ? 4 : 0;   // int8 x: the operands were 16 times the nibbles, 16-bit x: a sixteenth of them; exact
     float f[8];
     const float *sc = s_scale + (n - n0);
     const int *other = s_other + (n - n0);
     if constexpr (FP) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = fmaf(__int_as_float(other[j]), xs, v[j] * (1.0f / (1 << shift))) * sc[j];
+      for (int j = 0; j < 8; ++j) f[j] = fmaf(__int_as_float(other[j]), xs, v[j] * (float)(1 << shift)) * sc[j];
     } else {
       if (p.out_dtype == DT_I32) {
         int *dst = reinterpret_cast<int *>(p.out) + (long long)(m0 + row) * p.n + n;

@@ -266,3 +266,28 @@ def test_activation_on_4_bit_weights(device, x_type, override, counts, k, n, mus
         assert np.array_equal(got, O.f32_to_bf16_bits(ref.astype(np.float32)))
     else:
         assert (np.abs(O.bf16_bits_to_f32(got).astype(np.float64) - ref) <= 2.0 ** -7 * np.abs(ref) + slack * np.abs(pre) + 1e-30).all()
+
+
+@pytest.mark.parametrize("exponent", [119, -124, -130])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("counts,split", [([16, 3], 1), ([31, 2], 2)])
+def test_16_bit_activations_at_the_ends_of_float32(device, counts, split, bits, exponent):
+    """bfloat16 x around 2^exponent: sums up to 2^127, brought back by the scales, stay finite, and subnormal x and products are kept.
+    Bounds: float32 sums of 256 exact products (2^-16 of the terms' magnitudes), one bfloat16 rounding (half a step of 2^-133 where the
+    output is subnormal)."""
+    rng = np.random.default_rng(13)
+    e, m, k, n = len(counts), sum(counts), 256, 272
+    x = O.f32_to_bf16_bits(np.ldexp(rng.standard_normal((m, k)), exponent).astype(np.float32))
+    w = rng.integers(-8, 8, (e, k, n), dtype=np.int8)
+    scale = 2.0 ** -6 if exponent > 0 else 1.0
+    s = O.f32_to_bf16_bits(np.full((e, n), scale, np.float32))
+    out = _run(cabi.DT_BF16, bits, x, w, counts, split, {cabi.IN_ANTIQUANT_SCALE: to_dev(s)}, cabi.DT_BF16, antiquant_dtype=cabi.DT_BF16)
+    got = O.bf16_bits_to_f32(out.view(np.uint16)).astype(np.float64)
+    assert np.isfinite(got).all()
+    xv, r = O.bf16_bits_to_f32(x).astype(np.float64), 0
+    largest = 0.0
+    for i, c in enumerate(counts):
+        want, mag = xv[r:r + c] @ w[i].astype(np.float64), np.abs(xv[r:r + c]) @ np.abs(w[i].astype(np.float64))
+        assert (np.abs(got[r:r + c] - scale * want) <= 2.0 ** -8 * scale * np.abs(want) + 2.0 ** -16 * scale * mag + 2.0 ** -134).all()
+        largest, r = max(largest, np.abs(want).max()), r + c
+    assert exponent < 0 or 2.0 ** 124 < largest < 2.0 ** 128     # (sixteen times these sums is infinite)
