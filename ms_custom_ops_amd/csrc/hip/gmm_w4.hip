@@ -245,8 +245,10 @@ hipError_t launch_a8w4(const int8_t *x, const unsigned char *w, const int *group
   // (slots past the last group that holds rows leave at once: counting them all makes the shares of the columns larger, not smaller)
   // With several groups the launch ends with the largest one, which does rows x columns of work in its shares: more of them, by twice the average rows of a
   // group, let the others' CUs take part (172 rows over 64 experts, 8064 x 6128 701 -> 372 us; 106 rows, 5312 x 6064 431 -> 246; 12342 random
-  // shapes 0.95 of the time; one group is even whatever the shares)
-  const long long wanted = (W4_TARGET_WGS + slots - 1ll) / slots * (slots > 1 ? (2ll * m + slots - 1) / slots : 1);
+  // shapes 0.95 of the time; one group is even whatever the shares).  Up to half as many rows as experts, most groups hold one row and are even
+  // too: twice the shares are a second round of workgroups there (20 rows over 64 experts, 2816 x 1200 11.25 against 12.4 us; 600 random
+  // shapes of 2 to 64 rows, no more than experts: 6 slower by more than 3 % than a launch of 1024 workgroups, 54 with twice the shares everywhere).
+  const long long wanted = (W4_TARGET_WGS + slots - 1ll) / slots * (slots > 1 && 2ll * m > e ? (2ll * m + slots - 1) / slots : 1);
   const int shares = wanted < blocks ? (int)wanted : blocks, steps = (blocks + shares - 1) / shares;
   const dim3 grid((unsigned)((blocks + steps - 1) / steps), (unsigned)slots);
   const int rows = w4_rows(k, m);

@@ -158,6 +158,7 @@ def test_a8w4_malformed_group_list_is_clamped_like_the_other_kernels():
     (65, 96, 24, 3, 32, [65, 65, 65]),               # more than sixteen rows, three pieces: lanes shared by column segments
     (41, 4352, 2052, 5, 128, [1, 1, 18, 26, 41]),    # four pieces per lane, groups of one to three batches of rows, shares by the average rows
     (40, 8192, 100, 8, 256, [4, 9, 9, 13, 30, 30, 31, 40]),
+    (20, 2816, 840, 40, 256, None),                  # half as many rows as experts: shares of two column blocks, the last one of one
 ])
 def test_a8w4_column_shares_and_row_blocks(m, k, n, e, g, gl):
     """One float16 rounding (2^-11, or half its smallest step) of the exact value and at most 16 float32 roundings (a product with
