@@ -885,7 +885,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_a16w8_rows_kernel(const Gmm
   const int strip = blockIdx.x;
   // (grid.y enumerates the chunks that hold rows, group after group: a slot past the last one has nothing to do)
   int grp, mc, g_start, g_end;
-  if (!chunk_of_slot(p, (int)blockIdx.y, S::kRows, lane, grp, mc, g_start, g_end)) return;
+  if (!chunk_of_slot<false>(p, (int)blockIdx.y, S::kRows, lane, grp, mc, g_start, g_end)) return;
   const int m0 = g_start + mc * S::kRows;
   const int chunk_rows = min(S::kRows, g_end - m0);
 
@@ -1178,7 +1178,7 @@ __global__ void __launch_bounds__(ST_THREADS, 2) gmm_a16w8_rows32_kernel(const G
   const int strip = blockIdx.x;
   // (grid.y enumerates the chunks that hold rows, group after group: a slot past the last one has nothing to do)
   int grp, mc, g_start, g_end;
-  if (!chunk_of_slot(p, (int)blockIdx.y, S::kRows, lane, grp, mc, g_start, g_end)) return;
+  if (!chunk_of_slot<false>(p, (int)blockIdx.y, S::kRows, lane, grp, mc, g_start, g_end)) return;
   const int m0 = g_start + mc * S::kRows;
   const int chunk_rows = min(S::kRows, g_end - m0);
 
