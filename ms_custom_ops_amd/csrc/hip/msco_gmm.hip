@@ -688,7 +688,9 @@ void choose_plan(msco_gmm_op *op) {
       // 21.5; 3 rows, 7552 x 4256 15.4 -> 14.0), 64 x 128 0.991 (41 rows, 2720 x 1200 10.9 -> 9.6).  Its rounds are those of an XCD, which takes an
       // eighth of the tiles, rounded up, with all their slices: three slices of 81 to 85 tiles are 33 workgroups for 32 CUs.  Counted over the
       // chip that was one round.  7778 random shapes that this changes, 0.83 of the time, one slower by more than 0.05: 64 x 128, three
-      // slices -> two 0.77 (72 rows, 2688 x 5280, [E,N,K] 15.6 -> 11.3), 32 x 128, 62 to 64 tiles, three -> four 0.95.
+      // slices -> two 0.77 (72 rows, 2688 x 5280, [E,N,K] 15.6 -> 11.3), 32 x 128, 62 to 64 tiles, three -> four 0.95.  Four slices of 57 to
+      // 64 32 x 128 tiles leave no CU of an XCD idle, and the exchange is 2 dearer: 260 shapes, four slices against three K = 3000 .. 4000 1.045
+      // (23 rows, 3616 x 8048 11.6 / 11.0), to 5000 0.996, to 6500 0.95, beyond 0.93.
       const int cus = or_default(tuning().tile_target_wgs, num_cus > 0 ? num_cus : kTileTargetWorkgroups);
       const int cap = (int)std::max<int64_t>(1, ((k + 63) / 64) / kTileMinSlabs);
       // (several groups, more than 11 and up to 16 rows each on average: all of them hold rows, some of them more than a tile, and a second tile per CU costs what it
@@ -699,9 +701,11 @@ void choose_plan(msco_gmm_op *op) {
         const int64_t slabs = ((k + 63) / 64 + sl - 1) / sl;
         const bool one_small = e == 1 && (few || op->tile_cfg == TILE_64x128);
         const int64_t xcd_cus = std::max(1, cus / kNumXcd);
-        const int64_t rounds = e == 1 ? ((t + kNumXcd - 1) / kNumXcd * sl + xcd_cus - 1) / xcd_cus : (t * sl + cus - 1) / cus;
+        const int64_t xcd_tiles = (t + kNumXcd - 1) / kNumXcd;
+        const int64_t rounds = e == 1 ? (xcd_tiles * sl + xcd_cus - 1) / xcd_cus : (t * sl + cus - 1) / cus;
         const int64_t fifths = few && rounds > 1 ? (rounds + 1) / 2 * (e == 1 || full_groups ? 8 : 6) : rounds * 5;
-        const int64_t exchange = sl <= 1 ? 0 : one_small ? (int64_t)(2 + bm * bn / 2048) * sl + 2 : (int64_t)(4 + bm * bn / 2048) * sl - 2;
+        const int64_t full_xcd = e == 1 && few && sl == 4 && xcd_tiles * sl == xcd_cus ? 2 : 0;
+        const int64_t exchange = sl <= 1 ? 0 : one_small ? (int64_t)(2 + bm * bn / 2048) * sl + 2 + full_xcd : (int64_t)(4 + bm * bn / 2048) * sl - 2;
         return fifths * (slabs + 10 + exchange);
       };
       int want = 1;

@@ -23,7 +23,8 @@ def _plan(m, k, n, e=1, nk=False, packed=False):
     (72, 2688, 5120, True, False, "w8a8_tile_64x128", 3), (72, 2688, 5280, True, False, "w8a8_tile_64x128", 2),      # 80 and 84 tiles
     (72, 2688, 5280, False, True, "w8a8_tile_64x128", 2), (244, 2912, 2688, True, False, "w8a8_tile_64x128", 2),
     (40, 16384, 6144, False, True, "w8a8_tile_64x128", 5), (40, 16384, 6272, False, True, "w8a8_tile_64x128", 4),      # 48 and 49
-    (19, 3296, 8192, False, False, "w8a8_skinny_tile_32x128", 4), (19, 3296, 8320, False, False, "w8a8_skinny_tile_32x128", 3),   # 64 and 65
+    (19, 4864, 8192, False, False, "w8a8_skinny_tile_32x128", 4), (19, 4864, 8320, False, False, "w8a8_skinny_tile_32x128", 3),   # 64 and 65
+    (19, 4800, 8192, False, False, "w8a8_skinny_tile_32x128", 3), (23, 3616, 8048, True, False, "w8a8_skinny_tile_32x128", 3),    # four slices fill an XCD: 75 K blocks and fewer
     (4, 2272, 10240, False, False, "w8a8_skinny_tile_32x128", 3), (4, 2272, 10448, False, False, "w8a8_skinny_tile_32x128", 2)])
 def test_one_group(m, k, n, nk, packed, kernel, split):
     assert _plan(m, k, n, nk=nk, packed=packed) == (kernel, split)
