@@ -412,7 +412,12 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     const int64_t avg = (m + e - 1) / e, rows = avg + avg / 10;
     if (bits == 4 && avg + avg / 2 <= 64 && (n + best.cols - 1) / best.cols * std::min(e, m) * ((rows + 127) / 128) * best.split * 2 <= cus) return;
     // (the kernels for smaller chunks keep what is not clearly better here; 128-row chunks are always better off)
-    if (bits == 8 && family_fits && op->stream_tch <= 4 && 0.9 * rows_small_us(m, k, n, e, cus, op->stream_tch, is_packed(d)) < us) return;
+    // (nor what the model prices too low: a few rows on strips of 512 that N fills to less than four fifths, 17 shapes 1.13 of the time of the
+    // smaller chunks (128 experts, 2463 rows, 3168 x 640 1.49; where N fills them 40 shapes 0.98), and one row block per group on more than two
+    // 256-column workgroups per CU, 26 shapes 1.08 (16 experts, 179 rows, 1760 x 8640 50.6 -> 59.5 us; two row blocks and more 0.87))
+    const int64_t strips = (n + best.cols - 1) / best.cols, wgs = strips * std::min(e, m) * ((rows + 127) / 128) * best.split;
+    const bool priced_low = best.cols == 512 ? rows <= 24 && n * 5 < strips * 512 * 4 : best.sets == 1 && rows <= 16 && wgs > 2 * cus;
+    if (bits == 8 && family_fits && op->stream_tch <= 4 && (priced_low || 0.9 * rows_small_us(m, k, n, e, cus, op->stream_tch, is_packed(d)) < us)) return;
   }
   op->family = FAM_ROWS16;
   op->strip_cols = best.cols;
