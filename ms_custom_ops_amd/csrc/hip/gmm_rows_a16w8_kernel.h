@@ -41,7 +41,7 @@
 //     the other: a weight strip comes into one L2 once.
 //
 // What bounds it (4096 x 4096 x 11008, three rounds of tiles): 327 us = 1.13 PFLOP/s before the epilogue's
-// branches went (8 x 512 rows, 4096 x 14336: 456 -> 430 us with them gone).  Per 64 K positions and round 1.38 us, of which
+// branches went (8 x 512 rows, 4096 x 14336: 456 -> 437 us with them gone).  Per 64 K positions and round 1.38 us, of which
 // the MFMAs alone 0.94 (2048 cycles), fragment reads 0.05, conversions 0.17, operand requests 0.22; and 21 .. 25 us per round that do not
 // depend on K (first requests, epilogue, stores in step on all CUs).  Two workgroups of four waves x 256 columns per CU
 // overlap those but request x twice: 349 us.  The barrier in the middle of a block with the fragment reads running on: the same.

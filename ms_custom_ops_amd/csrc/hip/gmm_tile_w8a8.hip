@@ -3,8 +3,8 @@
 // One workgroup computes one BM x BN output tile of one group with v_mfma_i32_32x32x32_i8 (the int8
 // MFMA that issues at full rate on this part; measured: the 16x16x64 form sustains about half of it).
 // The large configuration uses 8 wavefronts (2 x 4, two per SIMD, a 128 x 64 sub-tile of accumulators
-// each), so that one wave's LDS reads and barrier waits are covered by the other wave's MFMAs; the
-// small configurations use 4 wavefronts (2 x 2).
+// each), so that one wave's LDS reads and barrier waits are covered by the other wave's MFMAs; 64 x 128
+// and 128 x 128 tiles use 4 wavefronts (2 x 2), 256 columns of up to 128 rows 4 side by side, 32 x 128 tiles 2.
 //
 //   * Tile scheduling on the device.  The tile -> (group, m-tile, n-tile) mapping is computed by
 //     walking group_list, so the host never reads it; the grid is sized from an upper bound and
