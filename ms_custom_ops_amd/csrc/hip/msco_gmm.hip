@@ -440,9 +440,10 @@ int64_t few_row_tiles(int64_t m, int64_t n, int64_t e) { return groups_hit(m, e)
 //   little to walk, 64 x 128 with 64-byte slabs and three workgroups per CU (16 experts, 162 rows, 864 x 4112 22.7 -> 15.3, 32 x 256: 18.8).
 // The decode kernels keep what leaves most CUs idle whatever the tile, because their 16 waves split K inside a workgroup: a handful of
 // rows over dozens of experts (64 experts, 1 row, 2272 x 800: 8.3 against 9.9; 5 rows, 800 x 1824: 8.0 against 8.8), one group of ten
-// tiles and a long K (1 row, 3744 x 1120: 9.5 against 10.4), and several groups where that is K / 192 tiles, at least ten (2 rows over 16 experts,
-// 7712 x 656: 13.6 against 16.9; 3082 such [E,K,N] shapes 0.93 of the time of 32 x 128 tiles, 0.85 to 0.97 from few tiles to the line; 1288 of
-// them had become slower by more than 5 % with those, 14 are left).  They also keep K below 512 (not measured).  On [E,N,K] weights several groups take 64 x 128
+// tiles and a long K (1 row, 3744 x 1120: 9.5 against 10.4), and several groups where that is K / 192 tiles, at least ten, of up to two rows for five
+// experts (2 rows over 16, 7712 x 656: 13.6 against 16.9; 157 [E,K,N] shapes of up to 0.3 rows per expert 0.93 of the time of 32 x 128 tiles, 64 of three
+// rows over eight 1.00; with more rows those have more tiles to share K: up to one row per expert 1.06, one to eleven 1.15; 63 rows over 8, 7680 x
+// 528: 20.8 against 15.5).  They also keep K below 512 (not measured).  On [E,N,K] weights several groups take 64 x 128
 // tiles already, which are as fast (60 shapes: 0.98), but for more than 32 experts and up to 64 rows (41 rows over 64 experts, 4352 x 688: 27.9 ->
 // 20.3; 52 rows, 544 x 10576: 17.2 -> 15.3 with 64 x 128 tiles), where the decode kernels' plan dates from launches with workgroups for experts
 // without rows.
@@ -452,7 +453,7 @@ void plan_few_rows(msco_gmm_op *op, int &family) {
   if (is_packed(op->desc) || k < 512 || (e == 1 ? m > 32 : m > 16 * e)) return;
   const int64_t tiles = few_row_tiles(m, n, e);
   if (e == 1 && !nk && m <= kSkinnyRows && tiles <= 10 && k >= 2048) return;
-  if (e > 1 && ((nk && family != FAM_SKINNY) || tiles <= 10 || (!nk && family == FAM_SKINNY && tiles * 192 <= k) || (e >= 32 && m <= 5))) return;
+  if (e > 1 && ((nk && family != FAM_SKINNY) || tiles <= 10 || (!nk && family == FAM_SKINNY && tiles * 192 <= k && m * 5 <= e * 2) || (e >= 32 && m <= 5))) return;
   family = FAM_TILE;
   op->tile_cfg = tiles * 8 <= cus * 9 ? TILE_32x128 : nk || k < 1024 ? TILE_64x128 : TILE_32x256;
 }
@@ -864,8 +865,9 @@ void choose_plan(msco_gmm_op *op) {
       // on some of them: 100 rows over 16 experts, 3776 x 1440 19.6 -> 20.6).
       // A slice of K holds 128 blocks of 64 bytes, with 16-bit x 64.  Beyond 64 the 16-bit kernel would take two slices of 9 to 16 blocks
       // per wave in the code for 16, most requests of a shorter one masked: slices of at most 32 blocks, eight per wave, instead (us, two
-      // slices -> three or four: 18 rows over 16 experts, 4288 x 2320 43.9 -> 30.6; 14 rows, one group, 4288 x 8288 22.1 -> 13.8; 4 rows over 16 experts,
-      // 4352 x 1136 15.7 -> 10.1; 96 rows over 16, 6016 x 1792 49.3 -> 35.1).  Up to 64 blocks one slice is as good.
+      // slices -> three, random routings: 18 rows over 16 experts, 4288 x 2320 44.1 -> 28.8; 14 rows, one group, 4288 x 8288 21.7 -> 14.4; 4 rows over 16
+      // experts, 4352 x 1136 12.0 -> 11.1; 96 rows over 16, 6016 x 1792 48.8 -> 38.7).  Up to 64 blocks one slice is as good.  (Where the two slices are
+      // one workgroup per CU they are 3 % faster on 38 grouped shapes, but slower on others: 140 where that rule applied 1.03 of the time, one group 1.02.)
       const int64_t col_groups = (n + 15) / 16, k_blocks = (k + 63) / 64;
       const int slice_blocks = is_w8a8(d) ? 128 : 64, fewest = (int)((k_blocks + slice_blocks - 1) / slice_blocks);
       const bool short_slices = !is_w8a8(d) && fewest > 1 && k_blocks <= 32 * kMaxSplitK;

@@ -39,7 +39,8 @@ def test_several_groups_on_32_row_tiles(m, k, n, e, split):
 
 @pytest.mark.parametrize("m,k,n,e,kernel", [
     (6, 5760, 560, 128, "w8a8_skinny_16w"), (6, 5744, 560, 128, "w8a8_skinny_tile_32x128"),      # 30 tiles, 30 times 192 and less
-    (2, 7712, 656, 16, "w8a8_skinny_16w"), (2, 4576, 1136, 16, "w8a8_skinny_16w"), (2, 3072, 1136, 16, "w8a8_skinny_tile_32x128")])
+    (2, 7712, 656, 16, "w8a8_skinny_16w"), (2, 4576, 1136, 16, "w8a8_skinny_16w"), (2, 3072, 1136, 16, "w8a8_skinny_tile_32x128"),
+    (6, 7712, 656, 16, "w8a8_skinny_16w"), (7, 7712, 656, 16, "w8a8_skinny_tile_32x128"), (63, 7680, 528, 8, "w8a8_skinny_tile_32x128")])      # up to two rows for five experts
 def test_few_tiles_and_a_long_k_stay_with_the_decode_kernels(m, k, n, e, kernel):
     assert _plan(m, k, n, e)[0] == kernel
 
