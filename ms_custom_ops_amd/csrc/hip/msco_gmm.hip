@@ -395,6 +395,10 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     const int64_t k_min = rows <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : rows <= 256 ? 768 : 1280;
     if (!(k >= k_min && avg >= 48 && (tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65) && n * 100 >= strips * 512 * 85)) return;
   } else {
+    // (strips of 512 not where N fills them to less than four fifths: 512 and 256 in one round take equally long by the model, but in 118 shapes of 22 to 2000 rows
+    // a group and N = 528 .. 2464 one set on 256 takes 0.87 of the time; from four fifths on 0.97)
+    const int64_t wide = (n + 511) / 512 * 512;
+    if (n * 5 < wide * 4) best = Rows16Form{256, 1, 1};
     double us = rows16_us(m, k, n, e, cus, is_packed(d), bits, best);
     for (int sets = 1; sets <= 2; ++sets)
       for (int split = 1; split <= 4 && split <= (k + 63) / 64; ++split) {
@@ -412,11 +416,10 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     const int64_t avg = (m + e - 1) / e, rows = avg + avg / 10;
     if (bits == 4 && avg + avg / 2 <= 64 && (n + best.cols - 1) / best.cols * std::min(e, m) * ((rows + 127) / 128) * best.split * 2 <= cus) return;
     // (the kernels for smaller chunks keep what is not clearly better here; 128-row chunks are always better off)
-    // (nor what the model prices too low: a few rows on strips of 512 that N fills to less than four fifths, 17 shapes 1.13 of the time of the
-    // smaller chunks (128 experts, 2463 rows, 3168 x 640 1.49; where N fills them 40 shapes 0.98), and one row block per group on more than two
-    // 256-column workgroups per CU, 26 shapes 1.08 (16 experts, 179 rows, 1760 x 8640 50.6 -> 59.5 us; two row blocks and more 0.87))
-    const int64_t strips = (n + best.cols - 1) / best.cols, wgs = strips * std::min(e, m) * ((rows + 127) / 128) * best.split;
-    const bool priced_low = best.cols == 512 ? rows <= 24 && n * 5 < strips * 512 * 4 : best.sets == 1 && rows <= 16 && wgs > 2 * cus;
+    // (nor what the model prices too low: one row block per group on more than two 256-column workgroups per CU, 26 shapes 1.08 of the time of the
+    // smaller chunks (16 experts, 179 rows, 1760 x 8640 50.6 -> 59.5 us; two row blocks and more 0.87))
+    const int64_t wgs = (n + best.cols - 1) / best.cols * std::min(e, m) * ((rows + 127) / 128) * best.split;
+    const bool priced_low = best.cols == 256 && best.sets == 1 && rows <= 16 && wgs > 2 * cus;
     if (bits == 8 && family_fits && op->stream_tch <= 4 && (priced_low || 0.9 * rows_small_us(m, k, n, e, cus, op->stream_tch, is_packed(d)) < us)) return;
   }
   op->family = FAM_ROWS16;

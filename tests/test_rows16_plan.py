@@ -31,8 +31,9 @@ def _plan(m, k, n, e, layout="kn", bits=8, override=0):
     (816, 6336, 544, 16, "kn", 8, "a16w8_rows128x256_2", 3),
     # packed weights, two sets: 256 workgroups are a round, 288 are two
     (210, 5472, 8176, 8, "packed", 8, "a16w8_rows128x256_2", 1), (210, 5472, 8816, 8, "packed", 8, "a16w8_rows128", 1),
-    # up to 24 rows a group not on strips of 512 that N fills to less than four fifths, one row block a group not on more than two workgroups per CU
-    (2463, 3168, 832, 128, "kn", 8, "a16w8_rows128", 1), (2463, 3168, 816, 128, "kn", 8, "a16w8_skinny_rows", 1),
+    # strips of 512 where N fills them to four fifths, one row block a group not on more than two 256-column workgroups per CU
+    (11501, 3328, 832, 128, "kn", 8, "a16w8_rows128", 1), (11501, 3328, 816, 128, "kn", 8, "a16w8_rows128x256", 1),
+    (11501, 3328, 832, 128, "kn", 4, "a16w4_rows128", 1), (11501, 3328, 816, 128, "kn", 4, "a16w4_rows128x256", 1),
     (103, 1856, 2912, 8, "packed", 8, "a16w8_rows128x256", 1), (179, 1760, 8640, 16, "packed", 8, "a16w8_stream_rows", 1),
     # more than 65535 pairs of expert and chunk: beyond the grids of the kernels with smaller chunks
     (200000, 1024, 512, 1024, "kn", 8, "a16w8_rows128", 1), (200000, 1024, 512, 1024, "kn", 4, "a16w4_rows128x256", 1)])
