@@ -395,6 +395,7 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     const int64_t k_min = rows <= 128 ? (is_packed(d) ? 1024 : 2048) : is_packed(d) ? 512 : rows <= 256 ? 768 : 1280;
     if (!(k >= k_min && avg >= 48 && (tiles >= 2 * cus || tiles * 100 >= rounds * cus * 65) && n * 100 >= strips * 512 * 85)) return;
   } else {
+    const int64_t avg = (m + e - 1) / e, rows = avg + avg / 10;
     // (strips of 512 not where N fills them to less than four fifths: 512 and 256 in one round take equally long by the model, but in 118 shapes of 22 to 2000 rows
     // a group and N = 528 .. 2464 one set on 256 takes 0.87 of the time; from four fifths on 0.97)
     const int64_t wide = (n + 511) / 512 * 512;
@@ -410,10 +411,13 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
           best = f;
         }
       }
+    // (two sets of waves hide one another's waits where a CU has one workgroup; in more than a round, counted with a mean routing, one set takes
+    // 0.93 of their time: 276 shapes, 8- and 4-bit weights; 5268 rows over 8 experts, 2688 x 4112 165 -> 145 us)
+    const int64_t groups = std::min(e, m);
+    if (best.sets == 2 && best.split == 1 && (double)((n + 255) / 256 * groups) * expected_row_tiles((double)m / (double)groups, 128.0) > 1.02 * (double)cus) best.sets = 1;
     // (4-bit weights that the register-transpose kernels can take: strips of 256 columns and 32-row chunks there are twice as many workgroups, which
     // counts where these fill no more than half of the chip: 8 experts, 330 rows, 4416 x 4096 39 against 48 us; 8138 random shapes of 30 to 42 rows per
     // group 0.83 of the time of what the model picked, 0.79 with a quarter of the chip, 0.85 with half of it)
-    const int64_t avg = (m + e - 1) / e, rows = avg + avg / 10;
     if (bits == 4 && avg + avg / 2 <= 64 && (n + best.cols - 1) / best.cols * std::min(e, m) * ((rows + 127) / 128) * best.split * 2 <= cus) return;
     // (the kernels for smaller chunks keep what is not clearly better here; 128-row chunks are always better off)
     // (nor what the model prices too low: one row block per group on more than two 256-column workgroups per CU, 26 shapes 1.08 of the time of the

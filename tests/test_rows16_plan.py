@@ -29,6 +29,9 @@ def _plan(m, k, n, e, layout="kn", bits=8, override=0):
     # strips of 512 columns where they fill the chip, of 256 where they do not, two sets of waves with a K split where those do not either
     (4096, 4096, 14336, 8, "packed", 8, "a16w8_rows128", 1), (131072, 1024, 1024, 128, "packed", 8, "a16w8_rows128x256", 1),
     (816, 6336, 544, 16, "kn", 8, "a16w8_rows128x256_2", 3),
+    # two sets of waves in one round (256 workgroups), one set beyond
+    (1600, 4096, 4096, 8, "kn", 8, "a16w8_rows128x256_2", 1), (1600, 4096, 4112, 8, "kn", 8, "a16w8_rows128x256", 1),
+    (1600, 4096, 4096, 8, "kn", 4, "a16w4_rows128x256_2", 1), (1600, 4096, 4112, 8, "kn", 4, "a16w4_rows128x256", 1),
     # packed weights, two sets: 256 workgroups are a round, 288 are two
     (210, 5472, 8176, 8, "packed", 8, "a16w8_rows128x256_2", 1), (210, 5472, 8816, 8, "packed", 8, "a16w8_rows128", 1),
     # strips of 512 where N fills them to four fifths, one row block a group not on more than two 256-column workgroups per CU
