@@ -19,7 +19,9 @@ INCLUDE = os.path.join(REPO_DIR, "include")
 
 BACKEND_LIB = os.path.join(LIB_DIR, "libmsco_gmm.so")
 PROBES_LIB = os.path.join(LIB_DIR, "libmsco_probes.so")   # measurement aids: not part of the operator library
-HIP_SOURCES = ["gmm_tile_w8a8.hip", "gmm_tile4_w8a8.hip", "gmm_tile4m_w8a8.hip", "gmm_rows_w8a8.hip", "gmm_skinny_w8a8.hip", "gmm_generic.hip", "gmm_stream.hip", "msco_gmm.hip", "moe_routing.hip", "gmm_w4.hip", "gmm_regt.hip", "gmm_rows_a16w8.hip",
+# (longest first: the persistent kernel's instantiations)
+TILE4M_SOURCES = ["gmm_tile4m_%s%s.hip" % (layout, out) for out in ("_bf16", "_f16", "_bf16_silu", "_f16_silu", "") for layout in ("packed", "nk", "kn")]
+HIP_SOURCES = TILE4M_SOURCES + ["gmm_tile_w8a8.hip", "gmm_tile4_w8a8.hip", "gmm_tile4m_w8a8.hip", "gmm_rows_w8a8.hip", "gmm_skinny_w8a8.hip", "gmm_generic.hip", "gmm_stream.hip", "msco_gmm.hip", "moe_routing.hip", "gmm_w4.hip", "gmm_regt.hip", "gmm_rows_a16w8.hip",
                "gmm_rows_a16w8_bf16_kn.hip", "gmm_rows_a16w8_f16_packed.hip", "gmm_rows_a16w8_f16_kn.hip",
                "gmm_rows_a16w4_bf16.hip", "gmm_rows_a16w4_f16.hip"]
 PROBE_SOURCES = ["probes.hip"]
@@ -75,14 +77,14 @@ ATTRIBUTION_BUILDS = {"noepi": 1, "nomfma": 2, "nomfma_noepi": 3, "nostore": 4,
 
 def build_attribution(verbose: bool = False):
     """Measurement builds of the backend, never the shipped one: lib/attr/libmsco_gmm_<name>.so is libmsco_gmm.so with
-    one part of the persistent tile kernels taken out (MSCO_TILE4_ATTR in gmm_tile4_w8a8.hip and gmm_tile4m_w8a8.hip), so that timing the rest
+    one part of the persistent tile kernels taken out (MSCO_TILE4_ATTR in gmm_tile4_w8a8.hip and gmm_tile4m_kernel.h), so that timing the rest
     says what that part costs.  Select one with MSCO_GMM_LIB=<path>; their results are wrong on purpose."""
     build_backend(verbose)
     hipcc = _hipcc()
     hip_dir = os.path.join(CSRC, "hip")
     out_dir = os.path.join(LIB_DIR, "attr")
     os.makedirs(out_dir, exist_ok=True)
-    tile4 = ("gmm_tile4_w8a8.hip", "gmm_tile4m_w8a8.hip")
+    tile4 = ["gmm_tile4_w8a8.hip"] + TILE4M_SOURCES
     others = [os.path.join(OBJ_DIR, s.replace(".hip", ".o")) for s in HIP_SOURCES if s not in tile4]
 
     def build_one(item):

@@ -7,9 +7,20 @@
 
 namespace msco {
 
+// Tile shapes of the persistent four-wave kernel: 32 xb rows x 32 wb columns.
+struct T4mShape { int xb, wb; };
+constexpr int T4M_SHAPES = 6;
+constexpr T4mShape kT4mShape[T4M_SHAPES] = {{8, 8}, {7, 8}, {6, 8}, {5, 8}, {4, 8}, {9, 7}};   // (the last one not on [E,K,N])
+// The shape of a launch: an index into kT4mShape, or negative: by the groups, which the device counts, and these modelled times
+// (t4m_pick in gmm_tile4m_kernel.h).  (Not part of GmmParams: every kernel would request them.)
+struct T4mPick {
+  int shape;
+  float us[T4M_SHAPES], idle;   // us of a round (0: no such shape); the share of a round that is free where a CU has no tile
+};
+
 enum TileCfg : int {
   TILE_256x256 = 0, TILE_128x128 = 1, TILE_64x128 = 2, TILE_128x256 = 3,
-  TILE_256x256_W4 = 4,   // persistent, four wavefronts with 128 x 128 accumulators each: gmm_tile4m_w8a8.hip (16 x 16 x 64 MFMAs)
+  TILE_256x256_W4 = 4,   // persistent, four wavefronts with accumulators for a quarter of the tile each: gmm_tile4m_kernel.h (16 x 16 x 64 MFMAs); T4mPick
   TILE_256x256_W4_MFMA32 = 5,   // the same on 32 x 32 x 32 MFMAs: gmm_tile4_w8a8.hip (never planned; kept to be measured against)
   TILE_ROWS256 = 6,   // packed weights only: chunks of up to 256 rows x strips of 256 columns, x through LDS, weights straight into MFMA operands: gmm_rows_w8a8.hip
   TILE_ROWS128 = 7,   // the same with chunks of up to 128 rows and two workgroups per CU
@@ -22,10 +33,10 @@ enum TileCfg : int {
 };
 
 // MFMA tile kernel for W8A8 (prefill shapes).  nk: weights stored [E,N,K]; packed: the packed layout (nk is ignored).
-hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool packed, hipStream_t stream);
+hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool packed, const T4mPick &pick, hipStream_t stream);   // pick: TILE_256x256_W4 only
 hipError_t launch_tile_a8w4(const GmmParams &p, int tile_cfg, hipStream_t stream);   // int8 x, 4-bit weights [E,K,N/2]
 const char *tile_cfg_name(int tile_cfg);
-hipError_t launch_tile4m_w8a8(const GmmParams &p, int layout, hipStream_t stream);  // layout 0 [E,N,K], 1 packed, 2 [E,K,N] (N % 16 == 0)
+hipError_t launch_tile4m_w8a8(const GmmParams &p, const T4mPick &pick, int layout, hipStream_t stream);  // layout 0 [E,N,K], 1 packed, 2 [E,K,N] (N % 16 == 0)
 hipError_t launch_tile4_w8a8(const GmmParams &p, int layout, hipStream_t stream);   // layout 0 [E,N,K], 1 packed, 2 [E,K,N] (N % 16 == 0)
 void tile_cfg_dims(int tile_cfg, int *bm, int *bn);
 // packed weights, several groups of a few dozen to a few hundred rows: chunks of 16 rbmax rows (rbmax = 8, 10 or 16), see gmm_rows_w8a8.hip;

@@ -74,6 +74,7 @@ struct T4Tile {
 // would put loads into the middle of the operand stream, and vector loads complete in order.
 // Order inside a group: panels of 8 m-tiles; inside a panel n-tile major, m-tile minor, so that
 // workgroups that run side by side share one streamed weight panel.
+template <int BM = T4_BM, int BN = T4_BN>
 __device__ __forceinline__ T4Tile t4_locate(const int *meta_end, const int *meta_upto, int e, int lid, int total,
                                             int n_tiles, int lane) {
   T4Tile t{0, 0, 0, 0, 0};
@@ -94,15 +95,15 @@ __device__ __forceinline__ T4Tile t4_locate(const int *meta_end, const int *meta
     }
   }
   constexpr int PANEL = 8;
-  const int m_tiles = (t.g_end - g_start + T4_BM - 1) / T4_BM;
+  const int m_tiles = (t.g_end - g_start + BM - 1) / BM;
   const int panel_tiles = PANEL * n_tiles;
   const int panel = t_in_group / panel_tiles;
   const int in_panel = t_in_group - panel * panel_tiles;
   const int panel_m = max(1, min(PANEL, m_tiles - panel * PANEL));
   const int nt = in_panel / panel_m;
   const int mt = panel * PANEL + in_panel % panel_m;
-  t.m0 = g_start + mt * T4_BM;
-  t.n0 = nt * T4_BN;
+  t.m0 = g_start + mt * BM;
+  t.n0 = nt * BN;
   return t;
 }
 

@@ -1,0 +1,6 @@
+// Persistent four-wave tile kernel, [E,K,N] weights, float16 output, no activation: see gmm_tile4m_kernel.h.
+#include "gmm_tile4m_kernel.h"
+
+namespace msco {
+hipError_t tile4m_kn_f16(const GmmParams &p, const T4mPick &pick, hipStream_t s) { return t4m_launch<1, 2, 0, true>(p, pick, s); }
+}  // namespace msco

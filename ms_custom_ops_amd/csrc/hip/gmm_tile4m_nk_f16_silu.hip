@@ -1,0 +1,6 @@
+// Persistent four-wave tile kernel, [E,N,K] weights, float16 output, silu and fast gelu: see gmm_tile4m_kernel.h.
+#include "gmm_tile4m_kernel.h"
+
+namespace msco {
+hipError_t tile4m_nk_f16_silu(const GmmParams &p, const T4mPick &pick, hipStream_t s) { return t4m_launch<1, 0, 2, true>(p, pick, s); }
+}  // namespace msco

@@ -713,14 +713,14 @@ static hipError_t launch_32_rows(const GmmParams &p, int bn, int layout, hipStre
 
 // nk: weights stored [E,N,K]; packed: the blocked layout; neither: [E,K,N] (N a multiple of 16, which the plan's
 // alignment rule guarantees for every MFMA kernel)
-hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool packed, hipStream_t stream) {
+hipError_t launch_tile_w8a8(const GmmParams &p, int tile_cfg, bool nk, bool packed, const T4mPick &pick, hipStream_t stream) {
   const int layout = packed ? 1 : nk ? 0 : 2;
   if (layout == 2 && p.n % 16 != 0) return hipErrorInvalidValue;
   // the persistent kernel needs at least four 128-byte K slabs per tile and a group table that fits in LDS; what it
   // cannot take runs the eight-wave kernel of the same tile shape
   if (tile_cfg == TILE_256x256_W4 || tile_cfg == TILE_256x256_W4_MFMA32) {
     if (p.k >= 512 && p.e <= 1024)
-      return tile_cfg == TILE_256x256_W4 ? launch_tile4m_w8a8(p, layout, stream) : launch_tile4_w8a8(p, layout, stream);
+      return tile_cfg == TILE_256x256_W4 ? launch_tile4m_w8a8(p, pick, layout, stream) : launch_tile4_w8a8(p, layout, stream);
     tile_cfg = TILE_256x256;
   }
   if (tile_cfg == TILE_ROWS256 || tile_cfg == TILE_ROWS128 || tile_cfg == TILE_ROWS160)

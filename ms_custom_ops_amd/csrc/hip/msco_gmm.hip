@@ -36,7 +36,8 @@ enum Override : int {
   OV_ROWS16_256 = 15,  // the same with strips of 256 columns
   OV_ROWS16_256X2 = 16, // ... and two sets of waves that take turns at the K blocks
   OV_TILE_32x128 = 17,  // a few rows on [E,K,N] and [E,N,K] weights (packed: 64 x 128 tiles)
-  OV_TILE_32x256 = 18   // ... on [E,K,N] weights ([E,N,K]: as 17)
+  OV_TILE_32x256 = 18,  // ... on [E,K,N] weights ([E,N,K]: as 17)
+  OV_W4_128 = 19, OV_W4_160 = 20, OV_W4_192 = 21, OV_W4_224 = 22, OV_W4_288 = 23   // the persistent kernel with tiles of that many rows
 };
 
 constexpr int64_t kSkinnyMaxRows = 64;   // total rows up to which the weight-streaming kernel is planned
@@ -87,6 +88,7 @@ struct msco_gmm_op {
   int64_t m = 0, k = 0, n = 0, e = 0;
   int family = FAM_NONE;
   int tile_cfg = 0;
+  int tile_shape = 0;        // persistent tile kernel: index into kT4mShape, negative: picked on the device from the groups
   int split_k = 1;
   int skinny_wide16 = 0;
   int skinny_cols = kSkinnyCols;
@@ -129,7 +131,7 @@ int check_desc(const msco_gmm_desc &d) {
   if (d.group_list_dtype != MSCO_DT_NONE && d.group_list_dtype != MSCO_DT_I32 && d.group_list_dtype != MSCO_DT_I64)
     return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_type != 0 && d.group_list_type != 1) return MSCO_ERR_INVALID_ARG;
-  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_TILE_32x256) return MSCO_ERR_INVALID_ARG;
+  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_W4_288) return MSCO_ERR_INVALID_ARG;
   if (d.weight_layout != MSCO_WL_ROW_MAJOR && d.weight_layout != MSCO_WL_PACKED) return MSCO_ERR_INVALID_ARG;
   if (d.force_split_k < 0) return MSCO_ERR_INVALID_ARG;
   if (d.act_type < MSCO_ACT_NONE || d.act_type > MSCO_ACT_SILU) return MSCO_ERR_INVALID_ARG;
@@ -507,6 +509,134 @@ bool plan_one_round(msco_gmm_op *op) {   // true: K is not to be split
   return false;
 }
 
+// Mean number of bm-row tiles of a group that holds `avg` rows on average and, in a random routing, scatters by about the root
+// of that; and their variance.
+struct TileMoments { double mean, var; };
+TileMoments row_tile_moments(double avg, double bm) {
+  const double sd = std::sqrt(std::max(avg, 1e-9));
+  double t = std::max(0.0, std::floor((avg - 5.0 * sd) / bm)), mean = t, square = t * t;
+  for (double rows = t * bm + 0.5; rows < avg + 5.0 * sd; rows += bm, t += 1.0) {
+    const double p = 0.5 * std::erfc((rows - avg) / (sd * std::sqrt(2.0)));   // P(more than t tiles)
+    mean += p;
+    square += p * (2.0 * t + 1.0);
+  }
+  return {std::max(mean, 1e-3), std::max(square - mean * mean, 0.0)};
+}
+
+// Rounds that tiles of bm rows x bn columns make, one per CU, and the share of them that the CUs are busy: `busy` is tiles / CUs.
+struct TileRounds { double rounds, busy; };
+TileRounds even_rounds(int64_t m, int64_t n, int64_t e, int64_t bm, int64_t bn, int64_t cus) {
+  const double nt = (double)((n + bn - 1) / bn);
+  if (e == 1) {
+    const int64_t t = (m + bm - 1) / bm * (int64_t)nt;
+    return {(double)((t + cus - 1) / cus), (double)t / (double)cus};
+  }
+  const double groups = (double)std::min(e, m);
+  const TileMoments g = row_tile_moments((double)m / groups, (double)bm);
+  const double mean = g.mean * groups, sd = std::sqrt(g.var * groups);
+  double rounds = 0.0;
+  for (double r = 0.0;; r += 1.0) {   // sum of P(more than r rounds): the row tiles are whole ones
+    const double need = std::floor((double)cus * r / nt) + 0.5;
+    const double p = sd < 1e-6 ? (mean > need ? 1.0 : 0.0) : 0.5 * std::erfc((need - mean) / (sd * std::sqrt(2.0)));
+    if (p < 1e-3) break;
+    rounds += p;
+  }
+  return {std::max(rounds, 1.0), mean * nt / (double)cus};
+}
+// ... with a popularity that falls as 1 / rank^z; groups of up to `lo` rows belong to another launch.
+TileRounds skewed_rounds(int64_t m, int64_t n, int64_t e, int64_t bm, int64_t bn, int64_t cus, double z, double lo) {
+  double sum = 0.0, t = 0.0;
+  for (int64_t i = 1; i <= e; ++i) sum += std::pow((double)i, -z);
+  for (int64_t i = 1; i <= e; ++i) {
+    const double avg = (double)m * std::pow((double)i, -z) / sum;
+    if (avg > lo) t += avg > 0.5 * (double)bm ? avg / (double)bm + 0.5 : std::min(avg, 1.0);
+  }
+  t *= (double)((n + bn - 1) / bn) / (double)cus;
+  return {std::max(1.0, t + 0.5), t};
+}
+
+// The persistent kernel on tiles of other shapes than 256 x 256 (kT4mShape), against each other and against the 128 x 256 and 128 x 128
+// tiles, by a model of the time in us: rounds of one tile per CU, each a part per 128-byte K slab and a fixed one; CUs without a tile
+// in the last round leave the others more of the clock and of the L2, hence `idle`.  The operand stream of a CU is what 512 rows of
+// either side take and the matrix pipe is busy for 64 blocks per wave, so a lower tile is dearer per product but wastes
+// less: of a group's last row tile, and of the last round.  Fitted to 1160 random shapes (1 to 128 groups, 100 rows per group to
+// 16384 rows, K = 512 .. 8192, N = 512 .. 14336, even and skewed routings, three layouts), every tile shape measured on all of them: off by
+// 6 .. 8 % (rms).  One group, picked here: 0.91 of the time of 256 x 256 tiles where those were planned.  Several: the device picks, as it
+// alone knows how even they are (t4m_pick).  us, before -> now: one group of 2048 rows, 4096 x 11008, [E,N,K] 94 -> 83 (192 x 256; 344 tiles
+// made two rounds on 172 CUs); 8 experts, 256 rows on average, 4096 x 14336, packed 160 -> 123 (288 x 224: 512 tiles for 672).
+// 128 x 256 and 128 x 128 tiles give way where the least time, over even and skewed routings, is 0.95 of theirs ([E,K,N]: 0.90, its model of them is off by
+// 7 %): 0.94 / 0.84 (packed), 0.86 / 0.82 ([E,N,K]), 0.92 ([E,K,N]) of their time; one group of 2037 rows, 3040 x 2896, [E,N,K] 34 -> 29.
+struct TileTime { double launch, idle, slab, fixed; };
+struct TileTimes { double launch, idle, slab[T4M_SHAPES], fixed[T4M_SHAPES]; TileTime tall, small; };   // small, tall: the 128 x 128 and 128 x 256 tiles
+constexpr TileTimes kTileTimes[3] = {   // [E,K,N], [E,N,K], packed
+    {5.3, 0.32, {1.416, 1.268, 1.126, 1.019, 0.864, 0.0}, {7.3, 6.6, 5.7, 4.65, 4.0, 0.0}, {7.7, 0.38, 1.019, 0.0}, {5.4, 0.45, 0.591, 1.5}},
+    {6.0, 0.33, {1.393, 1.205, 1.081, 0.974, 0.853, 1.363}, {6.7, 5.9, 5.0, 4.1, 3.2, 6.8}, {3.7, 0.34, 1.163, 4.0}, {4.6, 0.39, 0.599, 1.3}},
+    {5.6, 0.32, {1.322, 1.141, 0.986, 0.880, 0.750, 1.301}, {7.65, 7.3, 6.35, 5.4, 4.35, 8.0}, {3.9, 0.35, 0.902, 4.4}, {6.1, 0.58, 0.560, 0.6}}};
+
+bool tile_shapes_fit(const msco_gmm_desc &d) {   // shapes other than 256 x 256 are built for these outputs only
+  return d.out_dtype != MSCO_DT_I32 && (d.act_type == ACT_NONE || d.act_type == ACT_SILU || d.act_type == ACT_FAST_GELU);
+}
+
+void tile_shape_times(const msco_gmm_op *op, float *round_us, float *idle) {
+  const TileTimes &t = kTileTimes[layout_of(op->desc)];
+  for (int j = 0; j < T4M_SHAPES; ++j) round_us[j] = (float)((double)(2 * ((op->k + 255) / 256)) * t.slab[j] + t.fixed[j]);
+  *idle = (float)t.idle;
+}
+
+void plan_tile_shape(msco_gmm_op *op) {
+  const msco_gmm_desc &d = op->desc;
+  const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
+  const bool tall = op->tile_cfg == TILE_128x256, small = op->tile_cfg == TILE_128x128;
+  // (groups of 100 rows leave too much of a tile empty: 128 experts, 2576 columns, 108 rows 1.03, 32 experts, 1440 columns, 102 rows 1.15)
+  if (!(op->tile_cfg == TILE_256x256_W4 || tall || small) || k < 512 || e > 1024 || !tile_shapes_fit(d) || ((tall || small) && e > 1 && m < 160 * e)) return;
+  if (e > 1 && op->tile_cfg == TILE_256x256_W4) {
+    op->tile_shape = -1;
+    return;
+  }
+  const TileTimes &t = kTileTimes[layout_of(d)];
+  const double lo = e >= 16 && (is_packed(d) || d.transpose_b == 0) ? 64.0 : 0.0;   // (the second launch takes them)
+  float round_us[T4M_SHAPES], idle;
+  tile_shape_times(op, round_us, &idle);
+  // the least time of the shapes, for an even routing (z = 0) and for skewed ones
+  int best = 0;
+  double best_tiles = 0.0;
+  auto rounds = [&](int64_t bm, int64_t bn, double z, double from) {
+    return z == 0.0 ? even_rounds(m, n, e, bm, bn, cus) : skewed_rounds(m, n, e, bm, bn, cus, z, from);
+  };
+  auto least = [&](double z) {
+    double us = 0.0;
+    for (int j = 0; j < T4M_SHAPES; ++j) {
+      if (t.slab[j] <= 0.0) continue;
+      const TileRounds r = rounds(32 * kT4mShape[j].xb, 32 * kT4mShape[j].wb, z, lo);
+      const double u = t.launch + ((1.0 - idle) * r.rounds + idle * r.busy) * (double)round_us[j];
+      if (j == 0) us = u * (op->tile_cfg == TILE_256x256_W4 ? 0.97 : 1.0);
+      if (j == 0 || u < us) {
+        us = j == 0 ? us : u;
+        if (z == 0.0) { best = j; best_tiles = r.busy * (double)cus; }
+      }
+    }
+    return us;
+  };
+  double now = 0.0;
+  auto other = [&](double z) {
+    const TileTime &o = tall ? t.tall : t.small;
+    const TileRounds r = rounds(128, tall ? 256 : 128, z, 0.0);
+    return o.launch + ((1.0 - o.idle) * r.rounds + o.idle * r.busy) * ((double)k / 128.0 * o.slab + o.fixed);
+  };
+  double us = least(0.0);
+  if (tall || small) {
+    now = other(0.0);
+    if (e > 1) {
+      us = 0.5 * us + 0.25 * least(0.6) + 0.25 * least(1.2);
+      now = 0.5 * now + 0.25 * other(0.6) + 0.25 * other(1.2);
+    }
+    // (tiles for more than half of the CUs: with fewer, K splits of the others win)
+    if (best_tiles <= 140.0 || us >= (layout_of(d) == 0 ? 0.90 : 0.95) * now) return;
+  }
+  op->tile_cfg = TILE_256x256_W4;
+  op->tile_shape = e > 1 ? -1 : best;
+}
+
 void choose_plan(msco_gmm_op *op) {
   const msco_gmm_desc &d = op->desc;
   const int num_cus = op->num_cus;
@@ -521,6 +651,7 @@ void choose_plan(msco_gmm_op *op) {
   op->wide_k_slabs = 0;
   op->w_nontemporal = 0;
   op->small_group_rows = 0;
+  op->tile_shape = 0;
   op->shallow = false;
 
   int family;
@@ -649,11 +780,17 @@ void choose_plan(msco_gmm_op *op) {
   if (d.kernel_override == OV_AUTO && aligned && is_w8a8(d) && !is_w4(d)) {
     one_round = family == FAM_TILE && plan_one_round(op);
     plan_few_rows(op, family);
+    if (family == FAM_TILE && d.force_split_k == 0) plan_tile_shape(op);
   }
   switch (d.kernel_override) {
     case OV_TILE_256: family = FAM_TILE; op->tile_cfg = TILE_256x256; break;
     case OV_TILE_256_W4: family = FAM_TILE; op->tile_cfg = TILE_256x256_W4; break;
     case OV_TILE_256_W4_MFMA32: family = FAM_TILE; op->tile_cfg = TILE_256x256_W4_MFMA32; break;
+    case OV_W4_128: case OV_W4_160: case OV_W4_192: case OV_W4_224: case OV_W4_288:
+      family = FAM_TILE;
+      op->tile_cfg = TILE_256x256_W4;
+      if (tile_shapes_fit(d)) op->tile_shape = d.kernel_override == OV_W4_288 ? (layout_of(d) == 0 ? 0 : 5) : OV_W4_224 + 1 - d.kernel_override;
+      break;
     case OV_TILE_128: family = FAM_TILE; op->tile_cfg = TILE_128x128; break;
     case OV_TILE_128x256: family = FAM_TILE; op->tile_cfg = TILE_128x256; break;
     case OV_TILE_64: family = FAM_TILE; op->tile_cfg = TILE_64x128; break;
@@ -936,7 +1073,7 @@ void choose_plan(msco_gmm_op *op) {
   const char *fam = family == FAM_REGT ? (op->shallow ? "skinny_regt_shallow" : "skinny_regt") : family == FAM_ROWS16 ? (op->strip_cols == 512 ? "rows128" : op->wave_sets == 2 ? "rows128x256_2" : "rows128x256") : family == FAM_TILE ? (op->tile_cfg >= TILE_32x128 ? "skinny_tile" : "tile") : family == FAM_SKINNY ? "skinny" : "generic";
   std::snprintf(buf, sizeof(buf),
                 "msco_gmm plan: kernel=%s%s%s%s layout=%s m=%lld k=%lld n=%lld e=%lld split_k=%d strips=%d "
-                "workspace=%zu%s",
+                "workspace=%zu%s%s",
                 is_w4(d) ? (op->widen_bytes > 0 ? (is_w8a8(d) ? "a8w4_widened_" : "a16w4_widened_") : (is_w8a8(d) ? "a8w4_" : "a16w4_"))
                          : is_w8a8(d) ? "w8a8_" : "a16w8_", (family == FAM_SKINNY && is_packed(d)) ? (op->stream_tch > 1 ? "stream_rows" : "stream")
                 : (family == FAM_SKINNY && op->stream_tch > 1)    ? "skinny_rows" : fam,
@@ -944,7 +1081,9 @@ void choose_plan(msco_gmm_op *op) {
                 (family == FAM_SKINNY && op->skinny_wide16) ? "_16w" : "",
                 is_packed(d) ? "packed" : d.transpose_b ? "[E,N,K]" : "[E,K,N]", (long long)m, (long long)k, (long long)n, (long long)e,
                 op->split_k, op->n_strips, op->workspace_bytes,
-                op->small_group_rows > 0 ? (" small_groups=" + std::to_string(op->small_group_rows) + ":tile_64x128").c_str() : "");
+                op->small_group_rows > 0 ? (" small_groups=" + std::to_string(op->small_group_rows) + ":tile_64x128").c_str() : "",
+                family == FAM_TILE && op->tile_cfg == TILE_256x256_W4 && op->tile_shape != 0
+                    ? (op->tile_shape < 0 ? std::string(" tile_rows=by_groups") : " tile_rows=" + std::to_string(32 * kT4mShape[op->tile_shape].xb)).c_str() : "");
   op->info = buf;
 }
 
@@ -1184,6 +1323,8 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   hipError_t err = hipSuccess;
   const bool nk = d.transpose_b != 0;
   const int layout = layout_of(d);
+  T4mPick pick{h->tile_shape};
+  if (h->tile_shape < 0) tile_shape_times(h, pick.us, &pick.idle);
   if (h->family == FAM_REGT) {
     err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, h->shallow, s);
   } else if (h->family == FAM_ROWS16) {
@@ -1196,10 +1337,10 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
       small.split_k = 1;
       small.wide_k_slabs = 0;              // (128-byte slabs measured slower here: 340 against 336 us)
       small.w_nontemporal = layout == 2 || !nk;   // each small group's weights are read by one m-tile (packed, [E,K,N])
-      err = launch_tile_w8a8(big, h->tile_cfg, nk, layout == 2, s);
-      if (err == hipSuccess) err = launch_tile_w8a8(small, TILE_64x128, nk, layout == 2, s);
+      err = launch_tile_w8a8(big, h->tile_cfg, nk, layout == 2, pick, s);
+      if (err == hipSuccess) err = launch_tile_w8a8(small, TILE_64x128, nk, layout == 2, pick, s);
     } else if (h->family == FAM_TILE && is_w4(d) && h->widen_bytes == 0) err = launch_tile_a8w4(p, h->tile_cfg, s);
-    else if (h->family == FAM_TILE) err = launch_tile_w8a8(p, h->tile_cfg, nk, layout == 2, s);
+    else if (h->family == FAM_TILE) err = launch_tile_w8a8(p, h->tile_cfg, nk, layout == 2, pick, s);
     else if (h->family == FAM_SKINNY && layout == 2) err = h->stream_tch > 1 ? launch_streamm_w8a8(p, h->stream_tch, s) : launch_stream_w8a8(p, s);
     else if (h->family == FAM_SKINNY) err = launch_skinny_w8a8(p, nk, h->skinny_wide16 != 0, s);
     else err = launch_generic_w8a8(p, layout, s);

@@ -1,0 +1,111 @@
+"""The persistent four-wave kernel on tiles of 128, 160, 192 and 224 rows x 256 columns and of 288 x 224: exact results at the
+edges of the tiles (GPU), and what the plan takes them for (CPU).  Bar: 16-bit outputs bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+from ms_custom_ops_amd import cabi
+from oracle import gmm_oracle as O
+
+ROWS = {cabi.OV_W4_128: 128, cabi.OV_W4_160: 160, cabi.OV_W4_192: 192, cabi.OV_W4_224: 224, cabi.OV_W4_288: 288}
+LAYOUTS = ["packed", "nk", "kn"]
+
+
+def _run(seed, rows, k, n, override, layout, *, out="bf16", act=0):
+    from gpu_utils import run_w8a8
+    rng = np.random.default_rng(seed)
+    e, m = len(rows), sum(rows)
+    x, w = rng.integers(-128, 128, (m, k), dtype=np.int8), rng.integers(-128, 128, (e, k, n), dtype=np.int8)
+    bias = rng.integers(-1000, 1001, (e, n)).astype(np.int32)
+    scale, pt = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), rng.uniform(1e-3, 1e-2, m).astype(np.float32)
+    ends = np.cumsum(rows)
+    got, info = run_w8a8(x, w, ends, bias, scale, pt, out=out, override=override, transpose_b=layout == "nk", packed=layout == "packed",
+                         act_type=act, launches=2)
+    return got, info, (x, w, ends, bias, scale, pt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("override", list(ROWS))
+@pytest.mark.parametrize("k,n", [(512, 240), (656, 464), (1040, 1008)])   # fewest K slabs; K and N tails: columns of one wave, of both, several tiles
+def test_exact_at_the_edges(device, override, layout, k, n):
+    h = ROWS[override]
+    rows = [h, 0, 1, h + 1, h - 1, 17, 2 * h, h // 2, h // 2 + 1]
+    got, info, args = _run(k + n, rows, k, n, override, layout)
+    want = O.grouped_matmul_w8a8(*args)
+    assert "256x256x128_w4" in info and (("tile_rows=%d" % h) in info) == (h != 288 or layout != "kn"), info
+    assert np.array_equal(got, np.asarray(want).view(np.uint16)), info
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("override", list(ROWS))
+def test_more_tiles_than_compute_units(device, override, layout):
+    # the operand stream of a tile's last slabs runs into the next tile, in another group or panel; float16
+    got, info, args = _run(7, [700, 300, 90, 2050], 576, 5200, override, layout, out="f16")
+    want = O.grouped_matmul_w8a8(*args, out_dtype="f16")
+    assert np.array_equal(got, np.asarray(want).view(np.uint16)), info
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("override", list(ROWS))
+def test_silu_equals_the_256_row_tile(device, override, layout):
+    a, _, _ = _run(11, [150, 320], 640, 528, override, layout, act=cabi.ACT_SILU)
+    b, info, _ = _run(11, [150, 320], 640, 528, cabi.OV_TILE_256_W4, layout, act=cabi.ACT_SILU)
+    assert "tile_rows" not in info and np.array_equal(a, b)
+
+
+def _plan(m, k, n, e, layout, *, out=cabi.DT_BF16, act=0):
+    op = cabi.GmmOp(x_dtype=cabi.DT_I8, out_dtype=out, scale_dtype=cabi.DT_NONE if out == cabi.DT_I32 else cabi.DT_F32, transpose_b=int(layout == "nk"), act_type=act,
+                    weight_layout=int(layout == "packed"), **({} if e == 1 else dict(group_list_dtype=cabi.DT_I64)))
+    op.plan(m, k, n, e)
+    info = op.plan_info()
+    op.close()
+    return info
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("rows", [[256] * 4, [288, 280, 270, 186], [128, 128, 128, 640], [1024, 0, 0, 0], [0, 161, 383, 470], [1, 1, 1, 1]])
+def test_shape_picked_from_the_groups(device, layout, rows):
+    # one plan, group lists that the device gives different tiles; rows past the last boundary stay untouched
+    from gpu_utils import run_w8a8
+    rng = np.random.default_rng(5)
+    m, k, n, e = 1024, 512, 14336, 4
+    x, w = rng.integers(-128, 128, (m, k), dtype=np.int8), rng.integers(-128, 128, (e, k, n), dtype=np.int8)
+    scale, pt = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), rng.uniform(1e-3, 1e-2, m).astype(np.float32)
+    got, info = run_w8a8(x, w, rows, None, scale, pt, transpose_b=layout == "nk", packed=layout == "packed", group_list_type=1, launches=2)
+    assert "tile_rows=by_groups" in info, info
+    ends = np.cumsum(rows)
+    want = np.asarray(O.grouped_matmul_w8a8(x, w, ends, None, scale, pt)).view(np.uint16)
+    assert np.array_equal(got[:ends[-1]], want[:ends[-1]]) and (got[ends[-1]:] == 0x7FC0).all()
+
+
+@pytest.mark.gpu
+def test_shape_picked_over_more_than_64_groups(device):
+    from gpu_utils import run_w8a8
+    rng = np.random.default_rng(6)
+    e, k, n = 70, 512, 2064
+    rows = rng.integers(0, 500, e)
+    rows[3], rows[68] = 0, 900
+    m = int(rows.sum())
+    x, w = rng.integers(-128, 128, (m, k), dtype=np.int8), rng.integers(-128, 128, (e, k, n), dtype=np.int8)
+    scale, pt = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), rng.uniform(1e-3, 1e-2, m).astype(np.float32)
+    got, info = run_w8a8(x, w, np.cumsum(rows), None, scale, pt, packed=True, launches=2)
+    assert "tile_rows=by_groups" in info, info
+    assert np.array_equal(got, np.asarray(O.grouped_matmul_w8a8(x, w, np.cumsum(rows), None, scale, pt)).view(np.uint16))
+
+
+@pytest.mark.parametrize("m,k,n,e,layout,rows", [
+    (2048, 4096, 11008, 1, "nk", "192"), (2048, 4096, 11008, 1, "packed", "192"),    # 344 tiles of 256 rows, 473 of 192: two rounds either way
+    (16384, 4096, 14336, 1, "nk", ""),                                               # many rounds: the tile that reads least
+    (2029, 3040, 2896, 1, "nk", "128"),                                              # one round of 192 tiles in place of 128 x 256 ones
+    (2048, 4096, 14336, 8, "packed", "by_groups"), (8192, 4096, 14336, 8, "kn", "by_groups")])
+def test_the_plan(m, k, n, e, layout, rows):
+    info = _plan(m, k, n, e, layout)
+    assert "tile_256x256x128_w4" in info and (("tile_rows=" + rows) in info if rows else "tile_rows" not in info), info
+
+
+@pytest.mark.parametrize("kwargs", [dict(out=cabi.DT_I32), dict(act=cabi.ACT_RELU), dict(act=cabi.ACT_GELU_TANH)])
+def test_outputs_that_stay_on_256_rows(kwargs):
+    assert "tile_rows" not in _plan(2048, 4096, 11008, 1, "nk", **kwargs)
