@@ -141,7 +141,8 @@ typedef struct msco_gmm_desc {
                               * 14 weight-only: equal chunks of up to 128 rows x strips of 512 columns, 15 x strips of 256,
                               * 16 the same with two sets of waves that take turns at the K blocks, 17 32 x 128 and 18 32 x 256
                               * tiles ([E,N,K]: 17 for both; packed: 3), 19 .. 22 the persistent kernel with tiles of 128,
-                              * 160, 192, 224 rows x 256 columns, 23 of 288 rows x 224 columns ([E,K,N]: 6); float outputs without an
+                              * 160, 192, 224 rows x 256 columns, 23 of 288 rows x 224 columns ([E,K,N]: 6), 24 and 25 of 128
+                              * and 160 rows x 192 columns; float outputs without an
                               * activation or with silu or fast gelu (else: 6)
                               * (msco_gmm_plan_info names what was planned) */
   int32_t weight_layout;     /* MSCO_WL_ROW_MAJOR: as transpose_b says; MSCO_WL_PACKED: written by msco_pack_weight */

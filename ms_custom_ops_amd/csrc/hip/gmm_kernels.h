@@ -9,13 +9,15 @@ namespace msco {
 
 // Tile shapes of the persistent four-wave kernel: 32 xb rows x 32 wb columns.
 struct T4mShape { int xb, wb; };
-constexpr int T4M_SHAPES = 6;
-constexpr T4mShape kT4mShape[T4M_SHAPES] = {{8, 8}, {7, 8}, {6, 8}, {5, 8}, {4, 8}, {9, 7}};   // (the last one not on [E,K,N])
+constexpr int T4M_SHAPES = 8;
+constexpr T4mShape kT4mShape[T4M_SHAPES] = {{8, 8}, {7, 8}, {6, 8}, {5, 8}, {4, 8}, {9, 7}, {4, 6}, {5, 6}};
+constexpr bool t4m_has(int shape, int layout) { return layout != 2 || kT4mShape[shape].wb != 7; }   // layout 0 [E,N,K], 1 packed, 2 [E,K,N]
 // The shape of a launch: an index into kT4mShape, or negative: by the groups, which the device counts, and these modelled times
 // (t4m_pick in gmm_tile4m_kernel.h).  (Not part of GmmParams: every kernel would request them.)
 struct T4mPick {
   int shape;
-  float us[T4M_SHAPES], idle;   // us of a round (0: no such shape); the share of a round that is free where a CU has no tile
+  float us[T4M_SHAPES];   // of a round (0: no such shape)
+  float idle, empty;      // the share of a round that is free where a CU has no tile; of a tile, where its rows do not exist
 };
 
 enum TileCfg : int {

@@ -108,6 +108,13 @@ constexpr T4mOps t4m_ops(int quads, int reads, int parts, bool requests_last) {
   return o;
 }
 
+// The first operation that stands behind MFMA `slot` or a later one: spread evenly over the step's MFMAs, or (early) one behind each from the first on.
+constexpr int t4m_first_op(int slot, int mfmas, int ops, bool early) {
+  int j = 0;
+  while (j < ops && (early ? (j < mfmas ? j : mfmas - 1) : j * mfmas / ops) < slot) ++j;
+  return j;
+}
+
 }  // namespace
 
 // MODE: output type, 0 bf16, 1 f16, 2 int32 (raw accumulators plus bias).  WL: weight layout, 0 [E,N,K], 1 packed, 2 [E,K,N]
@@ -131,13 +138,14 @@ constexpr T4mOps t4m_ops(int quads, int reads, int parts, bool requests_last) {
 template <int MODE, int WL, int ACT, int XB, int WB>
 __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *smem, int start, int end, int carry) {
   constexpr bool PK = WL == 1, KN = WL == 2;
-  static_assert(!KN || WB == 8, "a K row of [E,K,N] weights is staged by sixteen lanes of 16 columns");
+  static_assert(WB <= 8 || !KN, "a K row of [E,K,N] weights is staged by sixteen lanes of 16 columns");
+  constexpr int WQ = KN ? 8 : WB;   // staging quads of the weights ([E,K,N]: 16 K rows each, whatever the columns)
   constexpr int BM = 32 * XB, BN = 32 * WB, WM = 16 * XB, WN = 16 * WB;   // tile and wave tile
   constexpr int X0 = (XB + 1) / 2, W0 = (WB + 1) / 2;                     // blocks of the first part of either operand
   constexpr int X_STAGE = t4m_x_stage(XB), W_STAGE = t4m_w_stage(WL, WB), W_BASE = 2 * X_STAGE;
   constexpr int PARAM_OFF = t4m_param_off(WL), META_OFF = t4m_meta_off(WL);
   static_assert(2 * (X_STAGE + W_STAGE) <= PARAM_OFF, "operand stages");
-  constexpr T4mQuads Q = t4m_quads(XB, WB);
+  constexpr T4mQuads Q = t4m_quads(XB, WQ);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -227,6 +235,7 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
     b_voff0 = PK   ? (unsigned)(((wave >> 1) * k_blocks + (wave & 1)) * 1024 + ln * 16)
               : KN ? (unsigned)(4 * wave + (ln >> 4)) * (unsigned)p.n + (unsigned)((ln & 15) * 16)   // K row 4 wave + lane / 16 of quad 0, chunk lane % 16
                    : (unsigned)d_row0 * (unsigned)p.k + d_chunk_w * 16;
+    if (KN && WB < 8 && (ln & 15) >= 2 * WB) b_voff0 |= T4_OOB;   // (columns of the next tile: not read)
     const int swz = (m16 >> 1) & 7;
     x_lane = (unsigned)((wave_m * WM + m16) * T4_BK + ((g4 ^ swz) << 4));
     const int w_row = 8 * (m16 >> 2) + (m16 & 3);   // fragment row m16 of blocks 0 and 1 is column w_row, w_row + 4 of the first 32
@@ -238,7 +247,7 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
     } else if constexpr (KN) {
       // address lane m16 of its block of 16 names K row m16 / 2 of the 16 that lane group g4 multiplies, chunk m16 % 2 of
       // the pair that holds the 32 columns of blocks 0 and 1, the half that holds an even block's columns
-      w_lane = (unsigned)(W_BASE + (16 * g4 + (m16 >> 1)) * T4M_KN_PITCH + (wave_n * 8 + (m16 & 1)) * 16 + (g4 & 1) * 8);
+      w_lane = (unsigned)(W_BASE + (16 * g4 + (m16 >> 1)) * T4M_KN_PITCH + (wave_n * WB + (m16 & 1)) * 16 + (g4 & 1) * 8);
     } else {
       // (an odd number of blocks puts the second wave's first column at 16 mod 32: bit 4 of its columns is flipped)
       w_lane = (unsigned)(W_BASE + (wave_n * WN + w_row) * T4_BK + ((g4 ^ (((m16 >> 1) & 1) | (((m16 >> 2) ^ ((wave_n * WB & 1) << 1)) << 1))) << 4));
@@ -260,7 +269,7 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
   const std::integral_constant<int, 3> c3;
 
   v4i acc[WB][XB];                       // [f: weight block][i: x block]
-  v4i stg[2][2][XB > WB ? XB : WB];      // staging quads: [slab parity][operand: 0 x, 1 w][u]
+  v4i stg[2][2][XB > WQ ? XB : WQ];      // staging quads: [slab parity][operand: 0 x, 1 w][u]
   v4i wf[2][W0], xf[2][X0];              // fragments: set 0 the first part's blocks, set 1 the second part's
 
   T4Tile nxt = cur;        // tile that follows `cur` in this workgroup's walk (loads run ahead into it)
@@ -360,11 +369,11 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
   // written to LDS and refilled (group 0: what steps 7 and 8 move) -------------------------------------------
   {
     static_for<XB>([&](auto u) { load_one(0, c0, c0, u); });
-    static_for<WB>([&](auto u) { load_one(0, c0, c1, u); });
+    static_for<WQ>([&](auto u) { load_one(0, c0, c1, u); });
     static_for<XB>([&](auto u) { load_one(1, c1, c0, u); });
-    static_for<WB>([&](auto u) { load_one(1, c1, c1, u); });
+    static_for<WQ>([&](auto u) { load_one(1, c1, c1, u); });
     static_for<XB>([&](auto u) { cycle_one(0, c0, c0, u); });
-    static_for<WB>([&](auto u) { cycle_one(0, c0, c1, u); });
+    static_for<WQ>([&](auto u) { cycle_one(0, c0, c1, u); });
     static_for<4>([&](auto j) {
       constexpr int J = decltype(j)::value;
       cycle_one(1, c1, std::integral_constant<int, Q.op[J]>{}, std::integral_constant<int, Q.u[J]>{});
@@ -483,18 +492,15 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
           constexpr bool EARLY = decltype(early_c)::value != 0;
           constexpr T4mOps O = t4m_ops(Q.count[STEP], decltype(nr_c)::value, decltype(parts_c)::value, EARLY);
           mfma_step(xm_c, fp_c, ip_c, [&](auto s_c) __attribute__((always_inline)) {
-            constexpr int S = decltype(s_c)::value;
-            static_for<O.n>([&](auto j_c) __attribute__((always_inline)) {
-              constexpr int J = decltype(j_c)::value, AT = EARLY ? (J < M ? J : M - 1) : J * M / O.n;
-              if constexpr (AT == S) {
-                constexpr int A = O.a[J], QI = Q.first[STEP] + A;
-                if constexpr (O.kind[J] == 0)
-                  put_half(st, p_c, std::integral_constant<int, Q.op[QI]>{}, std::integral_constant<int, Q.u[QI]>{}, std::integral_constant<int, O.b[J]>{});
-                else if constexpr (O.kind[J] == 1)
-                  rd(std::integral_constant<int, A>{}, std::integral_constant<int, O.b[J]>{});
-                else
-                  fill(p_c, std::integral_constant<int, Q.op[QI]>{}, std::integral_constant<int, Q.u[QI]>{});
-              }
+            constexpr int S = decltype(s_c)::value, FIRST = t4m_first_op(S, M, O.n, EARLY), NEXT = t4m_first_op(S + 1, M, O.n, EARLY);
+            static_for<NEXT - FIRST>([&](auto j_c) __attribute__((always_inline)) {
+              constexpr int J = FIRST + decltype(j_c)::value, A = O.a[J], QI = Q.first[STEP] + A;
+              if constexpr (O.kind[J] == 0)
+                put_half(st, p_c, std::integral_constant<int, Q.op[QI]>{}, std::integral_constant<int, Q.u[QI]>{}, std::integral_constant<int, O.b[J]>{});
+              else if constexpr (O.kind[J] == 1)
+                rd(std::integral_constant<int, A>{}, std::integral_constant<int, O.b[J]>{});
+              else
+                fill(p_c, std::integral_constant<int, Q.op[QI]>{}, std::integral_constant<int, Q.u[QI]>{});
             });
           });
         };
@@ -746,11 +752,12 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
 }
 
 // The tile shape with the least modelled time for these groups: rounds of one tile per CU, of which `idle` is free where CUs
-// have no tile (pick.us: us of a round, 0: no such shape).  Counted on the device, as only the device knows the groups: over 148 random shapes of 2
-// to 128 experts, even and skewed, what this picks takes 0.91 of the time of 256 x 256 tiles, 1.04 at worst; picked by the host from the
-// average group, 0.93 and 1.29.  Other shapes than 256 x 256 have to be 0.97 of it.
+// have no tile, less a part for rows that do not exist (their products are zeros).  Counted on the device, as only the device knows the groups:
+// over 199 random shapes of 4 to 128 experts, even and skewed, where 256 x 256 tiles were planned, what this picks takes 0.92 of their time, 1.12 at
+// worst; picked by the host from the average group, 0.93 and 1.3 at worst.  Other shapes than 256 x 256 have to be 0.94 of it: 5 of those 199 take more than
+// 1.02 of the time then, 9 where any less will do, and the mean is the same to 0.003.
 __device__ __forceinline__ int t4m_pick(const GmmParams &p, const T4mPick &pick, int lane, int start, int end, int carry) {
-  int tiles[T4M_SHAPES] = {};
+  int tiles[T4M_SHAPES] = {}, all_rows = 0;
   for (int g0 = 0; g0 < p.e; g0 += 64) {
     if (g0 > 0) group_rows_chunk(p, g0, lane, carry, start, end);
     const int rows = end - start;
@@ -763,6 +770,7 @@ __device__ __forceinline__ int t4m_pick(const GmmParams &p, const T4mPick &pick,
       tiles[j] += (int)(sum & 0xFFFFu);
       tiles[j + 1] += (int)(sum >> 16);
     }
+    all_rows += wave_bcast(wave_scan_add(live), 63);
   }
   int best = 0;
   float best_us = 0.0f;
@@ -770,8 +778,10 @@ __device__ __forceinline__ int t4m_pick(const GmmParams &p, const T4mPick &pick,
   for (int j = 0; j < T4M_SHAPES; ++j) {
     if (pick.us[j] <= 0.0f) continue;
     const int t = tiles[j] * ((p.n + 32 * kT4mShape[j].wb - 1) / (32 * kT4mShape[j].wb));
-    const float us = ((1.0f - pick.idle) * (float)((t + T4_MAX_WGS - 1) / T4_MAX_WGS) + pick.idle * (float)t * (1.0f / T4_MAX_WGS)) * pick.us[j];
-    if (j == 0) best_us = 0.97f * us;
+    const float rounds = (1.0f - pick.idle) * (float)((t + T4_MAX_WGS - 1) / T4_MAX_WGS) + pick.idle * (float)t * (1.0f / T4_MAX_WGS);
+    const float empty = 1.0f - (float)all_rows * __builtin_amdgcn_rcpf((float)max(1, tiles[j] * 32 * kT4mShape[j].xb));
+    const float us = rounds * pick.us[j] * (1.0f - pick.empty * empty);
+    if (j == 0) best_us = 0.94f * us;
     else if (us < best_us) { best = j; best_us = us; }
   }
   return __builtin_amdgcn_readfirstlane(best);
@@ -788,19 +798,18 @@ __global__ void __launch_bounds__(T4_NW * 64, 1) gmm_w8a8_tile4m_kernel(const Gm
     t4m_tiles<MODE, WL, ACT, 8, 8>(p, smem, start, end, carry);
   } else {
     const int shape = pick.shape >= 0 ? pick.shape : t4m_pick(p, pick, lane, start, end, carry);
-    if (shape == 0) t4m_tiles<MODE, WL, ACT, 8, 8>(p, smem, start, end, carry);
-    else if (shape == 1) t4m_tiles<MODE, WL, ACT, 7, 8>(p, smem, start, end, carry);
-    else if (shape == 2) t4m_tiles<MODE, WL, ACT, 6, 8>(p, smem, start, end, carry);
-    else if (shape == 3) t4m_tiles<MODE, WL, ACT, 5, 8>(p, smem, start, end, carry);
-    else if (shape == 4) t4m_tiles<MODE, WL, ACT, 4, 8>(p, smem, start, end, carry);
-    else if constexpr (WL != 2) t4m_tiles<MODE, WL, ACT, 9, 7>(p, smem, start, end, carry);
+    static_for<T4M_SHAPES>([&](auto j_c) __attribute__((always_inline)) {
+      constexpr int J = decltype(j_c)::value, XB = kT4mShape[J].xb, WB = kT4mShape[J].wb;
+      if constexpr (WL != 2 || WB != 7)
+        if (shape == J) t4m_tiles<MODE, WL, ACT, XB, WB>(p, smem, start, end, carry);
+    });
   }
 }
 
 template <int MODE, int WL, int ACT, bool SHAPES>
 static hipError_t t4m_launch(const GmmParams &p, const T4mPick &pick, hipStream_t stream) {
   // as many workgroups as any shape has tiles, one per CU at most; every non-empty group adds at most one partial tile
-  const long long bm = SHAPES ? 128 : 256, bn = SHAPES ? 224 : 256;
+  const long long bm = SHAPES ? 128 : 256, bn = SHAPES ? 192 : 256;
   const long long tiles_ub = ((p.m + bm - 1) / bm + p.e) * ((p.n + bn - 1) / bn);
   long long grid = ((tiles_ub + kNumXcd - 1) / kNumXcd) * kNumXcd;
   if (grid > T4_MAX_WGS) grid = T4_MAX_WGS;

@@ -21,7 +21,7 @@ hipError_t launch_tile4m_w8a8(const GmmParams &p, const T4mPick &pick, int layou
   if (p.k < 4 * T4_BK || p.e > T4_MAX_E || layout < 0 || layout > 2 || (layout == 2 && p.n % 16 != 0)) return hipErrorInvalidValue;
   const bool silu = p.act_type == ACT_SILU || p.act_type == ACT_FAST_GELU, any = (p.out_dtype == DT_BF16 || p.out_dtype == DT_F16) && (silu || p.act_type == ACT_NONE);
   if (!any && p.out_dtype != DT_BF16 && p.out_dtype != DT_F16 && p.out_dtype != DT_I32) return hipErrorInvalidValue;
-  if (pick.shape >= T4M_SHAPES || (pick.shape == T4M_SHAPES - 1 && layout == 2) || (!any && pick.shape != 0)) return hipErrorInvalidValue;
+  if (pick.shape >= T4M_SHAPES || (pick.shape >= 0 && !t4m_has(pick.shape, layout)) || (!any && pick.shape != 0)) return hipErrorInvalidValue;
 #define MSCO_T4M_RUN(LAYOUT) \
   (!any ? tile4m_##LAYOUT(p, pick, s) \
    : p.out_dtype == DT_BF16 ? (silu ? tile4m_##LAYOUT##_bf16_silu(p, pick, s) : tile4m_##LAYOUT##_bf16(p, pick, s)) \

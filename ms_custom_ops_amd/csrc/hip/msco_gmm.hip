@@ -37,7 +37,8 @@ enum Override : int {
   OV_ROWS16_256X2 = 16, // ... and two sets of waves that take turns at the K blocks
   OV_TILE_32x128 = 17,  // a few rows on [E,K,N] and [E,N,K] weights (packed: 64 x 128 tiles)
   OV_TILE_32x256 = 18,  // ... on [E,K,N] weights ([E,N,K]: as 17)
-  OV_W4_128 = 19, OV_W4_160 = 20, OV_W4_192 = 21, OV_W4_224 = 22, OV_W4_288 = 23   // the persistent kernel with tiles of that many rows
+  OV_W4_128 = 19, OV_W4_160 = 20, OV_W4_192 = 21, OV_W4_224 = 22, OV_W4_288 = 23,  // the persistent kernel with tiles of that many rows
+  OV_W4_128x192 = 24, OV_W4_160x192 = 25
 };
 
 constexpr int64_t kSkinnyMaxRows = 64;   // total rows up to which the weight-streaming kernel is planned
@@ -131,7 +132,7 @@ int check_desc(const msco_gmm_desc &d) {
   if (d.group_list_dtype != MSCO_DT_NONE && d.group_list_dtype != MSCO_DT_I32 && d.group_list_dtype != MSCO_DT_I64)
     return MSCO_ERR_UNSUPPORTED;
   if (d.group_list_type != 0 && d.group_list_type != 1) return MSCO_ERR_INVALID_ARG;
-  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_W4_288) return MSCO_ERR_INVALID_ARG;
+  if (d.kernel_override < OV_AUTO || d.kernel_override > OV_W4_160x192) return MSCO_ERR_INVALID_ARG;
   if (d.weight_layout != MSCO_WL_ROW_MAJOR && d.weight_layout != MSCO_WL_PACKED) return MSCO_ERR_INVALID_ARG;
   if (d.force_split_k < 0) return MSCO_ERR_INVALID_ARG;
   if (d.act_type < MSCO_ACT_NONE || d.act_type > MSCO_ACT_SILU) return MSCO_ERR_INVALID_ARG;
@@ -543,95 +544,111 @@ TileRounds even_rounds(int64_t m, int64_t n, int64_t e, int64_t bm, int64_t bn, 
   }
   return {std::max(rounds, 1.0), mean * nt / (double)cus};
 }
-// ... with a popularity that falls as 1 / rank^z; groups of up to `lo` rows belong to another launch.
-TileRounds skewed_rounds(int64_t m, int64_t n, int64_t e, int64_t bm, int64_t bn, int64_t cus, double z, double lo) {
+// ... with a popularity that falls as 1 / rank^z.
+TileRounds skewed_rounds(int64_t m, int64_t n, int64_t e, int64_t bm, int64_t bn, int64_t cus, double z) {
   double sum = 0.0, t = 0.0;
   for (int64_t i = 1; i <= e; ++i) sum += std::pow((double)i, -z);
   for (int64_t i = 1; i <= e; ++i) {
     const double avg = (double)m * std::pow((double)i, -z) / sum;
-    if (avg > lo) t += avg > 0.5 * (double)bm ? avg / (double)bm + 0.5 : std::min(avg, 1.0);
+    t += avg > 0.5 * (double)bm ? avg / (double)bm + 0.5 : std::min(avg, 1.0);
   }
   t *= (double)((n + bn - 1) / bn) / (double)cus;
   return {std::max(1.0, t + 0.5), t};
 }
 
-// The persistent kernel on tiles of other shapes than 256 x 256 (kT4mShape), against each other and against the 128 x 256 and 128 x 128
-// tiles, by a model of the time in us: rounds of one tile per CU, each a part per 128-byte K slab and a fixed one; CUs without a tile
-// in the last round leave the others more of the clock and of the L2, hence `idle`.  The operand stream of a CU is what 512 rows of
+// The persistent kernel on tiles of other shapes than 256 x 256 (kT4mShape), against each other and against the 128 x 256, 128 x 128 and
+// 64 x 128 tiles, by a model of the time in us: rounds of one tile per CU, each a part per 128-byte K slab (more where K rows do not start on
+// a line) and a fixed one; CUs without a tile in the last round leave the others more of the clock and of the L2, hence `idle`, and rows that do
+// not exist draw less power, hence `empty`; and the weights have to be read (us per MB).  The operand stream of a CU is what 512 rows of
 // either side take and the matrix pipe is busy for 64 blocks per wave, so a lower tile is dearer per product but wastes
-// less: of a group's last row tile, and of the last round.  Fitted to 1160 random shapes (1 to 128 groups, 100 rows per group to
-// 16384 rows, K = 512 .. 8192, N = 512 .. 14336, even and skewed routings, three layouts), every tile shape measured on all of them: off by
-// 6 .. 8 % (rms).  One group, picked here: 0.91 of the time of 256 x 256 tiles where those were planned.  Several: the device picks, as it
-// alone knows how even they are (t4m_pick).  us, before -> now: one group of 2048 rows, 4096 x 11008, [E,N,K] 94 -> 83 (192 x 256; 344 tiles
-// made two rounds on 172 CUs); 8 experts, 256 rows on average, 4096 x 14336, packed 160 -> 123 (288 x 224: 512 tiles for 672).
-// 128 x 256 and 128 x 128 tiles give way where the least time, over even and skewed routings, is 0.95 of theirs ([E,K,N]: 0.90, its model of them is off by
-// 7 %): 0.94 / 0.84 (packed), 0.86 / 0.82 ([E,N,K]), 0.92 ([E,K,N]) of their time; one group of 2037 rows, 3040 x 2896, [E,N,K] 34 -> 29.
-struct TileTime { double launch, idle, slab, fixed; };
-struct TileTimes { double launch, idle, slab[T4M_SHAPES], fixed[T4M_SHAPES]; TileTime tall, small; };   // small, tall: the 128 x 128 and 128 x 256 tiles
+// less: of a group's last row tile, and of the last round.  Fitted to 1900 random shapes (1 to 128 groups, 14 rows per group to
+// 32768 rows, K = 512 .. 8192, N = 512 .. 14336, even and skewed routings, weights from memory), every shape and tile measured on all of them: off by
+// 10 .. 16 % (rms), between shapes by less.  One group, picked here: 0.86 of the time of 256 x 256 tiles where those were planned.  Several: the device picks, as
+// it alone knows how even they are (t4m_pick).  us, before -> now: one group of 2048 rows, 4096 x 11008, [E,N,K] 94 -> 83 (192 x 256; 344 tiles
+// made two rounds on 172 CUs); 8 experts, 256 rows on average, 4096 x 14336, packed 160 -> 130 (288 x 224: 512 tiles for 672).
+// The smaller tiles give way where the least time, over even and skewed routings, is 0.93 of theirs ([E,K,N], several groups: 0.88) and the tiles are
+// more than 140 of 256 columns' worth (their K splits and second workgroups win below), several groups from 160 rows each on (128 experts, 2576 columns, 108 rows,
+// packed 1.03), on [E,N,K] from 20 rows each where K is 2048 or more (64 experts, 46 rows, 768 x 1792 1.19, 14 rows, 1984 x 1008 1.08),
+// 128 x 128 and 64 x 128 from K = 1536 (8 experts, 732 rows, 704 x 2608 1.17; one group of 2373 rows, 1120 x 1904 1.04).  1200 other shapes, of the time before: [E,N,K]
+// 0.93 with several groups (32 experts, 49 rows, 5824 x 2304 0.71; 8 experts, 109 rows, 1760 x 10656 0.72), 0.99 with one (573 rows, 4928 x 6544 0.66);
+// [E,K,N] 0.99 and 0.98 (1643 rows, 4608 x 2480 0.78); packed 0.99.
+struct TileTime { double launch, idle, slab, fixed, read, unaligned; };
+struct TileTimes { double launch, idle, read, unaligned, empty, slab[T4M_SHAPES], fixed[T4M_SHAPES]; TileTime tall, small, low; };   // 128 x 256, 128 x 128, 64 x 128 tiles
 constexpr TileTimes kTileTimes[3] = {   // [E,K,N], [E,N,K], packed
-    {5.3, 0.32, {1.416, 1.268, 1.126, 1.019, 0.864, 0.0}, {7.3, 6.6, 5.7, 4.65, 4.0, 0.0}, {7.7, 0.38, 1.019, 0.0}, {5.4, 0.45, 0.591, 1.5}},
-    {6.0, 0.33, {1.393, 1.205, 1.081, 0.974, 0.853, 1.363}, {6.7, 5.9, 5.0, 4.1, 3.2, 6.8}, {3.7, 0.34, 1.163, 4.0}, {4.6, 0.39, 0.599, 1.3}},
-    {5.6, 0.32, {1.322, 1.141, 0.986, 0.880, 0.750, 1.301}, {7.65, 7.3, 6.35, 5.4, 4.35, 8.0}, {3.9, 0.35, 0.902, 4.4}, {6.1, 0.58, 0.560, 0.6}}};
+    {4.73, 0.303, 0.251, 0.042, 0.128, {1.457, 1.283, 1.128, 1.019, 0.876, 0.0, 0.755, 0.870}, {7.15, 6.74, 5.99, 5.09, 4.30, 0.0, 3.28, 3.85},
+     {4.88, 0.313, 1.004, 2.76, 0.205, 0.058}, {4.40, 0.396, 0.585, 1.92, 0.212, 0.147}, {4.65, 0.414, 0.385, 0.72, 0.225, 0.178}},
+    {4.37, 0.314, 0.208, 0.144, 0.135, {1.367, 1.229, 1.080, 0.982, 0.859, 1.305, 0.685, 0.776}, {7.61, 6.71, 5.95, 5.08, 4.27, 7.61, 3.24, 3.83},
+     {4.00, 0.326, 1.124, 2.97, 0.249, 0.154}, {3.58, 0.501, 0.639, 1.87, 0.225, 0.182}, {4.16, 0.642, 0.447, 0.52, 0.251, 0.205}},
+    {5.00, 0.325, 0.197, 0.042, 0.150, {1.378, 1.205, 1.051, 0.939, 0.805, 1.313, 0.663, 0.738}, {7.90, 7.19, 6.38, 5.53, 4.51, 8.01, 3.34, 4.23},
+     {4.64, 0.386, 0.990, 2.98, 0.197, 0.045}, {4.53, 0.463, 0.568, 1.90, 0.146, 0.084}, {4.83, 0.542, 0.342, 0.70, 0.194, 0.060}}};
 
 bool tile_shapes_fit(const msco_gmm_desc &d) {   // shapes other than 256 x 256 are built for these outputs only
   return d.out_dtype != MSCO_DT_I32 && (d.act_type == ACT_NONE || d.act_type == ACT_SILU || d.act_type == ACT_FAST_GELU);
 }
 
-void tile_shape_times(const msco_gmm_op *op, float *round_us, float *idle) {
+void tile_shape_times(const msco_gmm_op *op, T4mPick &pick) {
   const TileTimes &t = kTileTimes[layout_of(op->desc)];
-  for (int j = 0; j < T4M_SHAPES; ++j) round_us[j] = (float)((double)(2 * ((op->k + 255) / 256)) * t.slab[j] + t.fixed[j]);
-  *idle = (float)t.idle;
+  const double slabs = (double)(2 * ((op->k + 255) / 256)) * (op->k % 128 != 0 ? 1.0 + t.unaligned : 1.0);
+  for (int j = 0; j < T4M_SHAPES; ++j) pick.us[j] = (float)(slabs * t.slab[j] + t.fixed[j]);
+  if (layout_of(op->desc) == 0) pick.us[5] = 0.0f;   // (288 x 224)
+  pick.idle = (float)t.idle;
+  pick.empty = (float)t.empty;
 }
 
 void plan_tile_shape(msco_gmm_op *op) {
   const msco_gmm_desc &d = op->desc;
   const int64_t m = op->m, k = op->k, n = op->n, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
-  const bool tall = op->tile_cfg == TILE_128x256, small = op->tile_cfg == TILE_128x128;
-  // (groups of 100 rows leave too much of a tile empty: 128 experts, 2576 columns, 108 rows 1.03, 32 experts, 1440 columns, 102 rows 1.15)
-  if (!(op->tile_cfg == TILE_256x256_W4 || tall || small) || k < 512 || e > 1024 || !tile_shapes_fit(d) || ((tall || small) && e > 1 && m < 160 * e)) return;
-  if (e > 1 && op->tile_cfg == TILE_256x256_W4) {
-    op->tile_shape = -1;
-    return;
+  const bool large = op->tile_cfg == TILE_256x256_W4, tall = op->tile_cfg == TILE_128x256, small = op->tile_cfg == TILE_128x128, low = op->tile_cfg == TILE_64x128;
+  const bool nk = layout_of(d) == 1;
+  if (!(large || tall || small || low) || k < ((small || low) ? 1536 : 512) || e > 1024 || !tile_shapes_fit(d)) return;
+  if (e > 1) {
+    if (large) {
+      op->tile_shape = -1;
+      return;
+    }
+    if (m < 160 * e && !(nk && m >= 20 * e && k >= 2048)) return;
   }
   const TileTimes &t = kTileTimes[layout_of(d)];
-  const double lo = e >= 16 && (is_packed(d) || d.transpose_b == 0) ? 64.0 : 0.0;   // (the second launch takes them)
-  float round_us[T4M_SHAPES], idle;
-  tile_shape_times(op, round_us, &idle);
-  // the least time of the shapes, for an even routing (z = 0) and for skewed ones
-  int best = 0;
-  double best_tiles = 0.0;
-  auto rounds = [&](int64_t bm, int64_t bn, double z, double from) {
-    return z == 0.0 ? even_rounds(m, n, e, bm, bn, cus) : skewed_rounds(m, n, e, bm, bn, cus, z, from);
+  T4mPick pick{};
+  tile_shape_times(op, pick);
+  const double mb = (double)(std::min(e, m) * k) * (double)n * 1e-6;
+  auto both = [](double tiles_us, double read_us) { return std::sqrt(std::sqrt(tiles_us * tiles_us * tiles_us * tiles_us + read_us * read_us * read_us * read_us)); };
+  auto rounds = [&](int64_t bm, int64_t bn, double z) {
+    return z == 0.0 ? even_rounds(m, n, e, bm, bn, cus) : skewed_rounds(m, n, e, bm, bn, cus, z);
   };
+  // the least time of the shapes, popularity falling as 1 / rank^z
+  int best = 0;
+  double best_tiles = 0.0;   // for an even routing, in tiles of 256 columns
   auto least = [&](double z) {
     double us = 0.0;
     for (int j = 0; j < T4M_SHAPES; ++j) {
-      if (t.slab[j] <= 0.0) continue;
-      const TileRounds r = rounds(32 * kT4mShape[j].xb, 32 * kT4mShape[j].wb, z, lo);
-      const double u = t.launch + ((1.0 - idle) * r.rounds + idle * r.busy) * (double)round_us[j];
-      if (j == 0) us = u * (op->tile_cfg == TILE_256x256_W4 ? 0.97 : 1.0);
-      if (j == 0 || u < us) {
-        us = j == 0 ? us : u;
-        if (z == 0.0) { best = j; best_tiles = r.busy * (double)cus; }
+      if (pick.us[j] <= 0.0f) continue;
+      const int64_t bm = 32 * kT4mShape[j].xb, bn = 32 * kT4mShape[j].wb;
+      const TileRounds r = rounds(bm, bn, z);
+      const double rows = r.busy * (double)cus / (double)((n + bn - 1) / bn) * (double)bm;   // of all tiles, whether they exist or not
+      const double u = t.launch + both(((1.0 - t.idle) * r.rounds + t.idle * r.busy) * (double)pick.us[j] * (1.0 - t.empty * std::max(0.0, 1.0 - (double)m / rows)), mb * t.read);
+      if (j > 0 && u >= us) continue;
+      us = j == 0 && large ? 0.97 * u : u;
+      if (z == 0.0) {
+        best = j;
+        best_tiles = r.busy * (double)cus * (double)bn / 256.0;
       }
     }
     return us;
   };
-  double now = 0.0;
-  auto other = [&](double z) {
-    const TileTime &o = tall ? t.tall : t.small;
-    const TileRounds r = rounds(128, tall ? 256 : 128, z, 0.0);
-    return o.launch + ((1.0 - o.idle) * r.rounds + o.idle * r.busy) * ((double)k / 128.0 * o.slab + o.fixed);
+  auto now = [&](double z) {
+    const TileTime &o = tall ? t.tall : small ? t.small : t.low;
+    const TileRounds r = rounds(low ? 64 : 128, tall ? 256 : 128, z);
+    return o.launch + both(((1.0 - o.idle) * r.rounds + o.idle * r.busy) * ((double)k / 128.0 * o.slab * (k % 128 != 0 ? 1.0 + o.unaligned : 1.0) + o.fixed), mb * o.read);
   };
   double us = least(0.0);
-  if (tall || small) {
-    now = other(0.0);
+  if (!large) {
+    double old = now(0.0);
     if (e > 1) {
       us = 0.5 * us + 0.25 * least(0.6) + 0.25 * least(1.2);
-      now = 0.5 * now + 0.25 * other(0.6) + 0.25 * other(1.2);
+      old = 0.5 * old + 0.25 * now(0.6) + 0.25 * now(1.2);
     }
-    // (tiles for more than half of the CUs: with fewer, K splits of the others win)
-    if (best_tiles <= 140.0 || us >= (layout_of(d) == 0 ? 0.90 : 0.95) * now) return;
+    if (best_tiles <= 140.0 || us >= (layout_of(d) == 0 && e > 1 ? 0.88 : 0.93) * old) return;
   }
   op->tile_cfg = TILE_256x256_W4;
   op->tile_shape = e > 1 ? -1 : best;
@@ -786,10 +803,12 @@ void choose_plan(msco_gmm_op *op) {
     case OV_TILE_256: family = FAM_TILE; op->tile_cfg = TILE_256x256; break;
     case OV_TILE_256_W4: family = FAM_TILE; op->tile_cfg = TILE_256x256_W4; break;
     case OV_TILE_256_W4_MFMA32: family = FAM_TILE; op->tile_cfg = TILE_256x256_W4_MFMA32; break;
-    case OV_W4_128: case OV_W4_160: case OV_W4_192: case OV_W4_224: case OV_W4_288:
+    case OV_W4_128: case OV_W4_160: case OV_W4_192: case OV_W4_224: case OV_W4_288: case OV_W4_128x192: case OV_W4_160x192:
       family = FAM_TILE;
       op->tile_cfg = TILE_256x256_W4;
-      if (tile_shapes_fit(d)) op->tile_shape = d.kernel_override == OV_W4_288 ? (layout_of(d) == 0 ? 0 : 5) : OV_W4_224 + 1 - d.kernel_override;
+      if (!tile_shapes_fit(d)) break;
+      op->tile_shape = d.kernel_override >= OV_W4_288 ? 5 + d.kernel_override - OV_W4_288 : OV_W4_224 + 1 - d.kernel_override;
+      if (layout_of(d) == 0 && d.kernel_override == OV_W4_288) op->tile_shape = 0;
       break;
     case OV_TILE_128: family = FAM_TILE; op->tile_cfg = TILE_128x128; break;
     case OV_TILE_128x256: family = FAM_TILE; op->tile_cfg = TILE_128x256; break;
@@ -1083,7 +1102,7 @@ void choose_plan(msco_gmm_op *op) {
                 op->split_k, op->n_strips, op->workspace_bytes,
                 op->small_group_rows > 0 ? (" small_groups=" + std::to_string(op->small_group_rows) + ":tile_64x128").c_str() : "",
                 family == FAM_TILE && op->tile_cfg == TILE_256x256_W4 && op->tile_shape != 0
-                    ? (op->tile_shape < 0 ? std::string(" tile_rows=by_groups") : " tile_rows=" + std::to_string(32 * kT4mShape[op->tile_shape].xb)).c_str() : "");
+                    ? (op->tile_shape < 0 ? std::string(" tile_rows=by_groups") : " tile_rows=" + std::to_string(32 * kT4mShape[op->tile_shape].xb) + (kT4mShape[op->tile_shape].wb == 6 ? "x192" : "")).c_str() : "");
   op->info = buf;
 }
 
@@ -1324,7 +1343,7 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   const bool nk = d.transpose_b != 0;
   const int layout = layout_of(d);
   T4mPick pick{h->tile_shape};
-  if (h->tile_shape < 0) tile_shape_times(h, pick.us, &pick.idle);
+  if (h->tile_shape < 0) tile_shape_times(h, pick);
   if (h->family == FAM_REGT) {
     err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, h->shallow, s);
   } else if (h->family == FAM_ROWS16) {
