@@ -101,7 +101,8 @@ def test_shape_picked_over_more_than_64_groups(device):
     (2048, 4096, 11008, 1, "nk", "192"), (2048, 4096, 11008, 1, "packed", "192"),    # 344 tiles of 256 rows, 473 of 192: two rounds either way
     (16384, 4096, 14336, 1, "nk", ""),                                               # many rounds: the tile that reads least
     (2029, 3040, 2896, 1, "nk", "128"),                                              # one round of 192 tiles in place of 128 x 256 ones
-    (2048, 4096, 14336, 8, "packed", "by_groups"), (8192, 4096, 14336, 8, "kn", "by_groups")])
+    (2048, 4096, 14336, 8, "packed", "by_groups"), (4096, 4096, 14336, 8, "kn", "by_groups"),
+    (8192, 4096, 14336, 8, "kn", "")])                                               # several groups, many rounds
 def test_the_plan(m, k, n, e, layout, rows):
     info = _plan(m, k, n, e, layout)
     assert "tile_256x256x128_w4" in info and (("tile_rows=" + rows) in info if rows else "tile_rows" not in info), info
