@@ -168,6 +168,16 @@ int64_t groups_hit(int64_t m, int64_t e) {
   return std::max<int64_t>(1, std::min<int64_t>(std::min(m, e), (int64_t)std::ceil(ed * (1.0 - q) + std::sqrt(std::max(var, 0.0)))));
 }
 
+// 4-bit weights, 16-bit x, several groups whose 128-row chunks on strips of 256 columns are at most a quarter of the chip: the
+// register-transpose kernels, whose 32-row chunks are four times as many workgroups, take less than the 128-row kernel with its K
+// splits.  They convert the weights once per 32 rows in place of 128, which costs more than that with a long K.  92 random shapes of
+// 30 to 230 rows per group 0.77 of the time, 1.07 at worst (us: 16 experts, 58 rows, 1440 x 576 23.8 -> 16.5; 8 experts, 110 rows,
+// 1856 x 784 28.0 -> 18.2); K of 3072 to 4096 0.88, 1.19 at worst; up to three eighths of the chip 0.85, 1.25 at worst.
+bool few_4bit_chunks(const msco_gmm_op *op) {
+  const int64_t m = op->m, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, avg = (m + e - 1) / e, rows = avg + avg / 10;
+  return is_w4(op->desc) && is_a16w8(op->desc) && e >= 8 && op->k >= 512 && op->k <= 3072 && (op->n + 255) / 256 * std::min(e, m) * ((rows + 127) / 128) * 4 <= cus;
+}
+
 // Row-major [E,K,N] weights transposed and converted in registers (gmm_regt.hip).  Called behind choose_plan's own pick:
 // takes the plan over where these kernels are the better ones, and sets up the widening where 4-bit weights go to a
 // kernel that reads int8.
@@ -187,7 +197,7 @@ void plan_regt(msco_gmm_op *op) {
   // more than a second and third pass over the nibbles (4 / 32 rows per group: 47 / 95 us in all).
   // Weight-only on 8-bit weights, one 16-row chunk per group: the decode form.
   const bool want = d.kernel_override == OV_REGT ||
-                    (d.kernel_override == OV_AUTO && bits == 4 && rows <= 64 && op->family != FAM_ROWS16) ||
+                    (d.kernel_override == OV_AUTO && bits == 4 && (rows <= 64 || few_4bit_chunks(op)) && op->family != FAM_ROWS16) ||
                     (op->family == FAM_SKINNY && bits == 8 && is_a16w8(d) && op->stream_tch == 1);
   // 4-bit weights, int8 x, more than one 16-row chunk per group: tiles that read the nibbles through LDS (4 / 16 / 32 rows
   // per group 52 / 53 / 58 us against 44 / 53 / 82 us in 32-row chunks)
@@ -387,7 +397,7 @@ void plan_rows16(msco_gmm_op *op, bool family_fits) {
     while (best.split > 1 && workspace(best) > kTileSplitMaxWorkspace) --best.split;
   } else if (d.kernel_override != OV_AUTO || d.force_split_k != 0 || (family_fits && op->stream_tch == 1)) {
     return;
-  } else if (bits == 4 && e >= 8 && k >= 512 && m <= 30 * e) {
+  } else if (bits == 4 && e >= 8 && k >= 512 && (m <= 30 * e || few_4bit_chunks(op))) {
     return;   // (the register-transpose kernels)
   } else if (e < 8 || k < 512) {
     // Outside what the model was fitted to (one group has kernels with a K split of its own): strips of 512 where they fill the chip and
