@@ -445,22 +445,24 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
       // which keeps every memory operation in its slot (scheduling barriers alone do not: instruction selection has
       // already moved loads by the time they act).  An accumulator block meets its
       // next MFMA a K half later: the compiler's wait counts cover the operands, nothing else needs wait states.
-      auto one_mfma = [&](auto f_c, auto i_c) __attribute__((always_inline)) {
+      // NEW: the tile's first products, which the accumulators take as they are.
+      auto one_mfma = [&](auto new_c, auto f_c, auto i_c) __attribute__((always_inline)) {
         constexpr int F = decltype(f_c)::value, I = decltype(i_c)::value;
         v4i &a = acc[F][I], &w = wf[F / W0][F % W0], &x = xf[I / X0][I % X0];   // (named first: operands of an asm statement do not capture)
 #if MSCO_TILE4_ATTR & 2
         asm volatile("" ::"v"(w), "v"(x));
 #else
-        asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(a) : "v"(w), "v"(x) : "memory");
+        if constexpr (decltype(new_c)::value != 0) asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, 0" : "=a"(a) : "v"(w), "v"(x) : "memory");
+        else asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(a) : "v"(w), "v"(x) : "memory");
 #endif
       };
-      auto mfma_step = [&](auto xm_c, auto fp_c, auto ip_c, auto &&slot) __attribute__((always_inline)) {
+      auto mfma_step = [&](auto new_c, auto xm_c, auto fp_c, auto ip_c, auto &&slot) __attribute__((always_inline)) {
         constexpr int FP = decltype(fp_c)::value, IP = decltype(ip_c)::value, NF = FP == 0 ? W0 : WB - W0, NI = IP == 0 ? X0 : XB - X0;
         constexpr bool XM = decltype(xm_c)::value != 0;
         __builtin_amdgcn_sched_barrier(0);
         static_for<NF * NI>([&](auto k_c) __attribute__((always_inline)) {
           constexpr int K = decltype(k_c)::value;
-          one_mfma(std::integral_constant<int, FP * W0 + (XM ? K % NF : K / NI)>{}, std::integral_constant<int, IP * X0 + (XM ? K / NF : K % NI)>{});
+          one_mfma(new_c, std::integral_constant<int, FP * W0 + (XM ? K % NF : K / NI)>{}, std::integral_constant<int, IP * X0 + (XM ? K / NF : K % NI)>{});
           slot(k_c);
           __builtin_amdgcn_sched_barrier(0);
         });
@@ -480,7 +482,7 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
       // The step before the barrier has its LDS traffic first, so that the wait before the barrier is short.
       // Behind the barrier every wave's part of the next slab is visible and nobody reads this stage any more: the first
       // quads of the slab after next go there.
-      auto slab = [&](auto stage, auto os, auto par_c, auto &&fill_a, auto &&fill_b) __attribute__((always_inline)) {
+      auto slab = [&](auto new_c, auto stage, auto os, auto par_c, auto &&fill_a, auto &&fill_b) __attribute__((always_inline)) {
         constexpr int PAR = decltype(par_c)::value;
         const std::integral_constant<int, PAR ^ 1> oth;
         // step STEP: MFMAs of (weight part FP, x part IP); NR fragment reads rd(b, part); its quads, staging parity p, to LDS
@@ -491,7 +493,7 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
           constexpr int M = (FP == 0 ? W0 : WB - W0) * (IP == 0 ? X0 : XB - X0);
           constexpr bool EARLY = decltype(early_c)::value != 0;
           constexpr T4mOps O = t4m_ops(Q.count[STEP], decltype(nr_c)::value, decltype(parts_c)::value, EARLY);
-          mfma_step(xm_c, fp_c, ip_c, [&](auto s_c) __attribute__((always_inline)) {
+          mfma_step(std::integral_constant<int, decltype(new_c)::value != 0 && STEP <= 4>{}, xm_c, fp_c, ip_c, [&](auto s_c) __attribute__((always_inline)) {
             constexpr int S = decltype(s_c)::value, FIRST = t4m_first_op(S, M, O.n, EARLY), NEXT = t4m_first_op(S + 1, M, O.n, EARLY);
             static_for<NEXT - FIRST>([&](auto j_c) __attribute__((always_inline)) {
               constexpr int J = FIRST + decltype(j_c)::value, A = O.a[J], QI = Q.first[STEP] + A;
@@ -535,10 +537,10 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
 #undef T4M_RX
 #undef T4M_RW
       };
-      // slab kt, its look-ahead anywhere (next tile, past K)
-      auto slab_any = [&](int kt, auto par_c) __attribute__((always_inline)) {
+      // slab kt, its look-ahead anywhere (next tile, past K); NEW: the tile's first
+      auto slab_any = [&](auto new_c, int kt, auto par_c) __attribute__((always_inline)) {
         const int stage = kt & 1;
-        slab(stage, stage ^ 1, par_c, [&](auto p_c, auto op_c, auto u_c) __attribute__((always_inline)) { load_one(kt + 3, p_c, op_c, u_c); },
+        slab(new_c, stage, stage ^ 1, par_c, [&](auto p_c, auto op_c, auto u_c) __attribute__((always_inline)) { load_one(kt + 3, p_c, op_c, u_c); },
              [&](auto p_c, auto op_c, auto u_c) __attribute__((always_inline)) { load_one(kt + 4, p_c, op_c, u_c); });
       };
       // slab kt in stage ST whose look-ahead stays inside the current tile and inside K; soff3 / soff4: K offsets of the
@@ -558,22 +560,18 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
           else stg[P][OP][U] = __builtin_amdgcn_raw_buffer_load_b128(rw_s, b_voff0 + U * b_step, PK ? soff * 16 : KN ? 0u : soff, 0);
 #endif
         };
-        slab(stage_c, os, par_c, [&](auto p_c, auto op_c, auto u_c) __attribute__((always_inline)) { refill(soff3, rw3, p_c, op_c, u_c); },
+        slab(c0, stage_c, os, par_c, [&](auto p_c, auto op_c, auto u_c) __attribute__((always_inline)) { refill(soff3, rw3, p_c, op_c, u_c); },
              [&](auto p_c, auto op_c, auto u_c) __attribute__((always_inline)) { refill(soff4, rw4, p_c, op_c, u_c); });
       };
+      // The tile's first slab is a copy of the general body whose first products replace the accumulators (slabs 0 and 1: the staging
+      // parities alternate).  Clearing them was 256 instructions of a lone wave in front of every tile, half a microsecond: one group of 4096
+      // rows, 1024 x 8192, [E,N,K] 46.6 -> 44.2 us; 16 experts, 400 rows, 1024 x 8192, [E,K,N] / packed 83.1 -> 80.4, 80.5 -> 78.9; 8 experts, 8192
+      // rows, 4096 x 14336, packed 420.2 -> 417.6.  (With a branch here that clears where K is short, accumulators spill in the K loops.)
+      slab_any(c1, 0, c1);
+      slab_any(c0, 1, c0);
       // slabs whose furthest request (group 0 of the slab five on) ends inside K run the compile-time body, two per round
       const int k_clean = max(0, ((p.k / T4_BK - 4) / 2) * 2);
-      int kt = 0;
-      {
-        // (a zero the compiler cannot see through: a constant vector of zeros gets hoisted out of the tile loop into
-        // registers the K loops do not have)
-        int zero = 0;
-        asm volatile("" : "+v"(zero));
-#pragma unroll
-        for (int f = 0; f < WB; ++f)
-#pragma unroll
-          for (int i = 0; i < XB; ++i) acc[f][i] = v4i{zero, zero, zero, zero};
-      }
+      int kt = 2;
       for (; kt < k_clean; kt += 2) {
         const unsigned kb = (unsigned)kt * T4_BK;
         slab_inside(c0, c1, kb + 3 * T4_BK, kb + 4 * T4_BK);
@@ -582,8 +580,8 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
       // the last slabs of the tile (their look-ahead runs into the next tile or past K) multiply every block: what
       // lands in blocks without rows is never stored
       for (; kt < k_slabs; kt += 2) {
-        slab_any(kt, c1);
-        slab_any(kt + 1, c0);
+        slab_any(c0, kt, c1);
+        slab_any(c0, kt + 1, c0);
       }
     }
     // ---- fused dequant epilogue ----------------------------------------------------------------------
