@@ -111,3 +111,11 @@ def test_the_plan(m, k, n, e, layout, rows):
 @pytest.mark.parametrize("kwargs", [dict(out=cabi.DT_I32), dict(act=cabi.ACT_RELU), dict(act=cabi.ACT_GELU_TANH)])
 def test_outputs_that_stay_on_256_rows(kwargs):
     assert "tile_rows" not in _plan(2048, 4096, 11008, 1, "nk", **kwargs)
+
+
+@pytest.mark.parametrize("rows", [257, 296])
+def test_groups_just_beyond_256_rows(rows):
+    assert "tile_rows=by_groups" in _plan(8 * rows, 4096, 14336, 8, "packed")
+    for kwargs in (dict(act=cabi.ACT_RELU), dict(out=cabi.DT_I32)):   # (256 x 256 tiles only: equal chunks of up to 160 rows)
+        assert "rows160" in _plan(8 * rows, 4096, 14336, 8, "packed", **kwargs)
+    assert "rows160" in _plan(8 * 297, 4096, 14336, 8, "packed")
