@@ -1,6 +1,6 @@
 // Grouped W8A8 GEMM, persistent register-heavy MFMA tile kernel for gfx950 on v_mfma_i32_32x32x32_i8: 256 x 256
 // output tiles, four wavefronts (one per SIMD), 128 x 128 accumulators per wavefront; every weight layout.  The plan
-// takes the 16 x 16 x 64 form of the same design (gmm_tile4m_w8a8.hip), which draws less power per multiply-add; this
+// takes the 16 x 16 x 64 form of the same design (gmm_tile4m_kernel.h), which draws less power per multiply-add; this
 // one runs only when it is forced (kernel_override 8), to be measured against.
 //
 // Why this shape.  A wavefront that owns 128 x 128 outputs reads 8 operand fragments from LDS for every

@@ -52,7 +52,7 @@ namespace {
 typedef int v2i __attribute__((ext_vector_type(2)));
 // A tile is 32 XB rows x 32 WB columns: XB x blocks and WB weight blocks of 16 x 16 per wave, 2 x 2 waves.
 // LDS: x stages 0 and 1, weight stages 0 and 1, two epilogue operand tables, the group table.  [E,K,N] weights
-// (WL == 2, WB == 8) lie in LDS as K rows of 256 column bytes at a pitch of 288 bytes (see the kernel's head).
+// (WL == 2) lie in LDS as K rows of 256 column bytes at a pitch of 288 bytes (see the kernel's head).
 constexpr int T4M_KN_PITCH = 288;
 constexpr int T4M_TABLE = 320;                                   // entries of an epilogue operand table: the longest tile edge
 constexpr int T4M_PARAM_BYTES = 3 * 4 * T4M_TABLE;
