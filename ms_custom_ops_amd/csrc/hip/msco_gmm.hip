@@ -172,7 +172,8 @@ int64_t groups_hit(int64_t m, int64_t e) {
 // register-transpose kernels, whose 32-row chunks are four times as many workgroups, take less than the 128-row kernel with its K
 // splits.  They convert the weights once per 32 rows in place of 128, which costs more than that with a long K.  92 random shapes of
 // 30 to 230 rows per group 0.77 of the time, 1.07 at worst (us: 16 experts, 58 rows, 1440 x 576 23.8 -> 16.5; 8 experts, 110 rows,
-// 1856 x 784 28.0 -> 18.2); K of 3072 to 4096 0.88, 1.19 at worst; up to three eighths of the chip 0.85, 1.25 at worst.
+// 1856 x 784 28.0 -> 18.2), 45 of 150 to 930 rows and up to 690 columns 0.70 and 1.01 (8 experts, 2000 rows, 1120 x 240 22.1 -> 14.5); K of
+// 3072 to 4096 0.88, 1.19 at worst; up to three eighths of the chip 0.85, 1.25 at worst.  The error against float64 is the same to six digits.
 bool few_4bit_chunks(const msco_gmm_op *op) {
   const int64_t m = op->m, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, avg = (m + e - 1) / e, rows = avg + avg / 10;
   return is_w4(op->desc) && is_a16w8(op->desc) && e >= 8 && op->k >= 512 && op->k <= 3072 && (op->n + 255) / 256 * std::min(e, m) * ((rows + 127) / 128) * 4 <= cus;
