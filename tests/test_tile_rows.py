@@ -119,3 +119,24 @@ def test_groups_just_beyond_256_rows(rows):
     for kwargs in (dict(act=cabi.ACT_RELU), dict(out=cabi.DT_I32)):   # (256 x 256 tiles only: equal chunks of up to 160 rows)
         assert "rows160" in _plan(8 * rows, 4096, 14336, 8, "packed", **kwargs)
     assert "rows160" in _plan(8 * 297, 4096, 14336, 8, "packed")
+
+
+def test_planning_takes_no_longer_for_many_groups():
+    # a server plans anew for every row count: the skewed routings that the plan looks at are not added up group by group (1024 groups took 15 times
+    # what 64 take; 4 is far from either side's noise)
+    import ctypes
+    import time
+
+    plan = cabi.load().msco_gmm_plan
+    best = {}
+    for e in (64, 1024):
+        op = cabi.GmmOp(x_dtype=cabi.DT_I8, out_dtype=cabi.DT_BF16, scale_dtype=cabi.DT_F32, transpose_b=1, group_list_dtype=cabi.DT_I64)
+        ws, times = ctypes.c_size_t(0), []
+        for step in range(200):
+            began = time.perf_counter()
+            plan(op._h, 40 * e + step, 4096, 2048, e, ctypes.byref(ws))
+            times.append(time.perf_counter() - began)
+        assert "by_groups" in op.plan_info()   # (the comparison with smaller tiles was made)
+        best[e] = min(times)
+        op.close()
+    assert best[1024] < 4 * best[64]
