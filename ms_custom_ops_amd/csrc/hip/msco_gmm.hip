@@ -777,23 +777,26 @@ void choose_plan(msco_gmm_op *op) {
     const bool rows_kernel_ok = is_packed(d) && e > 1 && k >= 1024 && ((n + 255) / 256) * std::min<int64_t>(e, m) >= num_cus;
     // The 160-row form again where a group is two or three equal chunks that share its weights through the L2.  All figures are
     // routings by the top-2 of random logits (groups as uneven as real ones), us, former plan -> this.
-    //   257 .. 296 rows per group on average, where the persistent kernel has 256-row tiles only (int32 output, relu, tanh gelu): it gives a group of
-    //   just more than 256 rows a second m-tile.  8 experts, K = 4096, N = 14336, 260 / 290 rows: 167 -> 149, 197 -> 160; 64 experts, 2048 x
-    //   1408, 260 / 275 / 290: 84 -> 79, 90 -> 82, 90 -> 89; 128 experts, 4096 x 1024, 270: 213 -> 188.  Its other shapes, picked from the groups, take 0.91
-    //   of these chunks' time (70 random shapes, 8 to 64 experts, even and skewed; 32 experts, 271 rows, 5344 x 1200 107 -> 82; worst 1.14: 8
-    //   experts, 268 rows, 4416 x 13440 171 -> 189).
+    //   257 .. 296 rows per group on average: the persistent kernel's 256-row tiles give a group of just more than 256 rows a second m-tile. 8 experts,
+    //   K = 4096, N = 14336, 260 / 290 rows: 167 -> 149, 197 -> 160; 64 experts, 2048 x 1408, 260 / 275 / 290: 84 -> 79, 90 -> 82, 90 -> 89; 128 experts, 4096
+    //   x 1024, 270: 213 -> 188.  Its other shapes, picked from the groups, take over where the outputs have them and few chunks leave uneven groups
+    //   nothing to even out with.  550 random shapes of 8 to 256 experts, shapes picked from the groups over chunks for even routings / popularity as
+    //   1 / rank^0.6 / 1 / rank^1.2: up to two chunk workgroups per CU, their one round, 0.93 / 0.79 / 0.87 (at worst 1.13); up to four 1.02 / 0.89 / 0.91 from
+    //   K = 4096 on (at worst 1.12; 8 experts, 4096 x 14336, 257 .. 296 rows 1.00 / 0.95 / 0.93), 1.05 / 0.95 / 0.97 below; more of them, K = 4096 and longer
+    //   1.01 / 1.00 / 0.99, shorter 1.05 / 1.01 / 1.00.  (256 x 256 tiles there: 1.18 .. 1.28 / 0.95 .. 1.05 / 0.96 .. 1.06.)
     //   297 .. 340 (three chunks): 8 experts, 4096 x 14336, 300 / 335 rows: 205 -> 177, 199 -> 189; 2816 x 5664, 330: 80 -> 72; 16 experts,
     //   4096 x 4096, 320: 112 -> 113; not beyond: 8 experts, 2816 x 5664, 400 rows 70 -> 77.
     //   192 .. 256 where larger tiles than 128 x 128 do not fill the chip but these workgroups do: 8 experts, 7168 x 4096, 200 / 250
     //   rows: 91 -> 73, 120 -> 79; 2816 x 4096, 200 / 250: 38 -> 33, 55 -> 37.  A short K needs the 250: 2048 x 4096, 210 / 250 rows 24.2 ->
     //   28.8, 36.6 -> 33.9; 16 experts, 2048 x 2048, 230 / 250: 29.9 -> 33.8, 36.4 -> 35.4.
-    // Popularity falling as 1 / rank^0.6 and 1 / rank^1.2 in place of even: the bands beyond 256 rows lie between 0.90 and 1.14, the third
+    // Popularity falling as 1 / rank^0.6 and 1 / rank^1.2 in place of even: the second band lies between 0.90 and 1.14, the third
     // between 1.0 and 1.5 times the former plan's speed; which it will be only the device knows.
     // Where 256-row tiles fill the chip, 256 rows on average and fewer stay with them: even groups of 240 rows, one m-tile each, take
     // 126 us there (8 experts, 4096 x 14336) and 141 us here; random routings of 256 rows on average 158 and 147 us.
     const int64_t row_wgs = ((n + 255) / 256) * std::min<int64_t>(e, m) * ((avg_rows + avg_rows / 20 + 159) / 160);
+    const bool by_groups = tile_shapes_fit(d) && d.force_split_k == 0 && row_wgs <= (k >= 4096 ? 4 : 2) * (num_cus > 0 ? num_cus : kDefaultCUs);   // (plan_tile_shape follows)
     const bool rows_chunks_ok = is_packed(d) && e > 1 && k >= 2048 &&
-                                ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172 && !tile_shapes_fit(d)) || (avg_rows > 296 && avg_rows <= 340 && n >= 4096 && row_wgs >= 256) ||
+                                ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172 && !by_groups) || (avg_rows > 296 && avg_rows <= 340 && n >= 4096 && row_wgs >= 256) ||
                                  (avg_rows >= 192 && avg_rows <= 256 && n >= 2048 && (k >= 2816 || avg_rows >= 250) && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));
     if (rows_kernel_ok && avg_rows <= 116) {
       op->tile_cfg = TILE_ROWS128;

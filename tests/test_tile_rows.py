@@ -140,3 +140,21 @@ def test_planning_takes_no_longer_for_many_groups():
         best[e] = min(times)
         op.close()
     assert best[1024] < 4 * best[64]
+
+
+@pytest.mark.parametrize("e,rows,k,n,by_groups", [
+    (8, 270, 2048, 8192, True), (8, 270, 2048, 8208, False), (16, 296, 4080, 4112, False),            # two chunk workgroups per CU
+    (16, 270, 4096, 8192, True), (16, 270, 4096, 8208, False), (16, 270, 4096, 14336, False),         # long K: four
+    # 256 x 256 tiles that make more than six rounds, where no shape would be picked
+    (64, 270, 2048, 3584, False), (128, 270, 2048, 1792, False), (32, 270, 2048, 7168, False), (64, 270, 4096, 4096, False), (1100, 270, 2048, 512, False)])
+def test_chunks_of_groups_beyond_256_rows(e, rows, k, n, by_groups):
+    # (out of the chunk kernels only into shapes that are picked from the groups)
+    info = _plan(e * rows, k, n, e, "packed")
+    assert ("tile_rows=by_groups" if by_groups else "rows160") in info, info
+
+
+def test_a_forced_k_split_keeps_the_chunks():
+    op = cabi.GmmOp(x_dtype=cabi.DT_I8, out_dtype=cabi.DT_BF16, scale_dtype=cabi.DT_F32, weight_layout=cabi.WL_PACKED, group_list_dtype=cabi.DT_I64, force_split_k=1)
+    op.plan(8 * 270, 4096, 8192, 8)
+    assert "rows160" in op.plan_info()   # (no shape is picked then)
+    op.close()
