@@ -168,12 +168,22 @@ int64_t groups_hit(int64_t m, int64_t e) {
   return std::max<int64_t>(1, std::min<int64_t>(std::min(m, e), (int64_t)std::ceil(ed * (1.0 - q) + std::sqrt(std::max(var, 0.0)))));
 }
 
-// 4-bit weights, 16-bit x, several groups whose 128-row chunks on strips of 256 columns are at most a quarter of the chip: the
+// Mean number of bm-row tiles of a group that holds `avg` rows on average: a random routing scatters them by about the root of that.
+double expected_row_tiles(double avg, double bm) {
+  const double sd = std::sqrt(std::max(avg, 1e-9));
+  const double sure = std::max(0.0, std::floor((avg - 5.0 * sd) / bm));
+  double tiles = sure;
+  for (double rows = sure * bm + 0.5; rows < avg + 5.0 * sd; rows += bm) tiles += 0.5 * std::erfc((rows - avg) / (sd * std::sqrt(2.0)));
+  return std::max(tiles, 1e-3);
+}
+
+// 4-bit weights, 16-bit x, several groups of more than 30 rows whose 128-row chunks on strips of 256 columns are at most a quarter of the chip: the
 // register-transpose kernels, whose 32-row chunks are four times as many workgroups, take less than the 128-row kernel with its K
-// splits.  They convert the weights once per 32 rows in place of 128, which costs more than that with a long K.  92 random shapes of
-// 30 to 230 rows per group 0.77 of the time, 1.07 at worst (us: 16 experts, 58 rows, 1440 x 576 23.8 -> 16.5; 8 experts, 110 rows,
-// 1856 x 784 28.0 -> 18.2), 45 of 150 to 930 rows and up to 690 columns 0.70 and 1.01 (8 experts, 2000 rows, 1120 x 240 22.1 -> 14.5); K of
-// 3072 to 4096 0.88, 1.19 at worst; up to three eighths of the chip 0.85, 1.25 at worst.  The error against float64 is the same to six digits.
+// splits.  They convert the weights once per 32 rows in place of 128, which costs more than that with a long K.  642 random
+// shapes of 31 to 1000 rows per group, even and skewed, 0.66 of the time, 1.01 at worst (us: 16 experts, 58 rows, 1440 x 576 23.8 -> 16.5; 8 experts,
+// 110 rows, 1856 x 784 28.0 -> 18.2; 8 experts, 2000 rows, 1120 x 240 22.1 -> 14.5; the chunks and strips that plan_regt counts for them are part of
+// it: 0.72 and 1.45 without).  Beyond, without those: up to three eighths of the chip 0.85 and 1.25, K of 3072 to 4096 0.88 and 1.19.  The error against
+// float64 is the same to six digits.
 bool few_4bit_chunks(const msco_gmm_op *op) {
   const int64_t m = op->m, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, avg = (m + e - 1) / e, rows = avg + avg / 10;
   return is_w4(op->desc) && is_a16w8(op->desc) && e >= 8 && op->k >= 512 && op->k <= 3072 && (op->n + 255) / 256 * std::min(e, m) * ((rows + 127) / 128) * 4 <= cus;
@@ -248,14 +258,20 @@ void plan_regt(msco_gmm_op *op) {
     // split for 16 chunks instead of 8 and 45.3 -> 37.0 us).  Few rows over many groups: the groups that a random routing hits where
     // the forms below are chosen by how full the chip is (32 experts, 52 rows, K = 6976, N = 1920, not full: 70.9 -> 65.2 us), as
     // many as there can be elsewhere (the other estimate there: 110 shapes at 0.98 to 1.13 of the time, 1.003 on average).
-    const int64_t active =
+    // Groups of more than 30 rows (few_4bit_chunks): those that a random routing makes, most groups ending in a chunk of their own.  A chip that an
+    // average group's would just fill, with or without a K split, takes a second round for the others (us; 128-row kernel, an average group's, these: 32
+    // experts, 54 rows, 3024 x 400 30.2 / 37.4 / 29.5; 32 experts, 174 rows, 560 x 208 15.3 / 17.0 / 12.5).
+    const bool few = d.kernel_override == OV_AUTO && m > 30 * e && few_4bit_chunks(op);
+    const int64_t active = few ? std::min<int64_t>(slots, (int64_t)std::ceil((double)std::min(m, e) * expected_row_tiles((double)m / (double)std::min(m, e), 16.0 * blocks))) :
       std::max<int64_t>(1, std::min<int64_t>(slots, (can_be_shallow ? groups_hit(m, e) : std::min<int64_t>(m, e)) * ((avg + 16 * blocks - 1) / (16 * blocks))));
     const int64_t cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs;
     // Strips of 512 columns (eight waves, twice as many neighbouring bytes per K row) while they fill most of the CUs
     // without a K split, strips of 256 (four waves) otherwise.  8 experts, K = 4096, N = 14336, 4 rows per group, 4-bit
     // weights: 44 against 51 us (int8 x), 47 against 52 us (bf16).  One group, N = 11008: 20 against 17 us.
     const int64_t wgs512 = ((n + 511) / 512) * active, wgs256 = ((n + 255) / 256) * active;
-    int64_t cols = wgs512 * 4 >= cus * 3 ? 512 : 256;
+    // (not for those groups, of which only up to 256 columns would give so many: 64 experts, 116 rows, 1504 x 112 42.3 us with half of the waves
+    // without columns, 26.7 with strips of 256)
+    int64_t cols = wgs512 * 4 >= cus * 3 && !few ? 512 : 256;
     // 8-bit weights: 512 columns take 0.9 of the time of two strips of 256, but their rounds on the chip are coarser: up to two they are
     // counted whole, the chip full with 31/32 of the CUs (256 columns: with 34/32, four of them fit a CU and fewer groups may be hit); beyond,
     // a half for the last one.  Strips of 512 / 256, us, the weights not in the caches: 48 rows over 32 experts, K = 2624, N = 4624 (more than one round): 96.6 / 72.4; 320 over 32, K = 832, N = 4688: 38.8 / 36.4; 288
@@ -308,15 +324,6 @@ void plan_regt(msco_gmm_op *op) {
     op->widen_bytes = (e * k * n + 255) / 256 * 256;
     op->workspace_bytes += (size_t)op->widen_bytes;
   }
-}
-
-// Mean number of bm-row tiles of a group that holds `avg` rows on average: a random routing scatters them by about the root of that.
-double expected_row_tiles(double avg, double bm) {
-  const double sd = std::sqrt(std::max(avg, 1e-9));
-  const double sure = std::max(0.0, std::floor((avg - 5.0 * sd) / bm));
-  double tiles = sure;
-  for (double rows = sure * bm + 0.5; rows < avg + 5.0 * sd; rows += bm) tiles += 0.5 * std::erfc((rows - avg) / (sd * std::sqrt(2.0)));
-  return std::max(tiles, 1e-3);
 }
 
 // Weight-only on packed or [E,K,N] weights beyond one 16-row chunk per group: the forms of the 128-row kernel

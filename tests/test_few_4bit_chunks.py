@@ -26,9 +26,33 @@ def test_the_rule(m, k, n, e, regt, dt):
     op.close()
 
 
+def test_chunks_that_a_random_routing_makes():
+    # 32 experts, 54 rows: 64 chunks of an average group's and 71 of a random routing; two strips of those twice are more than 256 workgroups
+    op, _ = _op(32 * 54, 3024, 400, 32, cabi.DT_BF16)
+    assert "split_k=1 strips=2" in op.plan_info(), op.plan_info()
+    op.close()
+
+
+def test_strips_are_no_wider_than_the_columns():
+    # partial tiles of a forced split show the strip: as wide for 256 chunks of 112 columns (strips of 512 "fill" the chip) as for 86
+    def bytes_of(rows, e):
+        op = cabi.GmmOp(x_dtype=cabi.DT_BF16, out_dtype=cabi.DT_BF16, weight_dtype=cabi.DT_I4, group_list_dtype=cabi.DT_I64, antiquant_dtype=cabi.DT_BF16,
+                        has_antiquant_offset=1, force_split_k=2)
+        try:
+            op.plan(rows * e, 1504, 112, e)
+        except cabi.BackendError:
+            pass   # (no device for the counters)
+        info = op.plan_info()
+        op.close()
+        assert "skinny_regt" in info and "strips=1" in info, info
+        return int(info.split("workspace=")[1].split()[0]) // (e + rows * e // 32)
+    assert bytes_of(114, 64) == bytes_of(54, 32)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
-@pytest.mark.parametrize("counts,k,n", [([130, 0, 33, 257, 1, 64, 32, 200], 1040, 512), ([5, 300, 31, 0, 90, 127, 128, 129], 2064, 272)])
+@pytest.mark.parametrize("counts,k,n", [([130, 0, 33, 257, 1, 64, 32, 200], 1040, 512), ([5, 300, 31, 0, 90, 127, 128, 129], 2064, 272),
+                                        ([0, 130, 33, 64, 65, 31, 96, 13] * 4, 720, 400), ([114, 0, 228, 115, 129, 1, 63, 97] * 8, 544, 112)])
 def test_against_float64(device, counts, k, n, dtype):
     # bound: one rounding of the output, and 1e-5 of the sum of the terms' magnitudes for K < 4096 float32 additions of 2^-24 each
     import torch
