@@ -1,5 +1,5 @@
 // Grouped W8A8 GEMM, persistent four-wave tile kernel for gfx950 on v_mfma_i32_16x16x64_i8: output tiles of 256 x 256 and,
-// for float outputs without an activation or with silu or fast gelu, of five other shapes (kT4mShape); four wavefronts (one per
+// for float outputs without an activation or with silu or fast gelu, of seven other shapes (kT4mShape); four wavefronts (one per
 // SIMD), each a quarter of the tile as up to 64 blocks of 16 x 16; weights stored [E,N,K], packed or [E,K,N].
 //
 // Why other shapes: a tile takes the same time whether its rows exist or not, and so does a round of the chip.  One group of 2048 rows,
@@ -138,7 +138,8 @@ constexpr int t4m_first_op(int slot, int mfmas, int ops, bool early) {
 template <int MODE, int WL, int ACT, int XB, int WB>
 __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *smem, int start, int end, int carry) {
   constexpr bool PK = WL == 1, KN = WL == 2;
-  static_assert(WB <= 8 || !KN, "a K row of [E,K,N] weights is staged by sixteen lanes of 16 columns");
+  static_assert(WB <= 8, "a K row of [E,K,N] weights is staged by sixteen lanes of 16 columns, a tile's column operands by one entry per thread");
+  static_assert(MODE != 2 || WB % 2 == 0, "int32 output is stored in pairs of blocks");
   constexpr int WQ = KN ? 8 : WB;   // staging quads of the weights ([E,K,N]: 16 K rows each, whatever the columns)
   constexpr int BM = 32 * XB, BN = 32 * WB, WM = 16 * XB, WN = 16 * WB;   // tile and wave tile
   constexpr int X0 = (XB + 1) / 2, W0 = (WB + 1) / 2;                     // blocks of the first part of either operand
@@ -393,7 +394,7 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
     {
       const unsigned lds = (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char *)table + wave * 256;
       const long long pg = p.scale_per_group ? (long long)cur.grp * p.n : 0;
-      // entry i of the tables; edges beyond 256 take a second pass of the first wave (entries past the edge: zeros, never read)
+      // entry i of the tables; rows beyond 256 take a second pass of the first wave (entries past the edge: zeros, never read)
       auto columns = [&](int i, unsigned at) __attribute__((always_inline)) {
         const int col = cur.n0 + i;
         if (p.scale_dtype == DT_NONE) {
@@ -422,7 +423,6 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
       };
       columns(tid, lds);
       rows(tid, lds);
-      if (BN > 256 && wave == 0) columns(256 + tid, lds + 1024);
       if (BM > 256 && wave == 0) rows(256 + tid, lds + 1024);
     }
 
@@ -605,7 +605,6 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
         // the table holds raw 16-bit patterns: widen them in place (one entry per thread)
         unsigned *mine = reinterpret_cast<unsigned *>(table) + tid;
         *mine = *mine << 16;
-        if (BN > 256 && wave == 0) mine[256] <<= 16;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         t4_barrier();
       }
@@ -641,7 +640,7 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
         voff_q[j] = (n_first + 4 < p.n ? v_lane : T4_OOB) + (unsigned)((32 * j + 4) * esize);   // (int32 output: second store)
       }
       if constexpr (ODD) {
-        if constexpr (!raw) sc[WB - 1] = *reinterpret_cast<const uint4 *>(tb_scale + 32 * PAIRS - 4 * g4);
+        sc[WB - 1] = *reinterpret_cast<const uint4 *>(tb_scale + 32 * PAIRS - 4 * g4);
         voff_p[PAIRS] = (n_base + 32 * PAIRS + 4 * g4 < p.n ? v_lane - (unsigned)(4 * g4 * esize) : T4_OOB) + (unsigned)(32 * PAIRS * esize);
       }
       // accumulators leave the accumulation file here and not earlier
@@ -724,13 +723,9 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
           int a4[4];
           fetch(std::integral_constant<int, WB - 1>{}, i_c, a4);
           const unsigned vp = voff_p[PAIRS] + (unsigned)I * row16;
-          if constexpr (raw) {
-            __builtin_amdgcn_raw_buffer_store_b128(v4i{a4[0], a4[1], a4[2], a4[3]}, rs_out, vp, 0, 0);
-          } else {
-            unsigned r0, r1;
-            finish(a4, sc[WB - 1], pt_i, r0, r1);
-            __builtin_amdgcn_raw_buffer_store_b64(v2i{(int)r0, (int)r1}, rs_out, vp, 0, 0);
-          }
+          unsigned r0, r1;
+          finish(a4, sc[WB - 1], pt_i, r0, r1);
+          __builtin_amdgcn_raw_buffer_store_b64(v2i{(int)r0, (int)r1}, rs_out, vp, 0, 0);
         }
       };
       if (bm_active == XB) {
@@ -751,9 +746,9 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
 
 // The tile shape with the least modelled time for these groups: rounds of one tile per CU, of which `idle` is free where CUs
 // have no tile, less a part for rows that do not exist (their products are zeros).  Counted on the device, as only the device knows the groups:
-// over 199 random shapes of 4 to 128 experts, even and skewed, where 256 x 256 tiles were planned, what this picks takes 0.92 of their time, 1.12 at
-// worst; picked by the host from the average group, 0.93 and 1.3 at worst.  Other shapes than 256 x 256 have to be 0.94 of it: 5 of those 199 take more than
-// 1.02 of the time then, 9 where any less will do, and the mean is the same to 0.003.
+// over 130 random shapes of 4 to 128 experts, even and skewed, where 256 x 256 tiles were planned, what this picks takes 0.93 of their time, 1.07 at
+// worst (16 experts, 3540 rows, 768 x 3280, [E,K,N] 24.5 -> 26.2 us), 5 of them more than 1.02; picked by the host from the average group, 1.3 at
+// worst.  Other shapes than 256 x 256 have to be 0.94 of it: where any less will do, twice as many take more than 1.02 of the time, and the mean is the same to 0.003.
 __device__ __forceinline__ int t4m_pick(const GmmParams &p, const T4mPick &pick, int lane, int start, int end, int carry) {
   int tiles[T4M_SHAPES] = {}, all_rows = 0;
   for (int g0 = 0; g0 < p.e; g0 += 64) {
