@@ -56,6 +56,47 @@ def test_silu_equals_the_256_row_tile(device, override, layout):
     assert "tile_rows" not in info and np.array_equal(a, b)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("override", list(ROWS))
+@pytest.mark.parametrize("form", ["bf16", "u64", "shared", "scalar", "bare"])
+def test_forms_of_the_epilogue_operands(device, form, override, layout):
+    # the tables of a tile: bfloat16 scales are widened in place, 64-bit ones read every other word, one row or one value for all
+    # groups, no scale per token (288 rows: the second pass of the first wave writes the ones); two tiles per workgroup's table or more
+    from gpu_utils import run_w8a8
+    h, k, n = ROWS[override], 528, 2320
+    rows = [h, 0, h - 1, 2 * h + 1, 16, 700]
+    rng = np.random.default_rng(h + len(form))
+    e, m = len(rows), sum(rows)
+    x, w = rng.integers(-128, 128, (m, k), dtype=np.int8), rng.integers(-128, 128, (e, k, n), dtype=np.int8)
+    scale, pt = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), rng.uniform(1e-3, 1e-2, m).astype(np.float32)
+    bias = rng.integers(-1000, 1001, (e, n)).astype(np.int32) if form in ("bf16", "u64") else None
+    given, kw = scale, {}
+    if form == "bf16":
+        given = O.f32_to_bf16_bits(scale)
+        scale, kw = O.bf16_bits_to_f32(given), dict(scale_dtype=cabi.DT_BF16)
+    elif form == "u64":
+        given, kw = O.encode_scale_int64(scale), dict(scale_dtype=cabi.DT_U64)
+    elif form in ("shared", "scalar"):
+        given, kw = (scale[0], dict(scale_per_group=0)) if form == "shared" else (scale[0, :1], dict(scale_per_group=0, scale_is_scalar=1))
+        scale = np.broadcast_to(given, (e, n))
+    if form in ("bf16", "scalar", "bare"):
+        pt = None
+    ends = np.cumsum(rows)
+    got, info = run_w8a8(x, w, ends, bias, given, pt, override=override, transpose_b=layout == "nk", packed=layout == "packed", launches=2, **kw)
+    want = O.grouped_matmul_w8a8(x, w, ends, bias, scale, pt)
+    assert "256x256x128_w4" in info and np.array_equal(got, np.asarray(want).view(np.uint16)), info
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("override", list(ROWS))
+def test_fast_gelu_equals_the_256_row_tile(device, override, layout):
+    a, _, _ = _run(12, [150, 320], 640, 528, override, layout, act=cabi.ACT_FAST_GELU, out="f16")
+    b, info, _ = _run(12, [150, 320], 640, 528, cabi.OV_TILE_256_W4, layout, act=cabi.ACT_FAST_GELU, out="f16")
+    assert "tile_rows" not in info and np.array_equal(a, b)
+
+
 def _plan(m, k, n, e, layout, *, out=cabi.DT_BF16, act=0):
     op = cabi.GmmOp(x_dtype=cabi.DT_I8, out_dtype=out, scale_dtype=cabi.DT_NONE if out == cabi.DT_I32 else cabi.DT_F32, transpose_b=int(layout == "nk"), act_type=act,
                     weight_layout=int(layout == "packed"), **({} if e == 1 else dict(group_list_dtype=cabi.DT_I64)))
@@ -80,6 +121,24 @@ def test_shape_picked_from_the_groups(device, layout, rows):
     ends = np.cumsum(rows)
     want = np.asarray(O.grouped_matmul_w8a8(x, w, ends, None, scale, pt)).view(np.uint16)
     assert np.array_equal(got[:ends[-1]], want[:ends[-1]]) and (got[ends[-1]:] == 0x7FC0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("bad,good,kind", [([300, 200, 5000, 1024], [300, 300, 1024, 1024], 0), ([-5, 512, 100, 700], [0, 512, 512, 700], 0),
+                                           ([300, 2000, 5, 7], [300, 1024, 1024, 1024], 1), ([-3, 10, 2 ** 40, 1], [0, 10, 1024, 1024], 1)])
+def test_shape_picked_from_malformed_groups(device, layout, bad, good, kind):
+    # decreasing boundaries, negative ones, ones past the last row: the tiles are counted from the clamped ranges that the kernel walks
+    from gpu_utils import run_w8a8
+    rng = np.random.default_rng(8)
+    m, k, n, e = 1024, 512, 14336, 4
+    x, w = rng.integers(-128, 128, (m, k), dtype=np.int8), rng.integers(-128, 128, (e, k, n), dtype=np.int8)
+    scale = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32)
+    kw = dict(transpose_b=layout == "nk", packed=layout == "packed")
+    got, info = run_w8a8(x, w, bad, None, scale, None, group_list_type=kind, **kw)
+    assert "tile_rows=by_groups" in info, info
+    want = np.asarray(O.grouped_matmul_w8a8(x, w, good, None, scale, None)).view(np.uint16)
+    assert np.array_equal(got[:good[-1]], want[:good[-1]]) and (got[good[-1]:] == 0x7FC0).all()
 
 
 @pytest.mark.gpu
