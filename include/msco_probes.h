@@ -1,5 +1,5 @@
 /* Measurement aids of the grouped-matmul backend -- a library of their own (libmsco_probes.so), so that the operator
- * library exports nothing but operators.  Neither has a counterpart in the reference; the benchmark quotes them next to
+ * library exports nothing but operators.  None has a counterpart in the reference; the benchmark quotes them next to
  * the kernels' rates.  Status codes are those of msco_gmm.h. */
 #ifndef MSCO_PROBES_H_
 #define MSCO_PROBES_H_
@@ -43,6 +43,15 @@ MSCO_API int msco_probe_mfma_issue(const void *operands, void *sink, void *clock
  * access pattern of the packed-layout decode kernels.  Its duration is the floor under any single-launch decode kernel
  * whose weights have that size.  `sink` receives workgroups * 256 int32 values of no meaning. */
 MSCO_API int msco_probe_read(const void *src, size_t bytes, void *sink, int32_t workgroups, void *stream);
+
+/* Which tile shape the persistent kernel takes for these groups where the plan leaves it to the device (plan information "tile_rows=by_groups"): every
+ * shape gives the same bits, so outputs do not show it.  One wavefront runs the kernel's own code over `group_list` (e <= 1024 int64 on the device, type as in
+ * msco_gmm_desc) and writes the index to `choice` (int32 on the device); groups of up to `rows_lo` rows are a second launch's.  layout: 0 [E,K,N], 1 [E,N,K], 2 packed;
+ * index: 0 256 x 256, 1 .. 4 224, 192, 160, 128 rows x 256 columns, 5 288 x 224, 6 and 7 128 and 160 x 192.  The second call evaluates the same rule on the
+ * host, from the rows of each group. */
+MSCO_API int msco_probe_tile_pick(int32_t layout, int32_t m, int32_t k, int32_t n, int32_t e, int32_t rows_lo, const void *group_list, int32_t group_list_type,
+                                  void *choice, void *stream);
+MSCO_API int msco_probe_tile_pick_host(int32_t layout, int32_t k, int32_t n, int32_t e, int32_t rows_lo, const int32_t *rows, int32_t *choice);
 
 #ifdef __cplusplus
 }

@@ -37,7 +37,7 @@ EXPORTED_SYMBOLS = ("msco_gmm_create", "msco_gmm_plan", "msco_gmm_launch", "msco
                     "msco_packed_weight_bytes", "msco_pack_weight", "msco_gmm_a8w4", "msco_unpack_int4",
                     "msco_moe_init_routing_v2_workspace_bytes", "msco_moe_init_routing_v2", "msco_moe_init_routing_v2_quant",
                     "msco_moe_token_unpermute", "msco_gmm_launch_static")
-PROBE_SYMBOLS = ("msco_probe_mfma_issue", "msco_probe_read")   # libmsco_probes.so, include/msco_probes.h
+PROBE_SYMBOLS = ("msco_probe_mfma_issue", "msco_probe_read", "msco_probe_tile_pick", "msco_probe_tile_pick_host")   # libmsco_probes.so, include/msco_probes.h
 STATIC_WORKSPACE_BYTES = 32 << 20
 PROBE_MFMA_WORKGROUPS, PROBE_MFMA_OPERAND_BYTES = 256, 8 * 256 * 16
 
@@ -73,6 +73,10 @@ def load_probes():
         lib.msco_probe_read.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p]
         lib.msco_probe_mfma_issue.restype = ctypes.c_int
         lib.msco_probe_mfma_issue.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]
+        lib.msco_probe_tile_pick.restype = ctypes.c_int
+        lib.msco_probe_tile_pick.argtypes = [ctypes.c_int32] * 6 + [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p]
+        lib.msco_probe_tile_pick_host.restype = ctypes.c_int
+        lib.msco_probe_tile_pick_host.argtypes = [ctypes.c_int32] * 5 + [ctypes.POINTER(ctypes.c_int32)] * 2
         _probes = lib
     return _probes
 
@@ -182,6 +186,21 @@ def probe_read(src: int, nbytes: int, sink: int, workgroups: int, stream: Option
     """Raw-pointer call of msco_probe_read (see include/msco_probes.h)."""
     vp = lambda v: ctypes.c_void_p(v if v else None)
     _check("msco_probe_read", load_probes().msco_probe_read(vp(src), nbytes, vp(sink), workgroups, vp(stream)))
+
+
+def probe_tile_pick(layout: int, m: int, k: int, n: int, e: int, rows_lo: int, group_list: int, group_list_type: int, choice: int,
+                    stream: Optional[int] = None):
+    """Raw-pointer call of msco_probe_tile_pick (see include/msco_probes.h)."""
+    vp = lambda v: ctypes.c_void_p(v if v else None)
+    _check("msco_probe_tile_pick", load_probes().msco_probe_tile_pick(layout, m, k, n, e, rows_lo, vp(group_list), group_list_type, vp(choice), vp(stream)))
+
+
+def probe_tile_pick_host(layout: int, k: int, n: int, rows: Sequence[int], rows_lo: int = 0) -> int:
+    """msco_probe_tile_pick_host: the index of the tile shape for groups of these rows."""
+    choice = ctypes.c_int32(-1)
+    _check("msco_probe_tile_pick_host", load_probes().msco_probe_tile_pick_host(
+        layout, k, n, len(rows), rows_lo, (ctypes.c_int32 * len(rows))(*[int(r) for r in rows]), ctypes.byref(choice)))
+    return choice.value
 
 
 def moe_init_routing_v2_workspace_bytes(num_rows: int, k: int, expert_num: int) -> int:

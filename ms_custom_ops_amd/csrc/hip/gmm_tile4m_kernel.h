@@ -749,6 +749,25 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
 // over 130 random shapes of 4 to 128 experts, even and skewed, where 256 x 256 tiles were planned, what this picks takes 0.93 of their time, 1.07 at
 // worst (16 experts, 3540 rows, 768 x 3280, [E,K,N] 24.5 -> 26.2 us), 5 of them more than 1.02; picked by the host from the average group, 1.3 at
 // worst.  Other shapes than 256 x 256 have to be 0.94 of it: where any less will do, twice as many take more than 1.02 of the time, and the mean is the same to 0.003.
+// tiles: row tiles of each shape; n: columns; inv: 1 / x.
+template <typename Inv>
+__host__ __device__ __forceinline__ int t4m_least(const T4mPick &pick, const int (&tiles)[T4M_SHAPES], int all_rows, int n, Inv &&inv) {
+  int best = 0;
+  float best_us = 0.0f;
+#pragma unroll
+  for (int j = 0; j < T4M_SHAPES; ++j) {
+    if (pick.us[j] <= 0.0f) continue;
+    const int t = tiles[j] * ((n + 32 * kT4mShape[j].wb - 1) / (32 * kT4mShape[j].wb));
+    const float rounds = (1.0f - pick.idle) * (float)((t + T4_MAX_WGS - 1) / T4_MAX_WGS) + pick.idle * (float)t * (1.0f / T4_MAX_WGS);
+    const int rows = tiles[j] * 32 * kT4mShape[j].xb;
+    const float empty = 1.0f - (float)all_rows * inv((float)(rows > 1 ? rows : 1));
+    const float us = rounds * pick.us[j] * (1.0f - pick.empty * empty);
+    if (j == 0) best_us = 0.94f * us;
+    else if (us < best_us) { best = j; best_us = us; }
+  }
+  return best;
+}
+
 __device__ __forceinline__ int t4m_pick(const GmmParams &p, const T4mPick &pick, int lane, int start, int end, int carry) {
   int tiles[T4M_SHAPES] = {}, all_rows = 0;
   for (int g0 = 0; g0 < p.e; g0 += 64) {
@@ -765,19 +784,7 @@ __device__ __forceinline__ int t4m_pick(const GmmParams &p, const T4mPick &pick,
     }
     all_rows += wave_bcast(wave_scan_add(live), 63);
   }
-  int best = 0;
-  float best_us = 0.0f;
-#pragma unroll
-  for (int j = 0; j < T4M_SHAPES; ++j) {
-    if (pick.us[j] <= 0.0f) continue;
-    const int t = tiles[j] * ((p.n + 32 * kT4mShape[j].wb - 1) / (32 * kT4mShape[j].wb));
-    const float rounds = (1.0f - pick.idle) * (float)((t + T4_MAX_WGS - 1) / T4_MAX_WGS) + pick.idle * (float)t * (1.0f / T4_MAX_WGS);
-    const float empty = 1.0f - (float)all_rows * __builtin_amdgcn_rcpf((float)max(1, tiles[j] * 32 * kT4mShape[j].xb));
-    const float us = rounds * pick.us[j] * (1.0f - pick.empty * empty);
-    if (j == 0) best_us = 0.94f * us;
-    else if (us < best_us) { best = j; best_us = us; }
-  }
-  return __builtin_amdgcn_readfirstlane(best);
+  return __builtin_amdgcn_readfirstlane(t4m_least(pick, tiles, all_rows, p.n, [](float x) { return __builtin_amdgcn_rcpf(x); }));
 }
 
 // SHAPES: all tile shapes (pick.shape, or by t4m_pick where that is negative), else 256 x 256.

@@ -14,6 +14,7 @@
 #include <string>
 
 #include "gmm_kernels.h"
+#include "gmm_tile_times.h"
 
 namespace {
 
@@ -597,7 +598,7 @@ class SkewedRouting {
 };
 
 // The persistent kernel on tiles of other shapes than 256 x 256 (kT4mShape), against each other and against the 128 x 256, 128 x 128 and
-// 64 x 128 tiles, by a model of the time in us: rounds of one tile per CU, each a part per 128-byte K slab (more where K rows do not start on
+// 64 x 128 tiles, by a model of the time in us (kTileTimes): rounds of one tile per CU, each a part per 128-byte K slab (more where K rows do not start on
 // a line) and a fixed one; CUs without a tile in the last round leave the others more of the clock and of the L2, hence `idle`, and rows that do
 // not exist draw less power, hence `empty`; and the weights have to be read (us per MB).  The operand stream of a CU is what 512 rows of
 // either side take and the matrix pipe is busy for 64 blocks per wave, so a lower tile is dearer per product but wastes
@@ -612,27 +613,8 @@ class SkewedRouting {
 // 128 x 128 and 64 x 128 from K = 1536 (8 experts, 732 rows, 704 x 2608 1.17; one group of 2373 rows, 1120 x 1904 1.04).  1200 other shapes, of the time before: [E,N,K]
 // 0.93 with several groups (32 experts, 49 rows, 5824 x 2304 0.71; 8 experts, 109 rows, 1760 x 10656 0.72), 0.99 with one (573 rows, 4928 x 6544 0.66);
 // [E,K,N] 0.99 and 0.98 (1643 rows, 4608 x 2480 0.78); packed 0.99.
-struct TileTime { double launch, idle, slab, fixed, read, unaligned; };
-struct TileTimes { double launch, idle, read, unaligned, empty, slab[T4M_SHAPES], fixed[T4M_SHAPES]; TileTime tall, small, low; };   // 128 x 256, 128 x 128, 64 x 128 tiles
-constexpr TileTimes kTileTimes[3] = {   // [E,K,N], [E,N,K], packed
-    {4.73, 0.303, 0.251, 0.042, 0.128, {1.457, 1.283, 1.128, 1.019, 0.876, 0.0, 0.755, 0.870}, {7.15, 6.74, 5.99, 5.09, 4.30, 0.0, 3.28, 3.85},
-     {4.88, 0.313, 1.004, 2.76, 0.205, 0.058}, {4.40, 0.396, 0.585, 1.92, 0.212, 0.147}, {4.65, 0.414, 0.385, 0.72, 0.225, 0.178}},
-    {4.37, 0.314, 0.208, 0.144, 0.135, {1.367, 1.229, 1.080, 0.982, 0.859, 1.305, 0.685, 0.776}, {7.61, 6.71, 5.95, 5.08, 4.27, 7.61, 3.24, 3.83},
-     {4.00, 0.326, 1.124, 2.97, 0.249, 0.154}, {3.58, 0.501, 0.639, 1.87, 0.225, 0.182}, {4.16, 0.642, 0.447, 0.52, 0.251, 0.205}},
-    {5.00, 0.325, 0.197, 0.042, 0.150, {1.378, 1.205, 1.051, 0.939, 0.805, 1.313, 0.663, 0.738}, {7.90, 7.19, 6.38, 5.53, 4.51, 8.01, 3.34, 4.23},
-     {4.64, 0.386, 0.990, 2.98, 0.197, 0.045}, {4.53, 0.463, 0.568, 1.90, 0.146, 0.084}, {4.83, 0.542, 0.342, 0.70, 0.194, 0.060}}};
-
 bool tile_shapes_fit(const msco_gmm_desc &d) {   // shapes other than 256 x 256 are built for these outputs only
   return d.out_dtype != MSCO_DT_I32 && (d.act_type == ACT_NONE || d.act_type == ACT_SILU || d.act_type == ACT_FAST_GELU);
-}
-
-void tile_shape_times(const msco_gmm_op *op, T4mPick &pick) {
-  const TileTimes &t = kTileTimes[layout_of(op->desc)];
-  const double slabs = (double)(2 * ((op->k + 255) / 256)) * (op->k % 128 != 0 ? 1.0 + t.unaligned : 1.0);
-  for (int j = 0; j < T4M_SHAPES; ++j) pick.us[j] = (float)(slabs * t.slab[j] + t.fixed[j]);
-  if (layout_of(op->desc) == 0) pick.us[5] = 0.0f;   // (288 x 224)
-  pick.idle = (float)t.idle;
-  pick.empty = (float)t.empty;
 }
 
 void plan_tile_shape(msco_gmm_op *op) {
@@ -652,7 +634,7 @@ void plan_tile_shape(msco_gmm_op *op) {
   }
   const TileTimes &t = kTileTimes[layout_of(d)];
   T4mPick pick{};
-  tile_shape_times(op, pick);
+  tile_shape_times(layout_of(d), k, pick);
   const double mb = (double)(std::min(e, m) * k) * (double)n * 1e-6;
   auto both = [](double tiles_us, double read_us) { return std::sqrt(std::sqrt(tiles_us * tiles_us * tiles_us * tiles_us + read_us * read_us * read_us * read_us)); };
   // the least time of the shapes, and that of the tile planned so far, for an even routing (null) or a skewed one
@@ -1391,7 +1373,7 @@ int msco_gmm_launch(msco_gmm_handle h, const void *const *inputs, void *out, voi
   const bool nk = d.transpose_b != 0;
   const int layout = layout_of(d);
   T4mPick pick{h->tile_shape};
-  if (h->tile_shape < 0) tile_shape_times(h, pick);
+  if (h->tile_shape < 0) tile_shape_times(layout, h->k, pick);
   if (h->family == FAM_REGT) {
     err = launch_regt(p, is_w4(d) ? 4 : 8, h->row_blocks, h->strip_cols, h->shallow, s);
   } else if (h->family == FAM_ROWS16) {

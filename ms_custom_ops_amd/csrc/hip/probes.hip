@@ -14,8 +14,14 @@
 // the same weight size.  Each workgroup reads one contiguous share of the buffer, its four wavefronts taking
 // neighbouring 1 KiB pieces (16 bytes per lane), eight loads in flight per wavefront, non-temporal loads: the access
 // pattern of the packed-layout decode kernels.
+//
+// 3. Which tile shape the persistent kernel picks for given groups: its own code on one wavefront, and the same rule on the host.
 #include "gmm_common.h"
+#include "gmm_tile4m_kernel.h"
+#include "gmm_tile_times.h"
 #include "msco_probes.h"
+
+#include <climits>
 
 #include <type_traits>
 
@@ -137,6 +143,14 @@ __global__ void __launch_bounds__(256, 1) probe_issue_kernel(const v4i *operands
   }
 }
 
+__global__ void __launch_bounds__(64) probe_tile_pick_kernel(const GmmParams p, const T4mPick pick, int *choice) {
+  const int lane = threadIdx.x & 63;
+  int carry = 0, start, end;
+  group_rows_chunk(p, 0, lane, carry, start, end);
+  const int shape = t4m_pick(p, pick, lane, start, end, carry);
+  if (lane == 0) *choice = shape;
+}
+
 }  // namespace
 }  // namespace msco
 
@@ -178,4 +192,39 @@ extern "C" int msco_probe_read(const void *src, size_t bytes, void *sink, int32_
   hipLaunchKernelGGL(msco::probe_read_kernel, dim3((unsigned)workgroups), dim3(256), 0, static_cast<hipStream_t>(stream),
                      static_cast<const unsigned char *>(src), (long long)bytes, static_cast<int *>(sink));
   return hipGetLastError() == hipSuccess ? MSCO_OK : MSCO_ERR_DEVICE;
+}
+
+extern "C" int msco_probe_tile_pick(int32_t layout, int32_t m, int32_t k, int32_t n, int32_t e, int32_t rows_lo, const void *group_list, int32_t group_list_type,
+                                    void *choice, void *stream) {
+  if (layout < 0 || layout > 2 || m < 0 || k < 512 || n < 1 || e < 1 || group_list == nullptr || choice == nullptr || group_list_type < 0 || group_list_type > 1)
+    return MSCO_ERR_INVALID_ARG;
+  if ((int64_t)m * k >= ((int64_t)1 << 31) || e > msco::T4_MAX_E) return MSCO_ERR_SHAPE;
+  msco::GmmParams p{};
+  p.m = m;
+  p.k = k;
+  p.n = n;
+  p.e = e;
+  p.group_list = group_list;
+  p.gl_dtype = msco::DT_I64;
+  p.gl_type = group_list_type;
+  p.rows_lo = rows_lo;
+  p.rows_hi = INT_MAX;
+  msco::T4mPick pick{-1};
+  msco::tile_shape_times(layout, k, pick);
+  hipLaunchKernelGGL(msco::probe_tile_pick_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), p, pick, static_cast<int *>(choice));
+  return hipGetLastError() == hipSuccess ? MSCO_OK : MSCO_ERR_DEVICE;
+}
+
+extern "C" int msco_probe_tile_pick_host(int32_t layout, int32_t k, int32_t n, int32_t e, int32_t rows_lo, const int32_t *rows, int32_t *choice) {
+  if (layout < 0 || layout > 2 || k < 512 || n < 1 || e < 1 || rows == nullptr || choice == nullptr) return MSCO_ERR_INVALID_ARG;
+  msco::T4mPick pick{-1};
+  msco::tile_shape_times(layout, k, pick);
+  int tiles[msco::T4M_SHAPES] = {}, all_rows = 0;
+  for (int32_t g = 0; g < e; ++g) {
+    if (rows[g] <= rows_lo || rows[g] <= 0) continue;
+    all_rows += rows[g];
+    for (int j = 0; j < msco::T4M_SHAPES; ++j) tiles[j] += (rows[g] + 32 * msco::kT4mShape[j].xb - 1) / (32 * msco::kT4mShape[j].xb);
+  }
+  *choice = msco::t4m_least(pick, tiles, all_rows, n, [](float x) { return 1.0f / x; });
+  return MSCO_OK;
 }

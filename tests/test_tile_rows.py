@@ -217,3 +217,43 @@ def test_a_forced_k_split_keeps_the_chunks():
     op.plan(8 * 270, 4096, 8192, 8)
     assert "rows160" in op.plan_info()   # (no shape is picked then)
     op.close()
+
+
+# The shape with the least modelled time: one whole round of the chip where only that shape makes one.  (columns, rows of the groups, groups of up to so
+# many rows left out, index into the shapes)
+ONE_ROUND = [(4096, [256] * 16, 0, 0), (4096, [224] * 16, 0, 1), (4096, [192] * 16, 0, 2), (4096, [160] * 16, 0, 3), (4096, [128] * 16, 0, 4),
+             (14336, [288] * 8, 0, 5), (14336, [257] * 8, 0, 5), (3072, [128] * 16, 0, 6), (3072, [160] * 16, 0, 7),
+             (512, [128] * 128, 0, 4), (512, [0] * 70 + [224] * 128, 0, 1),                                     # more than 64 groups
+             (4096, [224] * 16 + [64] * 100, 64, 1), (4096, [224] * 16 + [64] * 100, 0, 4), (4096, [0] * 8, 0, 0)]   # a second launch's groups do not count
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("n,rows,rows_lo,index", ONE_ROUND)
+def test_the_pick(layout, n, rows, rows_lo, index):
+    got = cabi.probe_tile_pick_host(["kn", "nk", "packed"].index(layout), 4096, n, rows, rows_lo)
+    assert got == index if index != 5 or layout != "kn" else got == 3   # (no 288 x 224 on [E,K,N])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_the_device_picks_as_the_host(device, layout):
+    # outputs do not show the shape; the kernel's counting (two counts to a sum, 64 groups at a time, clamped boundaries) and its rule do, on one wavefront
+    import torch
+    rng = np.random.default_rng(layout)
+    cases = [(n, rows, lo, np.cumsum(rows), 0, sum(rows)) for n, rows, lo, _ in ONE_ROUND]
+    for _ in range(60):
+        e, n = int(rng.choice([1, 2, 8, 63, 64, 65, 128, 300, 1024])), 16 * int(rng.integers(32, 900))
+        rows = (rng.gamma(rng.choice([0.3, 2.0, 20.0]), 1.0, e) * rng.choice([2, 15, 60])).astype(np.int64)
+        kind = int(rng.integers(2))
+        cases.append((n, rows, int(rng.choice([0, 64])), rows if kind else np.cumsum(rows), kind, int(rows.sum()) + int(rng.integers(3))))
+    cases += [(14336, [300, 0, 724, 0], 0, [300, 200, 5000, 1024], 0, 1024), (14336, [300, 724, 0, 0], 0, [300, 2000, 5, 7], 1, 1024)]
+    st, seen = torch.cuda.current_stream().cuda_stream, set()
+    for n, rows, lo, given, kind, m in cases:
+        choice, gl = torch.full((1,), -1, dtype=torch.int32, device="cuda:0"), torch.from_numpy(np.asarray(given, dtype=np.int64)).to("cuda:0")
+        cabi.probe_tile_pick(layout, m, 512, n, len(rows), lo, gl.data_ptr(), kind, choice.data_ptr(), st)
+        want = cabi.probe_tile_pick_host(layout, 512, n, rows, lo)
+        assert int(choice.item()) == want, (n, list(rows)[:8], lo, kind)
+        seen.add(want)
+    assert seen == set(range(8)) - ({5} if layout == 0 else set())
+    with pytest.raises(cabi.BackendError):
+        cabi.probe_tile_pick(layout, 128, 512, 512, 1025, 0, gl.data_ptr(), 0, choice.data_ptr(), st)
