@@ -565,8 +565,8 @@ __device__ __forceinline__ void t4m_tiles(const GmmParams &p, unsigned char *sme
       };
       // The tile's first slab is a copy of the general body whose first products replace the accumulators (slabs 0 and 1: the staging
       // parities alternate).  Clearing them was 256 instructions of a lone wave in front of every tile, half a microsecond: one group of 4096
-      // rows, 1024 x 8192, [E,N,K] 46.6 -> 44.2 us; 16 experts, 400 rows, 1024 x 8192, [E,K,N] / packed 83.1 -> 80.4, 80.5 -> 78.9; 8 experts, 8192
-      // rows, 4096 x 14336, packed 420.2 -> 417.6.  (With a branch here that clears where K is short, accumulators spill in the K loops.)
+      // rows, 1024 x 8192, [E,N,K] 46.6 -> 44.2 us; 16 experts, 400 rows, 1024 x 8192, [E,K,N] / packed 83.1 -> 80.4, 80.5 -> 78.9; where a tile's
+      // K loop is long, no more than noise (8 experts, 8192 rows, 4096 x 14336, packed 1.004).  (With a branch here that clears where K is short, accumulators spill in the K loops.)
       slab_any(c1, 0, c1);
       slab_any(c0, 1, c0);
       // slabs whose furthest request (group 0 of the slab five on) ends inside K run the compile-time body, two per round

@@ -183,7 +183,7 @@ double expected_row_tiles(double avg, double bm) {
 // splits.  They convert the weights once per 32 rows in place of 128, which costs more than that with a long K.  642 random
 // shapes of 31 to 1000 rows per group, even and skewed, 0.66 of the time, 1.01 at worst (us: 16 experts, 58 rows, 1440 x 576 23.8 -> 16.5; 8 experts,
 // 110 rows, 1856 x 784 28.0 -> 18.2; 8 experts, 2000 rows, 1120 x 240 22.1 -> 14.5; the chunks and strips that plan_regt counts for them are part of
-// it: 0.72 and 1.45 without).  Beyond, without those: up to three eighths of the chip 0.85 and 1.25, K of 3072 to 4096 0.88 and 1.19.  The error against
+// it: 0.72 and 1.32 without).  Beyond, without those: up to three eighths of the chip 0.85 and 1.25, K of 3072 to 4096 0.88 and 1.19.  The error against
 // float64 is the same to six digits.
 bool few_4bit_chunks(const msco_gmm_op *op) {
   const int64_t m = op->m, e = op->e, cus = op->num_cus > 0 ? op->num_cus : kDefaultCUs, avg = (m + e - 1) / e, rows = avg + avg / 10;
