@@ -626,8 +626,10 @@ void plan_tile_shape(msco_gmm_op *op) {
   if (e > 1) {
     if (large) {
       // (beyond six rounds the other shapes save nothing -- 19 shapes 0.99 of the time -- and counting them takes a microsecond or two: 64 experts,
-      // 49152 rows, 2048 x 2816, [E,K,N], skewed 327.7 / 326.0)
-      op->tile_shape = even_busy(m, n, e, 256, 256, cus) > 6.0 ? 0 : -1;
+      // 49152 rows, 2048 x 2816, [E,K,N], skewed 327.7 / 326.0; not packed groups of just more than 256 rows, of which 256 x 256 tiles make two: choose_plan)
+      const int64_t avg_rows = (m + e - 1) / e;
+      const bool just_beyond = is_packed(d) && avg_rows > 256 && avg_rows <= 296;
+      op->tile_shape = !just_beyond && even_busy(m, n, e, 256, 256, cus) > 6.0 ? 0 : -1;
       return;
     }
     if (m < 160 * e && !(nk && m >= 20 * e && k >= 2048)) return;
@@ -772,7 +774,10 @@ void choose_plan(msco_gmm_op *op) {
     //   nothing to even out with.  550 random shapes of 8 to 256 experts, shapes picked from the groups over chunks for even routings / popularity as
     //   1 / rank^0.6 / 1 / rank^1.2: up to two chunk workgroups per CU, their one round, 0.93 / 0.79 / 0.87 (at worst 1.13); up to four 1.02 / 0.89 / 0.91 from
     //   K = 4096 on (at worst 1.12; 8 experts, 4096 x 14336, 257 .. 296 rows 1.00 / 0.95 / 0.93), 1.05 / 0.95 / 0.97 below; more of them, K = 4096 and longer
-    //   1.01 / 1.00 / 0.99, shorter 1.05 / 1.01 / 1.00.  (256 x 256 tiles there: 1.18 .. 1.28 / 0.95 .. 1.05 / 0.96 .. 1.06.)
+    //   1.01 / 1.00 / 0.99, shorter 1.05 / 1.01 / 1.00.  (256 x 256 tiles there: 1.18 .. 1.28 / 0.95 .. 1.05 / 0.96 .. 1.06.)  More than 256 groups, whose every
+    //   chunk workgroup walks them all: the shapes, also beyond six rounds, up to 511 columns 0.86 / 0.85 / 0.66, more columns 0.96 / 0.97 / 0.86 (140 shapes; 256 x 256
+    //   tiles 1.01 / 0.86 / 0.66 and 1.19 / 0.97 / 0.86); beyond the persistent kernel's 1024 groups eight-wave tiles up to 511 columns, 0.92 / 0.70 / 0.60, not from 512 on,
+    //   1.31 / 0.99 / 1.19 (33 shapes).
     //   297 .. 340 (three chunks): 8 experts, 4096 x 14336, 300 / 335 rows: 205 -> 177, 199 -> 189; 2816 x 5664, 330: 80 -> 72; 16 experts,
     //   4096 x 4096, 320: 112 -> 113; not beyond: 8 experts, 2816 x 5664, 400 rows 70 -> 77.
     //   192 .. 256 where larger tiles than 128 x 128 do not fill the chip but these workgroups do: 8 experts, 7168 x 4096, 200 / 250
@@ -783,7 +788,8 @@ void choose_plan(msco_gmm_op *op) {
     // Where 256-row tiles fill the chip, 256 rows on average and fewer stay with them: even groups of 240 rows, one m-tile each, take
     // 126 us there (8 experts, 4096 x 14336) and 141 us here; random routings of 256 rows on average 158 and 147 us.
     const int64_t row_wgs = ((n + 255) / 256) * std::min<int64_t>(e, m) * ((avg_rows + avg_rows / 20 + 159) / 160);
-    const bool by_groups = tile_shapes_fit(d) && d.force_split_k == 0 && row_wgs <= (k >= 4096 ? 4 : 2) * (num_cus > 0 ? num_cus : kDefaultCUs);   // (plan_tile_shape follows)
+    const int64_t cus = num_cus > 0 ? num_cus : kDefaultCUs;
+    const bool by_groups = tile_shapes_fit(d) && d.force_split_k == 0 && (e <= 256 ? row_wgs <= (k >= 4096 ? 4 : 2) * cus : e <= 1024 || n < 512);   // (plan_tile_shape follows)
     const bool rows_chunks_ok = is_packed(d) && e > 1 && k >= 2048 &&
                                 ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172 && !by_groups) || (avg_rows > 296 && avg_rows <= 340 && n >= 4096 && row_wgs >= 256) ||
                                  (avg_rows >= 192 && avg_rows <= 256 && n >= 2048 && (k >= 2816 || avg_rows >= 250) && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));

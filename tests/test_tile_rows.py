@@ -156,6 +156,25 @@ def test_shape_picked_over_more_than_64_groups(device):
     assert np.array_equal(got, np.asarray(O.grouped_matmul_w8a8(x, w, np.cumsum(rows), None, scale, pt)).view(np.uint16))
 
 
+@pytest.mark.gpu
+def test_shape_picked_over_hundreds_of_groups(device):
+    # more than 256 packed groups of just more than 256 rows on average, some of them in the second launch: the bits of 256 x 256 tiles
+    from gpu_utils import run_w8a8
+    rng = np.random.default_rng(9)
+    e, k, n = 300, 2048, 80
+    rows = rng.poisson(290, e) * (rng.random(e) < 0.9)
+    rows[:5] = [0, 1, 64, 65, 900]
+    rows[-1] += e * 270 - rows.sum()
+    assert rows[-1] > 0
+    m = int(rows.sum())
+    x, w = rng.integers(-128, 128, (m, k), dtype=np.int8), rng.integers(-128, 128, (e, k, n), dtype=np.int8)
+    scale, pt = rng.uniform(1e-3, 1e-2, (e, n)).astype(np.float32), rng.uniform(1e-3, 1e-2, m).astype(np.float32)
+    a, info = run_w8a8(x, w, np.cumsum(rows), None, scale, pt, packed=True, launches=2)
+    assert "tile_rows=by_groups" in info and "small_groups=64" in info, info
+    b, info = run_w8a8(x, w, np.cumsum(rows), None, scale, pt, packed=True, override=cabi.OV_TILE_256_W4)
+    assert "tile_rows" not in info and np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("m,k,n,e,layout,rows", [
     (2048, 4096, 11008, 1, "nk", "192"), (2048, 4096, 11008, 1, "packed", "192"),    # 344 tiles of 256 rows, 473 of 192: two rounds either way
     (16384, 4096, 14336, 1, "nk", ""),                                               # many rounds: the tile that reads least
@@ -205,11 +224,17 @@ def test_planning_takes_no_longer_for_many_groups():
     (8, 270, 2048, 8192, True), (8, 270, 2048, 8208, False), (16, 296, 4080, 4112, False),            # two chunk workgroups per CU
     (16, 270, 4096, 8192, True), (16, 270, 4096, 8208, False), (16, 270, 4096, 14336, False),         # long K: four
     # 256 x 256 tiles that make more than six rounds, where no shape would be picked
-    (64, 270, 2048, 3584, False), (128, 270, 2048, 1792, False), (32, 270, 2048, 7168, False), (64, 270, 4096, 4096, False), (1100, 270, 2048, 512, False)])
+    (64, 270, 2048, 3584, False), (128, 270, 2048, 1792, False), (32, 270, 2048, 7168, False), (64, 270, 4096, 4096, False), (256, 270, 2048, 512, False),
+    (257, 270, 2048, 512, True), (1000, 290, 4096, 400, True),                                        # more than 256 groups: shapes, whatever the rounds
+    (1100, 270, 2048, 512, False)])
 def test_chunks_of_groups_beyond_256_rows(e, rows, k, n, by_groups):
     # (out of the chunk kernels only into shapes that are picked from the groups)
     info = _plan(e * rows, k, n, e, "packed")
     assert ("tile_rows=by_groups" if by_groups else "rows160") in info, info
+
+
+def test_more_groups_than_the_persistent_kernel_takes():
+    assert "256x256x64" in _plan(1100 * 270, 2048, 496, 1100, "packed")
 
 
 def test_a_forced_k_split_keeps_the_chunks():
