@@ -770,14 +770,13 @@ void choose_plan(msco_gmm_op *op) {
     // routings by the top-2 of random logits (groups as uneven as real ones), us, former plan -> this.
     //   257 .. 296 rows per group on average: the persistent kernel's 256-row tiles give a group of just more than 256 rows a second m-tile. 8 experts,
     //   K = 4096, N = 14336, 260 / 290 rows: 167 -> 149, 197 -> 160; 64 experts, 2048 x 1408, 260 / 275 / 290: 84 -> 79, 90 -> 82, 90 -> 89; 128 experts, 4096
-    //   x 1024, 270: 213 -> 188.  Its other shapes, picked from the groups, take over where the outputs have them and few chunks leave uneven groups
-    //   nothing to even out with.  550 random shapes of 8 to 256 experts, shapes picked from the groups over chunks for even routings / popularity as
-    //   1 / rank^0.6 / 1 / rank^1.2: up to two chunk workgroups per CU, their one round, 0.93 / 0.79 / 0.87 (at worst 1.13); up to four 1.02 / 0.89 / 0.91 from
-    //   K = 4096 on (at worst 1.12; 8 experts, 4096 x 14336, 257 .. 296 rows 1.00 / 0.95 / 0.93), 1.05 / 0.95 / 0.97 below; more of them, K = 4096 and longer
-    //   1.01 / 1.00 / 0.99, shorter 1.05 / 1.01 / 1.00.  (256 x 256 tiles there: 1.18 .. 1.28 / 0.95 .. 1.05 / 0.96 .. 1.06.)  More than 256 groups, whose every
-    //   chunk workgroup walks them all: the shapes, also beyond six rounds, up to 511 columns 0.86 / 0.85 / 0.66, more columns 0.96 / 0.97 / 0.86 (140 shapes; 256 x 256
-    //   tiles 1.01 / 0.86 / 0.66 and 1.19 / 0.97 / 0.86); beyond the persistent kernel's 1024 groups eight-wave tiles up to 511 columns, 0.92 / 0.70 / 0.60, not from 512 on,
-    //   1.31 / 0.99 / 1.19 (33 shapes).
+    //   x 1024, 270: 213 -> 188.  Its other shapes, picked from the groups in any number of rounds, take over where the outputs have them: uneven groups leave
+    //   CUs without chunks idle, tiles of 256 columns less so.  615 random shapes of 8 to 256 experts, shapes over chunks for even routings / popularity as 1 /
+    //   rank^0.6 / 1 / rank^1.2: up to two chunk workgroups per CU, their one round, 0.93 / 0.79 / 0.87 (at worst 1.13), up to four 1.04 / 0.94 / 0.94 (1.19), more of
+    //   them 1.01 / 1.00 / 0.98 from K = 2816 on (1.16) and 1.06 / 1.02 / 1.01 below, where the chunks stay.  (256 x 256 tiles alone 1.20 / 0.97 / 1.00; 8 experts, 4096 x
+    //   14336, 257 .. 296 rows: shapes 1.00 / 0.95 / 0.93.)  More than 256 groups, whose every chunk workgroup walks them all: up to 511 columns 0.86 / 0.85 / 0.66,
+    //   more columns 0.96 / 0.97 / 0.86 (140 shapes); beyond the persistent kernel's 1024 groups eight-wave tiles up to 511 columns, 0.92 / 0.70 / 0.60, not from
+    //   512 on, 1.31 / 0.99 / 1.19 (33 shapes).
     //   297 .. 340 (three chunks): 8 experts, 4096 x 14336, 300 / 335 rows: 205 -> 177, 199 -> 189; 2816 x 5664, 330: 80 -> 72; 16 experts,
     //   4096 x 4096, 320: 112 -> 113; not beyond: 8 experts, 2816 x 5664, 400 rows 70 -> 77.
     //   192 .. 256 where larger tiles than 128 x 128 do not fill the chip but these workgroups do: 8 experts, 7168 x 4096, 200 / 250
@@ -789,7 +788,7 @@ void choose_plan(msco_gmm_op *op) {
     // 126 us there (8 experts, 4096 x 14336) and 141 us here; random routings of 256 rows on average 158 and 147 us.
     const int64_t row_wgs = ((n + 255) / 256) * std::min<int64_t>(e, m) * ((avg_rows + avg_rows / 20 + 159) / 160);
     const int64_t cus = num_cus > 0 ? num_cus : kDefaultCUs;
-    const bool by_groups = tile_shapes_fit(d) && d.force_split_k == 0 && (e <= 256 ? row_wgs <= (k >= 4096 ? 4 : 2) * cus : e <= 1024 || n < 512);   // (plan_tile_shape follows)
+    const bool by_groups = tile_shapes_fit(d) && d.force_split_k == 0 && (e <= 256 ? k >= 2816 || row_wgs <= 4 * cus : e <= 1024 || n < 512);   // (plan_tile_shape follows)
     const bool rows_chunks_ok = is_packed(d) && e > 1 && k >= 2048 &&
                                 ((avg_rows > 256 && avg_rows <= 296 && row_wgs >= 172 && !by_groups) || (avg_rows > 296 && avg_rows <= 340 && n >= 4096 && row_wgs >= 256) ||
                                  (avg_rows >= 192 && avg_rows <= 256 && n >= 2048 && (k >= 2816 || avg_rows >= 250) && row_wgs >= 172 && row_wgs <= 256 && group_tiles(256, 256) < busy));

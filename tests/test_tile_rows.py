@@ -221,10 +221,10 @@ def test_planning_takes_no_longer_for_many_groups():
 
 
 @pytest.mark.parametrize("e,rows,k,n,by_groups", [
-    (8, 270, 2048, 8192, True), (8, 270, 2048, 8208, False), (16, 296, 4080, 4112, False),            # two chunk workgroups per CU
-    (16, 270, 4096, 8192, True), (16, 270, 4096, 8208, False), (16, 270, 4096, 14336, False),         # long K: four
-    # 256 x 256 tiles that make more than six rounds, where no shape would be picked
-    (64, 270, 2048, 3584, False), (128, 270, 2048, 1792, False), (32, 270, 2048, 7168, False), (64, 270, 4096, 4096, False), (256, 270, 2048, 512, False),
+    (16, 270, 2048, 8192, True), (16, 270, 2048, 8208, False), (16, 296, 2800, 8208, False), (16, 270, 2816, 8208, True),   # four chunk workgroups per CU; a long K
+    # 256 x 256 tiles that make more than six rounds
+    (64, 270, 2048, 3584, False), (128, 270, 2048, 1792, False), (32, 270, 2048, 7168, False), (256, 270, 2048, 528, False),
+    (16, 270, 4096, 14336, True), (64, 270, 4096, 4096, True),
     (257, 270, 2048, 512, True), (1000, 290, 4096, 400, True),                                        # more than 256 groups: shapes, whatever the rounds
     (1100, 270, 2048, 512, False)])
 def test_chunks_of_groups_beyond_256_rows(e, rows, k, n, by_groups):
